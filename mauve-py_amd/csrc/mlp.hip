@@ -15,6 +15,7 @@
 // bf16 rounding is round-to-nearest-even; products of two bf16 values are
 // exact in fp32; every sum accumulates in fp32.
 #include "mh_internal.hpp"
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <random>
@@ -154,17 +155,26 @@ __global__ __launch_bounds__(256) void features_kernel(const uint8_t *__restrict
 // ---- GEMM on MFMA ---------------------------------------------------------
 //
 // C[M x N] = A[M x K] . B[K x N], bf16 operands (fp32 sources are rounded on
-// load), fp32 accumulation with v_mfma_f32_16x16x16bf16.  A workgroup of 4
-// waves computes a 64x64 tile, each wave a 32x32 quarter as 2x2 MFMA blocks;
-// K advances 16 at a time through LDS.  Operand element (r, c) is at
-// p[(idx ? idx[r] : r) * s0 + c * s1]: strides give the transposes, idx
-// gathers rows (a batch of examples).
+// load), fp32 accumulation with v_mfma_f32_16x16x16bf16, k ascending.  A
+// workgroup of 4 waves computes a 64x64 tile, each wave a 32x32 quarter as 2x2
+// MFMA blocks; K advances 32 at a time through LDS, the next step's loads
+// issued before the current step's MFMAs.  An operand is laid out with either
+// its k or its other index contiguous (KC); a thread loads 8 consecutive
+// elements of that index at once, so a wavefront reads whole lines either way.
+// idx gathers rows of the memory layout (a batch of examples).  gridDim.z > 1
+// splits K: split z covers k in [z * kchunk, (z + 1) * kchunk) and writes its
+// own fp32 partial of EPI_F32 (summed by grad_reduce_kernel, z ascending).
+//
+// These products are small (rows x 272 x 256), so the kernel is bound by load
+// latency and by the workgroups in flight, not by MFMA.  One element a load
+// and no split of K, a 4,096-row batch's products took 1,121 us a pass (the
+// weight gradients' K is the row count: 8 and 20 workgroups); 8 elements a
+// load and K split at 128 rows they take 74 us.
 
 struct Operand {
     const void *p;
-    int64_t s0, s1;
+    int64_t ld;             // elements from one index of the outer (memory row) dimension to the next
     const uint32_t *idx;
-    int f32;
 };
 
 enum { EPI_F32 = 0, EPI_BIAS_RELU_BF16 = 1, EPI_MASK_BF16 = 2 };
@@ -172,7 +182,8 @@ enum { EPI_F32 = 0, EPI_BIAS_RELU_BF16 = 1, EPI_MASK_BF16 = 2 };
 struct Epilogue {
     int mode;
     const float *bias;      // per column (EPI_BIAS_RELU_BF16)
-    float *c32;             // EPI_F32
+    float *c32;             // EPI_F32; split z at c32 + z * zstride
+    int64_t zstride;
     uint16_t *cbf;          // bf16 outputs
     int64_t ldc;
     const uint16_t *mask;   // EPI_MASK_BF16: keep where mask > 0
@@ -182,52 +193,102 @@ struct Epilogue {
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ inline uint16_t load_op(const Operand &o, int64_t r, int64_t c)
+constexpr int GT = 64, GK = 32, GKP = GK + 4;   // tile, k step, padded LDS row
+
+// eight consecutive floats at any float address, eight bf16 at any bf16 address
+struct __attribute__((packed, aligned(4))) F8 { float v[8]; };
+struct __attribute__((packed, aligned(2))) H8 { uint16_t v[8]; };
+
+// Elements (outer, inner .. inner + 7) of an operand, as bf16; zeros past the bounds.
+template <bool F32>
+__device__ __forceinline__ void load8(const Operand &o, int outer, int n_outer, int inner, int n_inner, uint16_t *v)
 {
-    const int64_t rr = o.idx ? (int64_t)o.idx[r] : r;
-    const int64_t x = rr * o.s0 + c * o.s1;
-    return o.f32 ? to_bf16(static_cast<const float *>(o.p)[x]) : static_cast<const uint16_t *>(o.p)[x];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = 0;
+    if (outer >= n_outer || inner >= n_inner) return;
+    const int64_t row = o.idx ? (int64_t)o.idx[outer] : (int64_t)outer;
+    const int64_t at = row * o.ld + inner;
+    if (inner + 8 <= n_inner) {
+        if constexpr (F32) {
+            const F8 x = *reinterpret_cast<const F8 *>(static_cast<const float *>(o.p) + at);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = to_bf16(x.v[q]);
+        } else {
+            const H8 x = *reinterpret_cast<const H8 *>(static_cast<const uint16_t *>(o.p) + at);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = x.v[q];
+        }
+    } else {
+        for (int q = 0; q < 8 && inner + q < n_inner; ++q) {
+            if constexpr (F32) v[q] = to_bf16(static_cast<const float *>(o.p)[at + q]);
+            else v[q] = static_cast<const uint16_t *>(o.p)[at + q];
+        }
+    }
 }
 
-constexpr int GT = 64, GK = 16, GKP = GK + 4;   // tile, k step, padded LDS row
+// KC: k contiguous, memory row = m (or n); else m (or n) contiguous, memory row = k.
+// The thread's 8 elements of the 64 x 32 tile at (x0, k0); nx, k1 the bounds.
+template <bool KC, bool F32>
+__device__ __forceinline__ void tile_load(const Operand &o, int t, int x0, int nx, int k0, int k1, uint16_t *v)
+{
+    if constexpr (KC) load8<F32>(o, x0 + (t >> 2), nx, k0 + (t & 3) * 8, k1, v);
+    else load8<F32>(o, k0 + (t >> 3), k1, x0 + (t & 7) * 8, nx, v);
+}
 
-__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, Operand A, Operand Bo, Epilogue E)
+template <bool KC> __device__ __forceinline__ void tile_store(uint16_t (*s)[GKP], int t, const uint16_t *v)
+{
+    if constexpr (KC) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[t >> 2][(t & 3) * 8 + q] = v[q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[(t & 7) * 8 + q][t >> 3] = v[q];
+    }
+}
+
+template <bool AKC, bool AF32, bool BKC, bool BF32>
+__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, int kchunk, Operand A, Operand Bo, Epilogue E)
 {
     __shared__ uint16_t As[GT][GKP];   // [m][k]
     __shared__ uint16_t Bs[GT][GKP];   // [n][k]
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int m0 = blockIdx.x * GT, n0 = blockIdx.y * GT;
+    const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
     const int wm = (wv >> 1) * 32, wn = (wv & 1) * 32;
     f32x4 acc[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += GK) {
-        // 64x16 of A and 16x64 of B: 4 elements each per thread
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int e = t + 256 * q;          // 0..1023
-            const int r = e >> 4, c = e & 15;   // tile row (m or n), k
-            const int gm = m0 + r, gn = n0 + r, gk = k0 + c;
-            As[r][c] = (gm < M && gk < K) ? load_op(A, gm, gk) : (uint16_t)0;
-            Bs[r][c] = (gn < N && gk < K) ? load_op(Bo, gk, gn) : (uint16_t)0;
-        }
+    uint16_t va[8], vb[8];
+    tile_load<AKC, AF32>(A, t, m0, M, kb, ke, va);
+    tile_load<BKC, BF32>(Bo, t, n0, N, kb, ke, vb);
+    for (int k0 = kb; k0 < ke; k0 += GK) {
+        tile_store<AKC>(As, t, va);
+        tile_store<BKC>(Bs, t, vb);
         __syncthreads();
-        const int li = lane & 15, lk = (lane >> 4) * 4;
-        bf16x4 av[2], bv[2];
-#pragma unroll
-        for (int x = 0; x < 2; ++x) {
-            const uint16_t *pa = &As[wm + 16 * x + li][lk];
-            const uint16_t *pb = &Bs[wn + 16 * x + li][lk];
-            av[x] = bf16x4{(short)pa[0], (short)pa[1], (short)pa[2], (short)pa[3]};
-            bv[x] = bf16x4{(short)pb[0], (short)pb[1], (short)pb[2], (short)pb[3]};
+        if (k0 + GK < ke) {
+            tile_load<AKC, AF32>(A, t, m0, M, k0 + GK, ke, va);
+            tile_load<BKC, BF32>(Bo, t, n0, N, k0 + GK, ke, vb);
         }
+        const int li = lane & 15;
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
+        for (int kk = 0; kk < GK; kk += 16) {
+            const int lk = kk + (lane >> 4) * 4;
+            bf16x4 av[2], bv[2];
 #pragma unroll
-            for (int y = 0; y < 2; ++y)
-                acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[x], bv[y], acc[x][y], 0, 0, 0);
+            for (int x = 0; x < 2; ++x) {
+                const uint16_t *pa = &As[wm + 16 * x + li][lk];
+                const uint16_t *pb = &Bs[wn + 16 * x + li][lk];
+                av[x] = bf16x4{(short)pa[0], (short)pa[1], (short)pa[2], (short)pa[3]};
+                bv[x] = bf16x4{(short)pb[0], (short)pb[1], (short)pb[2], (short)pb[3]};
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[x], bv[y], acc[x][y], 0, 0, 0);
+        }
         __syncthreads();
     }
     // D[i][j] of a 16x16 block: lane holds column j = lane%16, rows 4*(lane/16) + 0..3
@@ -243,7 +304,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, Operand 
                 const float v = acc[x][y][q];
                 const int64_t o = (int64_t)gm * E.ldc + gn;
                 if (E.mode == EPI_F32) {
-                    E.c32[o] = v;
+                    E.c32[(int64_t)blockIdx.z * E.zstride + o] = v;
                 } else if (E.mode == EPI_BIAS_RELU_BF16) {
                     const float z = v + E.bias[gn];
                     E.cbf[o] = to_bf16(z > 0.f ? z : 0.f);
@@ -300,26 +361,46 @@ __global__ void head_back_kernel(const uint16_t *__restrict__ g, const uint16_t 
     dz2[e] = pos ? to_bf16(from_bf16(g[r]) * from_bf16(w3bf[k])) : (uint16_t)0;
 }
 
-// out[c] = sum_r v[r][c] (* w[r] when w is given), r ascending, fp32
-__global__ void colsum_kernel(const uint16_t *__restrict__ v, int rows, int cols, const uint16_t *__restrict__ w,
-                              float *__restrict__ out)
+// The column sums of the backward pass over the rows of split z = blockIdx.x
+// (kchunk rows), fp32, rows ascending: db1 = colsum dz1, db2 = colsum dz2, dw3
+// = g^T h2, db3 = sum g, into the split's partial gradient.  One thread a
+// column walking every row took 3,034 us for 4,096 rows (three launches of one
+// or two workgroups, a chain of dependent loads); a split's 128 rows, 8 loads
+// in flight, take 9 us.
+__global__ __launch_bounds__(256) void colsums_kernel(const uint16_t *__restrict__ dz1, const uint16_t *__restrict__ dz2,
+                                                      const uint16_t *__restrict__ h2, const uint16_t *__restrict__ gy,
+                                                      int rows, int kchunk, float *__restrict__ part)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= cols) return;
-    float s = 0.f;
-    for (int r = 0; r < rows; ++r) {
-        const float x = from_bf16(v[(int64_t)r * cols + c]);
-        s += w ? x * from_bf16(w[r]) : x;
+    static_assert(NH1 == 256 && NH2 == 128, "a thread a column of dz1; dz2 and h2 half the workgroup each");
+    const int t = threadIdx.x;
+    const int lo = blockIdx.x * kchunk, hi = min(rows, lo + kchunk);
+    float *out = part + (int64_t)blockIdx.x * NPARAM;
+    const bool head = t >= NH2;
+    const int c = head ? t - NH2 : t;
+    const uint16_t *v2 = head ? h2 : dz2;
+    float s1 = 0.f, s2 = 0.f, s3 = 0.f;
+#pragma unroll 8
+    for (int r = lo; r < hi; ++r) {
+        const float g = from_bf16(gy[r]);
+        const float x = from_bf16(v2[(int64_t)r * NH2 + c]);
+        s1 += from_bf16(dz1[(int64_t)r * NH1 + t]);
+        s2 += head ? x * g : x;
+        s3 += g;
     }
-    out[c] = s;
+    out[OFF_B1 + t] = s1;
+    out[(head ? OFF_W3 : OFF_B2) + c] = s2;
+    if (t == 0) out[OFF_B3] = s3;
 }
 
-__global__ void sum_bf16_kernel(const uint16_t *__restrict__ v, int n, float *__restrict__ out)
+// g = the sum of the splits' partial gradients, splits ascending
+__global__ void grad_reduce_kernel(const float *__restrict__ part, int nsplit, float *__restrict__ g)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= NPARAM) return;
     float s = 0.f;
-    for (int r = 0; r < n; ++r) s += from_bf16(v[r]);
-    out[0] = s;
+#pragma unroll 8
+    for (int z = 0; z < nsplit; ++z) s += part[(int64_t)z * NPARAM + x];
+    g[x] = s;
 }
 
 // Adam on the fp32 master weights, then the bf16 copies
@@ -376,6 +457,7 @@ struct mh_mlp {
     mh_context *ctx = nullptr;
     DevBuf p, m, v, g, wbf;
     DevBuf h1, h2, y, gy, dz1, dz2, loss, idx;
+    DevBuf part;          // partial gradients, one a split of the batch's rows
     uint64_t cap = 0;     // batch rows the activation buffers hold
     uint64_t step = 0;
     uint64_t seed = 0;
@@ -397,9 +479,21 @@ int mlp_reserve(mh_mlp *n, uint64_t rows)
     return MH_OK;
 }
 
-void launch_gemm(hipStream_t st, int M, int N, int K, const Operand &A, const Operand &B, const Epilogue &E)
+// Rows of a split of the weight gradients' K (= the batch's rows): 128, so that
+// a 2,048-row training batch gives dW1 320 workgroups and dW2 128, and at most
+// 64 splits (65,536 rows: 1,024 rows each).
+int grad_kchunk(int rows)
 {
-    hipLaunchKernelGGL(gemm_kernel, dim3((M + GT - 1) / GT, (N + GT - 1) / GT), dim3(256), 0, st, M, N, K, A, B, E);
+    const int per = (rows + 63) / 64;
+    return std::max(128, (per + GK - 1) / GK * GK);
+}
+
+template <bool AKC, bool AF32, bool BKC, bool BF32>
+void launch_gemm(hipStream_t st, int M, int N, int K, int kchunk, const Operand &A, const Operand &B, const Epilogue &E)
+{
+    hipLaunchKernelGGL((gemm_kernel<AKC, AF32, BKC, BF32>),
+                       dim3((M + GT - 1) / GT, (N + GT - 1) / GT, (K + kchunk - 1) / kchunk), dim3(256), 0, st, M, N, K,
+                       kchunk, A, B, E);
 }
 
 // forward over `rows` examples (features x rows, or x[idx[r]]): h1, h2, y
@@ -408,57 +502,57 @@ void mlp_forward_rows(mh_mlp *n, const float *x, const uint32_t *idx, int rows)
     hipStream_t st = n->ctx->stream;
     const float *p = n->p.as<float>();
     const uint16_t *wbf = n->wbf.as<uint16_t>();
-    Operand X{x, NIN, 1, idx, 1};
-    Operand W1t{wbf + BOFF_W1, 1, NIN, nullptr, 0};          // (k = in, n = out) at W1[out][in]
-    Epilogue e1{EPI_BIAS_RELU_BF16, p + OFF_B1, nullptr, n->h1.as<uint16_t>(), NH1, nullptr, 0};
-    launch_gemm(st, rows, NH1, NIN, X, W1t, e1);
-    Operand H1{n->h1.as<uint16_t>(), NH1, 1, nullptr, 0};
-    Operand W2t{wbf + BOFF_W2, 1, NH1, nullptr, 0};
-    Epilogue e2{EPI_BIAS_RELU_BF16, p + OFF_B2, nullptr, n->h2.as<uint16_t>(), NH2, nullptr, 0};
-    launch_gemm(st, rows, NH2, NH1, H1, W2t, e2);
+    Operand X{x, NIN, idx};
+    Operand W1t{wbf + BOFF_W1, NIN, nullptr};          // (k = in, n = out) at W1[out][in]
+    Epilogue e1{EPI_BIAS_RELU_BF16, p + OFF_B1, nullptr, 0, n->h1.as<uint16_t>(), NH1, nullptr, 0};
+    launch_gemm<true, true, true, false>(st, rows, NH1, NIN, NIN, X, W1t, e1);
+    Operand H1{n->h1.as<uint16_t>(), NH1, nullptr};
+    Operand W2t{wbf + BOFF_W2, NH1, nullptr};
+    Epilogue e2{EPI_BIAS_RELU_BF16, p + OFF_B2, nullptr, 0, n->h2.as<uint16_t>(), NH2, nullptr, 0};
+    launch_gemm<true, false, true, false>(st, rows, NH2, NH1, NH1, H1, W2t, e2);
     hipLaunchKernelGGL(head_kernel, dim3((rows + 255) / 256), dim3(256), 0, st, n->h2.as<uint16_t>(), rows,
                        wbf + BOFF_W3, p + OFF_B3, n->y.as<float>());
 }
 
 // loss and gradients of one batch into n->g (fp32, flat parameter layout)
-void mlp_backward_rows(mh_mlp *n, const float *x, const float *target, const uint32_t *idx, int rows)
+int mlp_backward_rows(mh_mlp *n, const float *x, const float *target, const uint32_t *idx, int rows)
 {
     hipStream_t st = n->ctx->stream;
     const uint16_t *wbf = n->wbf.as<uint16_t>();
-    float *g = n->g.as<float>();
     uint16_t *gy = n->gy.as<uint16_t>(), *h1 = n->h1.as<uint16_t>(), *h2 = n->h2.as<uint16_t>();
     uint16_t *dz1 = n->dz1.as<uint16_t>(), *dz2 = n->dz2.as<uint16_t>();
+    const int kc = grad_kchunk(rows), ns = (rows + kc - 1) / kc;
+    int rc;
+    if ((rc = n->part.ensure((size_t)ns * NPARAM * 4 + 64)) != MH_OK) return rc;
+    float *part = n->part.as<float>();
     hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, st, n->y.as<float>(), target, idx, rows, gy,
                        n->loss.as<float>());
-    // head: dw3 = g^T h2, db3 = sum g, dz2
-    hipLaunchKernelGGL(colsum_kernel, dim3((NH2 + 127) / 128), dim3(128), 0, st, h2, rows, NH2, gy, g + OFF_W3);
-    hipLaunchKernelGGL(sum_bf16_kernel, dim3(1), dim3(64), 0, st, gy, rows, g + OFF_B3);
     hipLaunchKernelGGL(head_back_kernel, dim3((unsigned)(((int64_t)rows * NH2 + 255) / 256)), dim3(256), 0, st, gy,
                        h2, rows, wbf + BOFF_W3, dz2);
-    // layer 2: dW2 = dz2^T h1 (M = NH2, N = NH1, K = rows), db2, dz1
+    // layer 2: dW2 = dz2^T h1 (M = NH2, N = NH1, K = rows), dz1
     {
-        Operand A{dz2, 1, NH2, nullptr, 0};       // (m = out2, k = row) at dz2[row][out2]
-        Operand B{h1, NH1, 1, nullptr, 0};        // (k = row, n = in2) at h1[row][in2]
-        Epilogue e{EPI_F32, nullptr, g + OFF_W2, nullptr, NH1, nullptr, 0};
-        launch_gemm(st, NH2, NH1, rows, A, B, e);
+        Operand A{dz2, NH2, nullptr};             // (m = out2, k = row) at dz2[row][out2]
+        Operand B{h1, NH1, nullptr};              // (k = row, n = in2) at h1[row][in2]
+        Epilogue e{EPI_F32, nullptr, part + OFF_W2, NPARAM, nullptr, NH1, nullptr, 0};
+        launch_gemm<false, false, false, false>(st, NH2, NH1, rows, kc, A, B, e);
     }
-    hipLaunchKernelGGL(colsum_kernel, dim3((NH2 + 127) / 128), dim3(128), 0, st, dz2, rows, NH2, nullptr,
-                       g + OFF_B2);
     {
-        Operand A{dz2, NH2, 1, nullptr, 0};       // (m = row, k = out2)
-        Operand B{wbf + BOFF_W2, NH1, 1, nullptr, 0};   // (k = out2, n = in2) at W2[out2][in2]
-        Epilogue e{EPI_MASK_BF16, nullptr, nullptr, dz1, NH1, h1, NH1};
-        launch_gemm(st, rows, NH1, NH2, A, B, e);
+        Operand A{dz2, NH2, nullptr};             // (m = row, k = out2)
+        Operand B{wbf + BOFF_W2, NH1, nullptr};   // (k = out2, n = in2) at W2[out2][in2]
+        Epilogue e{EPI_MASK_BF16, nullptr, nullptr, 0, dz1, NH1, h1, NH1};
+        launch_gemm<true, false, false, false>(st, rows, NH1, NH2, NH2, A, B, e);
     }
-    // layer 1: dW1 = dz1^T x (M = NH1, N = NIN, K = rows), db1
+    // layer 1: dW1 = dz1^T x (M = NH1, N = NIN, K = rows)
     {
-        Operand A{dz1, 1, NH1, nullptr, 0};
-        Operand B{x, NIN, 1, idx, 1};             // (k = row, n = feature) at x[idx[row]][feature]
-        Epilogue e{EPI_F32, nullptr, g + OFF_W1, nullptr, NIN, nullptr, 0};
-        launch_gemm(st, NH1, NIN, rows, A, B, e);
+        Operand A{dz1, NH1, nullptr};
+        Operand B{x, NIN, idx};                   // (k = row, n = feature) at x[idx[row]][feature]
+        Epilogue e{EPI_F32, nullptr, part + OFF_W1, NPARAM, nullptr, NIN, nullptr, 0};
+        launch_gemm<false, false, false, true>(st, NH1, NIN, rows, kc, A, B, e);
     }
-    hipLaunchKernelGGL(colsum_kernel, dim3((NH1 + 127) / 128), dim3(128), 0, st, dz1, rows, NH1, nullptr,
-                       g + OFF_B1);
+    // biases and the head: dw3 = g^T h2, db3 = sum g
+    hipLaunchKernelGGL(colsums_kernel, dim3(ns), dim3(256), 0, st, dz1, dz2, h2, gy, rows, kc, part);
+    hipLaunchKernelGGL(grad_reduce_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, st, part, ns, n->g.as<float>());
+    return MH_OK;
 }
 
 }  // namespace
@@ -572,7 +666,7 @@ int mh_mlp_grad(mh_context *ctx, mh_mlp *n, const float *d_x, const float *d_t, 
     int rc;
     if ((rc = mlp_reserve(n, rows)) != MH_OK) return rc;
     mlp_forward_rows(n, d_x, nullptr, (int)rows);
-    mlp_backward_rows(n, d_x, d_t, nullptr, (int)rows);
+    if ((rc = mlp_backward_rows(n, d_x, d_t, nullptr, (int)rows)) != MH_OK) return rc;
     MH_HIP(hipGetLastError());
     MH_HIP(hipMemcpyAsync(grads, n->g.ptr, NPARAM * 4, hipMemcpyDeviceToHost, ctx->stream));
     float l = 0.f;
@@ -608,7 +702,7 @@ int mh_mlp_train(mh_context *ctx, mh_mlp *n, const float *d_x, const float *d_t,
         for (uint64_t bi = 0; bi < nb; ++bi) {
             const uint32_t *idx = n->idx.as<uint32_t>() + bi * bs;
             mlp_forward_rows(n, d_x, idx, (int)bs);
-            mlp_backward_rows(n, d_x, d_t, idx, (int)bs);
+            if ((rc = mlp_backward_rows(n, d_x, d_t, idx, (int)bs)) != MH_OK) return rc;
             ++n->step;
             // cosine decay of the learning rate over the run
             const double prog = ((double)ep * nb + bi) / ((double)opt->epochs * nb);

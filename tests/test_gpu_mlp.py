@@ -105,6 +105,31 @@ def test_gradients_match_oracle(ctx, n):
     net.free()
 
 
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 8200])
+def test_gradients_at_the_row_split(ctx, n):
+    """The weight gradients sum the rows in splits of 128 (160 from 8,193 rows
+    on, for 64 splits at most): sizes about a split's edge and above the cap.
+    The bound is that of the other gradient test (an activation's bf16 rounding
+    may move by a unit, 2^-8 of it); the splits' sums add in a fixed order, so a
+    second call gives the same bits."""
+    rng = np.random.default_rng(500 + n)
+    p, x, t = _net_and_batch(rng, n)
+    net = mauvehip.Mlp(ctx, params=p)
+    dX, dT = ctx.alloc(x.nbytes + 16), ctx.alloc(t.nbytes + 16)
+    ctx.h2d(dX + 4, x)              # a float address that is not 16-byte aligned
+    ctx.h2d(dT, t)
+    loss, g = net.grad_device(dX + 4, dT, n)
+    wl, wg = mo.grad(p, x, t)
+    assert abs(loss - wl) <= 1e-3 * max(1.0, abs(wl))
+    for lo, hi in ((mo.OFF_W1, mo.OFF_B1), (mo.OFF_B1, mo.OFF_W2), (mo.OFF_W2, mo.OFF_B2), (mo.OFF_B2, mo.OFF_W3),
+                   (mo.OFF_W3, mo.OFF_B3), (mo.OFF_B3, mo.NPARAM)):
+        assert np.linalg.norm(g[lo:hi] - wg[lo:hi]) <= 2e-2 * max(np.linalg.norm(wg[lo:hi]), 1e-12), (lo, hi)
+    assert np.array_equal(net.grad_device(dX + 4, dT, n)[1], g)
+    for q in (dX, dT):
+        ctx.free(q)
+    net.free()
+
+
 def test_training_fits_a_smooth_target(ctx):
     """Adam on the device drives the loss of a learnable target down."""
     rng = np.random.default_rng(7)
