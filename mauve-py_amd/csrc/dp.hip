@@ -1,12 +1,13 @@
 // dp.hip -- batched NWSmall-exact affine-gap DP for gfx950.
 //
-// One wavefront per job.  The B axis is cut into stripes of 512 columns;
-// lane k owns columns [8k, 8k+8) of the stripe and walks down the rows of A
-// one step behind lane k-1 (anti-diagonal skew), so at step t lane k is on
-// row i = t - k + 1.  The right-edge values (M, D, I) of each lane's last
-// column move to lane k+1 with a DPP wave_shr:1 each step; lane 0 reads the
-// stripe's left boundary column from a per-job buffer written by lane 63 of
-// the previous stripe, 64 rows at a time.
+// One wavefront per job (or four narrow jobs a wavefront, one a 16-lane row).
+// The B axis is cut into stripes of 64 * COLS columns; lane k owns COLS
+// consecutive columns of the stripe and walks down the rows of A one step
+// behind lane k-1 (anti-diagonal skew), so at step t lane k is on row i = t -
+// k + 1.  The right-edge values of each lane's last column move to lane k+1
+// with a DPP wave_shr:1 each step; lane 0 reads the stripe's left boundary
+// column from a per-job buffer written by lane 63 of the previous stripe, 64
+// rows at a time.
 //
 // Scores are int32.  On this path every operand of the reference's float DP
 // is an integer (NUC_SP, -200 open/close halves, extend 0, MU/nucmx.cpp:8-25,
@@ -19,14 +20,11 @@
 //            tie order M, D, I                                      (111-142)
 // with the boundary rows/columns of 546-569, 579-595, 616-637 expressed as
 // virtual row/column 0 values, and the one-row case (LA == 1) where M(1,1)
-// carries close_A[0] and a 'D' trace bit (616-626; SetTermGaps leaves
-// close[0] alone for a length-1 profile, MU/termgaps.cpp:24).
+// carries close_A[0] (616-626; SetTermGaps leaves close[0] alone for a length-1
+// profile, MU/termgaps.cpp:24).
 //
-// Trace bits are the reference's 4-bit code (MU/types.h:26-46): bits 0-1 the
-// M source (MM=0, DM=1, IM=2), bit 2 MD, bit 3 MI.  Each lane writes one
-// 32-bit word (8 cells) per step, so a wavefront stores 256 contiguous bytes
-// per step; the word of cell (i, j) is at
-//   stripe*(LA+63)*64 + (i-1 + lane)*64 + lane,  lane = ((j-1) mod 512) / 8.
+// Each cell leaves a 4-bit record for the trace-back, which the same wavefront
+// runs right after its forward pass.
 #include "mh_internal.hpp"
 #include "dp_tune_table.h"
 #include <algorithm>
@@ -88,9 +86,9 @@ __host__ __device__ inline void stripe_rows(uint32_t la, uint32_t lb, uint32_t b
     r1 = (int)a1;
 }
 
-// Trace bytes of one job run by g lanes: per non-empty stripe (rows + g - 1)
-// steps of g lanes x cols/2 bytes.
-uint64_t dp_trace_bytes(uint32_t la, uint32_t lb, uint32_t band, uint32_t cols, uint32_t g)
+// Steps of one job run by g lanes of cols columns: rows + g - 1 per non-empty
+// stripe.  A step evaluates g * cols cells.
+static uint64_t dp_steps(uint32_t la, uint32_t lb, uint32_t band, uint32_t cols, uint32_t g)
 {
     const uint32_t sw = g * cols;
     const uint32_t ns = (lb + sw - 1) / sw;
@@ -100,7 +98,7 @@ uint64_t dp_trace_bytes(uint32_t la, uint32_t lb, uint32_t band, uint32_t cols, 
         stripe_rows(la, lb, band, sw, s, r0, r1);
         if (r1 >= r0) steps += (uint64_t)(r1 - r0 + 1) + (g - 1);
     }
-    return steps * g * (cols / 2);
+    return steps;
 }
 
 namespace {
@@ -125,33 +123,258 @@ __device__ __forceinline__ void static_for(std::integer_sequence<int, Cs...>, F 
     (f(std::integral_constant<int, Cs>{}), ...);
 }
 
-__device__ __forceinline__ int max3i(int a, int b, int c)
+// ---- the cell ---------------------------------------------------------------
+//
+// NWSmall's recurrences (see above) are evaluated in a form that keeps two
+// values a column instead of three and adds once a cell instead of three times.
+// With o the gap open (goh) and c the close (goh), both constant inside the
+// matrix, and
+//   E(i,j) = D(i,j) - o,   F(i,j) = I(i,j) - o,   N(i,j) = M(i,j) - (o + c),
+// the rules become
+//   H(i,j)   = max(N, E, F)(i,j)        the best source of M(i+1,j+1)
+//   N(i,j)   = s(i,j) + H(i-1,j-1),     M = N + (o + c)
+//   E(i+1,j) = max(E(i,j), M(i,j)),     F(i,j+1) = max(F(i,j), M(i,j)).
+// Each is the reference's comparison with both sides shifted alike, and all
+// values are integers, so scores and ties are the same.  The terminal gaps
+// (open 0 at the first position, no close at the last) only touch column 0, row
+// 0 and the final pick.
+//
+// A cell's trace record holds, for a walk that arrives at (i, j), the state it
+// continues in: bits 0-1 the source of H(i, j) for one that arrives by an M edge
+// from (i+1, j+1) (TAG_M, TAG_D, TAG_I), bit 2 set when D(i+1, j) opens from M(i, j),
+// bit 3 set when I(i, j+1) does.  The int32 cell keeps values times four with
+// the state in the two low bits (M 3, D 2, I 0): a maximum then breaks ties as
+// the reference does (M before D before I) and its low bits are the record's,
+// shifted into the trace word by one v_alignbit each, instead of compares and
+// selects.
+//
+// The forward pass is bound by VALU issue.  Per cell this takes 11.5 VALU
+// instructions: two adds (one an SDWA add that also picks the cell's 16-bit
+// score), one max3, two max, three v_alignbit, three that restore the tags, and
+// half a v_perm (the scores of two columns by A's letter).  Measured on MI355X:
+// the 16-column row step went from 348 instructions (compares, selects and s_nops
+// for the trace bits) to 199; 20,000 jobs of 5-500 columns from 1,697 to 992 us,
+// 4,000 of 10-20,000 from 113.8 to 75.9 ms (both with the walks below).
+enum : uint32_t { TAG_M = 3, TAG_D = 2, TAG_I = 0 };
+
+__device__ __forceinline__ uint32_t walk_next(uint32_t nib, int t)
 {
-    int r;
-    asm("v_max3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
+    if (t == 'M') return (nib & 3u) == TAG_M ? 'M' : ((nib & 3u) == TAG_D ? 'D' : 'I');
+    if (t == 'D') return (nib & 4u) ? 'M' : 'D';
+    return (nib & 8u) ? 'M' : 'I';
 }
+
+// does a walk in state t stay in it at a position with this record
+__device__ __forceinline__ bool walk_stays(uint32_t nib, int t)
+{
+    return t == 'M' ? (nib & 3u) == TAG_M : (t == 'D' ? (nib & 4u) == 0u : (nib & 8u) == 0u);
+}
+
+// bytes of a lane's records of one step: a nibble a column, in whole words a
+// lane can store at once
+__host__ __device__ constexpr uint32_t lane_bytes_of(uint32_t cols) { return cols <= 4 ? 2u : (cols <= 8 ? 4u : 8u); }
+
+template <int COLS> __device__ __forceinline__ void store_records(uint8_t *dst, const uint32_t *word)
+{
+    if constexpr (COLS <= 4) *reinterpret_cast<uint16_t *>(dst) = (uint16_t)word[0];
+    else if constexpr (COLS <= 8) *reinterpret_cast<uint32_t *>(dst) = word[0];
+    else *reinterpret_cast<uint2 *>(dst) = make_uint2(word[0], word[1]);
+}
+
+// Match scores: int32, NUC_SP (MU/nucmx.cpp:8-25) as packed_rows gives it, or
+// the 6 x 6 float table of operands with wildcard letters.
+struct ScoreArgs {
+    uint32_t lo[4], hi[4];     // int32: row a's scores times 4, 16 bits each (columns 0, 1 | 2, 3)
+    uint32_t sr[4];            // int32: row a's scores plus SBIAS, 8 bits each (sliding-window jobs)
+};
+
+constexpr int GOH = -200;      // half of the gap open (MU/profilefrommsa.cpp:291-292)
+
+// int32 cells: values times 4 plus the state's tag
+struct IntCell {
+    static constexpr int OC = 4 * (2 * GOH);
+    static constexpr int NEGV = -(1 << 30);
+    __device__ static int neg_h() { return NEGV | 3; }
+    __device__ static int neg_e() { return NEGV | 2; }
+    __device__ static int neg_f() { return NEGV; }
+    // H(0,0): the source of M(1,1) is M(0,0) = 0; with LA == 1 the reference
+    // gives M(1,1) the close of the one position (MU/nwsmall.cpp:616-626)
+    __device__ static int corner(int la) { return 4 * (la == 1 ? GOH : 0) - OC + 3; }
+    // H(i,0) and H(0,j): D(i,0) = I(0,j) = 0, closed
+    __device__ static int edge() { return 4 * GOH - OC + 3; }
+
+    template <int COLS> struct Lane {
+        int H[COLS], E[COLS], F[COLS];   // row i: H(i,j), E(i+1,j), F(i,j+1)
+        uint32_t sel[(COLS + 1) / 2];    // byte selectors of two columns' scores
+        uint32_t word[COLS > 8 ? 2 : 1];
+    };
+    template <int COLS, class Code> __device__ static void init(Lane<COLS> &s, Code &&code, bool top, bool first)
+    {
+#pragma unroll
+        for (int c = 0; c < COLS; c += 2) {
+            const uint32_t b0 = code(c) & 3u, b1 = c + 1 < COLS ? code(c + 1) & 3u : 0u;
+            s.sel[c / 2] = (2u * b0) | ((2u * b0 + 1u) << 8) | ((2u * b1) << 16) | ((2u * b1 + 1u) << 24);
+        }
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            s.H[c] = top ? edge() : neg_h();
+            s.E[c] = neg_e();
+            s.F[c] = neg_f();
+        }
+        (void)first;
+        for (uint32_t &w : s.word) w = 0;
+    }
+    // the row operand of A's letter
+    __device__ static void operand(const ScoreArgs &sc, uint32_t code, int &lo, int &hi)
+    {
+        lo = (int)((code & 2) ? ((code & 1) ? sc.lo[3] : sc.lo[2]) : ((code & 1) ? sc.lo[1] : sc.lo[0]));
+        hi = (int)((code & 2) ? ((code & 1) ? sc.hi[3] : sc.hi[2]) : ((code & 1) ? sc.hi[1] : sc.hi[0]));
+    }
+    // one row: diagH = H(i-1, first column - 1), f = F(i, first column)
+    template <int COLS>
+    __device__ static __forceinline__ void row(Lane<COLS> &s, const float *, int lo, int hi, int diagH, int f)
+    {
+        // (N of column c + 1 is taken before H of column c changes, so that no
+        // register is copied)
+        uint32_t p = __builtin_amdgcn_perm((uint32_t)hi, (uint32_t)lo, s.sel[0]);
+        int n = diagH + (int)(int16_t)(p & 0xFFFFu);
+        static_for(std::make_integer_sequence<int, COLS>{}, [&](auto ic) {
+            constexpr int c = decltype(ic)::value;
+            constexpr int w = c >> 3;
+            const int m = n + OC;
+            const int h = max(max(n, s.E[c]), f);
+            s.word[w] = __builtin_amdgcn_alignbit((uint32_t)h, s.word[w], 2);
+            if constexpr (c + 1 < COLS) {
+                if constexpr ((c & 1) == 1) p = __builtin_amdgcn_perm((uint32_t)hi, (uint32_t)lo, s.sel[(c + 1) / 2]);
+                n = s.H[c] + ((c & 1) ? (int)(int16_t)(p & 0xFFFFu) : (int)p >> 16);
+            }
+            s.H[c] = h | 3;
+            const int x = max(s.E[c], m);
+            s.word[w] = __builtin_amdgcn_alignbit((uint32_t)x, s.word[w], 1);
+            s.E[c] = x & ~1;
+            const int y = max(f, m);
+            s.word[w] = __builtin_amdgcn_alignbit((uint32_t)y, s.word[w], 1);
+            f = y & ~3;
+            s.F[c] = f;
+        });
+        if constexpr ((COLS & 7) != 0) s.word[COLS >> 3] >>= 32 - 4 * (COLS & 7);
+    }
+    // the final pick (MU/nwsmall.cpp:641-656) of the cell with values h, e, f
+    // and record nib: M(LA,LB), D and I without their close.  e and f hold
+    // max(E, M) and max(F, M); the record's bits say which, and an M that
+    // neither shows and that is not H's source is below D or I.
+    __device__ static void pick(int h, int e, int f, uint32_t nib, int, int, int, int &score, int &edge_out)
+    {
+        constexpr int NONE = -(1 << 30);
+        const int hv = h >> 2, ev = e >> 2, fv = f >> 2;
+        const int M = (nib & 4u) ? ev : ((nib & 8u) ? fv : ((nib & 3u) == TAG_M ? hv + 2 * GOH : NONE));
+        const int D = (nib & 4u) ? NONE : ev + GOH, I = (nib & 8u) ? NONE : fv + GOH;
+        score = M;
+        edge_out = 'M';
+        if (D > score) { score = D; edge_out = 'D'; }
+        if (I > score) { score = I; edge_out = 'I'; }
+    }
+};
+
+// Cells whose values carry no tag: float for operands with wildcard letters
+// (fractional scores, added in the reference's order: M = s + best, D and I
+// closed before the comparison, so every value and tie is its float), and
+// int32 for jobs whose scores times four could leave 32 bits.  H(i,j) =
+// max(M, D + c, I + c), E(i+1,j) = max(D, M + o), F(i,j+1) = max(I, M + o).
+template <class T> struct CmpCell {
+    static constexpr bool FLT = std::is_same<T, float>::value;
+    static constexpr T G = (T)GOH;
+    __device__ static T neg() { return FLT ? (T)-1e37f : (T)-(1 << 29); }     // MINUS_INFINITY, MU/intmath.h:46
+    __device__ static int bits(T v)
+    {
+        if constexpr (FLT) return __float_as_int(v);
+        else return v;
+    }
+    __device__ static T val(int b)
+    {
+        if constexpr (FLT) return __int_as_float(b);
+        else return b;
+    }
+    __device__ static int neg_h() { return bits(neg()); }
+    __device__ static int neg_e() { return bits(neg()); }
+    __device__ static int neg_f() { return bits(neg()); }
+    __device__ static int corner(int la) { return bits(la == 1 ? G : (T)0); }
+    __device__ static int edge() { return bits(G); }
+
+    template <int COLS> struct Lane {
+        int H[COLS], E[COLS], F[COLS];   // row i: H(i,j), D(i+1,j), I(i,j+1)
+        T M[COLS], D[COLS], I[COLS];     // row i
+        uint8_t code[COLS];
+        uint32_t word[COLS > 8 ? 2 : 1];
+    };
+    template <int COLS, class Code> __device__ static void init(Lane<COLS> &s, Code &&code, bool top, bool)
+    {
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            s.code[c] = (uint8_t)code(c);
+            s.H[c] = top ? edge() : neg_h();
+            s.E[c] = neg_e();
+            s.F[c] = neg_f();
+            s.M[c] = s.D[c] = s.I[c] = neg();
+        }
+        for (uint32_t &w : s.word) w = 0;
+    }
+    __device__ static void operand(const ScoreArgs &, uint32_t code, int &lo, int &hi)
+    {
+        lo = 6 * (int)code;
+        hi = 0;
+    }
+    template <int COLS>
+    __device__ static __forceinline__ void row(Lane<COLS> &s, const float *table, int lo, int, int diagH, int f)
+    {
+#pragma clang fp contract(off)
+        T dh = val(diagH), fi = val(f);
+        static_for(std::make_integer_sequence<int, COLS>{}, [&](auto ic) {
+            constexpr int c = decltype(ic)::value;
+            constexpr int w = c >> 3, sh = 4 * (c & 7);
+            const T sc = (T)table[lo + s.code[c]];
+            const T m = sc + dh, d = val(s.E[c]), i = fi;
+            const T a = m + G, dc = d + G, ic2 = i + G;
+            const T h = max(max(m, dc), ic2);
+            uint32_t nib = m == h ? (uint32_t)TAG_M : (dc == h ? (uint32_t)TAG_D : (uint32_t)TAG_I);
+            dh = val(s.H[c]);
+            s.H[c] = bits(h);
+            if (a >= d) nib |= 4u;
+            s.E[c] = bits(a >= d ? a : d);
+            if (a >= i) nib |= 8u;
+            fi = a >= i ? a : i;
+            s.F[c] = bits(fi);
+            s.M[c] = m;
+            s.D[c] = d;
+            s.I[c] = i;
+            s.word[w] = (sh == 0 ? 0u : s.word[w]) | (nib << sh);
+        });
+    }
+    // M, D, I of the final cell
+    __device__ static void pick(int, int, int, uint32_t, int M, int D, int I, int &score, int &edge_out)
+    {
+        T s = val(M);
+        edge_out = 'M';
+        if (val(D) > s) { s = val(D); edge_out = 'D'; }
+        if (val(I) > s) { s = val(I); edge_out = 'I'; }
+        if constexpr (FLT) score = (int)rintf(s);
+        else score = s;
+    }
+};
 
 // One job per G lanes: a wavefront (G = 64), or each 16-lane DPP row of a
 // wavefront (G = 16: four jobs at once, for jobs at most 16*COLS columns wide,
 // whose skew and column padding would leave most of a wavefront idle).  In
-// what follows "64" is G.  D and I are kept shifted by the close half (goh):
-// D' = D + goh and I' = I + goh, so the M recurrence reads them without an
-// add; every comparison is between two values shifted alike, so ties and
-// trace bits are unchanged.  Per row a lane runs two passes over its COLS
-// columns: M and D right to left (each needs only the previous row's values of
-// its own and the left column), then I left to right (it chains along the
-// row).  Both update the registers in place.
-//
-// Stripe s computes rows [r0, r1] (stripe_rows); at step t lane k is on row
-// r0 + t - k.  Cells outside those rows are outside the computed region and
-// read as NEG, so a banded job is the exact DP restricted to that region;
-// with band 0 every stripe runs all rows.  Lanes outside their row range sit
-// out the step (exec mask).  Trace bits are the reference's 4-bit code
-// (MU/types.h:26-46): bits 0-1 the M source (MM=0, DM=1, IM=2), bit 2 MD,
-// bit 3 MI; each lane stores COLS/2 bytes per step, so a wavefront stores
-// 32*COLS contiguous bytes per step.  Cell (i, j) of lane k, column c is at
-// byte  stripe_base + ((i - r0 + k)*64 + k)*COLS/2 + c/2, nibble c%2.
+// what follows "64" is G.  Stripe s computes rows [r0, r1] (stripe_rows); at
+// step t lane k is on row r0 + t - k.  Cells outside those rows are outside
+// the computed region and read as minus infinity, so a banded job is the exact
+// DP restricted to that region; with band 0 every stripe runs all rows.  Lanes
+// outside their row range sit out the step (exec mask).  Two values a row move
+// to the next lane: H of the lane's last column (the diagonal source of the
+// next lane's first column on the row below) and F past it.  Each lane stores
+// lane_bytes_of(COLS) bytes of records per step, so a wavefront stores 512
+// contiguous bytes (16 columns a lane).  Cell (i, j) of lane k, column c is at
+// byte  stripe_base + ((i - r0 + k)*64 + k)*lane_bytes + c/2, nibble c%2.
 //
 // PIPE: the job's stripes are shared by P wavefronts, wavefront p0 taking
 // stripes p0, p0 + P, ...: stripe s reads the boundary column that stripe
@@ -172,34 +395,40 @@ __device__ __forceinline__ int max3i(int a, int b, int c)
 // parts of the one job a bin whose parts are not all taken; those are far
 // fewer than the resident wavefronts.
 // The result is the same as one wavefront's.
+//
+// Returns whether this wavefront (this row of it) computed the final cell;
+// score and edge are then the final pick in every lane of the group.
 constexpr uint32_t DP_SPIN_MAX = 1u << 22;
 
-template <int COLS, int G, bool PIPE = false>
-__device__ __forceinline__ void dp_job(const DevJob &jb, const uint8_t *__restrict__ A,
-                                       const uint8_t *__restrict__ B, uint8_t *__restrict__ tb,
-                                       int *__restrict__ bnd, DpOut *__restrict__ out, uint32_t sr0,
-                                       uint32_t sr1, uint32_t sr2, uint32_t sr3, int goh, int (*lds_in)[64],
-                                       int (*lds_out)[64], int p0 = 0, int P = 1,
+// LDS of one wavefront: the rows a group's first lane takes in, and the
+// boundary column its last lane hands on
+struct DpLds {
+    int4 in[64];        // H(i, j0 - 1), F(i, j0), A's row operand (two words)
+    int2 out[64];
+    int fin[6][64];
+};
+
+template <class CELL, int COLS, int G, bool PIPE = false>
+__device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restrict__ A, const uint8_t *__restrict__ B,
+                                       uint8_t *__restrict__ tb, int *__restrict__ bnd, const ScoreArgs &sc,
+                                       const float *table, DpLds &lds, int &score, int &edge, int p0 = 0, int P = 1,
                                        uint32_t *__restrict__ err = nullptr)
 {
     constexpr int STRIPE_W = G * COLS;
-    constexpr int NW = (COLS + 7) / 8;               // 32-bit trace words per lane per step
-    constexpr int LANE_BYTES = COLS / 2;
+    constexpr int LANE_BYTES = (int)lane_bytes_of(COLS);
     const int lane = (int)threadIdx.x & (G - 1);
     const int gb = (int)threadIdx.x & ~(G - 1);    // the job's slots in the LDS rows
     const int la = (int)jb.la, lb = (int)jb.lb;
     const uint8_t *a = A + jb.a_off;
     const uint8_t *b = B + jb.b_off;
     const int nr = (la + 63) & ~63;
-    int *bM = bnd + jb.bnd_off;
-    int *bD = bM + nr;
-    int *bI = bD + nr;
+    int *bH = bnd + jb.bnd_off;
+    int *bF = bH + nr;
     uint8_t *tbj = tb + jb.tb_off;
     const int nstripes = (lb + STRIPE_W - 1) / STRIPE_W;
     const int fin_lane = ((lb - 1) % STRIPE_W) / COLS;
     const int fin_col = (lb - 1) % COLS;
-    const int go2 = 2 * goh;
-    int finM = NEG, finD = NEG, finI = NEG;
+    bool fin = false;
     int prev_r0 = 1, prev_r1 = 0;     // rows of the previous stripe's last column held in bnd
     uint64_t tbs = 0;                 // byte offset of the stripe's trace block
     bool gave_up = false;             // PIPE: a wait ran past its bound
@@ -222,8 +451,8 @@ __device__ __forceinline__ void dp_job(const DevJob &jb, const uint8_t *__restri
                 if (a1 >= a0) tbs += (uint64_t)(a1 - a0 + G) * G * LANE_BYTES;
             }
             unsigned long long *pb = reinterpret_cast<unsigned long long *>(bnd + jb.bnd_off);
-            pin = pb + (size_t)((s + 1) & 1) * 3 * nr;
-            pout = pb + (size_t)(s & 1) * 3 * nr;
+            pin = pb + (size_t)((s + 1) & 1) * 2 * nr;
+            pout = pb + (size_t)(s & 1) * 2 * nr;
         }
         if (r1 < r0) {
             prev_r0 = 1;
@@ -232,13 +461,11 @@ __device__ __forceinline__ void dp_job(const DevJob &jb, const uint8_t *__restri
         }
         // PIPE: until every lane with want set holds the words stripe s - 1
         // wrote for row i (tag s), fetch them again
-        auto settle = [&](bool want, int i, unsigned long long &wM, unsigned long long &wD,
-                          unsigned long long &wI) {
+        auto settle = [&](bool want, int i, unsigned long long &wH, unsigned long long &wF) {
             if constexpr (PIPE) {
                 uint32_t spins = 0;
                 for (;;) {
-                    const bool bad = want && ((uint32_t)(wM >> 32) != (uint32_t)s ||
-                                              (uint32_t)(wD >> 32) != (uint32_t)s || (uint32_t)(wI >> 32) != (uint32_t)s);
+                    const bool bad = want && ((uint32_t)(wH >> 32) != (uint32_t)s || (uint32_t)(wF >> 32) != (uint32_t)s);
                     if (__ballot(bad) == 0 || gave_up) break;
                     if (++spins > DP_SPIN_MAX) {
                         if (lane == 0) atomicOr(err, 1u);
@@ -247,9 +474,8 @@ __device__ __forceinline__ void dp_job(const DevJob &jb, const uint8_t *__restri
                     }
                     __builtin_amdgcn_s_sleep(2);
                     if (bad) {
-                        wM = __hip_atomic_load(pin + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        wD = __hip_atomic_load(pin + nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        wI = __hip_atomic_load(pin + 2 * nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        wH = __hip_atomic_load(pin + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        wF = __hip_atomic_load(pin + nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
                 }
             }
@@ -264,241 +490,149 @@ __device__ __forceinline__ void dp_job(const DevJob &jb, const uint8_t *__restri
         const bool last_stripe = (s == nstripes - 1);
         const bool top0 = (r0 == 1);
 
-        uint32_t bsh[COLS];
-#pragma unroll
-        for (int c = 0; c < COLS; ++c) bsh[c] = (c < ncols) ? 8u * (uint32_t)b[jl - 1 + c] : 0u;
-
-        // the row above the stripe: virtual row 0 (M = NEG, D' = NEG + goh,
-        // I' = 0 + goh) when the stripe starts at row 1, else outside (NEG)
-        int Mp[COLS], Dp[COLS], Ip[COLS];
-#pragma unroll
-        for (int c = 0; c < COLS; ++c) {
-            Mp[c] = NEG;
-            Dp[c] = top0 ? NEG + goh : NEG;
-            Ip[c] = top0 ? goh : NEG;
-        }
-        // the cell above-left of the lane's first column: M(0,0) = 0 for column 1,
-        // virtual row 0 for other columns of row 0, the previous stripe's last
-        // column (row r0-1) for lane 0 when it holds that row, else outside
-        int lpM = NEG, lpD = NEG, lpI = NEG;
+        // the row above the stripe: row 0 when the stripe starts at row 1, else outside
+        typename CELL::template Lane<COLS> st;
+        CELL::template init<COLS>(st, [&](int c) { return c < ncols ? (uint32_t)b[jl - 1 + c] : 0u; }, top0, s == 0);
+        // H above-left of the lane's first column: the corner for column 1,
+        // row 0 for other columns of row 1, the previous stripe's last column
+        // (row r0-1) for lane 0 when it holds that row, else outside
+        int lpH = CELL::neg_h();
         if (top0) {
-            lpM = jl == 1 ? 0 : NEG;
-            lpD = NEG + goh;
-            lpI = jl == 1 ? NEG + goh : goh;
+            lpH = jl == 1 ? CELL::corner(la) : CELL::edge();
         } else if constexpr (PIPE) {
             const int i = r0 - 1;
             const bool want = lane == 0 && s > 0 && i >= prev_r0 && i <= prev_r1;
-            unsigned long long wM = 0, wD = 0, wI = 0;
+            unsigned long long wH = 0, wF = 0;
             if (want) {
-                wM = __hip_atomic_load(pin + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                wD = __hip_atomic_load(pin + nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                wI = __hip_atomic_load(pin + 2 * nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                wH = __hip_atomic_load(pin + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                wF = __hip_atomic_load(pin + nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            settle(want, i, wM, wD, wI);
-            if (want) {
-                lpM = (int)(uint32_t)wM;
-                lpD = (int)(uint32_t)wD;
-                lpI = (int)(uint32_t)wI;
-            }
+            settle(want, i, wH, wF);
+            if (want) lpH = (int)(uint32_t)wH;
         } else if (lane == 0 && s > 0 && r0 - 1 >= prev_r0 && r0 - 1 <= prev_r1) {
-            lpM = bM[r0 - 2];
-            lpD = bD[r0 - 2];
-            lpI = bI[r0 - 2];
+            lpH = bH[r0 - 2];
         }
-        int outM = NEG, outD = NEG, outI = NEG, acode = 0;
-        const int ob2_0 = (jl == 1) ? goh : go2;      // open_B[j-1] + goh for the lane's first column
+        int outH = CELL::neg_h(), outF = CELL::neg_f(), rlo = 0, rhi = 0;
 
         // lane 0's inputs, G rows per chunk: column jl-1 of the previous stripe
-        // where it computed that row (else NEG), or column 0 (M = NEG,
-        // D' = 0 + goh, I' = NEG + goh); and the A codes.  The next chunk is
-        // loaded one chunk ahead.
-        // (PIPE: the words are fetched here, for rows this stripe computes,
-        // and settled before use)
-        unsigned long long wM = 0, wD = 0, wI = 0;
+        // where it computed that row, column 0, or outside; and A's letters.
+        // The next chunk is loaded one chunk ahead.  (PIPE: the words are
+        // fetched here, for rows this stripe computes, and settled before use)
+        unsigned long long wH = 0, wF = 0;
         bool want = false;
         int wrow = 0;
-        auto left_in = [&](int x, int &m, int &d, int &ii, int &ac) {
+        auto left_in = [&](int x, int &h, int &f, uint32_t &ac) {
             const int i = r0 + x;
-            if (s == 0) {
-                m = NEG; d = goh; ii = NEG + goh;
-            } else if (i >= prev_r0 && i <= prev_r1) {
+            h = s == 0 ? CELL::edge() : CELL::neg_h();
+            f = CELL::neg_f();
+            if constexpr (PIPE) want = false;
+            if (s > 0 && i >= prev_r0 && i <= prev_r1) {
                 if constexpr (PIPE) {
                     want = i <= r1;
                     wrow = i;
                     if (want) {
-                        wM = __hip_atomic_load(pin + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        wD = __hip_atomic_load(pin + nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        wI = __hip_atomic_load(pin + 2 * nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        wH = __hip_atomic_load(pin + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        wF = __hip_atomic_load(pin + nr + i - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
-                    m = NEG; d = NEG; ii = NEG;
                 } else {
-                    m = bM[i - 1]; d = bD[i - 1]; ii = bI[i - 1];
-                }
-            } else {
-                if constexpr (PIPE) want = false;
-                m = NEG; d = NEG; ii = NEG;
-            }
-            ac = i <= r1 ? a[i - 1] : 0;
-        };
-        // PIPE: the fetched words, once settled, as the lane's inputs
-        auto take = [&](int &m, int &d, int &ii) {
-            if constexpr (PIPE) {
-                settle(want, wrow, wM, wD, wI);
-                if (want) {
-                    m = (int)(uint32_t)wM;
-                    d = (int)(uint32_t)wD;
-                    ii = (int)(uint32_t)wI;
+                    h = bH[i - 1];
+                    f = bF[i - 1];
                 }
             }
+            ac = i <= r1 ? a[i - 1] : 0u;
         };
-        int nM, nD, nI, nA;
-        left_in(lane, nM, nD, nI, nA);
+        int nH, nF;
+        uint32_t nA;
+        left_in(lane, nH, nF, nA);
 
         const int nsteps = nrows + nl - 1;
+        const uint32_t my_rows = lane < nl ? (uint32_t)nrows : 0u;
+        uint8_t *dst = tbj + tbs + (size_t)lane * LANE_BYTES;
         for (int t = 0; t < nsteps; ++t) {
             const int q = t & (G - 1);
             if (q == 0) {
-                take(nM, nD, nI);
-                lds_in[0][gb + lane] = nM;
-                lds_in[1][gb + lane] = nD;
-                lds_in[2][gb + lane] = nI;
-                lds_in[3][gb + lane] = nA;
-                left_in(t + G + lane, nM, nD, nI, nA);
-            }
-            const int rM = shr1_group<G>(outM, lds_in[0][gb + q]);
-            const int rD = shr1_group<G>(outD, lds_in[1][gb + q]);
-            const int rI = shr1_group<G>(outI, lds_in[2][gb + q]);
-            const int ra = shr1_group<G>(acode, lds_in[3][gb + q]);
-            acode = ra;
-
-            const int i = r0 + t - lane;
-            if (i >= r0 && i <= r1 && lane < nl) {
-            const uint32_t srow = (ra & 2) ? ((ra & 1) ? sr3 : sr2) : ((ra & 1) ? sr1 : sr0);
-            const int oa2 = (i == 1) ? goh : go2;   // open_A[i-1] + goh
-            uint32_t word[NW];
-#pragma unroll
-            for (int w = 0; w < NW; ++w) word[w] = 0;
-            // pass 1, right to left: D'(i,j) and M(i,j) from row i-1
-            static_for(std::make_integer_sequence<int, COLS>{}, [&](auto ic) {
-                constexpr int c = COLS - 1 - decltype(ic)::value;
-                constexpr uint32_t K = 1u << (4 * (c & 7));
-                const int md = Mp[c] + oa2;
-                const bool tD = md >= Dp[c];
-                const int Dn = max(md, Dp[c]);
-                const int dM = c ? Mp[c > 0 ? c - 1 : 0] : lpM;
-                const int dD = c ? Dp[c > 0 ? c - 1 : 0] : lpD;
-                const int dI = c ? Ip[c > 0 ? c - 1 : 0] : lpI;
-                const int best = max3i(dM, dD, dI);
-                uint32_t srcK = (dM != best) ? ((dD == best) ? K : 2u * K) : 0u;
-                const int sc = (int)__builtin_amdgcn_ubfe(srow, bsh[c], 8) - SBIAS;
-                int Mn = sc + best;
-                if (c == 0 && la == 1 && jl == 1 && i == 1) {
-                    // one-row quirk: with LA == 1, M(1,1) carries close_A[0] and a 'D' bit
-                    Mn = sc + goh;
-                    srcK = K;
+                if constexpr (PIPE) {
+                    settle(want, wrow, wH, wF);
+                    if (want) {
+                        nH = (int)(uint32_t)wH;
+                        nF = (int)(uint32_t)wF;
+                    }
                 }
-                Mp[c] = Mn;
-                Dp[c] = Dn;
-                word[c >> 3] |= srcK | (tD ? 4u * K : 0u);
-            });
-            // pass 2, left to right: I'(i,j) from I'(i,j-1) and M(i,j-1)
-            int iL = rI, mL = rM;
-            static_for(std::make_integer_sequence<int, COLS>{}, [&](auto ic) {
-                constexpr int c = decltype(ic)::value;
-                constexpr uint32_t K = 1u << (4 * (c & 7));
-                const int mi = mL + (c == 0 ? ob2_0 : go2);
-                const bool tI = mi >= iL;
-                iL = max(mi, iL);
-                Ip[c] = iL;
-                mL = Mp[c];
-                word[c >> 3] |= tI ? 8u * K : 0u;
-            });
-            outM = Mp[COLS - 1];
-            outD = Dp[COLS - 1];
-            outI = Ip[COLS - 1];
-            lpM = rM;
-            lpD = rD;
-            lpI = rI;
-            uint8_t *dst = tbj + tbs + ((size_t)t * G + lane) * LANE_BYTES;
-            if constexpr (COLS == 16) {
-                *reinterpret_cast<uint2 *>(dst) = make_uint2(word[0], word[1]);
-            } else if constexpr (COLS == 8) {
-                *reinterpret_cast<uint32_t *>(dst) = word[0];
-            } else if constexpr (COLS == 4) {
-                *reinterpret_cast<uint16_t *>(dst) = (uint16_t)word[0];
-            } else if constexpr (COLS == 12) {
-                // 6 bytes a lane: 2-byte aligned
-                uint16_t *h = reinterpret_cast<uint16_t *>(dst);
-                h[0] = (uint16_t)word[0];
-                h[1] = (uint16_t)(word[0] >> 16);
-                h[2] = (uint16_t)word[1];
-            } else {
-                // an odd number of bytes a lane (6, 10 or 14 columns): byte stores
-#pragma unroll
-                for (int y = 0; y < LANE_BYTES; ++y) dst[y] = (uint8_t)(word[y >> 2] >> (8 * (y & 3)));
+                int lo, hi;
+                CELL::operand(sc, nA, lo, hi);
+                lds.in[gb + lane] = make_int4(nH, nF, lo, hi);
+                left_in(t + G + lane, nH, nF, nA);
             }
+            const int4 in = lds.in[gb + q];
+            const int rH = shr1_group<G>(outH, in.x);
+            const int rF = shr1_group<G>(outF, in.y);
+            rlo = shr1_group<G>(rlo, in.z);
+            rhi = shr1_group<G>(rhi, in.w);
+            if ((uint32_t)(t - lane) < my_rows) {
+                CELL::template row<COLS>(st, table, rlo, rhi, lpH, rF);
+                lpH = rH;
+                outH = st.H[COLS - 1];
+                outF = st.F[COLS - 1];
+                store_records<COLS>(dst, st.word);
             }
+            dst += G * LANE_BYTES;
             if (!last_stripe) {
                 // the last lane just finished relative row t-(G-1) of the stripe's last column
                 const int xl = t - (G - 1);
-                if (lane == G - 1 && xl >= 0 && xl < nrows) {
-                    const int slot = gb + (xl & (G - 1));
-                    lds_out[0][slot] = outM;
-                    lds_out[1][slot] = outD;
-                    lds_out[2][slot] = outI;
-                }
+                if (lane == G - 1 && xl >= 0 && xl < nrows) lds.out[gb + (xl & (G - 1))] = make_int2(outH, outF);
                 if (xl >= 0 && xl < nrows && ((xl & (G - 1)) == G - 1 || xl == nrows - 1)) {
                     const int x = (xl & ~(G - 1)) + lane;
                     if (x < nrows) {
                         const int r = r0 - 1 + x;
+                        const int2 v = lds.out[gb + lane];
                         if constexpr (PIPE) {
                             const unsigned long long tag = (unsigned long long)(uint32_t)(s + 1) << 32;
-                            __hip_atomic_store(pout + r, tag | (uint32_t)lds_out[0][gb + lane], __ATOMIC_RELAXED,
+                            __hip_atomic_store(pout + r, tag | (uint32_t)v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            __hip_atomic_store(pout + nr + r, tag | (uint32_t)v.y, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
-                            __hip_atomic_store(pout + nr + r, tag | (uint32_t)lds_out[1][gb + lane], __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                            __hip_atomic_store(pout + 2 * nr + r, tag | (uint32_t)lds_out[2][gb + lane],
-                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         } else {
-                            bM[r] = lds_out[0][gb + lane];
-                            bD[r] = lds_out[1][gb + lane];
-                            bI[r] = lds_out[2][gb + lane];
+                            bH[r] = v.x;
+                            bF[r] = v.y;
                         }
                     }
                 }
             }
         }
-        if (last_stripe && r1 == la && lane == fin_lane) {
+        if (last_stripe) {
             // the lane's registers hold row LA, the last it computed: the
-            // final cell's values, picked by way of LDS (the last stripe
-            // stages no boundary there), so that no per-column select on
-            // fin_col is held through the step loop
+            // final cell's values, picked by way of LDS, so that no
+            // per-column select on fin_col is held through the step loop
+            fin = true;
+            int sco = CELL::neg_e(), ed = 'M';
+            if (lane == fin_lane && r1 == la) {
+                static_assert(COLS <= G, "a column a slot");
 #pragma unroll
-            for (int c = 0; c < COLS; ++c) {
-                lds_out[0][gb + c] = Mp[c];
-                lds_out[1][gb + c] = Dp[c];
-                lds_out[2][gb + c] = Ip[c];
+                for (int c = 0; c < COLS; ++c) {
+                    lds.fin[0][gb + c] = st.H[c];
+                    lds.fin[1][gb + c] = st.E[c];
+                    lds.fin[2][gb + c] = st.F[c];
+                    if constexpr (!std::is_same<CELL, IntCell>::value) {
+                        lds.fin[3][gb + c] = CELL::bits(st.M[c]);
+                        lds.fin[4][gb + c] = CELL::bits(st.D[c]);
+                        lds.fin[5][gb + c] = CELL::bits(st.I[c]);
+                    }
+                }
+                const uint32_t w = COLS > 8 && fin_col >= 8 ? st.word[COLS > 8 ? 1 : 0] : st.word[0];
+                const int k = gb + fin_col;
+                CELL::pick(lds.fin[0][k], lds.fin[1][k], lds.fin[2][k], (w >> (4 * (fin_col & 7))) & 15u,
+                           lds.fin[3][k], lds.fin[4][k], lds.fin[5][k], sco, ed);
             }
-            finM = lds_out[0][gb + fin_col];
-            finD = lds_out[1][gb + fin_col];
-            finI = lds_out[2][gb + fin_col];
+            score = __shfl(sco, gb + fin_lane, 64);
+            edge = __shfl(ed, gb + fin_lane, 64);
         }
         prev_r0 = r0;
         prev_r1 = r1;
         tbs += (uint64_t)(nrows + G - 1) * G * LANE_BYTES;
-        if constexpr (!PIPE) __threadfence();
+        // the next stripe reads the boundary column, and the walk the records,
+        // that other lanes of this wavefront wrote
+        if constexpr (!PIPE) __threadfence_block();
     }
-    // (PIPE: the wavefront that ran the last stripe)
-    if (lane == fin_lane && (!PIPE || (p0 < nstripes && (nstripes - 1 - p0) % P == 0))) {
-        // back to unshifted D and I for the final pick, MU/nwsmall.cpp:641-656
-        finD -= goh;
-        finI -= goh;
-        int score = finM, edge = 'M';
-        if (finD > score) { score = finD; edge = 'D'; }
-        if (finI > score) { score = finI; edge = 'I'; }
-        out->score = score;
-        out->edge = edge;
-    }
+    return fin;
 }
 
 
@@ -506,7 +640,8 @@ __device__ __forceinline__ void dp_job(const DevJob &jb, const uint8_t *__restri
 // (DevJob::cols = GROUP_TAG + COLS, COLS even from 4 to 16: the narrowest
 // stripe that holds the job).
 constexpr uint32_t GROUP_TAG = 32;
-constexpr uint32_t ROWS_MAX_LB = 256;   // widest job run four to a wavefront
+constexpr uint32_t ROWS_MAX_LB = 256;     // widest job run four to a wavefront
+constexpr uint32_t ROWS_MAX_WALK = 1024;  // a + b from which a job takes a wavefront to itself
 
 // ---- one round of jobs: a length-binned work queue ----------------------
 //
@@ -532,22 +667,11 @@ enum : uint32_t { QK_STRIPE = 0, QK_ROWS = 1, QK_WINDOW = QK_ROWS + ROW_SHAPES, 
 constexpr int DPQ_MAXB = 48;
 constexpr int DPQ_CURSORS = DPQ_MAXB;
 
+// (Behind it in device memory: DPQ_CURSORS cursors, zeroed at the start of every
+// round, the last of them the round's wait-bound error flag.)
 struct DpRound {
-    const DevJob *jobs;
-    DpOut *outs;
-    const uint8_t *A, *B;
-    uint8_t *tb;
-    int *bnd;
-    uint8_t *paths;
-    mh_dp_result *res;
-    uint32_t *dev;
-    uint32_t *cursor;          // DPQ_CURSORS counters, zeroed at the start of every round; the last
-                               // one is the round's wait-bound error flag
-    uint32_t sr[4];
-    int32_t goh;
     uint32_t nbins;
-    uint32_t nwave;            // jobs [0, nwave) walk back on a wavefront each
-    uint32_t n;                // jobs in the round
+    float table[DP_NCLASS * DP_NCLASS];   // match scores of cells without a tag
     uint32_t kind[DPQ_MAXB], first[DPQ_MAXB], count[DPQ_MAXB];
     uint32_t item0[DPQ_MAXB + 1];   // the bins' first items in queue order (prefix sums)
 };
@@ -605,10 +729,10 @@ __device__ __forceinline__ int row_shr_old(int v, int old, int n)
 template <int C>
 __device__ __forceinline__ void dp_window_job(const DevJob &jb, const uint8_t *__restrict__ A,
                                               const uint8_t *__restrict__ B, uint8_t *__restrict__ tb,
-                                              DpOut *__restrict__ out, uint32_t sr0, uint32_t sr1, uint32_t sr2,
-                                              uint32_t sr3, int goh)
+                                              const ScoreArgs &sa, int &score, int &edge)
 {
     constexpr int WD = 64 * C;
+    constexpr int goh = GOH;
     constexpr int RPD = 8 / C;   // rows per trace word
     const int lane = threadIdx.x;
     const int la = (int)jb.la, lb = (int)jb.lb;
@@ -712,7 +836,7 @@ __device__ __forceinline__ void dp_window_job(const DevJob &jb, const uint8_t *_
             anext = (i + 63 + lane < la) ? a[i + 63 + lane] : 0;
         }
         const int ra = __builtin_amdgcn_readlane(achunk, (i - 1) & 63);
-        const uint32_t srow = (ra & 2) ? ((ra & 1) ? sr3 : sr2) : ((ra & 1) ? sr1 : sr0);
+        const uint32_t srow = (ra & 2) ? ((ra & 1) ? sa.sr[3] : sa.sr[2]) : ((ra & 1) ? sa.sr[1] : sa.sr[0]);
         const int oa2 = (i == 1) ? goh : go2;   // open_A[i-1] + goh
         // diagonal inputs of the lane's first column: lane k-1's last column
         // of the previous row, or the cell left of the window for lane 0
@@ -728,7 +852,7 @@ __device__ __forceinline__ void dp_window_job(const DevJob &jb, const uint8_t *_
             const int dM = c ? Mp[c > 0 ? c - 1 : 0] : dM0;
             const int dD = c ? Dp[c > 0 ? c - 1 : 0] : dD0;
             const int dI = c ? Ip[c > 0 ? c - 1 : 0] : dI0;
-            const int best = max3i(dM, dD, dI);
+            const int best = max(max(dM, dD), dI);
             uint32_t srcK = (dM != best) ? ((dD == best) ? K : 2u * K) : 0u;
             const int sc = (int)__builtin_amdgcn_ubfe(srow, bsh[c], 8) - SBIAS;
             int Mn = sc + best;
@@ -785,131 +909,89 @@ __device__ __forceinline__ void dp_window_job(const DevJob &jb, const uint8_t *_
         }
         bprev = bi;
     }
-    if (lane == 63) {
-        finD -= goh;
-        finI -= goh;
-        int score = finM, edge = 'M';
-        if (finD > score) { score = finD; edge = 'D'; }
-        if (finI > score) { score = finI; edge = 'I'; }
-        out->score = score;
-        out->edge = edge;
-    }
+    // the final pick, in lane 63
+    finD -= goh;
+    finI -= goh;
+    score = finM;
+    edge = 'M';
+    if (finD > score) { score = finD; edge = 'D'; }
+    if (finI > score) { score = finI; edge = 'I'; }
 }
 
-// Narrow jobs (lb <= 16): one lane per job.  The lane keeps a whole row of
-// M, D' and I' in registers and walks the rows of A, with the same two
-// register passes per row as dp_job; columns past lb are computed and
-// ignored (nothing flows leftwards).  The left boundary is column 0 and the
-// top row 0, as for the first stripe of dp_job.  Trace: 8 bytes per row,
-// cell (i, j) at byte (i-1)*8 + (j-1)/2, nibble (j-1)%2.
+// Narrow jobs (lb <= 16): one lane per job.  The lane keeps a whole row in
+// registers and walks the rows of A with dp_job's row step; columns past lb are
+// computed and ignored (nothing flows leftwards).  The left boundary is column
+// 0 and the top row 0, as for the first stripe of dp_job.  Trace: 8 bytes per
+// row, cell (i, j) at byte (i-1)*8 + (j-1)/2, nibble (j-1)%2.
 constexpr int TINY_LB = 16;
 constexpr uint32_t TINY_COLS_TAG = 1;   // DevJob::cols of a one-lane job
 
 __device__ __forceinline__ void tiny_job(const DevJob &jb, const uint8_t *__restrict__ A,
                                          const uint8_t *__restrict__ B, uint8_t *__restrict__ tb,
-                                         DpOut *__restrict__ out, uint32_t sr0, uint32_t sr1, uint32_t sr2,
-                                         uint32_t sr3, int goh)
+                                         const ScoreArgs &sc, int &score, int &edge)
 {
     const int la = (int)jb.la, lb = (int)jb.lb;
     const uint8_t *a = A + jb.a_off;
     const uint8_t *b = B + jb.b_off;
     uint8_t *tbj = tb + jb.tb_off;
-    const int go2 = 2 * goh;
-    uint32_t bsh[TINY_LB];
-#pragma unroll
-    for (int c = 0; c < TINY_LB; ++c) bsh[c] = c < lb ? 8u * (uint32_t)b[c] : 0u;
-    int Mp[TINY_LB], Dp[TINY_LB], Ip[TINY_LB];
-#pragma unroll
-    for (int c = 0; c < TINY_LB; ++c) {   // row 0: M = NEG, D' = NEG + goh, I' = 0 + goh
-        Mp[c] = NEG;
-        Dp[c] = NEG + goh;
-        Ip[c] = goh;
-    }
-    int finM = NEG, finD = NEG, finI = NEG;
+    IntCell::Lane<TINY_LB> st;
+    IntCell::init<TINY_LB>(st, [&](int c) { return c < lb ? (uint32_t)b[c] : 0u; }, true, true);
+    int diag = IntCell::corner(la);
     for (int i = 1; i <= la; ++i) {
-        const int ra = a[i - 1];
-        const uint32_t srow = (ra & 2) ? ((ra & 1) ? sr3 : sr2) : ((ra & 1) ? sr1 : sr0);
-        const int oa2 = (i == 1) ? goh : go2;
-        // column 0: (i-1, 0) is M(0,0) = 0 on row 1, else M = NEG, D' = 0 + goh
-        const int lpM = (i == 1) ? 0 : NEG, lpD = (i == 1) ? NEG + goh : goh, lpI = NEG + goh;
-        uint32_t word[2] = {0u, 0u};
-        static_for(std::make_integer_sequence<int, TINY_LB>{}, [&](auto ic) {
-            constexpr int c = TINY_LB - 1 - decltype(ic)::value;
-            constexpr uint32_t K = 1u << (4 * (c & 7));
-            const int md = Mp[c] + oa2;
-            const bool tD = md >= Dp[c];
-            const int Dn = max(md, Dp[c]);
-            const int dM = c ? Mp[c > 0 ? c - 1 : 0] : lpM;
-            const int dD = c ? Dp[c > 0 ? c - 1 : 0] : lpD;
-            const int dI = c ? Ip[c > 0 ? c - 1 : 0] : lpI;
-            const int best = max3i(dM, dD, dI);
-            uint32_t srcK = (dM != best) ? ((dD == best) ? K : 2u * K) : 0u;
-            const int sc = (int)__builtin_amdgcn_ubfe(srow, bsh[c], 8) - SBIAS;
-            int Mn = sc + best;
-            if (c == 0 && la == 1 && i == 1) {
-                // one-row quirk: with LA == 1, M(1,1) carries close_A[0] and a 'D' bit
-                Mn = sc + goh;
-                srcK = K;
-            }
-            Mp[c] = Mn;
-            Dp[c] = Dn;
-            word[c >> 3] |= srcK | (tD ? 4u * K : 0u);
-        });
-        // column 0 on row i: M = NEG, I' = NEG + goh; open_B[0] + goh = goh
-        int iL = NEG + goh, mL = NEG;
-        static_for(std::make_integer_sequence<int, TINY_LB>{}, [&](auto ic) {
-            constexpr int c = decltype(ic)::value;
-            constexpr uint32_t K = 1u << (4 * (c & 7));
-            const int mi = mL + (c == 0 ? goh : go2);
-            const bool tI = mi >= iL;
-            iL = max(mi, iL);
-            Ip[c] = iL;
-            mL = Mp[c];
-            word[c >> 3] |= tI ? 8u * K : 0u;
-        });
-        *reinterpret_cast<uint2 *>(tbj + (size_t)(i - 1) * 8) = make_uint2(word[0], word[1]);
-        if (i == la) {
-#pragma unroll
-            for (int c = 0; c < TINY_LB; ++c)
-                if (c == lb - 1) { finM = Mp[c]; finD = Dp[c]; finI = Ip[c]; }
-        }
+        int lo, hi;
+        IntCell::operand(sc, a[i - 1], lo, hi);
+        IntCell::row<TINY_LB>(st, nullptr, lo, hi, diag, IntCell::neg_f());
+        diag = IntCell::edge();
+        store_records<TINY_LB>(tbj + (size_t)(i - 1) * 8, st.word);
     }
-    finD -= goh;
-    finI -= goh;
-    int score = finM, edge = 'M';
-    if (finD > score) { score = finD; edge = 'D'; }
-    if (finI > score) { score = finI; edge = 'I'; }
-    out->score = score;
-    out->edge = edge;
+    int h = 0, e = 0, f = 0;
+#pragma unroll
+    for (int c = 0; c < TINY_LB; ++c)
+        if (c == lb - 1) { h = st.H[c]; e = st.E[c]; f = st.F[c]; }
+    const uint32_t w = lb > 8 ? st.word[1] : st.word[0];
+    IntCell::pick(h, e, f, (w >> (4 * ((lb - 1) & 7))) & 15u, 0, 0, 0, score, edge);
 }
 
-__device__ __forceinline__ int xchar(uint32_t bits, int t)
+__device__ __forceinline__ void put_result(const DevJob &jb, bool ok, int score, int pos, int64_t maxdev,
+                                           mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev)
 {
-    if (t == 'M') { const uint32_t v = bits & 3u; return v == 0 ? 'M' : (v == 1 ? 'D' : (v == 2 ? 'I' : '?')); }
-    if (t == 'D') return (bits & 4u) ? 'M' : 'D';
-    return (bits & 8u) ? 'M' : 'I';
+    mh_dp_result r;
+    r.score = score;
+    r.path_len = ok ? jb.la + jb.lb - (uint32_t)pos : 0u;
+    r.path_start = jb.path_off + (uint64_t)pos;
+    res[jb.user] = r;
+    if (dev) dev[jb.user] = ok ? (uint32_t)((maxdev + jb.la - 1) / jb.la) : 0xFFFFFFFFu;
 }
 
-// BitTraceBack, MU/bittraceback.cpp:138-209: one thread per job walks the
-// trace bits from (LA, LB) and writes the edges backwards into the job's
-// path slot.  It also records the path's largest distance from the
-// corner-to-corner line, ceil(max |i*LB - j*LA| / LA) over the visited
-// positions, which is the band label and the edge test of a banded job.
-__device__ __forceinline__ void traceback_thread_job(const DevJob *__restrict__ jobs,
-                                                     const DpOut *__restrict__ outs,
-                                                     const uint8_t *__restrict__ tb, uint8_t *__restrict__ paths,
-                                                     mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev,
-                                                     uint32_t x)
+// BitTraceBack (MU/bittraceback.cpp:138-209) by the G lanes that computed the
+// job (64 lanes for a job whose stripes other wavefronts computed): the walk
+// from (LA, LB) writes the edges backwards into the job's path slot and records
+// the path's largest distance from the corner-to-corner line, ceil(max |i*LB -
+// j*LA| / LA) over the visited positions, which is the band label and the edge
+// test of a banded job.
+//
+// A step reads the records of the next G positions in the walk's direction (M
+// along the diagonal, D up the column, I along the row) at once, a lane each;
+// a ballot finds the first whose record leaves the state, and the walk moves
+// there.  So it costs one round of loads per run of one state (or per G
+// positions, or stripe), and runs are long: substitutions do not end one, only
+// indels do.  It follows the forward pass on the same wavefront, whose records
+// are still in the L2, while other wavefronts compute.  (20,000 jobs of 5 to 500
+// columns walked by a thread each in a kernel of its own: 424 us after a forward
+// pass of 648 us; together now 407 us.)
+template <int G>
+__device__ __forceinline__ void walk_group(const DevJob &jb, const uint8_t *tb, uint8_t *__restrict__ paths,
+                                           mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev, int score,
+                                           int edge)
 {
-    const DevJob jb = jobs[x];
+    const int lane = (int)threadIdx.x & (G - 1), gb = (int)threadIdx.x & 63 & ~(G - 1);
     const int la = (int)jb.la, lb = (int)jb.lb;
-    // stripe layouts: G lanes per job (16 for the row-packed jobs) of cols columns
-    const bool rows16 = jb.cols > GROUP_TAG && jb.cols < WINDOW_TAG;
-    const int G = rows16 ? 16 : 64;
-    const int cols = rows16 ? (int)(jb.cols - GROUP_TAG) : (int)jb.cols, sw = G * cols, lane_bytes = cols / 2;
+    const int cols = G == 16 ? (int)(jb.cols - GROUP_TAG) : (int)jb.cols, sw = G * cols;
+    const int lane_bytes = (int)lane_bytes_of((uint32_t)cols);
+    const uint32_t inv = (65536u + (uint32_t)cols - 1u) / (uint32_t)cols;   // x / cols = x * inv >> 16 below 4096
     const uint8_t *tj = tb + jb.tb_off;
     uint8_t *slot = paths + jb.path_off;
-    // trace block of the last stripe: the sum over the stripes before it
+    // the trace block of the last stripe: the sum over the stripes before it
     int cur = (lb - 1) / sw, r0 = 1, r1 = 0;
     uint64_t base = 0;
     for (int s = 0; s < cur; ++s) {
@@ -918,253 +1000,178 @@ __device__ __forceinline__ void traceback_thread_job(const DevJob *__restrict__ 
         if (a1 >= a0) base += (uint64_t)(a1 - a0 + G) * G * lane_bytes;
     }
     stripe_rows(jb.la, jb.lb, jb.band, sw, cur, r0, r1);
-    // stripe layout: column j-1 = cur*sw + k*cols + c, tracked without
-    // divisions; dnum = i*lb - j*la, tracked as the walk moves
-    const bool stripes = jb.cols != TINY_COLS_TAG && jb.cols <= WINDOW_TAG;
-    int k = stripes ? ((lb - 1) % sw) / cols : 0, c = stripes ? (lb - 1) % cols : 0;
-    int64_t dnum = 0;
-    int pos = la + lb;
-    int i = la, j = lb;
-    int type = outs[x].edge;
+    int i = la, j = lb, pos = la + lb, type = edge;
+    int co = (lb - 1) - cur * sw;        // j's column in its stripe, from 0
+    int64_t dnum = 0, maxdev = 0;        // i*lb - j*la
     bool ok = true;
-    int64_t maxdev = 0;
-    for (;;) {
-        if (stripes && i > 0 && j > 0) {
-            // Look ahead along the run that keeps the walk's state (M along the
-            // diagonal, D up, I along the row): the bytes of up to TB_AHEAD of
-            // its cells in this stripe are loaded at once, and the walk moves
-            // over all but the last cell that keeps the state (the step below
-            // takes that one), instead of one dependent load per cell.
-            constexpr int TB_AHEAD = 8;
-            uint32_t by[TB_AHEAD], sh[TB_AHEAD];
-            int cnt = 0, kl = k, cc = c;
-            bool go = true;
-#pragma unroll
-            for (int d = 0; d < TB_AHEAD; ++d) {
-                const int ci = i - (type == 'I' ? 0 : d);
-                if (d > 0 && type != 'D' && --cc < 0) {
-                    cc = cols - 1;
-                    if (--kl < 0) go = false;
-                }
-                if (ci < r0 || ci > r1 || ci < 1) go = false;
-                by[d] = 0;
-                sh[d] = 4u * (uint32_t)(cc & 1);
-                if (go) {
-                    by[d] = tj[base + ((uint64_t)(ci - r0 + kl) * G + kl) * lane_bytes + (cc >> 1)];
-                    cnt = d + 1;
-                }
+    while (i > 0 && j > 0) {
+        const int up = type != 'I', left = type != 'D';
+        if (left && co == 0 && cur > 0) {
+            // the next position lies in the previous stripe: back over its trace block
+            --cur;
+            stripe_rows(jb.la, jb.lb, jb.band, sw, cur, r0, r1);
+            if (r1 >= r0) base -= (uint64_t)(r1 - r0 + G) * G * lane_bytes;
+            co = sw;
+        }
+        const int ci = i - (up ? 1 + lane : 0), o = co - (left ? 1 + lane : 0);
+        const bool in = ci >= 1 && ci >= r0 && ci <= r1 && o >= 0;
+        uint32_t nib = 0;
+        if (in) {
+            const int kl = (int)(((uint32_t)o * inv) >> 16), c = o - kl * cols;
+            const uint32_t byte = tj[base + ((uint64_t)(ci - r0 + kl) * G + kl) * lane_bytes + (c >> 1)];
+            nib = (byte >> (4 * (c & 1))) & 15u;
+        }
+        uint64_t vm = __ballot(in), sm = __ballot(in && walk_stays(nib, type));
+        if constexpr (G < 64) {
+            vm = (vm >> gb) & ((1ull << (G & 63)) - 1);
+            sm = (sm >> gb) & ((1ull << (G & 63)) - 1);
+        }
+        const int cnt = ~vm ? __builtin_ctzll(~vm) : 64, n = ~sm ? __builtin_ctzll(~sm) : 64;
+        const uint32_t nn = (uint32_t)__shfl((int)nib, gb + (n < G ? n : 0), 64);
+        int e, next;
+        if (n < cnt) {
+            e = n + 1;
+            next = (int)walk_next(nn, type);
+        } else if (cnt > 0) {
+            e = cnt;
+            next = type;
+        } else {
+            // onto row 0 or column 0 (by an M edge, or along the edge itself), or out of the region
+            e = 1;
+            const int i1 = i - up, j1 = j - left;
+            if ((i1 > 0 && j1 > 0) || (type == 'D' && j1 > 0) || (type == 'I' && i1 > 0)) {
+                ok = false;
+                break;
             }
-            // stay mask over the loaded cells; n = the leading run of ones
-            const uint32_t bit = type == 'M' ? 3u : (type == 'D' ? 4u : 8u);
-            uint32_t mask = 0;
+            next = type;
+        }
+        if (lane < e) slot[pos - 1 - lane] = (uint8_t)type;
+        pos -= e;
+        const int64_t dd = (up ? -(int64_t)lb : 0) + (left ? (int64_t)la : 0);
+        const int64_t d1 = dnum + dd, d2 = dnum + (int64_t)e * dd;
+        maxdev = max(maxdev, max(d1 < 0 ? -d1 : d1, d2 < 0 ? -d2 : d2));
+        dnum = d2;
+        if (up) i -= e;
+        if (left) {
+            j -= e;
+            co -= e;
+        }
+        type = next;
+    }
+    if (ok) {
+        // along the edge to the corner
+        const int rest = i + j;
+        const uint8_t t = i > 0 ? 'D' : 'I';
+        for (int x = lane; x < rest; x += G) slot[pos - 1 - x] = t;
+        pos -= rest;
+    }
+    if (lane == 0) put_result(jb, ok, score, pos, maxdev, res, dev);
+}
+
+// The walk of a one-lane job by its lane, eight positions looked at at once.
+__device__ __forceinline__ void walk_tiny(const DevJob &jb, const uint8_t *tb, uint8_t *__restrict__ paths,
+                                          mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev, int score,
+                                          int edge)
+{
+    constexpr int AHEAD = 8;
+    const int la = (int)jb.la, lb = (int)jb.lb;
+    const uint8_t *tj = tb + jb.tb_off;
+    uint8_t *slot = paths + jb.path_off;
+    int i = la, j = lb, pos = la + lb, type = edge;
+    int64_t dnum = 0, maxdev = 0;
+    bool ok = true;
+    while (i > 0 && j > 0) {
+        const int up = type != 'I', left = type != 'D';
+        uint32_t nib[AHEAD];
 #pragma unroll
-            for (int d = 0; d < TB_AHEAD; ++d)
-                if (d < cnt && ((by[d] >> sh[d]) & bit) == 0u) mask |= 1u << d;
-            const int n = (int)__builtin_ctz(~mask);
-            if (n >= 2) {
-                const int adv = n - 1;
-                for (int d = 0; d < adv; ++d) slot[pos - 1 - d] = (uint8_t)type;
-                pos -= adv;
-                const int64_t st = type == 'M' ? (int64_t)la - lb : (type == 'D' ? -(int64_t)lb : (int64_t)la);
-                const int64_t d1 = dnum + st, d2 = dnum + (int64_t)adv * st;
-                maxdev = max(maxdev, max(d1 < 0 ? -d1 : d1, d2 < 0 ? -d2 : d2));
-                dnum = d2;
-                if (type != 'I') i -= adv;
-                if (type != 'D') {
-                    j -= adv;
-                    for (int d = 0; d < adv; ++d)
-                        if (--c < 0) {
-                            c = cols - 1;
-                            --k;
-                        }
-                }
+        for (int d = 0; d < AHEAD; ++d) {
+            const int ci = i - up * (1 + d), cj = j - left * (1 + d);
+            nib[d] = 16;
+            if (ci >= 1 && cj >= 1) nib[d] = ((uint32_t)tj[(uint64_t)(ci - 1) * 8 + ((cj - 1) >> 1)] >> (4 * ((cj - 1) & 1))) & 15u;
+        }
+        int e = 0, next = type;
+        bool stay = true;
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d)
+            if (stay && nib[d] < 16) {
+                ++e;
+                stay = walk_stays(nib[d], type);
+                if (!stay) next = (int)walk_next(nib[d], type);
+            } else {
+                stay = false;
+            }
+        if (e == 0) {
+            e = 1;
+            const int i1 = i - up, j1 = j - left;
+            if ((type == 'D' && j1 > 0) || (type == 'I' && i1 > 0)) {
+                ok = false;
+                break;
             }
         }
+        for (int d = 0; d < e; ++d) slot[pos - 1 - d] = (uint8_t)type;
+        pos -= e;
+        const int64_t dd = (up ? -(int64_t)lb : 0) + (left ? (int64_t)la : 0);
+        const int64_t d1 = dnum + dd, d2 = dnum + (int64_t)e * dd;
+        maxdev = max(maxdev, max(d1 < 0 ? -d1 : d1, d2 < 0 ? -d2 : d2));
+        dnum = d2;
+        i -= up * e;
+        j -= left * e;
+        type = next;
+    }
+    if (ok) {
+        const uint8_t t = i > 0 ? 'D' : 'I';
+        for (int rest = i + j; rest > 0; --rest) slot[--pos] = t;
+    }
+    put_result(jb, ok, score, pos, maxdev, res, dev);
+}
+
+// The walk of a sliding-window job by one lane; its records are the
+// reference's code at the cell the walk leaves (dp_window_job).
+__device__ __forceinline__ void walk_window(const DevJob &jb, const uint8_t *tb, uint8_t *__restrict__ paths,
+                                            mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev, int score,
+                                            int edge)
+{
+    const int la = (int)jb.la, lb = (int)jb.lb;
+    const uint32_t *tj = reinterpret_cast<const uint32_t *>(tb + jb.tb_off);
+    uint8_t *slot = paths + jb.path_off;
+    const int C = (int)jb.cols - (int)WINDOW_TAG, rpd = 8 / C;
+    int pos = la + lb, i = la, j = lb, type = edge;
+    int64_t dnum = 0, maxdev = 0;
+    bool ok = true;
+    for (;;) {
         slot[--pos] = (uint8_t)type;
         uint32_t nib = 0;
         if (i > 0 && j > 0) {
-            if (jb.cols == TINY_COLS_TAG) {
-                const uint8_t byte = tj[(uint64_t)(i - 1) * 8 + ((j - 1) >> 1)];
-                nib = (byte >> (4 * ((j - 1) & 1))) & 15u;
-            } else if (jb.cols > WINDOW_TAG) {
-                const int C = (int)jb.cols - (int)WINDOW_TAG, rpd = 8 / C;
-                const int xw = j - window_base(la, lb, 64 * C, i) - 1;
-                if (xw < 0 || xw >= 64 * C) { ok = false; break; }
-                const uint32_t w = reinterpret_cast<const uint32_t *>(tj)[(uint64_t)((i - 1) / rpd) * 64 + xw / C];
-                nib = (w >> (4 * (C * ((i - 1) % rpd) + xw % C))) & 15u;
-            } else {
-                if (i < r0 || i > r1) { ok = false; break; }
-                const uint8_t byte = tj[base + ((uint64_t)(i - r0 + k) * G + k) * lane_bytes + (c >> 1)];
-                nib = (byte >> (4 * (c & 1))) & 15u;
-            }
+            const int xw = j - window_base(la, lb, 64 * C, i) - 1;
+            if (xw < 0 || xw >= 64 * C) { ok = false; break; }
+            const uint32_t w = tj[(uint64_t)((i - 1) / rpd) * 64 + xw / C];
+            nib = (w >> (4 * (C * ((i - 1) % rpd) + xw % C))) & 15u;
         }
-        const int nx = xchar(nib, type);
-        bool left = false;
-        if (type == 'M') { if (i == 0 || j == 0) { ok = false; break; } --i; --j; dnum += (int64_t)la - lb; left = true; }
-        else if (type == 'D') { if (i == 0) { ok = false; break; } --i; dnum -= lb; }
-        else { if (j == 0) { ok = false; break; } --j; dnum += la; left = true; }
-        if (stripes && left && j > 0 && --c < 0) {
-            c = cols - 1;
-            if (--k < 0) {   // into the previous stripe: step back over its trace block
-                k = G - 1;
-                --cur;
-                stripe_rows(jb.la, jb.lb, jb.band, sw, cur, r0, r1);
-                if (r1 >= r0) base -= (uint64_t)(r1 - r0 + G) * G * lane_bytes;
-            }
+        int nx;
+        if (type == 'M') {
+            const uint32_t v = nib & 3u;
+            nx = v == 0 ? 'M' : (v == 1 ? 'D' : (v == 2 ? 'I' : '?'));
+            if (i == 0 || j == 0) { ok = false; break; }
+            --i;
+            --j;
+            dnum += (int64_t)la - lb;
+        } else if (type == 'D') {
+            nx = (nib & 4u) ? 'M' : 'D';
+            if (i == 0) { ok = false; break; }
+            --i;
+            dnum -= lb;
+        } else {
+            nx = (nib & 8u) ? 'M' : 'I';
+            if (j == 0) { ok = false; break; }
+            --j;
+            dnum += la;
         }
         maxdev = max(maxdev, dnum < 0 ? -dnum : dnum);
         if (i == 0 && j == 0) break;
         if (pos == 0 || nx == '?') { ok = false; break; }
         type = nx;
     }
-    mh_dp_result r;
-    r.score = outs[x].score;
-    r.path_len = ok ? (uint32_t)(la + lb - pos) : 0u;
-    r.path_start = jb.path_off + (uint64_t)pos;
-    res[jb.user] = r;
-    if (dev) dev[jb.user] = ok ? (uint32_t)((maxdev + la - 1) / la) : 0xFFFFFFFFu;
-}
-
-// The same trace-back for stripe-layout jobs by one wavefront per job.  The
-// walk itself is sequential (all lanes run it in step), but its trace bytes
-// come from LDS: the wave loads a tile of 128 steps x 128 columns of the
-// current stripe (128 segments of 64 contiguous bytes, 16-byte aligned) in
-// one round of loads and refills it only when the walk leaves it, which
-// replaces a dependent global load per step with one per ~100 steps.
-constexpr int TBC_STEPS = 128, TBC_SEG = 64;
-constexpr uint32_t WAVE_WALK_MIN = 1024;   // a + b above which a job's walk gets a wavefront
-
-__device__ __forceinline__ void traceback_wave_job(const DevJob *__restrict__ jobs, const DpOut *__restrict__ outs,
-                                                   const uint8_t *__restrict__ tb, uint8_t *__restrict__ paths,
-                                                   mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev,
-                                                   uint32_t x, uint8_t *__restrict__ cache)
-{
-    const int lane = threadIdx.x;
-    const DevJob jb = jobs[x];
-    const int la = (int)jb.la, lb = (int)jb.lb;
-    // G lanes a step: 64, or 16 for the row-packed layout
-    const bool rows16 = jb.cols > GROUP_TAG;
-    const int G = rows16 ? 16 : 64;
-    const int cols = rows16 ? (int)(jb.cols - GROUP_TAG) : (int)jb.cols, sw = G * cols, lane_bytes = cols / 2;
-    const int K = TBC_SEG / lane_bytes < G ? TBC_SEG / lane_bytes : G;   // lanes a cached step holds
-    const int P = K * lane_bytes / 16;                                   // 16-byte parts a cached step
-    const int kalign = 16 / lane_bytes;      // segment starts on a 16-byte boundary
-    const uint8_t *tj = tb + jb.tb_off;
-    uint8_t *slot = paths + jb.path_off;
-    int cur = (lb - 1) / sw, r0 = 1, r1 = 0;
-    uint64_t base = 0;
-    for (int s = 0; s < cur; ++s) {
-        int a0, a1;
-        stripe_rows(jb.la, jb.lb, jb.band, sw, s, a0, a1);
-        if (a1 >= a0) base += (uint64_t)(a1 - a0 + G) * G * lane_bytes;
-    }
-    stripe_rows(jb.la, jb.lb, jb.band, sw, cur, r0, r1);
-    int c_s = -1, c_tlo = 0, c_thi = -1, c_klo = 0;   // cached stripe, steps and first lane
-    const int kshift = kalign == 2 ? 1 : (kalign == 4 ? 2 : 3);
-    // column j-1 = cur*sw + k*cols + c, tracked without divisions; dnum =
-    // i*lb - j*la, tracked as the walk moves
-    int k = ((lb - 1) % sw) / cols, c = (lb - 1) % cols;
-    int64_t dnum = 0;
-    int pos = la + lb;
-    int i = la, j = lb;
-    int type = outs[x].edge;
-    bool ok = true;
-    int64_t maxdev = 0;
-    const int cshift = cols == 4 ? 2 : (cols == 8 ? 3 : 4);
-    for (;;) {
-        // A run of cells that keep the walk's state (M from M along the
-        // diagonal, D from D up the column, I from I along the row): lane l
-        // reads the l-th cell of the run from the cached tile, and the walk
-        // moves over all but the last good cell at once (the step below takes
-        // that one, so the run never leaves the stripe or the tile).
-        if (i > 0 && j > 0 && cur == c_s) {
-            const int ci = i - (type == 'I' ? 0 : lane);
-            const int off = k * cols + c - (type == 'D' ? 0 : lane);
-            bool good = ci >= r0 && ci <= r1 && ci >= 1 && off >= 0;
-            if (good) {
-                const int kl = off >> cshift, cl = off & (cols - 1);
-                const int t = ci - r0 + kl;
-                good = t >= c_tlo && t <= c_thi && kl >= c_klo && kl < c_klo + K;
-                if (good) {
-                    const uint32_t nb =
-                        ((uint32_t)cache[(t - c_tlo) * TBC_SEG + (kl - c_klo) * lane_bytes + (cl >> 1)] >>
-                         (4 * (cl & 1))) & 15u;
-                    good = type == 'M' ? (nb & 3u) == 0u : (type == 'D' ? (nb & 4u) == 0u : (nb & 8u) == 0u);
-                }
-            }
-            const uint64_t bad = __ballot(!good);
-            const int n = bad ? (int)__builtin_ctzll(bad) : 64;
-            if (n >= 2) {
-                const int adv = n - 1;
-                if (lane < adv) slot[pos - 1 - lane] = (uint8_t)type;
-                pos -= adv;
-                const int64_t st = type == 'M' ? (int64_t)la - lb : (type == 'D' ? -(int64_t)lb : (int64_t)la);
-                const int64_t d1 = dnum + st, d2 = dnum + (int64_t)adv * st;
-                maxdev = max(maxdev, max(d1 < 0 ? -d1 : d1, d2 < 0 ? -d2 : d2));
-                dnum = d2;
-                if (type != 'I') i -= adv;
-                if (type != 'D') {
-                    j -= adv;
-                    const int o = k * cols + c - adv;
-                    k = o >> cshift;
-                    c = o & (cols - 1);
-                }
-            }
-        }
-        --pos;
-        if (lane == 0) slot[pos] = (uint8_t)type;
-        uint32_t nib = 0;
-        if (i > 0 && j > 0) {
-            if (i < r0 || i > r1) { ok = false; break; }
-            const int t = i - r0 + k;
-            if (cur != c_s || t < c_tlo || t > c_thi || k < c_klo || k >= c_klo + K) {
-                c_s = cur;
-                c_thi = t;
-                c_tlo = t - TBC_STEPS + 1 < 0 ? 0 : t - TBC_STEPS + 1;
-                const int kl = (((k >> kshift) + 1) << kshift) - K;
-                c_klo = kl < 0 ? 0 : kl;
-                const int nseg = c_thi - c_tlo + 1;
-                __syncthreads();
-                for (int e = lane; e < nseg * P; e += 64) {
-                    const int seg = e / P, part = e - seg * P;
-                    const uint8_t *src = tj + base + ((uint64_t)(c_tlo + seg) * G + c_klo) * lane_bytes + part * 16;
-                    *reinterpret_cast<uint4 *>(cache + seg * TBC_SEG + part * 16) = *reinterpret_cast<const uint4 *>(src);
-                }
-                __syncthreads();
-            }
-            // one LDS byte read by every lane; made wave-uniform so the walk's
-            // bookkeeping runs on the scalar unit
-            const uint32_t byte = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)cache[(t - c_tlo) * TBC_SEG + (k - c_klo) * lane_bytes + (c >> 1)]);
-            nib = (byte >> (4 * (c & 1))) & 15u;
-        }
-        const int nx = xchar(nib, type);
-        bool left = false;
-        if (type == 'M') { if (i == 0 || j == 0) { ok = false; break; } --i; --j; dnum += (int64_t)la - lb; left = true; }
-        else if (type == 'D') { if (i == 0) { ok = false; break; } --i; dnum -= lb; }
-        else { if (j == 0) { ok = false; break; } --j; dnum += la; left = true; }
-        if (left && j > 0 && --c < 0) {
-            c = cols - 1;
-            if (--k < 0) {   // into the previous stripe: step back over its trace block
-                k = G - 1;
-                --cur;
-                stripe_rows(jb.la, jb.lb, jb.band, sw, cur, r0, r1);
-                if (r1 >= r0) base -= (uint64_t)(r1 - r0 + G) * G * lane_bytes;
-            }
-        }
-        maxdev = max(maxdev, dnum < 0 ? -dnum : dnum);
-        if (i == 0 && j == 0) break;
-        if (pos == 0 || nx == '?') { ok = false; break; }
-        type = nx;
-    }
-    if (lane == 0) {
-        mh_dp_result r;
-        r.score = outs[x].score;
-        r.path_len = ok ? (uint32_t)(la + lb - pos) : 0u;
-        r.path_start = jb.path_off + (uint64_t)pos;
-        res[jb.user] = r;
-        if (dev) dev[jb.user] = ok ? (uint32_t)((maxdev + la - 1) / la) : 0xFFFFFFFFu;
-    }
+    put_result(jb, ok, score, pos, maxdev, res, dev);
 }
 
 // ---- the round's launches ------------------------------------------------
@@ -1175,78 +1182,89 @@ __global__ __launch_bounds__(64) void dp_queue_reset(uint32_t *__restrict__ curs
 }
 
 // The forward kernels' arguments: every pointer restrict-qualified (so that
-// job records and the bin table are read with scalar loads), the bin table in
-// the round's descriptor.
+// job records and the bin table are read with scalar loads; the walk reads the
+// trace the same wavefront wrote, through tb itself), the bin table in the
+// round's descriptor.
 #define DP_FWD_PARAMS                                                                                            \
     const DevJob *__restrict__ jobs, DpOut *__restrict__ outs, const uint8_t *__restrict__ A,                      \
-        const uint8_t *__restrict__ B, uint8_t *__restrict__ tb, int *__restrict__ bnd,                          \
-        const DpRound *__restrict__ rd, uint32_t *__restrict__ cursor, uint32_t sr0, uint32_t sr1, uint32_t sr2, \
-        uint32_t sr3, int goh
-#define DP_FWD_ARGS jobs, outs, A, B, tb, bnd, rd, cursor, sr0, sr1, sr2, sr3, goh
+        const uint8_t *__restrict__ B, uint8_t *tb, int *__restrict__ bnd, const DpRound *__restrict__ rd,       \
+        uint32_t *__restrict__ cursor, uint8_t *__restrict__ paths, mh_dp_result *__restrict__ res,              \
+        uint32_t *__restrict__ dev, ScoreArgs sc
+#define DP_FWD_ARGS jobs, outs, A, B, tb, bnd, rd, cursor, paths, res, dev, sc
 
-template <int MAXC>
-__device__ __forceinline__ void run_item(DP_FWD_PARAMS, uint32_t kind, uint32_t first, uint32_t count,
-                                         uint32_t item, int (*lds_in)[64], int (*lds_out)[64])
+// one work item: the forward pass of its jobs and their walks (a pipelined
+// part only its stripes; the job's walk waits for the others, dp_tb_wave)
+template <class CELL, int MAXC>
+__device__ __forceinline__ void run_item(DP_FWD_PARAMS, const float *table, uint32_t kind, uint32_t first,
+                                         uint32_t count, uint32_t item, DpLds &lds)
 {
+    int score = 0, edge = 'M';
     if (kind >= QK_PIPE) {
         const uint32_t P = kind - QK_PIPE + 2;
         const uint32_t x = first + item / P;
         const int p0 = (int)(item % P);
         const DevJob jb = jobs[x];
         uint32_t *err = cursor + (DPQ_CURSORS - 1);
-        if constexpr (MAXC >= 16) {
-            if (jb.cols == 16) {
-                dp_job<16, 64, true>(jb, A, B, tb, bnd, &outs[x], sr0, sr1, sr2, sr3, goh, lds_in, lds_out, p0, (int)P,
-                                     err);
-                return;
-            }
+        bool fin = false;
+        if (MAXC >= 16 && jb.cols == 16) {
+            if constexpr (MAXC >= 16)
+                fin = dp_job<CELL, 16, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
+        } else if (jb.cols == 8) {
+            fin = dp_job<CELL, 8, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
+        } else {
+            fin = dp_job<CELL, 4, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
         }
-        if (jb.cols == 8)
-            dp_job<8, 64, true>(jb, A, B, tb, bnd, &outs[x], sr0, sr1, sr2, sr3, goh, lds_in, lds_out, p0, (int)P,
-                                err);
-        else
-            dp_job<4, 64, true>(jb, A, B, tb, bnd, &outs[x], sr0, sr1, sr2, sr3, goh, lds_in, lds_out, p0, (int)P,
-                                err);
+        if (fin && threadIdx.x == 0) {
+            outs[x].score = score;
+            outs[x].edge = edge;
+        }
     } else if (kind == QK_STRIPE) {
-        const uint32_t x = first + item;
-        const DevJob jb = jobs[x];
-        if constexpr (MAXC >= 16) {
-            if (jb.cols == 16) {
-                dp_job<16, 64>(jb, A, B, tb, bnd, &outs[x], sr0, sr1, sr2, sr3, goh, lds_in, lds_out);
-                return;
-            }
+        const DevJob jb = jobs[first + item];
+        if (MAXC >= 16 && jb.cols == 16) {
+            if constexpr (MAXC >= 16) dp_job<CELL, 16, 64>(jb, A, B, tb, bnd, sc, table, lds, score, edge);
+        } else if (jb.cols == 8) {
+            dp_job<CELL, 8, 64>(jb, A, B, tb, bnd, sc, table, lds, score, edge);
+        } else {
+            dp_job<CELL, 4, 64>(jb, A, B, tb, bnd, sc, table, lds, score, edge);
         }
-        if (jb.cols == 8)
-            dp_job<8, 64>(jb, A, B, tb, bnd, &outs[x], sr0, sr1, sr2, sr3, goh, lds_in, lds_out);
-        else
-            dp_job<4, 64>(jb, A, B, tb, bnd, &outs[x], sr0, sr1, sr2, sr3, goh, lds_in, lds_out);
+        walk_group<64>(jb, tb, paths, res, dev, score, edge);
     } else if (kind == QK_WINDOW) {
-        const uint32_t x = first + item;
-        const DevJob jb = jobs[x];
-        switch (jb.cols - WINDOW_TAG) {
-        case 1: dp_window_job<1>(jb, A, B, tb, &outs[x], sr0, sr1, sr2, sr3, goh); break;
-        case 2: dp_window_job<2>(jb, A, B, tb, &outs[x], sr0, sr1, sr2, sr3, goh); break;
-        case 4: dp_window_job<4>(jb, A, B, tb, &outs[x], sr0, sr1, sr2, sr3, goh); break;
-        default: dp_window_job<8>(jb, A, B, tb, &outs[x], sr0, sr1, sr2, sr3, goh); break;
+        if constexpr (std::is_same<CELL, IntCell>::value) {
+            const DevJob jb = jobs[first + item];
+            switch (jb.cols - WINDOW_TAG) {
+            case 1: dp_window_job<1>(jb, A, B, tb, sc, score, edge); break;
+            case 2: dp_window_job<2>(jb, A, B, tb, sc, score, edge); break;
+            case 4: dp_window_job<4>(jb, A, B, tb, sc, score, edge); break;
+            default: dp_window_job<8>(jb, A, B, tb, sc, score, edge); break;
+            }
+            __threadfence_block();
+            if (threadIdx.x == 63) walk_window(jb, tb, paths, res, dev, score, edge);
         }
     } else if (kind == QK_TINY) {
-        const uint32_t x = first + item * 64 + threadIdx.x;
-        if (x < first + count) tiny_job(jobs[x], A, B, tb, &outs[x], sr0, sr1, sr2, sr3, goh);
+        if constexpr (std::is_same<CELL, IntCell>::value) {
+            const uint32_t x = first + item * 64 + threadIdx.x;
+            if (x < first + count) {
+                const DevJob jb = jobs[x];
+                tiny_job(jb, A, B, tb, sc, score, edge);
+                __threadfence_block();
+                walk_tiny(jb, tb, paths, res, dev, score, edge);
+            }
+        }
     } else {
         // four jobs of one shape, one per 16-lane row; a row past the bin's end sits out
         const uint32_t x = first + item * 4 + (threadIdx.x >> 4);
         if (x >= first + count) return;
         const DevJob jb = jobs[x];
-        DpOut *o = &outs[x];
         switch (kind - QK_ROWS) {
-        case 0: if constexpr (MAXC >= 16) dp_job<16, 16>(jb, A, B, tb, bnd, o, sr0, sr1, sr2, sr3, goh, lds_in, lds_out); break;
-        case 1: if constexpr (MAXC >= 14) dp_job<14, 16>(jb, A, B, tb, bnd, o, sr0, sr1, sr2, sr3, goh, lds_in, lds_out); break;
-        case 2: if constexpr (MAXC >= 12) dp_job<12, 16>(jb, A, B, tb, bnd, o, sr0, sr1, sr2, sr3, goh, lds_in, lds_out); break;
-        case 3: if constexpr (MAXC >= 10) dp_job<10, 16>(jb, A, B, tb, bnd, o, sr0, sr1, sr2, sr3, goh, lds_in, lds_out); break;
-        case 4: dp_job<8, 16>(jb, A, B, tb, bnd, o, sr0, sr1, sr2, sr3, goh, lds_in, lds_out); break;
-        case 5: dp_job<6, 16>(jb, A, B, tb, bnd, o, sr0, sr1, sr2, sr3, goh, lds_in, lds_out); break;
-        default: dp_job<4, 16>(jb, A, B, tb, bnd, o, sr0, sr1, sr2, sr3, goh, lds_in, lds_out); break;
+        case 0: if constexpr (MAXC >= 16) dp_job<CELL, 16, 16>(jb, A, B, tb, bnd, sc, table, lds, score, edge); break;
+        case 1: if constexpr (MAXC >= 14) dp_job<CELL, 14, 16>(jb, A, B, tb, bnd, sc, table, lds, score, edge); break;
+        case 2: if constexpr (MAXC >= 12) dp_job<CELL, 12, 16>(jb, A, B, tb, bnd, sc, table, lds, score, edge); break;
+        case 3: if constexpr (MAXC >= 10) dp_job<CELL, 10, 16>(jb, A, B, tb, bnd, sc, table, lds, score, edge); break;
+        case 4: dp_job<CELL, 8, 16>(jb, A, B, tb, bnd, sc, table, lds, score, edge); break;
+        case 5: dp_job<CELL, 6, 16>(jb, A, B, tb, bnd, sc, table, lds, score, edge); break;
+        default: dp_job<CELL, 4, 16>(jb, A, B, tb, bnd, sc, table, lds, score, edge); break;
         }
+        walk_group<16>(jb, tb, paths, res, dev, score, edge);
     }
 }
 
@@ -1258,11 +1276,17 @@ __device__ __forceinline__ void run_item(DP_FWD_PARAMS, uint32_t kind, uint32_t 
 // (workgroup w takes item w; workgroups start in that order), which needs no
 // cursor.  The host picks the variant a round's shapes allow, by the tuning
 // table.
-template <int MAXC, int WPE, bool PERSIST>
+template <class CELL, int MAXC, int WPE, bool PERSIST>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void dp_fwd(DP_FWD_PARAMS)
 {
-    __shared__ int lds_in[4][64];
-    __shared__ int lds_out[3][64];
+    __shared__ DpLds lds;
+    __shared__ float table_s[DP_NCLASS * DP_NCLASS];
+    const float *table = nullptr;
+    if constexpr (!std::is_same<CELL, IntCell>::value) {
+        if (threadIdx.x < DP_NCLASS * DP_NCLASS) table_s[threadIdx.x] = rd->table[threadIdx.x];
+        __syncthreads();
+        table = table_s;
+    }
     const uint32_t nb = rd->nbins;
     if constexpr (!PERSIST) {
         const uint32_t w = blockIdx.x;
@@ -1277,7 +1301,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
             if (threadIdx.x == 0) v = atomicAdd(&cursor[b], 1u);
             item = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
         }
-        run_item<MAXC>(DP_FWD_ARGS, rd->kind[b], rd->first[b], rd->count[b], item, lds_in, lds_out);
+        run_item<CELL, MAXC>(DP_FWD_ARGS, table, rd->kind[b], rd->first[b], rd->count[b], item, lds);
     } else {
         uint32_t b = 0;
         for (;;) {
@@ -1290,47 +1314,40 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                 if ((uint64_t)item * qk_per_item(rd->kind[b]) < rd->count[b]) break;
             }
             if (b >= nb) return;
-            run_item<MAXC>(DP_FWD_ARGS, rd->kind[b], rd->first[b], rd->count[b], item, lds_in, lds_out);
+            run_item<CELL, MAXC>(DP_FWD_ARGS, table, rd->kind[b], rd->first[b], rd->count[b], item, lds);
         }
     }
 }
 
-// Trace-backs: the jobs with long walks a wavefront each (workgroup x walks
-// job x), the others a thread each.  Their pointers come as arguments (not
-// from the round's descriptor): with every pointer restrict-qualified the
-// walk's job record is read with scalar loads and its bookkeeping stays on the
-// scalar unit.
+// The walks of the pipelined jobs (the first npipe of the table), a wavefront
+// each, once the forward launch has ended.
 __global__ __launch_bounds__(64) void dp_tb_wave(const DevJob *__restrict__ jobs, const DpOut *__restrict__ outs,
                                                  const uint8_t *__restrict__ tb, uint8_t *__restrict__ paths,
                                                  mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev,
-                                                 const uint32_t *__restrict__ idx, uint32_t nwave)
+                                                 uint32_t npipe)
 {
-    __shared__ __align__(16) uint8_t cache[TBC_STEPS * TBC_SEG];
-    if (blockIdx.x >= nwave) return;
-    traceback_wave_job(jobs, outs, tb, paths, res, dev, idx[blockIdx.x], cache);
+    if (blockIdx.x >= npipe) return;
+    const DevJob jb = jobs[blockIdx.x];
+    walk_group<64>(jb, tb, paths, res, dev, outs[blockIdx.x].score, outs[blockIdx.x].edge);
 }
 
-__global__ __launch_bounds__(64) void dp_tb_thread(const DevJob *__restrict__ jobs, const DpOut *__restrict__ outs,
-                                                   const uint8_t *__restrict__ tb, uint8_t *__restrict__ paths,
-                                                   mh_dp_result *__restrict__ res, uint32_t *__restrict__ dev,
-                                                   const uint32_t *__restrict__ idx, uint32_t first, uint32_t n)
-{
-    const uint32_t t = first + blockIdx.x * 64 + threadIdx.x;
-    if (t >= n) return;
-    traceback_thread_job(jobs, outs, tb, paths, res, dev, idx[t]);
-}
-
-// NUC_SP (MU/nucmx.cpp:8-25) rows packed as biased bytes: row a, column b at
-// bits [8b, 8b+8) holding NUC_SP[a][b] + 65.
-void packed_rows(uint32_t r[4])
+// NUC_SP (MU/nucmx.cpp:8-25) as the kernels take it (ScoreArgs)
+void packed_rows(ScoreArgs &sc)
 {
     static const int hoxd[4][4] = {{91, -114, -31, -123},
                                    {-114, 100, -125, -31},
                                    {-31, -125, 100, -114},
                                    {-123, -31, -114, 91}};
     for (int a = 0; a < 4; ++a) {
-        r[a] = 0;
-        for (int b = 0; b < 4; ++b) r[a] |= (uint32_t)(hoxd[a][b] + 60 + SBIAS) << (8 * b);
+        uint32_t h[4];
+        sc.sr[a] = 0;
+        for (int b = 0; b < 4; ++b) {
+            const int v = hoxd[a][b] + 60;
+            sc.sr[a] |= (uint32_t)(v + SBIAS) << (8 * b);
+            h[b] = (uint32_t)(uint16_t)(int16_t)(4 * v);
+        }
+        sc.lo[a] = h[0] | (h[1] << 16);
+        sc.hi[a] = h[2] | (h[3] << 16);
     }
 }
 
@@ -1343,6 +1360,7 @@ struct DpItem {
     uint32_t band;    // 0 = full matrix
     uint32_t cols;
     uint64_t tb_bytes;
+    uint64_t cells;   // of the region evaluated, padding included
 };
 
 // Relative cost per computed cell of the stripe shapes, used to pick a banded
@@ -1556,17 +1574,28 @@ struct FwdVariant {
     int maxc, wpe;
     bool persist;
 };
+#define MH_FWD(CELL, MAXC, WPE, PERSIST) \
+    {reinterpret_cast<const void *>(&dp_fwd<CELL, MAXC, WPE, PERSIST>), MAXC, WPE, PERSIST}
 const FwdVariant FWD_VARIANTS[] = {
-    {reinterpret_cast<const void *>(&dp_fwd<16, 3, false>), 16, 3, false},
-    {reinterpret_cast<const void *>(&dp_fwd<8, 4, false>), 8, 4, false},
-    {reinterpret_cast<const void *>(&dp_fwd<16, 2, false>), 16, 2, false},
-    {reinterpret_cast<const void *>(&dp_fwd<16, 3, true>), 16, 3, true},
-    {reinterpret_cast<const void *>(&dp_fwd<16, 2, true>), 16, 2, true},
-    {reinterpret_cast<const void *>(&dp_fwd<8, 4, true>), 8, 4, true},
-    {reinterpret_cast<const void *>(&dp_fwd<16, 4, false>), 16, 4, false},
+    MH_FWD(IntCell, 16, 3, false), MH_FWD(IntCell, 8, 4, false), MH_FWD(IntCell, 16, 2, false),
+    MH_FWD(IntCell, 16, 3, true),  MH_FWD(IntCell, 16, 2, true), MH_FWD(IntCell, 8, 4, true),
+    MH_FWD(IntCell, 16, 4, false),
+    // jobs whose scores times four could leave 32 bits
+    MH_FWD(CmpCell<int>, 16, 2, false),
 };
-constexpr int N_FWD_VARIANTS = (int)(sizeof(FWD_VARIANTS) / sizeof(FWD_VARIANTS[0]));
-static_assert(N_FWD_VARIANTS <= MH_DP_MAX_VARIANTS, "context graph slots");
+#undef MH_FWD
+constexpr int N_ALL_VARIANTS = (int)(sizeof(FWD_VARIANTS) / sizeof(FWD_VARIANTS[0]));
+constexpr int N_FWD_VARIANTS = N_ALL_VARIANTS - 1;   // of the tagged int32 cells
+constexpr int VARIANT_LONG = N_FWD_VARIANTS;
+static_assert(N_ALL_VARIANTS <= MH_DP_MAX_VARIANTS, "context graph slots");
+
+// The cells a run of jobs takes: tagged int32 (values times four), int32
+// without a tag.  The tagged form holds |score| < 2^28: a score is at
+// most 160 a position of the shorter operand, and a reachable cell of a band at
+// least -65 a position, so 225 * 2^20 < 2^28 keeps both apart from minus
+// infinity.  Longer jobs (only banded ones can be) keep untagged values.
+enum class DpCells { TAGGED, LONG };
+constexpr uint32_t TAGGED_MAX = 1u << 20;
 static_assert(DP_TUNE_WIDE_VARIANT < N_FWD_VARIANTS && DP_TUNE_NARROW_VARIANT < N_FWD_VARIANTS, "tuning table");
 
 static int dp_variant_for(bool wide)
@@ -1608,13 +1637,8 @@ static int resident_grid(mh_context *ctx, const void *fn, unsigned *grid)
     return MH_OK;
 }
 
-// grid sizes of a round: forward (items, or the resident grid of a
-// persistent variant), wavefront trace-backs, thread trace-backs
-struct RoundGrids {
-    unsigned fwd, tbw, tbt;
-};
-
-static int round_grids(mh_context *ctx, int v, uint64_t items, uint32_t nwave, uint32_t n, RoundGrids *g)
+// forward grid of a round: its items, or the resident grid of a persistent variant
+static int fwd_grid(mh_context *ctx, int v, uint64_t items, unsigned *g)
 {
     if (FWD_VARIANTS[v].persist) {
         if (!ctx->dp_fwd_grid[v]) {
@@ -1623,18 +1647,16 @@ static int round_grids(mh_context *ctx, int v, uint64_t items, uint32_t nwave, u
             if ((rc = resident_grid(ctx, FWD_VARIANTS[v].fn, &r)) != MH_OK) return rc;
             ctx->dp_fwd_grid[v] = r;
         }
-        g->fwd = ctx->dp_fwd_grid[v];
+        *g = ctx->dp_fwd_grid[v];
     } else {
         MH_CHECK(items < (1ull << 31), MH_ERR_INVALID, "too many DP work items in one round");
-        g->fwd = (unsigned)std::max<uint64_t>(1, items);
+        *g = (unsigned)std::max<uint64_t>(1, items);
     }
-    g->tbw = std::max(1u, nwave);
-    g->tbt = std::max(1u, (n - nwave + 63) / 64);
     return MH_OK;
 }
 
-// the forward kernels' arguments of a round (DP_FWD_PARAMS)
-struct FwdArgs {
+// the kernels' arguments of a round (DP_FWD_PARAMS; dp_tb_wave)
+struct RoundArgs {
     const DevJob *jobs;
     DpOut *outs;
     const uint8_t *A, *B;
@@ -1642,52 +1664,34 @@ struct FwdArgs {
     int *bnd;
     const DpRound *rd;
     uint32_t *cursor;
-    uint32_t sr0, sr1, sr2, sr3;
-    int goh;
-    void *args[13];
+    uint8_t *paths;
+    mh_dp_result *res;
+    uint32_t *dev;
+    ScoreArgs sc;
+    uint32_t npipe;
+    void *fwd[12], *walk[7];
     void set()
     {
-        void *a[13] = {&jobs, &outs, &A, &B, &tb, &bnd, &rd, &cursor, &sr0, &sr1, &sr2, &sr3, &goh};
-        std::memcpy(args, a, sizeof(a));
+        void *a[12] = {&jobs, &outs, &A, &B, &tb, &bnd, &rd, &cursor, &paths, &res, &dev, &sc};
+        void *w[7] = {&jobs, &outs, &tb, &paths, &res, &dev, &npipe};
+        std::memcpy(fwd, a, sizeof(a));
+        std::memcpy(walk, w, sizeof(w));
     }
 };
 
-static int launch_fwd(mh_context *ctx, FwdArgs &a, int v, unsigned grid)
+static int launch_fwd(mh_context *ctx, RoundArgs &a, int v, unsigned grid)
 {
     a.set();
     hipLaunchKernelGGL(dp_queue_reset, dim3(1), dim3(64), 0, ctx->stream, a.cursor);
-    MH_HIP(hipLaunchKernel(FWD_VARIANTS[v].fn, dim3(grid), dim3(64), a.args, 0, ctx->stream));
+    MH_HIP(hipLaunchKernel(FWD_VARIANTS[v].fn, dim3(grid), dim3(64), a.fwd, 0, ctx->stream));
     MH_HIP(hipGetLastError());
     return MH_OK;
 }
 
-// the trace-back kernels' arguments of a round
-struct TbArgs {
-    const DevJob *jobs;
-    const DpOut *outs;
-    const uint8_t *tb;
-    uint8_t *paths;
-    mh_dp_result *res;
-    uint32_t *dev;
-    const uint32_t *idx;
-    uint32_t nwave, first, n;
-    void *wave[8];
-    void *thread[9];
-    void set()
-    {
-        void *w[8] = {&jobs, &outs, &tb, &paths, &res, &dev, &idx, &nwave};
-        void *t[9] = {&jobs, &outs, &tb, &paths, &res, &dev, &idx, &first, &n};
-        std::memcpy(wave, w, sizeof(w));
-        std::memcpy(thread, t, sizeof(t));
-    }
-};
-
-static int launch_tb(mh_context *ctx, TbArgs &a, const RoundGrids &g)
+static int launch_walks(mh_context *ctx, RoundArgs &a)
 {
     a.set();
-    MH_HIP(hipLaunchKernel(reinterpret_cast<const void *>(&dp_tb_wave), dim3(g.tbw), dim3(64), a.wave, 0,
-                           ctx->stream));
-    MH_HIP(hipLaunchKernel(reinterpret_cast<const void *>(&dp_tb_thread), dim3(g.tbt), dim3(64), a.thread, 0,
+    MH_HIP(hipLaunchKernel(reinterpret_cast<const void *>(&dp_tb_wave), dim3(a.npipe), dim3(64), a.walk, 0,
                            ctx->stream));
     MH_HIP(hipGetLastError());
     return MH_OK;
@@ -1748,50 +1752,35 @@ static int set_node(hipGraphExec_t exec, hipGraphNode_t node, unsigned grid, voi
     return MH_OK;
 }
 
-// The round's forward launch (queue reset + forward kernel) and its
-// trace-backs, timed apart; from graphs captured once per context (the
+// The round's forward launch (queue reset + forward kernel) and the walks of
+// its pipelined jobs, timed apart; from graphs captured once per context (the
 // descriptor's address is fixed; a round sets the nodes' grids) or launched
 // directly.
-static int dp_launch_round(mh_context *ctx, const DpRound *d_round, int v, bool graph, const RoundGrids &g,
-                           FwdArgs &fwa, TbArgs &tba)
+static int dp_launch_round(mh_context *ctx, int v, bool graph, unsigned grid, RoundArgs &a)
 {
     int rc;
-    if (graph && d_round != ctx->dp_round.as<DpRound>()) graph = false;
+    if (graph && a.rd != ctx->dp_round.as<DpRound>()) graph = false;
     if (graph && !ctx->dp_graph_fwd[v]) {
         const void *fns[1] = {FWD_VARIANTS[v].fn};
         if ((rc = capture(ctx, &ctx->dp_graph_fwd_src[v], &ctx->dp_graph_fwd[v], fns, &ctx->dp_graph_fwd_node[v], 1,
-                          [&] { return launch_fwd(ctx, fwa, v, g.fwd); })) != MH_OK)
-            return rc;
-    }
-    if (graph && !ctx->dp_graph_tb) {
-        const void *fns[2] = {reinterpret_cast<const void *>(&dp_tb_wave),
-                              reinterpret_cast<const void *>(&dp_tb_thread)};
-        if ((rc = capture(ctx, &ctx->dp_graph_tb_src, &ctx->dp_graph_tb, fns, ctx->dp_graph_tb_node, 2,
-                          [&] { return launch_tb(ctx, tba, g); })) != MH_OK)
+                          [&] { return launch_fwd(ctx, a, v, grid); })) != MH_OK)
             return rc;
     }
     if (graph) {
-        fwa.set();
-        tba.set();
-        if ((rc = set_node(ctx->dp_graph_fwd[v], ctx->dp_graph_fwd_node[v], g.fwd, fwa.args)) != MH_OK) return rc;
-        if ((rc = set_node(ctx->dp_graph_tb, ctx->dp_graph_tb_node[0], g.tbw, tba.wave)) != MH_OK) return rc;
-        if ((rc = set_node(ctx->dp_graph_tb, ctx->dp_graph_tb_node[1], g.tbt, tba.thread)) != MH_OK) return rc;
+        a.set();
+        if ((rc = set_node(ctx->dp_graph_fwd[v], ctx->dp_graph_fwd_node[v], grid, a.fwd)) != MH_OK) return rc;
     }
     {
         TimedLaunch tl(ctx, "dp_forward");
         if (graph) {
             MH_HIP(hipGraphLaunch(ctx->dp_graph_fwd[v], ctx->stream));
-        } else if ((rc = launch_fwd(ctx, fwa, v, g.fwd)) != MH_OK) {
+        } else if ((rc = launch_fwd(ctx, a, v, grid)) != MH_OK) {
             return rc;
         }
     }
-    {
+    if (a.npipe) {
         TimedLaunch tl(ctx, "dp_traceback");
-        if (graph) {
-            MH_HIP(hipGraphLaunch(ctx->dp_graph_tb, ctx->stream));
-        } else if ((rc = launch_tb(ctx, tba, g)) != MH_OK) {
-            return rc;
-        }
+        if ((rc = launch_walks(ctx, a)) != MH_OK) return rc;
     }
     return MH_OK;
 }
@@ -1799,7 +1788,7 @@ static int dp_launch_round(mh_context *ctx, const DpRound *d_round, int v, bool 
 static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
                         const std::vector<uint64_t> &slot, std::vector<DpItem> &items, uint8_t *d_paths,
                         mh_dp_result *d_results, uint32_t *d_dev, uint64_t *cells,
-                        const FixedScratch *fx = nullptr)
+                        const FixedScratch *fx = nullptr, DpCells form = DpCells::TAGGED)
 {
     const uint64_t nitems = items.size();
     if (nitems == 0) return MH_OK;
@@ -1868,8 +1857,8 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             if ((rc0 = ctx->dp_tb.ensure(need + 256)) != MH_OK) return rc0;
         }
     }
-    uint32_t sr[4];
-    packed_rows(sr);
+    RoundArgs ra;
+    packed_rows(ra.sc);
     // pipelined stripe jobs: wavefronts a job by the round's size (up to
     // DP_PIPE_MAX), or MH_DP_PIPE (0 or 1 keeps one wavefront a job); the
     // no-allocation path keeps one
@@ -1959,7 +1948,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
         for (uint64_t z = 0; z < n64 && !wide; ++z) wide = items[first + z].cols == 16;
         for (int q = 0; q < 4; ++q)
             if (rows_at[q + 2] > rows_at[q + 1]) wide = true;
-        const int variant = dp_variant_for(wide);
+        const int variant = form == DpCells::TAGGED ? dp_variant_for(wide) : VARIANT_LONG;
         // Pipelined stripe jobs.  A round with fewer work items than the
         // forward launch's wavefront slots ends on its longest jobs' latency
         // with SIMDs idle: its 64-lane stripe jobs then run on P_j wavefronts
@@ -2033,28 +2022,11 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
         DevJob *dj = nullptr;
         std::vector<DevJob> host_jobs;
         if (fx) {
-            host_jobs.resize(n + (n * 4 + sizeof(DevJob) - 1) / sizeof(DevJob));
+            host_jobs.resize(n);
             dj = host_jobs.data();
         } else {
-            const int rc0 = pinned_jobs(ctx, n * sizeof(DevJob) + n * 4 + 64, (void **)&dj);
+            const int rc0 = pinned_jobs(ctx, n * sizeof(DevJob) + 64, (void **)&dj);
             if (rc0 != MH_OK) return rc0;
-        }
-        // trace-back order: the jobs whose walks are long and whose layout the
-        // wavefront walk reads (64-lane stripes; 16-lane stripes of 4 or 8
-        // columns a lane) walk on a wavefront each, the others on a thread each
-        uint32_t *tbi = reinterpret_cast<uint32_t *>(dj + n);
-        uint64_t nwave = 0;
-        {
-            auto wave_walk = [&](const DpItem &it) {
-                if (jobs[it.job].a_len + jobs[it.job].b_len < WAVE_WALK_MIN) return false;
-                if (it.cols == TINY_COLS_TAG || it.cols >= WINDOW_TAG) return false;
-                return it.cols < GROUP_TAG || it.cols == GROUP_TAG + 4 || it.cols == GROUP_TAG + 8;
-            };
-            for (uint64_t x = 0; x < n; ++x)
-                if (wave_walk(items[first + x])) tbi[nwave++] = (uint32_t)x;
-            uint64_t t = nwave;
-            for (uint64_t x = 0; x < n; ++x)
-                if (!wave_walk(items[first + x])) tbi[t++] = (uint32_t)x;
         }
         uint64_t tw = 0, bo = 0, bo_pipe = 0;
         for (uint64_t x = 0; x < n; ++x) {
@@ -2079,7 +2051,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
                 bo += 3 * bnd_ints(it);
                 bo_pipe = bo;
             }
-            if (cells) *cells += 2 * it.tb_bytes;
+            if (cells) *cells += it.cells;
         }
         DevJob *d_jobs;
         DpOut *d_outs;
@@ -2110,28 +2082,13 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             d_bnd = ctx->dp_bnd.as<int>();
             d_round = ctx->dp_round.as<DpRound>();
         }
-        uint32_t *d_tbi = reinterpret_cast<uint32_t *>(d_outs + n);
         MH_HIP(hipMemcpyAsync(d_jobs, dj, n * sizeof(DevJob), hipMemcpyHostToDevice, ctx->stream));
-        MH_HIP(hipMemcpyAsync(d_tbi, tbi, n * 4, hipMemcpyHostToDevice, ctx->stream));
         // the pipelined jobs' boundary words (the first jobs') start untagged
         if (bo_pipe) MH_HIP(hipMemsetAsync(d_bnd, 0, bo_pipe * 4, ctx->stream));
-        // the round's descriptor: pointers, the trace-back split and the queue's bins
+        // the round's descriptor: the queue's bins
         DpRound hr;
         std::memset(&hr, 0, sizeof(hr));
-        hr.jobs = d_jobs;
-        hr.outs = d_outs;
-        hr.A = d_a;
-        hr.B = d_b;
-        hr.tb = d_tb;
-        hr.bnd = d_bnd;
-        hr.paths = d_paths;
-        hr.res = d_results;
-        hr.dev = d_dev;
-        hr.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(d_round) + sizeof(DpRound));
-        for (int k = 0; k < 4; ++k) hr.sr[k] = sr[k];
-        hr.goh = -200;
-        hr.nwave = (uint32_t)nwave;
-        hr.n = (uint32_t)n;
+        if (form != DpCells::TAGGED) dp_score6(hr.table);
         auto add_bin = [&](uint32_t kind, uint64_t b0, uint64_t cnt) {
             if (cnt == 0) return;
             hr.kind[hr.nbins] = kind;
@@ -2174,52 +2131,39 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             nitems_q += (hr.count[q] + per - 1) / per;
         }
         hr.item0[hr.nbins] = (uint32_t)nitems_q;
-        RoundGrids grids;
+        unsigned grid = 0;
         {
             int rc;
-            if ((rc = round_grids(ctx, variant, nitems_q, hr.nwave, hr.n, &grids)) != MH_OK) return rc;
+            if ((rc = fwd_grid(ctx, variant, nitems_q, &grid)) != MH_OK) return rc;
         }
-        FwdArgs fwa;
-        fwa.jobs = d_jobs;
-        fwa.outs = d_outs;
-        fwa.A = d_a;
-        fwa.B = d_b;
-        fwa.tb = d_tb;
-        fwa.bnd = d_bnd;
-        fwa.rd = d_round;
-        fwa.cursor = hr.cursor;
-        fwa.sr0 = sr[0];
-        fwa.sr1 = sr[1];
-        fwa.sr2 = sr[2];
-        fwa.sr3 = sr[3];
-        fwa.goh = -200;
-        TbArgs tba;
-        tba.jobs = d_jobs;
-        tba.outs = d_outs;
-        tba.tb = d_tb;
-        tba.paths = d_paths;
-        tba.res = d_results;
-        tba.dev = d_dev;
-        tba.idx = d_tbi;
-        tba.nwave = hr.nwave;
-        tba.first = hr.nwave;
-        tba.n = hr.n;
+        ra.jobs = d_jobs;
+        ra.outs = d_outs;
+        ra.A = d_a;
+        ra.B = d_b;
+        ra.tb = d_tb;
+        ra.bnd = d_bnd;
+        ra.rd = d_round;
+        ra.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(d_round) + sizeof(DpRound));
+        ra.paths = d_paths;
+        ra.res = d_results;
+        ra.dev = d_dev;
+        ra.npipe = (uint32_t)npipe;
         if (fx) {
             MH_HIP(hipMemcpyAsync(d_round, &hr, sizeof(hr), hipMemcpyHostToDevice, ctx->stream));
             int rc;
-            if ((rc = dp_launch_round(ctx, d_round, variant, false, grids, fwa, tba)) != MH_OK) return rc;
+            if ((rc = dp_launch_round(ctx, variant, false, grid, ra)) != MH_OK) return rc;
         } else {
             int rc;
             if ((rc = dp_round_staging(ctx)) != MH_OK) return rc;
             std::memcpy(ctx->dp_round_host, &hr, sizeof(hr));
             MH_HIP(hipMemcpyAsync(d_round, ctx->dp_round_host, sizeof(hr), hipMemcpyHostToDevice, ctx->stream));
-            if ((rc = dp_launch_round(ctx, d_round, variant, dp_use_graph(), grids, fwa, tba)) != MH_OK) return rc;
+            if ((rc = dp_launch_round(ctx, variant, dp_use_graph(), grid, ra)) != MH_OK) return rc;
         }
         // the host job table is reused by the next round
         MH_HIP(hipStreamSynchronize(ctx->stream));
         if (npipe) {
             uint32_t err = 0;
-            MH_HIP(hipMemcpyAsync(&err, hr.cursor + (DPQ_CURSORS - 1), 4, hipMemcpyDeviceToHost, ctx->stream));
+            MH_HIP(hipMemcpyAsync(&err, ra.cursor + (DPQ_CURSORS - 1), 4, hipMemcpyDeviceToHost, ctx->stream));
             MH_HIP(hipStreamSynchronize(ctx->stream));
             MH_CHECK(err == 0, MH_ERR_DEVICE, "DP: a pipelined stripe's wait ran past its limit");
         }
@@ -2268,34 +2212,36 @@ static int dp_check_jobs(const mh_dp_job *jobs, uint64_t njobs, std::vector<uint
     return MH_OK;
 }
 
-static DpItem make_item(const mh_dp_job &jb, uint32_t job, uint32_t band, int force, bool rerun = false)
+static DpItem make_item(const mh_dp_job &jb, uint32_t job, uint32_t band, int force, bool rerun = false,
+                        bool tiny = true)
 {
     DpItem it;
     it.job = job;
     it.cols = dp_cols_for(jb.a_len, jb.b_len, band, force, rerun);
     it.band = dp_effective_band(jb.a_len, jb.b_len, band, it.cols);
     if (it.band == 0 && band != 0) it.cols = dp_cols_for(jb.a_len, jb.b_len, 0, force);
-    if (it.band == 0 && !force && jb.b_len <= (uint32_t)TINY_LB) {
+    if (it.band == 0 && !force && tiny && jb.b_len <= (uint32_t)TINY_LB) {
         it.cols = TINY_COLS_TAG;
         it.tb_bytes = (uint64_t)jb.a_len * 8;
+        it.cells = 2 * it.tb_bytes;
         return it;
     }
-    if (it.band == 0 && !force && jb.b_len <= ROWS_MAX_LB && jb.a_len + jb.b_len < WAVE_WALK_MIN &&
+    if (it.band == 0 && !force && jb.b_len <= ROWS_MAX_LB && jb.a_len + jb.b_len < ROWS_MAX_WALK &&
         shape_table()[dp_tune_class(jb.b_len)] == 0) {
         // four jobs per wavefront, one stripe each of the fewest columns a lane
         // (an even number from 4 to 16) that holds the job
-        const uint32_t c = std::max(4u, 2u * ((jb.b_len + 31) / 32));
-        it.cols = GROUP_TAG + c;
-        it.tb_bytes = dp_trace_bytes(jb.a_len, jb.b_len, 0, c, 16);
-        return it;
+        it.cols = GROUP_TAG + std::max(4u, 2u * ((jb.b_len + 31) / 32));
     }
-    it.tb_bytes = it.cols > GROUP_TAG ? dp_trace_bytes(jb.a_len, jb.b_len, it.band, it.cols - GROUP_TAG, 16)
-                                      : dp_trace_bytes(jb.a_len, jb.b_len, it.band, it.cols, 64);
+    const uint32_t g = it.cols > GROUP_TAG ? 16u : 64u, c = it.cols > GROUP_TAG ? it.cols - GROUP_TAG : it.cols;
+    const uint64_t steps = dp_steps(jb.a_len, jb.b_len, it.band, c, g);
+    it.tb_bytes = steps * g * lane_bytes_of(c);
+    it.cells = steps * g * c;
     if (it.band) {
         const uint32_t wc = dp_window_cols(jb.a_len, jb.b_len, it.band, dp_force_kind());
         if (wc) {
             it.cols = WINDOW_TAG + wc;
             it.tb_bytes = (uint64_t)((jb.a_len + 8 / wc - 1) / (8 / wc)) * 256;
+            it.cells = 2 * it.tb_bytes;
         }
     }
     return it;
@@ -2321,7 +2267,7 @@ uint64_t dp_item_cells(uint32_t la, uint32_t lb, uint32_t band)
     const DpItem it = make_item(mh_dp_job{0, 0, la, lb}, 0, band, dp_force_cols());
     if (it.cols > WINDOW_TAG) return (uint64_t)la * 64 * (it.cols - WINDOW_TAG);
     if (it.cols == TINY_COLS_TAG) return (uint64_t)la * lb;
-    return 2 * it.tb_bytes;
+    return it.cells;
 }
 
 // The jobs whose operands hold letters other than A, C, G, T (class > 3):
@@ -2344,6 +2290,26 @@ static int split_wild(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, c
         if (mx[j] > 3) out.push_back((uint32_t)j);
     }
     return MH_OK;
+}
+
+// dp_run_items over the items' two forms of cells
+static int dp_run_forms(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
+                        const std::vector<uint64_t> &slot, std::vector<DpItem> &items, uint8_t *d_paths,
+                        mh_dp_result *d_results, uint32_t *d_dev, uint64_t *cells, const FixedScratch *fx = nullptr)
+{
+    auto tagged = [&](const DpItem &it) {
+        return it.cols > WINDOW_TAG || std::min(jobs[it.job].a_len, jobs[it.job].b_len) <= TAGGED_MAX;
+    };
+    std::vector<DpItem> longs;
+    for (const DpItem &it : items)
+        if (!tagged(it)) longs.push_back(it);
+    if (!longs.empty()) {
+        items.erase(std::remove_if(items.begin(), items.end(), [&](const DpItem &it) { return !tagged(it); }),
+                    items.end());
+        const int rc = dp_run_items(ctx, d_a, d_b, jobs, slot, longs, d_paths, d_results, d_dev, cells, fx, DpCells::LONG);
+        if (rc != MH_OK) return rc;
+    }
+    return dp_run_items(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, d_dev, cells, fx, DpCells::TAGGED);
 }
 
 // drops the items of the float-DP jobs (items[j] is job j's)
@@ -2375,7 +2341,7 @@ int dp_run(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_
     make_items(jobs, njobs, nullptr, items);
     drop_wild(items, wj);
     host_time(ctx, "host_dp_plan", now_ms() - tp0);
-    if ((rc = dp_run_items(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, nullptr, nullptr)) != MH_OK)
+    if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, nullptr, nullptr)) != MH_OK)
         return rc;
     return dp_run_float(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, nullptr, nullptr, nullptr);
 }
@@ -2401,7 +2367,7 @@ int dp_run_noalloc(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, cons
     std::vector<DpItem> items;
     make_items(jobs, njobs, nullptr, items);
     drop_wild(items, wj);
-    if ((rc = dp_run_items(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, nullptr, nullptr, &fx)) != MH_OK)
+    if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, nullptr, nullptr, &fx)) != MH_OK)
         return rc;
     return dp_run_float(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, nullptr, nullptr, &fx);
 }
@@ -2452,7 +2418,7 @@ int dp_run_banded(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const
     drop_wild(items, wj);
     host_time(ctx, "host_dp_plan", now_ms() - tp0);
     const int force = dp_force_cols();
-    if ((rc = dp_run_items(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, d_dev, &st.cells)) != MH_OK)
+    if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, d_dev, &st.cells)) != MH_OK)
         return rc;
     if ((rc = dp_run_float(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, d_dev, &st.cells, nullptr)) != MH_OK)
         return rc;
@@ -2479,7 +2445,7 @@ int dp_run_banded(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const
                 }
             }
         if (!again.empty()) {
-            if ((rc = dp_run_items(ctx, d_a, d_b, jobs, slot, again, d_paths, d_results, d_dev, &st.cells)) != MH_OK)
+            if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, again, d_paths, d_results, d_dev, &st.cells)) != MH_OK)
                 return rc;
             MH_HIP(hipMemcpyAsync(dev.data(), d_dev, njobs * 4, hipMemcpyDeviceToHost, ctx->stream));
             MH_HIP(hipStreamSynchronize(ctx->stream));
@@ -2492,7 +2458,7 @@ int dp_run_banded(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const
                     ++st.rerun_full;
                 }
             if (!full.empty()) {
-                if ((rc = dp_run_items(ctx, d_a, d_b, jobs, slot, full, d_paths, d_results, d_dev, &st.cells)) != MH_OK)
+                if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, full, d_paths, d_results, d_dev, &st.cells)) != MH_OK)
                     return rc;
                 MH_HIP(hipStreamSynchronize(ctx->stream));
                 host_time(ctx, "band_pass3", now_ms() - tq);

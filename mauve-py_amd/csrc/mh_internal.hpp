@@ -93,7 +93,7 @@ struct KernelTimer {
 
 }  // namespace mh
 
-#define MH_DP_MAX_VARIANTS 8   // forward kernel variants of the DP (dp.hip)
+#define MH_DP_MAX_VARIANTS 9   // forward kernel variants of the DP (dp.hip)
 
 struct mh_context {
     int device = 0;
@@ -110,9 +110,9 @@ struct mh_context {
     // persistent grids
     mh::DevBuf dp_round;
     void *dp_round_host = nullptr;
-    hipGraph_t dp_graph_fwd_src[MH_DP_MAX_VARIANTS] = {}, dp_graph_tb_src = nullptr;
-    hipGraphExec_t dp_graph_fwd[MH_DP_MAX_VARIANTS] = {}, dp_graph_tb = nullptr;
-    hipGraphNode_t dp_graph_fwd_node[MH_DP_MAX_VARIANTS] = {}, dp_graph_tb_node[2] = {};
+    hipGraph_t dp_graph_fwd_src[MH_DP_MAX_VARIANTS] = {};
+    hipGraphExec_t dp_graph_fwd[MH_DP_MAX_VARIANTS] = {};
+    hipGraphNode_t dp_graph_fwd_node[MH_DP_MAX_VARIANTS] = {};
     unsigned dp_fwd_grid[MH_DP_MAX_VARIANTS] = {};
     mh::DevBuf ml_jobs, ml_y;   // learned band: job table, network outputs + bands
     // seed-matching scratch

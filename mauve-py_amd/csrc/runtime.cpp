@@ -346,8 +346,6 @@ void mh_destroy(mh_context *ctx)
         if (g) (void)hipGraphExecDestroy(g);
     for (hipGraph_t &g : ctx->dp_graph_fwd_src)
         if (g) (void)hipGraphDestroy(g);
-    if (ctx->dp_graph_tb) (void)hipGraphExecDestroy(ctx->dp_graph_tb);
-    if (ctx->dp_graph_tb_src) (void)hipGraphDestroy(ctx->dp_graph_tb_src);
     if (ctx->dp_round_host) (void)hipHostFree(ctx->dp_round_host);
     ctx->dp_round.release();
     ctx->dp_tb.release();

@@ -151,3 +151,23 @@ def test_fallback_chain(ctx):
         full_p, full_s = po.nwsmall(a, b)
         assert int(res[k]["score"]) <= int(full_s)
     assert n2 > 0 and st.rerun_doubled + st.rerun_full > 0
+
+
+def test_scores_past_the_tagged_range(ctx):
+    """Operands above 2^20 positions run cells without state tags (their
+    scores times four could leave 32 bits); 2^20 is the last tagged size.
+    Sparse substitutions: the path is the diagonal and the score its sum."""
+    nuc = np.array([[91, -114, -31, -123], [-114, 100, -125, -31], [-31, -125, 100, -114], [-123, -31, -114, 91]]) + 60
+    rng = np.random.default_rng(3)
+    for n in (1 << 20, (1 << 20) + 1):
+        a = rng.integers(0, 4, n, dtype=np.uint8)
+        b = a.copy()
+        hit = rng.random(n) < 0.01
+        b[hit] = (b[hit] + 1) % 4
+        jobs = mauvehip.make_jobs([0], [n], [0], [n])
+        paths, res, dev, st = mauvehip.global_align_banded(ctx, a, b, jobs, np.array([4], dtype=np.uint32),
+                                                           flags=mauvehip.BAND_NO_FALLBACK)
+        assert st.banded == 1
+        assert int(res[0]["path_len"]) == n and int(dev[0]) == 0
+        assert (paths[int(res[0]["path_start"]):][:n] == ord("M")).all()
+        assert int(res[0]["score"]) == int(nuc[a, b].sum())
