@@ -281,6 +281,10 @@ struct IntCell {
 // closed before the comparison, so every value and tie is its float), and
 // int32 for jobs whose scores times four could leave 32 bits.  H(i,j) =
 // max(M, D + c, I + c), E(i+1,j) = max(D, M + o), F(i,j+1) = max(I, M + o).
+// Bound by latency: such jobs are few.  2,000 jobs of 10-1,000 columns, one in
+// twenty with wildcard letters: 943 ms with a thread a wildcard job (rows and a
+// byte a cell in device memory, one dependent access after another), 1.65 ms
+// with these cells in dp_job's wavefronts.
 template <class T> struct CmpCell {
     static constexpr bool FLT = std::is_same<T, float>::value;
     static constexpr T G = (T)GOH;
@@ -1580,21 +1584,21 @@ const FwdVariant FWD_VARIANTS[] = {
     MH_FWD(IntCell, 16, 3, false), MH_FWD(IntCell, 8, 4, false), MH_FWD(IntCell, 16, 2, false),
     MH_FWD(IntCell, 16, 3, true),  MH_FWD(IntCell, 16, 2, true), MH_FWD(IntCell, 8, 4, true),
     MH_FWD(IntCell, 16, 4, false),
-    // jobs whose scores times four could leave 32 bits
-    MH_FWD(CmpCell<int>, 16, 2, false),
+    // jobs whose scores times four could leave 32 bits; jobs with wildcard letters
+    MH_FWD(CmpCell<int>, 16, 2, false), MH_FWD(CmpCell<float>, 16, 2, false),
 };
 #undef MH_FWD
 constexpr int N_ALL_VARIANTS = (int)(sizeof(FWD_VARIANTS) / sizeof(FWD_VARIANTS[0]));
-constexpr int N_FWD_VARIANTS = N_ALL_VARIANTS - 1;   // of the tagged int32 cells
-constexpr int VARIANT_LONG = N_FWD_VARIANTS;
+constexpr int N_FWD_VARIANTS = N_ALL_VARIANTS - 2;   // of the tagged int32 cells
+constexpr int VARIANT_LONG = N_FWD_VARIANTS, VARIANT_FLOAT = N_FWD_VARIANTS + 1;
 static_assert(N_ALL_VARIANTS <= MH_DP_MAX_VARIANTS, "context graph slots");
 
 // The cells a run of jobs takes: tagged int32 (values times four), int32
-// without a tag.  The tagged form holds |score| < 2^28: a score is at
+// without a tag, float.  The tagged form holds |score| < 2^28: a score is at
 // most 160 a position of the shorter operand, and a reachable cell of a band at
 // least -65 a position, so 225 * 2^20 < 2^28 keeps both apart from minus
 // infinity.  Longer jobs (only banded ones can be) keep untagged values.
-enum class DpCells { TAGGED, LONG };
+enum class DpCells { TAGGED, LONG, FLOAT };
 constexpr uint32_t TAGGED_MAX = 1u << 20;
 static_assert(DP_TUNE_WIDE_VARIANT < N_FWD_VARIANTS && DP_TUNE_NARROW_VARIANT < N_FWD_VARIANTS, "tuning table");
 
@@ -1785,6 +1789,24 @@ static int dp_launch_round(mh_context *ctx, int v, bool graph, unsigned grid, Ro
     return MH_OK;
 }
 
+// ints of the boundary columns of an item's job (rounded up: two values a row)
+static uint64_t item_bnd_ints(const DpItem &it, const mh_dp_job *jobs)
+{
+    // one-lane and window jobs hand no column over; a job of 16-lane
+    // stripes does when it has more than one (banded jobs)
+    if (it.cols == TINY_COLS_TAG || it.cols >= WINDOW_TAG) return 0ull;
+    const uint64_t sw = it.cols > GROUP_TAG ? 16ull * (it.cols - GROUP_TAG) : 64ull * it.cols;
+    const uint64_t ns = (jobs[it.job].b_len + sw - 1) / sw;
+    return ns > 1 ? 3ull * ((jobs[it.job].a_len + 63) & ~63ull) : 0ull;
+}
+
+// footprint in a fixed scratch of a round of `cnt` jobs with trace bytes
+// tbb (each rounded up to 16) and bi boundary ints
+static uint64_t fixed_need(uint64_t cnt, uint64_t tbb, uint64_t bi)
+{
+    return DP_ROUND_BYTES + align256(cnt * (sizeof(DevJob) + sizeof(DpOut) + 4)) + align256(bi * 4) + tbb + 256;
+}
+
 static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
                         const std::vector<uint64_t> &slot, std::vector<DpItem> &items, uint8_t *d_paths,
                         mh_dp_result *d_results, uint32_t *d_dev, uint64_t *cells,
@@ -1815,19 +1837,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
         items.swap(sorted);
     }
     host_time(ctx, "host_dp_sort", now_ms() - ts0);
-    auto bnd_ints = [&](const DpItem &it) {
-        // one-lane and window jobs hand no column over; a job of 16-lane
-        // stripes does when it has more than one (banded jobs)
-        if (it.cols == TINY_COLS_TAG || it.cols >= WINDOW_TAG) return 0ull;
-        const uint64_t sw = it.cols > GROUP_TAG ? 16ull * (it.cols - GROUP_TAG) : 64ull * it.cols;
-        const uint64_t ns = (jobs[it.job].b_len + sw - 1) / sw;
-        return ns > 1 ? 3ull * ((jobs[it.job].a_len + 63) & ~63ull) : 0ull;
-    };
-    // footprint in a fixed scratch of a round of `cnt` jobs with trace bytes
-    // tbb (each rounded up to 16) and bi boundary ints
-    auto fixed_need = [&](uint64_t cnt, uint64_t tbb, uint64_t bi) {
-        return DP_ROUND_BYTES + align256(cnt * (sizeof(DevJob) + sizeof(DpOut) + 4)) + align256(bi * 4) + tbb + 256;
-    };
+    auto bnd_ints = [&](const DpItem &it) { return item_bnd_ints(it, jobs); };
     if (fx) {
         for (const DpItem &it : items)
             MH_CHECK(fixed_need(1, (it.tb_bytes + 15) & ~15ull, bnd_ints(it)) <= fx->bytes, MH_ERR_INVALID,
@@ -1948,7 +1958,8 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
         for (uint64_t z = 0; z < n64 && !wide; ++z) wide = items[first + z].cols == 16;
         for (int q = 0; q < 4; ++q)
             if (rows_at[q + 2] > rows_at[q + 1]) wide = true;
-        const int variant = form == DpCells::TAGGED ? dp_variant_for(wide) : VARIANT_LONG;
+        const int variant = form == DpCells::TAGGED ? dp_variant_for(wide)
+                                                    : (form == DpCells::FLOAT ? VARIANT_FLOAT : VARIANT_LONG);
         // Pipelined stripe jobs.  A round with fewer work items than the
         // forward launch's wavefront slots ends on its longest jobs' latency
         // with SIMDs idle: its 64-lane stripe jobs then run on P_j wavefronts
@@ -2312,6 +2323,33 @@ static int dp_run_forms(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
     return dp_run_items(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, d_dev, cells, fx, DpCells::TAGGED);
 }
 
+// The jobs `which` (indices into jobs), whose operands hold wildcard letters:
+// the full DP in float cells.  In the fixed scratch a job keeps the limit it has
+// always had, that of a float row set and a byte a cell (dp_float.hip); a long
+// thin job whose records would not fit there (a lane's share of a step is at
+// least 2 bytes) takes that form still, a thread a job.
+static int dp_run_wild(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
+                       const std::vector<uint64_t> &slot, const std::vector<uint32_t> &which, uint8_t *d_paths,
+                       mh_dp_result *d_results, uint32_t *d_dev, uint64_t *cells, const FixedScratch *fx)
+{
+    if (which.empty()) return MH_OK;
+    const int force = dp_force_cols();
+    std::vector<DpItem> items;
+    std::vector<uint32_t> thin;
+    int rc;
+    for (uint32_t j : which) {
+        if (fx && (rc = dp_float_fits(jobs, j, fx)) != MH_OK) return rc;
+        DpItem it = make_item(jobs[j], j, 0, force, false, false);
+        it.cells = (uint64_t)jobs[j].a_len * jobs[j].b_len;
+        if (fx && fixed_need(1, (it.tb_bytes + 15) & ~15ull, item_bnd_ints(it, jobs)) > fx->bytes) thin.push_back(j);
+        else items.push_back(it);
+    }
+    if ((rc = dp_run_items(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, d_dev, cells, fx, DpCells::FLOAT)) !=
+        MH_OK)
+        return rc;
+    return thin.empty() ? MH_OK : dp_run_float_threads(ctx, d_a, d_b, jobs, slot, thin, d_paths, d_results, fx);
+}
+
 // drops the items of the float-DP jobs (items[j] is job j's)
 static void drop_wild(std::vector<DpItem> &items, const std::vector<uint32_t> &wild)
 {
@@ -2343,7 +2381,7 @@ int dp_run(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_
     host_time(ctx, "host_dp_plan", now_ms() - tp0);
     if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, nullptr, nullptr)) != MH_OK)
         return rc;
-    return dp_run_float(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, nullptr, nullptr, nullptr);
+    return dp_run_wild(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, nullptr, nullptr, nullptr);
 }
 
 int dp_run_noalloc(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs, uint64_t njobs,
@@ -2369,7 +2407,7 @@ int dp_run_noalloc(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, cons
     drop_wild(items, wj);
     if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, nullptr, nullptr, &fx)) != MH_OK)
         return rc;
-    return dp_run_float(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, nullptr, nullptr, &fx);
+    return dp_run_wild(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, nullptr, nullptr, &fx);
 }
 
 int dp_run_banded(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs, uint64_t njobs,
@@ -2420,7 +2458,7 @@ int dp_run_banded(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const
     const int force = dp_force_cols();
     if ((rc = dp_run_forms(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, d_dev, &st.cells)) != MH_OK)
         return rc;
-    if ((rc = dp_run_float(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, d_dev, &st.cells, nullptr)) != MH_OK)
+    if ((rc = dp_run_wild(ctx, d_a, d_b, jobs, slot, wj, d_paths, d_results, d_dev, &st.cells, nullptr)) != MH_OK)
         return rc;
     if (!(flags & MH_BAND_NO_FALLBACK) && st.banded) {
         // edge fallback: a banded path that reaches distance W is rerun with

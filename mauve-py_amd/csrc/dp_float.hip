@@ -9,14 +9,16 @@
 // each base; DNA counts are not normalised (MU/params.cpp:296-310).  The
 // position's m_AAScores (MU/profilefrommsa.cpp:279-285), SortCounts' order
 // (159-183) and ScoreProfPos2SPN (MU/scorepp.cpp:80-92) then give fractional
-// match scores, and NWSmall (MU/nwsmall.cpp:500-670) adds them in float.  An
-// int32 DP cannot reproduce that rounding, so such jobs run here: one thread
-// per job does NWSmall's float recurrences in the reference's order of
-// operations (no contraction into fused multiply-adds), keeps the 4-bit
-// trace of every cell (MU/types.h:26-46), and walks it back as BitTraceBack
-// (MU/bittraceback.cpp:138-209).  Operand classes: 0-3 A,C,G,T (U as T),
-// 4 'X', 5 any other letter.  Such jobs are rare (N runs in assemblies); the
-// A/C/G/T jobs of a batch keep the int32 kernels.
+// match scores, and NWSmall (MU/nwsmall.cpp:500-670) adds them in float.  The
+// tagged int32 cells cannot reproduce that rounding, so such jobs run dp.hip's
+// forward pass with float cells (CmpCell<float>), which take the 6 x 6 score
+// table made here.  Operand classes: 0-3 A,C,G,T (U as T), 4 'X', 5 any other
+// letter.
+//
+// The kernel below, one thread a job, is left for the no-allocation entry
+// point's long thin jobs: its scratch is 16 bytes a column and a byte a cell,
+// where the wavefronts' records take at least 32 bytes a row, so some jobs fit
+// the fixed scratch only in this form.
 #include "mh_internal.hpp"
 
 #include <algorithm>
@@ -332,27 +334,26 @@ int dp_code_max(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const m
     return MH_OK;
 }
 
-int dp_run_float(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
-                 const std::vector<uint64_t> &slot, const std::vector<uint32_t> &which, uint8_t *d_paths,
-                 mh_dp_result *d_results, uint32_t *d_dev, uint64_t *cells, const FixedScratch *fx)
+static uint64_t float_need(uint64_t cnt, uint64_t bytes)
 {
-    if (which.empty()) return MH_OK;
+    return ((cnt * sizeof(FloatJob) + 255) & ~255ull) + bytes + 256;
+}
+
+int dp_float_fits(const mh_dp_job *jobs, uint32_t j, const FixedScratch *fx)
+{
+    MH_CHECK(float_need(1, float_job_bytes(jobs[j].a_len, jobs[j].b_len)) <= fx->bytes, MH_ERR_INVALID,
+             "DP job " + std::to_string(j) + " (" + std::to_string(jobs[j].a_len) + " x " +
+                 std::to_string(jobs[j].b_len) + ", letters other than A,C,G,T) needs more than the " +
+                 std::to_string(fx->bytes >> 20) + " MiB scratch of the no-allocation entry point");
+    return MH_OK;
+}
+
+int dp_run_float_threads(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
+                         const std::vector<uint64_t> &slot, const std::vector<uint32_t> &which, uint8_t *d_paths,
+                         mh_dp_result *d_results, const FixedScratch *fx)
+{
     const Score6 &S = score6();
     const uint64_t jt = sizeof(FloatJob);
-    auto need = [&](uint64_t cnt, uint64_t bytes) { return ((cnt * jt + 255) & ~255ull) + bytes + 256; };
-    uint64_t budget;
-    if (fx) {
-        budget = fx->bytes;
-        for (uint32_t j : which)
-            MH_CHECK(need(1, float_job_bytes(jobs[j].a_len, jobs[j].b_len)) <= budget, MH_ERR_INVALID,
-                     "DP job " + std::to_string(j) + " (" + std::to_string(jobs[j].a_len) + " x " +
-                         std::to_string(jobs[j].b_len) + ", letters other than A,C,G,T) needs more than the " +
-                         std::to_string(fx->bytes >> 20) + " MiB scratch of the no-allocation entry point");
-    } else {
-        size_t free_b = 0, total_b = 0;
-        MH_HIP(hipMemGetInfo(&free_b, &total_b));
-        budget = (uint64_t)((free_b + ctx->dp_fl.bytes) * 0.5);
-    }
     std::vector<FloatJob> hj;
     size_t first = 0;
     while (first < which.size()) {
@@ -362,7 +363,7 @@ int dp_run_float(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const 
         while (last < which.size()) {
             const mh_dp_job &q = jobs[which[last]];
             const uint64_t b = float_job_bytes(q.a_len, q.b_len);
-            if (last > first && need(last - first + 1, bytes + b) > budget) break;
+            if (last > first && float_need(last - first + 1, bytes + b) > fx->bytes) break;
             FloatJob f;
             f.a_off = q.a_off;
             f.b_off = q.b_off;
@@ -374,24 +375,15 @@ int dp_run_float(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const 
             f.pad_ = 0;
             hj.push_back(f);
             bytes += b;
-            if (cells) *cells += (uint64_t)q.a_len * q.b_len;
             ++last;
         }
         const uint64_t n = last - first, tbytes = (n * jt + 255) & ~255ull;
-        uint8_t *base;
-        if (fx) {
-            base = fx->ptr;
-        } else {
-            int rc;
-            if ((rc = ctx->dp_fl.ensure(tbytes + bytes + 256)) != MH_OK) return rc;
-            base = ctx->dp_fl.as<uint8_t>();
-        }
-        FloatJob *d_jobs = reinterpret_cast<FloatJob *>(base);
+        FloatJob *d_jobs = reinterpret_cast<FloatJob *>(fx->ptr);
         MH_HIP(hipMemcpyAsync(d_jobs, hj.data(), n * jt, hipMemcpyHostToDevice, ctx->stream));
         {
             TimedLaunch tl(ctx, "dp_float");
             hipLaunchKernelGGL(dp_float_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, ctx->stream, d_jobs,
-                               (int)n, d_a, d_b, base + tbytes, S, d_paths, d_results, d_dev);
+                               (int)n, d_a, d_b, fx->ptr + tbytes, S, d_paths, d_results, (uint32_t *)nullptr);
             MH_HIP(hipGetLastError());
         }
         // the host job table is reused by the next round

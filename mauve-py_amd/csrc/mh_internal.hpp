@@ -93,7 +93,7 @@ struct KernelTimer {
 
 }  // namespace mh
 
-#define MH_DP_MAX_VARIANTS 9   // forward kernel variants of the DP (dp.hip)
+#define MH_DP_MAX_VARIANTS 10   // forward kernel variants of the DP (dp.hip)
 
 struct mh_context {
     int device = 0;
@@ -104,7 +104,7 @@ struct mh_context {
     std::vector<hipEvent_t> event_pool;
     // DP scratch
     mh::DevBuf dp_tb, dp_bnd, dp_jobs, dp_a, dp_b, dp_paths, dp_res, dp_dev;
-    mh::DevBuf dp_wild, dp_fl;   // operand scan; the float DP's job table and rows
+    mh::DevBuf dp_wild;   // operand scan
     // DP rounds: the descriptor and queue cursors (fixed address), its pinned
     // host copy, the launches captured as graphs per forward variant, and the
     // persistent grids
@@ -204,10 +204,13 @@ struct FixedScratch {
 int dp_code_max(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs, uint64_t njobs,
                 const FixedScratch *fx, std::vector<uint8_t> &out);
 // NWSmall in float for the jobs `which` (indices into jobs; slot = path slot
-// starts); cells (nullable) accumulates la * lb.
-int dp_run_float(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
-                 const std::vector<uint64_t> &slot, const std::vector<uint32_t> &which, uint8_t *d_paths,
-                 mh_dp_result *d_results, uint32_t *d_dev, uint64_t *cells, const FixedScratch *fx);
+// starts) in the fixed scratch, a thread a job: the long thin jobs whose
+// records the other form could not hold there.
+int dp_run_float_threads(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
+                         const std::vector<uint64_t> &slot, const std::vector<uint32_t> &which, uint8_t *d_paths,
+                         mh_dp_result *d_results, const FixedScratch *fx);
+// MH_ERR_INVALID when job j (with wildcard letters) is above the fixed scratch's limit
+int dp_float_fits(const mh_dp_job *jobs, uint32_t j, const FixedScratch *fx);
 // the 6 x 6 float match scores of the classes (row = A's class)
 void dp_score6(float *out);
 // The no-allocation DP: the same schedule and kernels with every scratch

@@ -119,3 +119,73 @@ def test_ascii_to_codes_classes(ctx):
     finally:
         ctx.free(d)
         ctx.free(c)
+
+
+def _wild_pairs(shapes, seed):
+    rng = np.random.default_rng(seed)
+    pairs = []
+    for la, lb in shapes:
+        n = max(la, lb)
+        a = rng.choice(list("ACGT"), n)
+        b = np.where(rng.random(n) < 0.12, rng.choice(list("ACGT"), n), a)
+        for s in (a, b):
+            s[rng.integers(0, n, 1 + n // 60)] = rng.choice(list("NXR"))
+        a[0] = "N"
+        if n > 40:
+            b = np.concatenate([b[:n // 3], rng.choice(list("ACGT"), 7), b[n // 3:]])
+        pairs.append(("".join(a[:la]), "".join(b[:lb])))
+    return pairs
+
+
+# sizes about the edges of the row shapes, lanes and stripes, one row, one column
+SHAPES = [(la, lb) for la in (1, 2, 17, 65, 300) for lb in (1, 2, 16, 17, 63, 64, 65, 128, 129, 255, 256, 257, 511, 513)]
+SHAPES += [(1100, 60), (900, 1025), (1500, 2100), (1, 3000), (3000, 1)]
+
+
+@pytest.mark.parametrize("pipe", ["1", "2", None])
+def test_float_cells_at_the_shapes_edges(ctx, pipe):
+    """Wildcard jobs on every row-packed and stripe shape, their stripes on one
+    wavefront, two, or as many as the round gives: the oracle's float paths and
+    scores, bit for bit (the cells add in the reference's order)."""
+    pairs = _wild_pairs(SHAPES, 31)
+    a, b, jobs = _pack(pairs)
+    old = os.environ.get("MH_DP_PIPE")
+    if pipe is None:
+        os.environ.pop("MH_DP_PIPE", None)
+    else:
+        os.environ["MH_DP_PIPE"] = pipe
+    try:
+        paths, res = mauvehip.global_align(ctx, a, b, jobs)
+    finally:
+        if old is None:
+            os.environ.pop("MH_DP_PIPE", None)
+        else:
+            os.environ["MH_DP_PIPE"] = old
+    for j, (x, y) in enumerate(pairs):
+        op, osc = po.nwsmall(x, y)
+        assert mauvehip.path_of(paths, res, j) == op, (j, len(x), len(y))
+        assert int(res[j]["score"]) == int(np.rint(np.float32(osc))), (j, len(x), len(y))
+
+
+def test_thin_job_in_the_fixed_scratch(ctx):
+    """A wildcard job whose records would not fit the no-allocation scratch,
+    while a byte a cell does: still accepted there, the same result."""
+    n = 2_100_000
+    rng = np.random.default_rng(8)
+    y = "".join(np.where(rng.random(n) < 0.01, "N", rng.choice(list("ACGT"), n)))
+    a, b, jobs = _pack([("C", y)])
+    dA, dB = ctx.alloc(len(a) + 16), ctx.alloc(len(b) + 16)
+    dP, dR = ctx.alloc(n + 16), ctx.alloc(64)
+    try:
+        ctx.h2d(dA, a)
+        ctx.h2d(dB, b)
+        op, osc = po.nwsmall("C", y)
+        for name in ("mh_dp_align_device", "mh_dp_align_device_noalloc"):
+            mauvehip._check(getattr(ctx.L, name)(ctx.h, dA, dB, jobs.ctypes.data, 1, dP, dR))
+            p = ctx.d2h(np.zeros(n + 16, np.uint8), dP)
+            r = ctx.d2h(np.zeros(1, mauvehip.DP_RESULT_DTYPE), dR)
+            assert mauvehip.path_of(p, r, 0) == op, name
+            assert int(r[0]["score"]) == int(np.rint(np.float32(osc))), name
+    finally:
+        for q in (dA, dB, dP, dR):
+            ctx.free(q)
