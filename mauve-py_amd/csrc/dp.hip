@@ -172,11 +172,15 @@ __device__ __forceinline__ bool walk_stays(uint32_t nib, int t)
 
 // bytes of a lane's records of one step: a nibble a column, in whole words a
 // lane can store at once
-__host__ __device__ constexpr uint32_t lane_bytes_of(uint32_t cols) { return cols <= 4 ? 2u : (cols <= 8 ? 4u : 8u); }
+__host__ __device__ constexpr uint32_t lane_bytes_of(uint32_t cols)
+{
+    return cols <= 2 ? 1u : (cols <= 4 ? 2u : (cols <= 8 ? 4u : 8u));
+}
 
 template <int COLS> __device__ __forceinline__ void store_records(uint8_t *dst, const uint32_t *word)
 {
-    if constexpr (COLS <= 4) *reinterpret_cast<uint16_t *>(dst) = (uint16_t)word[0];
+    if constexpr (COLS <= 2) *dst = (uint8_t)word[0];
+    else if constexpr (COLS <= 4) *reinterpret_cast<uint16_t *>(dst) = (uint16_t)word[0];
     else if constexpr (COLS <= 8) *reinterpret_cast<uint32_t *>(dst) = word[0];
     else *reinterpret_cast<uint2 *>(dst) = make_uint2(word[0], word[1]);
 }
@@ -398,7 +402,8 @@ template <class T> struct CmpCell {
 // running, so a part waits only on parts that run or have run, except the
 // parts of the one job a bin whose parts are not all taken; those are far
 // fewer than the resident wavefronts.
-// The result is the same as one wavefront's.
+// The result is the same as one wavefront's.  The boundary moves CH rows at a
+// time, each chunk's rows as soon as its steps are done.
 //
 // Returns whether this wavefront (this row of it) computed the final cell;
 // score and edge are then the final pick in every lane of the group.
@@ -409,6 +414,7 @@ constexpr uint32_t DP_SPIN_MAX = 1u << 22;
 struct DpLds {
     int4 in[64];        // H(i, j0 - 1), F(i, j0), A's row operand (two words)
     int2 out[64];
+    int2 idle[64];
     int fin[6][64];
 };
 
@@ -420,6 +426,7 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
 {
     constexpr int STRIPE_W = G * COLS;
     constexpr int LANE_BYTES = (int)lane_bytes_of(COLS);
+    constexpr int CH = G == 64 && COLS >= 8 ? 32 : 16;   // steps of a chunk
     const int lane = (int)threadIdx.x & (G - 1);
     const int gb = (int)threadIdx.x & ~(G - 1);    // the job's slots in the LDS rows
     const int la = (int)jb.la, lb = (int)jb.lb;
@@ -435,6 +442,7 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
     bool fin = false;
     int prev_r0 = 1, prev_r1 = 0;     // rows of the previous stripe's last column held in bnd
     uint64_t tbs = 0;                 // byte offset of the stripe's trace block
+    int counted = 0;                  // PIPE: the stripes whose blocks it counts
     bool gave_up = false;             // PIPE: a wait ran past its bound
 
     for (int s = PIPE ? p0 : 0; s < nstripes; s += PIPE ? P : 1) {
@@ -448,10 +456,9 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
             prev_r0 = 1;
             prev_r1 = 0;
             if (s > 0) stripe_rows(jb.la, jb.lb, jb.band, STRIPE_W, s - 1, prev_r0, prev_r1);
-            tbs = 0;
-            for (int q = 0; q < s; ++q) {
+            for (; counted < s; ++counted) {
                 int a0, a1;
-                stripe_rows(jb.la, jb.lb, jb.band, STRIPE_W, q, a0, a1);
+                stripe_rows(jb.la, jb.lb, jb.band, STRIPE_W, counted, a0, a1);
                 if (a1 >= a0) tbs += (uint64_t)(a1 - a0 + G) * G * LANE_BYTES;
             }
             unsigned long long *pb = reinterpret_cast<unsigned long long *>(bnd + jb.bnd_off);
@@ -518,10 +525,11 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
         }
         int outH = CELL::neg_h(), outF = CELL::neg_f(), rlo = 0, rhi = 0;
 
-        // lane 0's inputs, G rows per chunk: column jl-1 of the previous stripe
-        // where it computed that row, column 0, or outside; and A's letters.
-        // The next chunk is loaded one chunk ahead.  (PIPE: the words are
-        // fetched here, for rows this stripe computes, and settled before use)
+        // lane 0's inputs, CH rows per chunk (a lane a row): column jl-1 of the
+        // previous stripe where it computed that row, column 0, or outside;
+        // and A's letters.  The next chunk is loaded one chunk ahead.  (PIPE: the
+        // words are fetched here, for rows this stripe computes, and settled
+        // before use)
         unsigned long long wH = 0, wF = 0;
         bool want = false;
         int wrow = 0;
@@ -529,7 +537,9 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
             const int i = r0 + x;
             h = s == 0 ? CELL::edge() : CELL::neg_h();
             f = CELL::neg_f();
+            ac = 0;
             if constexpr (PIPE) want = false;
+            if (CH < G && lane >= CH) return;
             if (s > 0 && i >= prev_r0 && i <= prev_r1) {
                 if constexpr (PIPE) {
                     want = i <= r1;
@@ -543,7 +553,7 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
                     f = bF[i - 1];
                 }
             }
-            ac = i <= r1 ? a[i - 1] : 0u;
+            if (i <= r1) ac = a[i - 1];
         };
         int nH, nF;
         uint32_t nA;
@@ -551,9 +561,18 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
 
         const int nsteps = nrows + nl - 1;
         const uint32_t my_rows = lane < nl ? (uint32_t)nrows : 0u;
-        uint8_t *dst = tbj + tbs + (size_t)lane * LANE_BYTES;
+        uint8_t *dst = tbj + tbs;
+        const uint32_t dst_lane = (uint32_t)lane * LANE_BYTES;
+        // The last lane's values go to the step's slot of the chunk (the other
+        // lanes' to a slot no one reads).
+        int2 *const out_slot = lane == G - 1 ? &lds.out[gb] : &lds.idle[threadIdx.x & 63];
+        const int out_next = lane == G - 1 ? 1 : 0;
+        // (nothing loaded above is waited for inside the step loop, where the
+        // wait would be for the last step's store too)
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+        int4 ahead = make_int4(0, 0, 0, 0);
         for (int t = 0; t < nsteps; ++t) {
-            const int q = t & (G - 1);
+            const int q = t & (CH - 1);
             if (q == 0) {
                 if constexpr (PIPE) {
                     settle(want, wrow, wH, wF);
@@ -561,13 +580,26 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
                         nH = (int)(uint32_t)wH;
                         nF = (int)(uint32_t)wF;
                     }
+                    // A SIMD gives its oldest wavefront every slot it can use, and
+                    // the parts of a job wait for the slowest of them: each
+                    // wavefront's priority falls with its progress, modulo four
+                    // chunks, so that those that fell behind go first.
+                    switch ((t / CH) & 3) {
+                    case 0: __builtin_amdgcn_s_setprio(3); break;
+                    case 1: __builtin_amdgcn_s_setprio(2); break;
+                    case 2: __builtin_amdgcn_s_setprio(1); break;
+                    default: __builtin_amdgcn_s_setprio(0); break;
+                    }
                 }
                 int lo, hi;
                 CELL::operand(sc, nA, lo, hi);
-                lds.in[gb + lane] = make_int4(nH, nF, lo, hi);
-                left_in(t + G + lane, nH, nF, nA);
+                if (CH == G || lane < CH) lds.in[gb + lane] = make_int4(nH, nF, lo, hi);
+                left_in(t + CH + lane, nH, nF, nA);
+                ahead = lds.in[gb];
             }
-            const int4 in = lds.in[gb + q];
+            // row r0 + t - lane of every lane that has one
+            const int4 in = ahead;
+            ahead = lds.in[gb + ((q + 1) & (CH - 1))];   // the next step's
             const int rH = shr1_group<G>(outH, in.x);
             const int rF = shr1_group<G>(outF, in.y);
             rlo = shr1_group<G>(rlo, in.z);
@@ -577,31 +609,29 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
                 lpH = rH;
                 outH = st.H[COLS - 1];
                 outF = st.F[COLS - 1];
-                store_records<COLS>(dst, st.word);
+                store_records<COLS>(dst + dst_lane, st.word);
             }
             dst += G * LANE_BYTES;
-            if (!last_stripe) {
-                // the last lane just finished relative row t-(G-1) of the stripe's last column
-                const int xl = t - (G - 1);
-                if (lane == G - 1 && xl >= 0 && xl < nrows) lds.out[gb + (xl & (G - 1))] = make_int2(outH, outF);
-                if (xl >= 0 && xl < nrows && ((xl & (G - 1)) == G - 1 || xl == nrows - 1)) {
-                    const int x = (xl & ~(G - 1)) + lane;
-                    if (x < nrows) {
-                        const int r = r0 - 1 + x;
-                        const int2 v = lds.out[gb + lane];
-                        if constexpr (PIPE) {
-                            const unsigned long long tag = (unsigned long long)(uint32_t)(s + 1) << 32;
-                            __hip_atomic_store(pout + r, tag | (uint32_t)v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            __hip_atomic_store(pout + nr + r, tag | (uint32_t)v.y, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                        } else {
-                            bH[r] = v.x;
-                            bF[r] = v.y;
-                        }
+            out_slot[q * out_next] = make_int2(outH, outF);
+            if ((q == CH - 1 || t == nsteps - 1) && !last_stripe && (CH == G || lane < CH)) {
+                // the rows of the stripe's last column that this chunk finished
+                const int x = t - q - (G - 1) + lane;
+                if (x >= 0 && x < nrows) {
+                    const int r = r0 - 1 + x;
+                    const int2 v = lds.out[gb + lane];
+                    if constexpr (PIPE) {
+                        const unsigned long long tag = (unsigned long long)(uint32_t)(s + 1) << 32;
+                        __hip_atomic_store(pout + r, tag | (uint32_t)v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(pout + nr + r, tag | (uint32_t)v.y, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    } else {
+                        bH[r] = v.x;
+                        bF[r] = v.y;
                     }
                 }
             }
         }
+        if constexpr (PIPE) __builtin_amdgcn_s_setprio(0);
         if (last_stripe) {
             // the lane's registers hold row LA, the last it computed: the
             // final cell's values, picked by way of LDS, so that no
@@ -631,7 +661,7 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
         }
         prev_r0 = r0;
         prev_r1 = r1;
-        tbs += (uint64_t)(nrows + G - 1) * G * LANE_BYTES;
+        if constexpr (!PIPE) tbs += (uint64_t)(nrows + G - 1) * G * LANE_BYTES;
         // the next stripe reads the boundary column, and the walk the records,
         // that other lanes of this wavefront wrote
         if constexpr (!PIPE) __threadfence_block();
@@ -663,12 +693,13 @@ constexpr uint32_t ROWS_MAX_WALK = 1024;  // a + b from which a job takes a wave
 // launches of a round take one pointer and are captured in a graph once per
 // context; a round only sets the grid sizes of the graph's nodes.
 constexpr int ROW_SHAPES = 7;
-// QK_PIPE + P - 2 (P = 2 .. 8): 64-lane stripe jobs whose stripes P
+// QK_PIPE + P - 1 (P = 1 .. DP_PIPE_MAX): 64-lane stripe jobs whose stripes P
 // wavefronts share (an item is one wavefront's part: job first + item / P,
 // part item % P)
 enum : uint32_t { QK_STRIPE = 0, QK_ROWS = 1, QK_WINDOW = QK_ROWS + ROW_SHAPES, QK_TINY = QK_WINDOW + 1,
                   QK_PIPE = QK_TINY + 1 };
-constexpr int DPQ_MAXB = 48;
+constexpr uint32_t DP_PIPE_MAX = 32;
+constexpr int DPQ_MAXB = 72;
 constexpr int DPQ_CURSORS = DPQ_MAXB;
 
 // (Behind it in device memory: DPQ_CURSORS cursors, zeroed at the start of every
@@ -928,7 +959,7 @@ __device__ __forceinline__ void dp_window_job(const DevJob &jb, const uint8_t *_
 // 0 and the top row 0, as for the first stripe of dp_job.  Trace: 8 bytes per
 // row, cell (i, j) at byte (i-1)*8 + (j-1)/2, nibble (j-1)%2.
 constexpr int TINY_LB = 16;
-constexpr uint32_t TINY_COLS_TAG = 1;   // DevJob::cols of a one-lane job
+constexpr uint32_t TINY_COLS_TAG = 128;   // DevJob::cols of a one-lane job
 
 __device__ __forceinline__ void tiny_job(const DevJob &jb, const uint8_t *__restrict__ A,
                                          const uint8_t *__restrict__ B, uint8_t *__restrict__ tb,
@@ -1204,7 +1235,7 @@ __device__ __forceinline__ void run_item(DP_FWD_PARAMS, const float *table, uint
 {
     int score = 0, edge = 'M';
     if (kind >= QK_PIPE) {
-        const uint32_t P = kind - QK_PIPE + 2;
+        const uint32_t P = kind - QK_PIPE + 1;
         const uint32_t x = first + item / P;
         const int p0 = (int)(item % P);
         const DevJob jb = jobs[x];
@@ -1215,6 +1246,11 @@ __device__ __forceinline__ void run_item(DP_FWD_PARAMS, const float *table, uint
                 fin = dp_job<CELL, 16, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
         } else if (jb.cols == 8) {
             fin = dp_job<CELL, 8, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
+        } else if (std::is_same<CELL, IntCell>::value && jb.cols <= 2) {
+            if constexpr (std::is_same<CELL, IntCell>::value) {
+                if (jb.cols == 2) fin = dp_job<CELL, 2, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
+                else fin = dp_job<CELL, 1, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
+            }
         } else {
             fin = dp_job<CELL, 4, 64, true>(jb, A, B, tb, bnd, sc, table, lds, score, edge, p0, (int)P, err);
         }
@@ -1294,9 +1330,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     const uint32_t nb = rd->nbins;
     if constexpr (!PERSIST) {
         const uint32_t w = blockIdx.x;
-        uint32_t b = 0;
-        while (b + 1 < nb && w >= rd->item0[b + 1]) ++b;
-        if (b >= nb || w >= rd->item0[nb]) return;
+        if (nb == 0 || w >= rd->item0[nb]) return;
+        uint32_t b = 0;    // the last bin that starts at or before item w
+        for (uint32_t len = nb; len > 1;) {
+            const uint32_t half = len >> 1;
+            if (rd->item0[b + half] <= w) { b += half; len -= half; }
+            else len = half;
+        }
         uint32_t item = w - rd->item0[b];
         if (rd->kind[b] >= QK_PIPE) {
             // a ticket, so that the parts of a job are taken in order by
@@ -1365,6 +1405,7 @@ struct DpItem {
     uint32_t cols;
     uint64_t tb_bytes;
     uint64_t cells;   // of the region evaluated, padding included
+    uint32_t parts;   // wavefronts that share its stripes (0: not pipelined)
 };
 
 // Relative cost per computed cell of the stripe shapes, used to pick a banded
@@ -1807,6 +1848,113 @@ static uint64_t fixed_need(uint64_t cnt, uint64_t tbb, uint64_t bi)
     return DP_ROUND_BYTES + align256(cnt * (sizeof(DevJob) + sizeof(DpOut) + 4)) + align256(bi * 4) + tbb + 256;
 }
 
+// Pipelined stripe jobs.  Where the longest job takes longer on its own wavefront
+// than the round's work shared evenly by the forward launch's wavefront slots,
+// SIMDs would be idle at the end.  Then the jobs above a quarter of a slot's share
+// spread their stripes over several wavefronts, and a long banded job of 16-lane
+// stripes (a quarter of a wavefront, its stripes one after the other) takes all 64
+// lanes, with a quarter of the columns a lane: the same stripes, so the same
+// region.  A job's time is its steps times the instructions of a step; with P
+// wavefronts it is that of ceil(stripes / P) stripes.  A quarter, since an even end
+// is worth more than the lags between parts (46.4 ms on the 4,000 jobs below;
+// spreading the jobs above 0.4, 0.6, 0.8 and 1.05 shares 47.9, 50.0, 53.6 and 58.6;
+// parts of a whole share 52.3, of two 58.4); equal jobs are left alone (3,072 of
+// 2,048 columns 4.9 ms, spread 5.3).  A banded job's stripe starts when the one
+// before it has sent the row the stripe starts at, its row shift and the lanes'
+// skew later, so more parts than a stripe's steps over that lag would only wait.
+// Pipelined jobs start first.  items[0, n): the round's stripe jobs (every lane
+// shape), longest first; other: its remaining wavefronts.  MH_DP_PIPE = P (p_env)
+// instead gives P wavefronts to the first 64-lane jobs with at least P stripes,
+// as many as the idle slots hold.
+//
+// Measured, with the parts' priorities (dp_job): 4,000 jobs of 10-20,000 columns
+// (at most 8 parts a job, all the round's wavefronts fitting the slots together,
+// before) 75.9 -> 46.4 ms, a learned band's run over 6,000 such jobs 55.8 -> 19.7
+// ms.  Left: a part alone on its SIMD issues an instruction every six cycles
+// instead of four, and a banded job's stripes wait for each other (9 ms for 20,000
+// columns).
+static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_t other, uint64_t simds, int wpe,
+                       int p_env)
+{
+    auto group = [](const DpItem &it) { return it.cols > GROUP_TAG; };
+    auto cols_of = [&](const DpItem &it) { return group(it) ? it.cols - GROUP_TAG : it.cols; };
+    double est = 0;     // wavefronts of the round as it stands
+    bool wide = false;
+    for (uint64_t x = 0; x < n; ++x) {
+        est += group(items[x]) ? 0.25 : 1.0;
+        if (cols_of(items[x]) > 8) wide = true;
+    }
+    const bool tagged = wpe < 0;     // (only these cells have the one- and two-column lanes)
+    if (tagged) wpe = FWD_VARIANTS[dp_variant_for(wide)].wpe;
+    const double slots = std::max(1.0, (double)(simds * (uint64_t)wpe) - (double)other);
+    if (p_env > 1) {
+        if (est >= slots) return;
+        double used = est;
+        for (uint64_t x = 0; x < n; ++x) {
+            DpItem &it = items[x];
+            const uint64_t ns = (jobs[it.job].b_len + 64ull * it.cols - 1) / (64ull * it.cols);
+            if (group(it) || ns < (uint64_t)p_env || used + p_env - 1 > slots) continue;
+            it.parts = (uint32_t)p_env;
+            used += p_env - 1;
+        }
+        return;
+    }
+    // instructions of a step: about 24 around the cells, 12.4 a cell
+    auto step_cost = [](uint32_t cols) { return 24.0 + 12.4 * cols; };
+    struct Opt {
+        double own, stripe;    // time on its own; of one stripe when pipelined
+        uint32_t ns, pmax;
+        float weight;
+    };
+    std::vector<Opt> opt(n);
+    double total = 0, longest = 0;
+    for (uint64_t x = 0; x < n; ++x) {
+        const DpItem &it = items[x];
+        const mh_dp_job &jb = jobs[it.job];
+        const uint32_t c = cols_of(it), g = group(it) ? 16 : 64, sw = g * c;
+        Opt &o = opt[x];
+        const double steps = (double)(it.cells / ((uint64_t)g * c));
+        o.own = steps * step_cost(c);
+        o.ns = (jb.b_len + sw - 1) / sw;
+        o.weight = group(it) ? 0.25f : 1.0f;
+        o.pmax = 0;
+        const bool widen = tagged && group(it) && it.band != 0 && (c == 4 || c == 8);
+        if (o.ns > 1 && (g == 64 || widen)) {
+            const uint32_t c2 = widen ? c / 4 : c;
+            const double rows = steps / o.ns - (g - 1);
+            o.stripe = (rows + 63) * step_cost(c2);
+            o.pmax = std::min(DP_PIPE_MAX, o.ns);
+            if (it.band) {
+                const double lag = (double)jb.a_len * sw / jb.b_len + 63 + (c2 <= 2 ? 16 : 64);
+                o.pmax = std::min<uint32_t>(o.pmax, (uint32_t)std::max(1.0, std::ceil((rows + 63) / lag)));
+            }
+        }
+        total += o.own * o.weight;
+        longest = std::max(longest, o.own);
+    }
+    const double share = total / slots, T = 0.25 * share;
+    if (longest <= 1.1 * share) return;
+    auto parts_of = [&](const Opt &o, bool up) -> uint32_t {
+        if (o.own <= T || !o.pmax) return 0;
+        const double m = std::max(1.0, up ? std::ceil(T / o.stripe) : std::floor(T / o.stripe));   // stripes a part
+        return std::min<uint32_t>(o.pmax, (uint32_t)std::ceil(o.ns / m));
+    };
+    // parts past the slots would run after the others: fewer, longer ones then
+    double all = 0;
+    for (const Opt &o : opt) all += parts_of(o, false);
+    const bool up = all > slots;
+    for (uint64_t x = 0; x < n; ++x) {
+        DpItem &it = items[x];
+        const uint32_t p = parts_of(opt[x], up);
+        if (!p || (p == 1 && !group(it))) continue;
+        it.parts = p;
+        if (group(it)) {
+            it.cols = (it.cols - GROUP_TAG) / 4;
+            it.tb_bytes = dp_steps(jobs[it.job].a_len, jobs[it.job].b_len, it.band, it.cols, 64) * 64 * lane_bytes_of(it.cols);
+        }
+    }
+}
+
 static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
                         const std::vector<uint64_t> &slot, std::vector<DpItem> &items, uint8_t *d_paths,
                         mh_dp_result *d_results, uint32_t *d_dev, uint64_t *cells,
@@ -1872,7 +2020,6 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
     // pipelined stripe jobs: wavefronts a job by the round's size (up to
     // DP_PIPE_MAX), or MH_DP_PIPE (0 or 1 keeps one wavefront a job); the
     // no-allocation path keeps one
-    constexpr uint32_t DP_PIPE_MAX = 8;
     int pipe_env = -1;
     if (const char *e = getenv("MH_DP_PIPE")) pipe_env = std::max(0, std::min((int)DP_PIPE_MAX, atoi(e)));
     int ncu = 0;
@@ -1881,7 +2028,6 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
 
     uint64_t first = 0;
     std::vector<DpItem> shaped;
-    std::vector<uint8_t> pj;   // wavefronts of each stripe job of a round
     while (first < nitems) {
         // one round: as many jobs (in schedule order) as fit the trace budget
         uint64_t tbb = 0, bi = 0, last = first;
@@ -1908,8 +2054,12 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
                               [](const DpItem &it) { return it.cols < WINDOW_TAG; });
         uint64_t nstripe = 0;
         while (nstripe < nbig && items[first + nstripe].cols < WINDOW_TAG) ++nstripe;
-        // wavefront stripes, then the row-packed jobs by shape (16, 14, ..., 4
-        // columns a lane), each in order: a stable bucket pass
+        if (!fx && ncu > 0)
+            plan_parts(jobs, items.data() + first, nstripe, (nbig - nstripe) + (n - nbig + 63) / 64,
+                       (uint64_t)ncu * 4, form == DpCells::TAGGED ? -1 : FWD_VARIANTS[VARIANT_FLOAT].wpe, pipe_env);
+        // wavefront stripes (the pipelined ones first, most parts first), then
+        // the row-packed jobs by shape (16, 14, ..., 4 columns a lane), each in
+        // order: a stable bucket pass
         auto shape = [](const DpItem &it) {
             return it.cols < GROUP_TAG ? 0 : 1 + (int)(GROUP_TAG + 16 - it.cols) / 2;
         };
@@ -1953,6 +2103,8 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             std::copy(shaped.begin(), shaped.end(), items.begin() + (ptrdiff_t)b0);
         }
         const uint64_t n64 = rows_at[1];   // rows_at[1..]: the row jobs, 16 columns a lane first
+        std::stable_sort(items.begin() + (ptrdiff_t)first, items.begin() + (ptrdiff_t)(first + n64),
+                         [](const DpItem &x, const DpItem &y) { return x.parts > y.parts; });
         // the forward variant: the wide one when a shape wider than 8 columns a lane is in the round
         bool wide = false;
         for (uint64_t z = 0; z < n64 && !wide; ++z) wide = items[first + z].cols == 16;
@@ -1960,76 +2112,10 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             if (rows_at[q + 2] > rows_at[q + 1]) wide = true;
         const int variant = form == DpCells::TAGGED ? dp_variant_for(wide)
                                                     : (form == DpCells::FLOAT ? VARIANT_FLOAT : VARIANT_LONG);
-        // Pipelined stripe jobs.  A round with fewer work items than the
-        // forward launch's wavefront slots ends on its longest jobs' latency
-        // with SIMDs idle: its 64-lane stripe jobs then run on P_j wavefronts
-        // each.  P_j = ceil(W_j / T) (W_j the job's trace bytes, a measure of
-        // its cells), at most DP_PIPE_MAX and the job's stripes, with the
-        // smallest T whose parts fit the slots; so the parts are of about
-        // one size.  MH_DP_PIPE = P instead gives P wavefronts to the first
-        // jobs with at least P stripes, as many as the idle slots hold.
-        // Pipelined jobs go to the front of the queue, most parts first.
         uint64_t npipe = 0;
-        pj.assign(n64, 1);
-        if (!fx && ncu > 0) {
-            uint64_t items_est = n64 + (nbig - nstripe) + (n - nbig + 63) / 64;
-            for (int q = 0; q < ROW_SHAPES; ++q) items_est += (rows_at[q + 2] - rows_at[q + 1] + 3) / 4;
-            const uint64_t slots = (uint64_t)ncu * 4 * (uint64_t)FWD_VARIANTS[variant].wpe;
-            auto nstr = [&](const DpItem &it) {
-                const uint64_t sw = 64ull * it.cols;
-                return (jobs[it.job].b_len + sw - 1) / sw;
-            };
-            if (items_est < slots && pipe_env > 1) {
-                const uint64_t kmax = (slots - items_est) / (uint64_t)(pipe_env - 1);
-                for (uint64_t x = 0, k = 0; x < n64 && k < kmax; ++x)
-                    if (nstr(items[first + x]) >= (uint64_t)pipe_env) {
-                        pj[x] = (uint8_t)pipe_env;
-                        ++k;
-                    }
-            } else if (items_est < slots) {
-                const uint64_t room = slots - (items_est - n64);   // wavefronts for the stripe jobs
-                auto parts = [&](double T, bool set) {
-                    uint64_t tot = 0;
-                    for (uint64_t x = 0; x < n64; ++x) {
-                        const DpItem &it = items[first + x];
-                        const uint64_t cap = std::min<uint64_t>(DP_PIPE_MAX, nstr(it));
-                        const uint64_t q = std::max<uint64_t>(1, std::min<uint64_t>(cap, (uint64_t)std::ceil((double)it.tb_bytes / T)));
-                        tot += q;
-                        if (set) pj[x] = (uint8_t)q;
-                    }
-                    return tot;
-                };
-                double wmax = 1;
-                for (uint64_t x = 0; x < n64; ++x) wmax = std::max(wmax, (double)items[first + x].tb_bytes);
-                double lo = wmax / (2.0 * DP_PIPE_MAX), hi = wmax;   // parts(hi) = n64 <= room
-                for (int it = 0; it < 48; ++it) {
-                    const double mid = 0.5 * (lo + hi);
-                    (parts(mid, false) <= room ? hi : lo) = mid;
-                }
-                parts(hi, true);
-            }
-            for (uint64_t x = 0; x < n64; ++x) npipe += pj[x] > 1;
-            if (npipe) {
-                // most parts first, each part count in order; then the others
-                shaped.clear();
-                std::vector<uint8_t> pj2;
-                for (uint32_t P = DP_PIPE_MAX; P >= 2; --P)
-                    for (uint64_t x = 0; x < n64; ++x)
-                        if (pj[x] == P) {
-                            shaped.push_back(items[first + x]);
-                            pj2.push_back((uint8_t)P);
-                        }
-                for (uint64_t x = 0; x < n64; ++x)
-                    if (pj[x] <= 1) {
-                        shaped.push_back(items[first + x]);
-                        pj2.push_back(1);
-                    }
-                std::copy(shaped.begin(), shaped.end(), items.begin() + (ptrdiff_t)first);
-                pj.swap(pj2);
-                // (a count under the timers' names: pipelined jobs a round)
-                host_time(ctx, "dp_pipe_jobs", (double)npipe);
-            }
-        }
+        while (npipe < n64 && items[first + npipe].parts) ++npipe;
+        // (a count under the timers' names: pipelined jobs a round)
+        if (npipe) host_time(ctx, "dp_pipe_jobs", (double)npipe);
         DevJob *dj = nullptr;
         std::vector<DevJob> host_jobs;
         if (fx) {
@@ -2112,8 +2198,8 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             // the pipelined jobs first, a bin for each part count, an item a part
             for (uint64_t x = 0; x < npipe;) {
                 uint64_t y = x + 1;
-                while (y < npipe && pj[y] == pj[x]) ++y;
-                add_bin(QK_PIPE + (pj[x] - 2u), x, (y - x) * pj[x]);
+                while (y < npipe && items[first + y].parts == items[first + x].parts) ++y;
+                add_bin(QK_PIPE + (items[first + x].parts - 1u), x, (y - x) * items[first + x].parts);
                 x = y;
             }
             auto cls = [](uint64_t v) { return v ? (63 - __builtin_clzll(v)) / 2 : 0; };
@@ -2171,13 +2257,10 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             if ((rc = dp_launch_round(ctx, variant, dp_use_graph(), grid, ra)) != MH_OK) return rc;
         }
         // the host job table is reused by the next round
+        uint32_t err = 0;
+        if (npipe) MH_HIP(hipMemcpyAsync(&err, ra.cursor + (DPQ_CURSORS - 1), 4, hipMemcpyDeviceToHost, ctx->stream));
         MH_HIP(hipStreamSynchronize(ctx->stream));
-        if (npipe) {
-            uint32_t err = 0;
-            MH_HIP(hipMemcpyAsync(&err, ra.cursor + (DPQ_CURSORS - 1), 4, hipMemcpyDeviceToHost, ctx->stream));
-            MH_HIP(hipStreamSynchronize(ctx->stream));
-            MH_CHECK(err == 0, MH_ERR_DEVICE, "DP: a pipelined stripe's wait ran past its limit");
-        }
+        MH_CHECK(err == 0, MH_ERR_DEVICE, "DP: a pipelined stripe's wait ran past its limit");
         first = last;
     }
     return MH_OK;
@@ -2228,6 +2311,7 @@ static DpItem make_item(const mh_dp_job &jb, uint32_t job, uint32_t band, int fo
 {
     DpItem it;
     it.job = job;
+    it.parts = 0;
     it.cols = dp_cols_for(jb.a_len, jb.b_len, band, force, rerun);
     it.band = dp_effective_band(jb.a_len, jb.b_len, band, it.cols);
     if (it.band == 0 && band != 0) it.cols = dp_cols_for(jb.a_len, jb.b_len, 0, force);
@@ -2276,8 +2360,8 @@ uint64_t dp_item_cells(uint32_t la, uint32_t lb, uint32_t band)
 {
     if (la == 0 || lb == 0) return 0;
     const DpItem it = make_item(mh_dp_job{0, 0, la, lb}, 0, band, dp_force_cols());
-    if (it.cols > WINDOW_TAG) return (uint64_t)la * 64 * (it.cols - WINDOW_TAG);
     if (it.cols == TINY_COLS_TAG) return (uint64_t)la * lb;
+    if (it.cols > WINDOW_TAG) return (uint64_t)la * 64 * (it.cols - WINDOW_TAG);
     return it.cells;
 }
 

@@ -123,6 +123,44 @@ def test_pipelined_banded_matches_region_oracle(ctx, dp_env, cols):
         assert got == ref, P
 
 
+def test_narrow_banded_stripes_over_all_lanes(ctx, dp_env):
+    """Jobs of 16-lane stripes that the round spreads take all 64 lanes, one or
+    two columns a lane, over the same stripes: columns at a stripe's edges, one
+    row, rows at the chunks' edges, operands far from square."""
+    rng = np.random.default_rng(730)
+    shapes = [(1, 300), (15, 129), (16, 128), (17, 65), (400, 63), (900, 64), (1023, 1025), (700, 641), (1600, 1500),
+              (2100, 1000), (1000, 2300)]
+    pairs = [_related(rng, la, lb, 0.05) for la, lb in shapes for _ in range(3)]
+    bands = np.array([2, 9, 40] * len(shapes), dtype=np.uint32)
+    A, B, jobs = _batch(pairs)
+    os.environ.pop("MH_DP_COLS", None)
+    os.environ["MH_DP_BAND_KIND"] = "stripes"
+    got = {}
+    for P in ("1", "auto"):
+        if P == "auto":
+            os.environ.pop("MH_DP_PIPE", None)
+        else:
+            os.environ["MH_DP_PIPE"] = P
+        ctx.set_timing(True)
+        ctx.reset_kernel_times()
+        paths, res, dev, st = mauvehip.global_align_banded(ctx, A, B, jobs, bands, flags=mauvehip.BAND_NO_FALLBACK)
+        assert (_pipe_parts(ctx) > 0) == (P == "auto")
+        ctx.set_timing(False)
+        got[P] = [(mauvehip.path_of(paths, res, k), int(res[k]["score"]), int(dev[k]), int(res[k]["path_len"]))
+                  for k in range(len(pairs))]
+    narrow = 0
+    for k, (a, b) in enumerate(pairs):
+        eff, kind, width = mauvehip.band_region(len(a), len(b), 2 * int(bands[k]))
+        narrow += kind == mauvehip.REGION_STRIPES and width <= 128 and len(b) > width
+        p, sc, dv = po.nwsmall_region(a, b, eff, width if kind == mauvehip.REGION_STRIPES else 0)
+        if p is None:
+            assert got["auto"][k][3] == 0
+        else:
+            assert got["auto"][k][:3] == (p, sc, dv), (k, len(a), len(b), int(bands[k]))
+    assert narrow > 10
+    assert got["1"] == got["auto"]
+
+
 def test_pipelined_prefix_with_many_small_jobs(ctx, dp_env):
     """A round whose work items nearly fill the slots pipes only a prefix of
     its stripe jobs; the output equals the unpipelined one."""
