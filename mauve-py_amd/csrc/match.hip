@@ -2014,14 +2014,14 @@ __global__ void uq_chain_fill_kernel(const uint32_t *__restrict__ is_head, const
     ext_len[s] = ext_len[h];
 }
 
-// ---- AddHashEntry of the unique seeds, one bucket per thread --------------
+// ---- AddHashEntry of the unique seeds, one bucket per wavefront -----------
 // AddHashEntry (LM/MemHash.cpp:209-251) keeps each of the 40000 buckets a
 // vector sorted by MheCompare and inserts with std::lower_bound; buckets never
-// interact, so each is replayed literally by one thread, its seeds in HashMatch
-// order (a stable sort by bucket): the seed is looked up, a collision when the
-// entry at the lower bound compares equal, else the seed's extension (offset
-// kept, mersize 0) goes in at its own lower bound.  The bucket's vector holds
-// seed indices (an entry is its seed's extension).
+// interact, so each is replayed literally by one wavefront, its seeds in
+// HashMatch order (a stable sort by bucket): the seed is looked up, a collision
+// when the entry at the lower bound compares equal, else the seed's extension
+// (offset kept, mersize 0) goes in at its own lower bound.  The bucket's vector
+// leaves the kernel as seed indices (an entry is its seed's extension).
 
 struct UqSeeds {
     const int32_t *sst, *est;   // seed starts, extension starts (k a seed)
@@ -2048,15 +2048,255 @@ template <class E> __device__ __forceinline__ void uq_entry(const UqSeeds &q, ui
 }
 
 __global__ void uq_bucket_kernel(const int64_t *__restrict__ off, uint64_t ns, uint64_t *__restrict__ key,
-                                 uint32_t *__restrict__ val, uint32_t *__restrict__ cnt)
+                                 uint32_t *__restrict__ val)
 {
     const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= ns) return;
     const int64_t m = off[x] % 40000;
-    const uint32_t b = (uint32_t)(m < 0 ? m + 40000 : m);
-    key[x] = b;
+    key[x] = (uint64_t)(m < 0 ? m + 40000 : m);
     val[x] = (uint32_t)x;
-    atomicAdd(&cnt[b], 1u);
+}
+
+// start[q] = the first sorted seed of bucket q or a later one, start[nb] = ns
+// (a counter per bucket took 1.7 ms of atomics at 7 million seeds)
+__global__ void uq_bstart_kernel(const uint64_t *__restrict__ sk, uint64_t ns, uint32_t nb, uint32_t *__restrict__ start)
+{
+    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= ns) return;
+    const uint32_t q = (uint32_t)sk[r];
+    for (uint32_t t = r == 0 ? 0 : (uint32_t)sk[r - 1] + 1; t <= q; ++t) start[t] = (uint32_t)r;
+    if (r + 1 == ns)
+        for (uint32_t t = q + 1; t <= nb; ++t) start[t] = (uint32_t)ns;
+}
+
+// What MheCompare reads of an entry first: the first present genome's start,
+// the length, and in one word the offset (|off| < 15 * 2^32), the presence
+// mask and the LDS slot with all the starts.
+struct alignas(16) UqHead {
+    int32_t sf;
+    uint32_t len;
+    uint64_t w;      // offset << 26 | mask << 10 | slot
+};
+
+__device__ __forceinline__ uint32_t uq_norm(int32_t s, uint32_t len, uint32_t mersize)
+{
+    return s < 0 ? 0u - (uint32_t)s + len - mersize : (uint32_t)s;
+}
+
+// MheCompare both ways: -1 when the stored entry a (mersize 0) is below q, 1
+// when q is below a, 0 when neither.  The lowest genome present in one only
+// decides (the entry that holds it is the larger: FirstStart and the presence
+// tests alike), then containment, then the starts in genome order
+// (LM/MatchHashEntry.h:121-143); the first present genome's nearly always
+// settles the last two, and the other starts are read only when it does not.
+// Genomes below 2^29 bases, so that the differences of starts and lengths, and
+// of those, stay within 32 bits.
+template <int K>
+__device__ __forceinline__ int uq_cmp(const UqHead &a, const UqHead &q, uint32_t qmers, const int32_t *__restrict__ bodies,
+                                      const int32_t (&sq)[K])
+{
+    const uint64_t x = a.w ^ q.w;
+    const uint32_t md = (uint32_t)(x >> 10) & 0xFFFFu;
+    if (md) return ((uint32_t)(q.w >> 10) & md & (0u - md)) ? -1 : 1;
+    const uint32_t na = uq_norm(a.sf, a.len, 0), nq = uq_norm(q.sf, q.len, qmers);
+    const int32_t diff = q.sf - a.sf, dlen = (int32_t)q.len - (int32_t)a.len;
+    // by the first genome: a contains q, q contains a
+    bool ab = diff >= 0 && dlen + diff <= 0, ba = diff <= 0 && dlen + diff >= 0;
+    if ((x >> 26) == 0 && (ab || ba)) {
+        const int32_t *sa = bodies + (uint32_t)(a.w & 1023u) * K;
+        const int32_t diff_rc = dlen + diff;
+#pragma unroll
+        for (int g = 0; g < K; ++g) {
+            const int32_t as = sa[g], bs = sq[g], di = bs - as;
+            const bool skip = as == 0 || di == diff, rc = di == diff_rc;      // (absent in both: 0)
+            ab = ab && (skip || (bs < 0 && rc));
+            ba = ba && (skip || (as < 0 && rc));
+        }
+        if (ab || ba) return 0;
+    }
+    if (na == nq) {
+        const int32_t *sa = bodies + (uint32_t)(a.w & 1023u) * K;
+        int res = 0;
+#pragma unroll
+        for (int g = K - 1; g >= 0; --g) {
+            const uint32_t ma = uq_norm(sa[g], a.len, 0), mq = uq_norm(sq[g], q.len, qmers);
+            if (sa[g] != 0 && ma != mq) res = ma < mq ? -1 : 1;
+        }
+        return res;
+    }
+    return na < nq ? -1 : 1;
+}
+
+// std::lower_bound of one entry e by the whole wavefront, one probe each of the
+// next six levels of the probe tree a lane, the path taken from a ballot.
+template <int K>
+__device__ __forceinline__ uint32_t uq_insert_at(const UqHead *head, const int32_t *body, uint32_t n, const UqHead &e,
+                                                 const int32_t (&es)[K])
+{
+    const int node = threadIdx.x + 1;                    // heap index of this lane's probe, 1..63
+    const int lvl = 31 - __builtin_clz((unsigned)node);
+    uint32_t first = 0, len = n;
+    while (len > 0) {
+        uint32_t f = first, l = node < 64 ? len : 0;
+        for (int bt = lvl - 1; bt >= 0; --bt) {
+            const uint32_t half = l >> 1;
+            if ((node >> bt) & 1) {                      // the probe was below e: right half
+                f += half + 1;
+                l = l ? l - half - 1 : 0;
+            } else {
+                l = half;
+            }
+        }
+        bool lt = false;
+        if (l > 0) lt = uq_cmp<K>(head[f + (l >> 1)], e, 0, body, es) < 0;
+        const uint64_t below = __ballot(lt);             // bit node - 1
+        for (int s = 0, at = 1; s < 6 && len > 0; ++s) {
+            const uint32_t half = len >> 1;
+            if ((below >> (at - 1)) & 1ull) {
+                first += half + 1;
+                len -= half + 1;
+                at = 2 * at + 1;
+            } else {
+                len = half;
+                at = 2 * at;
+            }
+        }
+    }
+    return first;
+}
+
+// One wavefront per bucket, 64 seeds at a time, one a lane.  Every lane runs
+// its own seed's lower bound against the vector as it stands, with libstdc++'s
+// probe sequence (MheCompare is not a strict weak order, so the probes must be
+// exactly those).  The lanes before the first that is no collision have seen
+// the vector the replay would show them and are done; that seed's extension
+// goes in, and the lanes after it search again.  Four of five seeds are collisions in eight genomes of 5 Mb.
+// The end of a range is always n or the last probe that was not below the seed,
+// so the comparison there is the one at the result.
+//
+// The work is a chain of dependent reads (a seed's probes, and a bucket's
+// insertions), so everything probed lies in LDS: a 16-byte head an entry in the
+// vector's order, shifted on insertion, and the starts by slot.  CAP entries
+// fit; a seed that would be the next one ends the kernel's part of the bucket,
+// which uq_replay_rest_kernel takes on from there.  Buckets come largest first.
+// Eight genomes of 5 Mb (7.05 million seeds, 1.41 million matches, at most 966
+// in a bucket): 12.0 ms; the search by 63 lanes, one probe each of the next
+// six levels, on entries in device memory, took 104.5, its 128 GB of scattered
+// reads.
+template <int K, int CAP>
+__global__ __launch_bounds__(64) void uq_replay_kernel(UqSeeds q, const uint32_t *__restrict__ list,
+                                                       const uint32_t *__restrict__ order,
+                                                       const uint32_t *__restrict__ bstart, uint32_t *__restrict__ vec,
+                                                       uint32_t *__restrict__ nent, uint32_t *__restrict__ resume,
+                                                       unsigned long long *__restrict__ coll)
+{
+    static_assert(CAP % 256 == 0 || CAP == 128 || CAP == 64, "chunks of the shift");
+    static_assert(CAP <= 1024, "ten bits of slot");
+    constexpr int SH = CAP < 256 ? CAP / 64 : 4;       // chunks of 64 entries a step of the shift
+    __shared__ UqHead head[CAP];
+    __shared__ int32_t body[CAP * K];
+    __shared__ uint32_t xs[CAP];
+    const uint32_t b = list[blockIdx.x];
+    const int lane = threadIdx.x;
+    const uint32_t y0 = bstart[b], y1 = bstart[b + 1];
+    uint32_t ne = 0, stop = y1;
+    unsigned long long c = 0;
+    for (uint32_t base = y0; base < y1 && stop == y1; base += 64) {
+        const bool valid = base + lane < y1;
+        const uint32_t x = order[valid ? base + lane : base];
+        int32_t cs[K], es[K];
+        uint32_t cm = 0, em = 0;
+        UqHead ch, eh;
+        ch.sf = 0;
+        eh.sf = 0;
+#pragma unroll
+        for (int g = K - 1; g >= 0; --g) {
+            cs[g] = g < q.k ? q.sst[(uint64_t)x * q.k + g] : 0;
+            es[g] = g < q.k ? q.est[(uint64_t)x * q.k + g] : 0;
+            if (cs[g]) {
+                cm |= 1u << g;
+                ch.sf = cs[g];
+            }
+            if (es[g]) {
+                em |= 1u << g;
+                eh.sf = es[g];
+            }
+        }
+        const uint64_t off = (uint64_t)q.off[x] << 26;
+        ch.len = (uint32_t)q.sl;
+        ch.w = off | ((uint64_t)cm << 10);
+        eh.len = q.elen[x];
+        eh.w = off | ((uint64_t)em << 10);
+        int done = 0;
+        while (done < 64) {
+            const bool active = valid && lane >= done;
+            uint32_t f = 0, l = active ? ne : 0;
+            bool eq = false;
+            for (uint32_t lv = ne; lv > 0; lv >>= 1)       // (each probe at least halves the range)
+                if (l > 0) {
+                    const uint32_t half = l >> 1;
+                    const int r = uq_cmp<K>(head[f + half], ch, (uint32_t)q.sl, body, cs);
+                    f = r < 0 ? f + half + 1 : f;
+                    l = r < 0 ? l - half - 1 : half;
+                    eq = r < 0 ? eq : r == 0;
+                }
+            const bool hit = f != ne && eq;
+            const uint64_t live = __ballot(active), in = __ballot(active && !hit);
+            if (!in) {
+                c += __builtin_popcountll(live);
+                break;
+            }
+            const int j = __builtin_ctzll(in);
+            c += __builtin_popcountll(live & ((1ull << j) - 1));
+            if (ne == (uint32_t)CAP) {
+                stop = base + j;
+                break;
+            }
+            UqHead e;
+            int32_t ej[K];
+            e.sf = __builtin_amdgcn_readlane(eh.sf, j);
+            e.len = (uint32_t)__builtin_amdgcn_readlane((int)eh.len, j);
+            e.w = (uint32_t)__builtin_amdgcn_readlane((int)eh.w, j) |
+                  (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(eh.w >> 32), j) << 32;
+#pragma unroll
+            for (int g = 0; g < K; ++g) ej[g] = __builtin_amdgcn_readlane(es[g], j);
+            const uint32_t pos = uq_insert_at<K>(head, body, ne, e, ej);
+            // shift [pos, ne) up by one from the end; every read of a step
+            // before its writes
+            for (int32_t top = (int32_t)ne; top > (int32_t)pos; top -= 64 * SH) {
+                UqHead t[SH];
+#pragma unroll
+                for (int u = 0; u < SH; ++u) {
+                    const int32_t i = top - 64 * (u + 1) + lane;
+                    if (i >= (int32_t)pos) t[u] = head[i];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int u = 0; u < SH; ++u) {
+                    const int32_t i = top - 64 * (u + 1) + lane;
+                    if (i >= (int32_t)pos) head[i + 1] = t[u];
+                }
+                __syncthreads();
+            }
+            if (lane == j) {
+                eh.w |= ne;
+                head[pos] = eh;
+#pragma unroll
+                for (int g = 0; g < K; ++g) body[ne * K + g] = es[g];
+                xs[ne] = x;
+            }
+            __syncthreads();
+            ++ne;
+            done = j + 1;
+        }
+    }
+    uint32_t *v = vec + y0;
+    for (uint32_t i = lane; i < ne; i += 64) v[i] = xs[head[i].w & 1023u];
+    if (lane == 0) {
+        nent[b] = ne;
+        resume[b] = stop;
+        if (c) atomicAdd(coll, c);
+    }
 }
 
 // std::lower_bound over the bucket's vector v[0, n) for q, with libstdc++'s
@@ -2123,25 +2363,28 @@ __device__ uint32_t uq_lower_bound(const UqSeeds &q, const uint32_t *__restrict_
     return first;
 }
 
-// One wavefront per bucket: std::lower_bound's probes as above (the
-// comparisons are the reference's, one at a time, by the first lane); the
-// insertion's shift of the vector's tail runs across the wave, 64 entries a
-// step from the end (every lane reads its entry before any lane writes).
+// The rest of the buckets that outgrew LDS, one wavefront each: std::lower_bound's
+// probes as above; the insertion's shift of the vector's tail runs across the
+// wave, 64 entries a step from the end (every lane reads its entry before any
+// lane writes).
 template <class E>
-__global__ __launch_bounds__(64) void uq_replay_kernel(UqSeeds q, const uint32_t *__restrict__ order,
-                                                       const uint32_t *__restrict__ bstart, uint32_t *__restrict__ vec,
-                                                       uint32_t *__restrict__ nent,
-                                                       unsigned long long *__restrict__ coll)
+__global__ __launch_bounds__(64) void uq_replay_rest_kernel(UqSeeds q, const uint32_t *__restrict__ list,
+                                                            const uint32_t *__restrict__ order,
+                                                            const uint32_t *__restrict__ bstart,
+                                                            uint32_t *__restrict__ vec, uint32_t *__restrict__ nent,
+                                                            const uint32_t *__restrict__ resume,
+                                                            unsigned long long *__restrict__ coll)
 {
     __shared__ E tree[64];
-    const uint32_t b = blockIdx.x;
+    const uint32_t b = list[blockIdx.x];
     const int lane = threadIdx.x;
-    const uint32_t y0 = bstart[b], y1 = bstart[b + 1];
-    uint32_t *v = vec + y0;
-    uint32_t ne = 0;
+    const uint32_t y0 = resume[b], y1 = bstart[b + 1];
+    if (y0 == y1) return;
+    uint32_t *v = vec + bstart[b];
+    uint32_t ne = nent[b];
     unsigned long long c = 0;
     E cand, at_it;
-    if (y0 < y1) uq_entry(q, order[y0], false, cand);
+    uq_entry(q, order[y0], false, cand);
     for (uint32_t y = y0; y < y1; ++y) {
         const uint32_t x = order[y];
         uint32_t pos = 0xFFFFFFFFu;     // insertion point, or none (a collision)
@@ -2259,6 +2502,11 @@ static int uq_extend_by_chains(mh_context *ctx, const int32_t *d_sst, uint64_t S
     return MH_OK;
 }
 
+// Buckets of 2^UQ_LARGE seeds or more have 1,024 entries in LDS, of 2^UQ_SMALL
+// or more 256, the others 128, one a seed.  (Another bin of 512 fills the CUs
+// better but runs after the first: 13.8 against 12.0 ms for the three.)
+constexpr int UQ_LARGE = 9, UQ_SMALL = 7;
+
 int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRanges &live, UniqueSeeds *out)
 {
     MH_CHECK(k >= 2 && k <= EXT_MAXK && k <= PLAN_MAXK, MH_ERR_UNSUPPORTED, "UniqueMatchFinder takes 2 to 16 genomes");
@@ -2329,7 +2577,9 @@ int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRa
     std::memset(&env, 0, sizeof(env));
     env.seed_len = sl;
     env.mer_mask = w >= 32 ? ~0ull : (~0ull << (64 - 2 * w));
+    uint64_t longest = 0;
     for (int g = 0; g < k; ++g) {
+        longest = std::max<uint64_t>(longest, smls[g]->len);
         env.kp[g] = smls[g]->d_keys_pos;
         env.n[g] = smls[g]->n;
         env.L[g] = (int64_t)smls[g]->len;
@@ -2366,26 +2616,41 @@ int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRa
     MH_HIP(hipStreamSynchronize(ctx->stream));
     MH_CHECK(err == 0, MH_ERR_UNSUPPORTED, "seed extension left the sorted mer lists");
     // AddHashEntry, bucket by bucket: seeds ordered by bucket (stable), bucket
-    // starts, one thread per bucket, the list in bucket order
+    // starts, one wavefront per bucket, the list in bucket order
     const double t0 = now_ms();
     constexpr uint32_t NB = 40000;
     if ((rc = b[0].ensure(S * 8 * 2 + 64)) != MH_OK) return rc;
-    if ((rc = b[2].ensure(S * 4 * 2 + (NB + 1) * 4 * 3 + NB * 8 + 256)) != MH_OK) return rc;
+    if ((rc = b[2].ensure(S * 4 * 2 + (NB + 1) * 4 * 4 + NB * 8 + 256)) != MH_OK) return rc;
     uint64_t *bk0 = b[0].as<uint64_t>(), *bk1 = bk0 + S;
     uint32_t *bv0 = b[2].as<uint32_t>(), *bv1 = bv0 + S;
-    uint32_t *bcnt = bv1 + S, *bst = bcnt + (NB + 1), *nent = bst + (NB + 1);
-    uint64_t *outpos = reinterpret_cast<uint64_t *>((reinterpret_cast<uintptr_t>(nent + NB + 1) + 7) & ~(uintptr_t)7);
-    MH_HIP(hipMemsetAsync(bcnt, 0, (NB + 1) * 4, ctx->stream));
-    hipLaunchKernelGGL(uq_bucket_kernel, dim3((unsigned)((S + 255) / 256)), dim3(256), 0, ctx->stream, d_off, S,
-                       bk0, bv0, bcnt);
+    uint32_t *bst = bv1 + S, *blist = bst + (NB + 1), *nent = blist + NB, *resume = nent + NB;
+    uint64_t *outpos = reinterpret_cast<uint64_t *>((reinterpret_cast<uintptr_t>(resume + NB) + 7) & ~(uintptr_t)7);
+    const dim3 sgrid((unsigned)((S + 255) / 256));
+    hipLaunchKernelGGL(uq_bucket_kernel, sgrid, dim3(256), 0, ctx->stream, d_off, S, bk0, bv0);
     uint64_t *ok;
     uint32_t *order;
     if ((rc = radix_sort_kv(ctx, bk0, bv0, bk1, bv1, S, 16, &ok, &order)) != MH_OK) return rc;
-    std::vector<uint32_t> hc(NB + 1, 0), hs(NB + 1, 0);
-    MH_HIP(hipMemcpyAsync(hc.data(), bcnt, NB * 4, hipMemcpyDeviceToHost, ctx->stream));
+    hipLaunchKernelGGL(uq_bstart_kernel, sgrid, dim3(256), 0, ctx->stream, ok, S, NB, bst);
+    MH_HIP(hipGetLastError());
+    std::vector<uint32_t> hs(NB + 1), hl(NB);
+    MH_HIP(hipMemcpyAsync(hs.data(), bst, (NB + 1) * 4, hipMemcpyDeviceToHost, ctx->stream));
     MH_HIP(hipStreamSynchronize(ctx->stream));
-    for (uint32_t q = 0; q < NB; ++q) hs[q + 1] = hs[q] + hc[q];
-    MH_HIP(hipMemcpyAsync(bst, hs.data(), (NB + 1) * 4, hipMemcpyHostToDevice, ctx->stream));
+    // the buckets by seeds, largest power of two first
+    uint32_t at2[34] = {0};
+    auto cls = [&](uint32_t q) {
+        const uint32_t n = hs[q + 1] - hs[q];
+        return n ? __builtin_clz(n) : 32;       // 0 the largest
+    };
+    for (uint32_t q = 0; q < NB; ++q) ++at2[cls(q) + 1];
+    for (int t = 0; t < 33; ++t) at2[t + 1] += at2[t];
+    uint32_t first[33];
+    std::memcpy(first, at2, sizeof(first));
+    for (uint32_t q = 0; q < NB; ++q) hl[first[cls(q)]++] = q;
+    // (class t holds n < 2^(32 - t))
+    const uint32_t n_large = at2[32 - UQ_LARGE], n_small = at2[32 - UQ_SMALL], n_some = at2[32];
+
+    MH_HIP(hipMemcpyAsync(blist, hl.data(), NB * 4, hipMemcpyHostToDevice, ctx->stream));
+    MH_HIP(hipMemsetAsync(nent, 0, NB * 4, ctx->stream));
     uint32_t *vec = order == bv0 ? bv1 : bv0;     // the other value buffer: S slots
     unsigned long long *d_coll = reinterpret_cast<unsigned long long *>(ok == bk0 ? bk1 : bk0);
     MH_HIP(hipMemsetAsync(d_coll, 0, 8, ctx->stream));
@@ -2398,12 +2663,25 @@ int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRa
     qs.sl = sl;
     {
         TimedLaunch tl(ctx, "partition");
-        if (k <= 8)
-            hipLaunchKernelGGL((uq_replay_kernel<EntT<8, int32_t>>), dim3(NB), dim3(64), 0, ctx->stream, qs, order, bst, vec,
-                               nent, d_coll);
-        else
-            hipLaunchKernelGGL(uq_replay_kernel<EntU>, dim3(NB), dim3(64), 0, ctx->stream, qs, order, bst, vec, nent,
-                               d_coll);
+        auto bin = [&](auto kern, uint32_t lo, uint32_t hi) {
+            if (lo < hi)
+                hipLaunchKernelGGL(kern, dim3(hi - lo), dim3(64), 0, ctx->stream, qs, blist + lo, order, bst, vec, nent,
+                                   resume, d_coll);
+        };
+        if (longest >= (1u << 29)) {     // (uq_cmp's differences past 32 bits)
+            MH_HIP(hipMemcpyAsync(resume, bst, NB * 4, hipMemcpyDeviceToDevice, ctx->stream));
+            bin(uq_replay_rest_kernel<EntU>, 0, n_some);
+        } else if (k <= 8) {
+            bin(uq_replay_kernel<8, 1024>, 0, n_large);
+            bin(uq_replay_kernel<8, 256>, n_large, n_small);
+            bin(uq_replay_kernel<8, 128>, n_small, n_some);
+            bin(uq_replay_rest_kernel<EntT<8, int32_t>>, 0, n_small);
+        } else {
+            bin(uq_replay_kernel<16, 1024>, 0, n_large);
+            bin(uq_replay_kernel<16, 256>, n_large, n_small);
+            bin(uq_replay_kernel<16, 128>, n_small, n_some);
+            bin(uq_replay_rest_kernel<EntU>, 0, n_small);
+        }
         MH_HIP(hipGetLastError());
     }
     std::vector<uint32_t> hn(NB);

@@ -129,3 +129,21 @@ def test_unique_chain_walks_equal_every_seed_walk(ctx, monkeypatch, seed):
     assert st0.collisions == st1.collisions
     assert st0.walks == st0.seed_tuples
     assert 0 < st1.walks < st0.walks
+
+
+@pytest.mark.parametrize("ng,n", [(2, 1500), (3, 5000), (3, 60000), (9, 4000), (9, 24000)])
+def test_unique_many_entries_of_one_bucket(ctx, ng, n):
+    """Genomes that differ by substitutions only have every seed of a genome
+    set at one offset, so one bucket: fewer entries than the smallest bin's
+    capacity, several chunks of an insertion's shift, and more entries than
+    LDS holds (2,000 and more), for up to eight genomes and above."""
+    rng = np.random.default_rng(n + ng)
+    base = rng.integers(0, 4, n)
+    seqs = []
+    for g in range(ng):
+        t = base.copy()
+        hit = rng.random(n) < 0.03
+        t[hit] = (t[hit] + rng.integers(1, 4, int(hit.sum()))) % 4
+        seqs.append("".join("ACGT"[x] for x in t))
+    st = _check(ctx, seqs, (1 << 13) - 1)
+    assert st.matches > n // 40
