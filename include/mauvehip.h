@@ -134,8 +134,8 @@ typedef struct {
     int64_t matches;         /* entries in the match list                    */
     int64_t repeat_runs;     /* SearchRange restarts after runs above
                                 MER_REPEAT_LIMIT (LM/MatchFinder.cpp:253-276)  */
-    int64_t walks;           /* seeds extended by the step-by-step walk      */
-    int64_t long_walks;      /* of those, walks finished per diagonal        */
+    int64_t walks;           /* seeds extended by a walk of their own        */
+    int64_t long_walks;      /* of those, long walks a whole block finished  */
 } mh_match_stats;
 
 /* Replaces PairwiseMatchFinder/MemHash::FindMatches (LM/MemHash.cpp:109-127,

@@ -1,10 +1,42 @@
-// extend.hpp -- ungapped seed extension of two genomes, shared by the device
-// kernels and host-side checks of them.
+// extend.hpp -- ungapped seed extension over k genomes, on the device.
 //
-// ExtEnv describes the two sorted mer lists by position (GetDnaSeedMer
-// values, LM/SortedMerList.h) and the sequence lengths.  extend2 is the
-// reference's ExtendMatch (LM/MatchFinder.h:218-374) for one seed.
+// ExtendMatch (LM/MatchFinder.h:218-374) moves a match's two ends through the
+// genomes a seed holds.  A step matches when the masked windows of all of them
+// agree.  Within one round each end takes seed-length jumps while the next
+// window matches, then, step by step, moves to the furthest matching window
+// within one seed length (or stays); rounds repeat while either end made a
+// single step.  An end's moves depend only on its own position (the room to the
+// sequence ends and the windows read are functions of it), and an end whose
+// single-step phase found nothing finds nothing again.  So an end moves from
+// matching window to matching window, never past a seed length without one,
+// and stops where the next seed length of windows holds none: wherever it
+// stepped in between, it stops at the last matching window before the first
+// run of a seed length of windows that do not match or leave a sequence.  Two
+// seeds of the same genomes on one diagonal (each start of the one the same
+// distance from the other's) at most a seed length apart therefore extend to
+// the same match, and one of them is walked for both.
+//
+// The reference compares GetDnaSeedMer values: the smaller of the masked window
+// and its reverse complement, and which of the two it was.  Under a palindromic
+// pattern (the seed families all are) that is a comparison of the windows
+// themselves: for two genomes in one orientation, equal masked windows; in
+// opposite orientations, the masked window equal to the other's reverse
+// complement and not its own (a window that is its own reverse complement
+// counts as forward in both).  So a walk reads the packed sequences (reversed
+// genomes' from their packed reverse complement), 64 characters a genome, and
+// has 32 windows' outcomes from shifting the differing characters' bits by the
+// pattern.  Other patterns compare the values by position (PAL false).
+//
+// A thread's walk is bound by the latency of its scattered reads; a walk over a
+// long stretch is a chain of them, which a block cuts to one for 32,000
+// windows.  Measured, against walks step by step of eight bytes a position from
+// seeds exactly a seed length apart (and, for two genomes, the long ones by
+// pointer jumping over every window of their diagonals): eight genomes of 5 Mb
+// 1.3 ms (34.3), two of 200 kb 63 us (a 105 us walk and 0.72 ms of jumping).
 #pragma once
+#if defined(__HIP__)
+#include <hip/hip_runtime.h>
+#endif
 #include <cstdint>
 
 #if defined(__HIPCC__)
@@ -17,352 +49,237 @@
 
 namespace mh {
 
-enum : int { EXT_OK = 0, EXT_ERR = 1, EXT_LONG = 2 };
-
-struct ExtEnv {
-    const uint64_t *kp0, *kp1;   // GetDnaSeedMer by position
-    uint64_t n0, n1;              // SMLLength
-    int64_t L0, L1;               // sequence lengths
-    int seed_len;
-    uint64_t mer_mask;            // GetSeedMask(): top 2*weight bits
-};
-
-MH_HD inline bool lookup(const ExtEnv &e, int g, int64_t pos1, int64_t len, int64_t start, uint64_t &mer, int &parity)
-{
-    int64_t p = pos1;
-    if (p < 0) p = -p + len - e.seed_len;
-    const int64_t idx = p - 1;
-    const uint64_t n = g ? e.n1 : e.n0;
-    if (idx < 0 || (uint64_t)idx >= n) return false;
-    const uint64_t k = (g ? e.kp1 : e.kp0)[idx];
-    parity = start < 0 ? (int)(k & 1ull) : (int)!(k & 1ull);
-    mer = k & e.mer_mask;
-    return true;
-}
-
-// ExtendMatch, LM/MatchFinder.h:218-374, for a two-genome seed (both starts
-// present, linear sequences).  EXT_ERR if it would read outside the lists
-// (the reference reads out of bounds there; never seen in practice) or runs
-// more than 8 (L0 + L1) steps; EXT_LONG once it has run more than `budget`
-// steps (0: no budget), leaving st and len mid-walk.
-MH_HD inline int extend2(const ExtEnv &e, int64_t st[2], int64_t &len, int64_t budget)
-{
-    const int64_t Lg[2] = {e.L0, e.L1};
-    int jump = e.seed_len;
-    uint32_t extend_limit = 0, extend_attempts = 0;
-    bool extend_again = false;
-    int64_t guard = 0;
-    const int64_t guard_max = 8 * (e.L0 + e.L1) + 64;
-    for (int dir = 0; dir < 4; ++dir) {
-        int64_t maxlen = dir >= 2 ? (int64_t)e.seed_len : (int64_t)4294967295ll;
-        for (int x = 0; x < 2; ++x) {
-            if (st[x] < 0) {
-                const int64_t rc_len = Lg[x] - len + st[x] + 1;
-                if (rc_len < maxlen) maxlen = rc_len;
-            } else if (st[x] - 1 < maxlen) {
-                maxlen = st[x] - 1;
-            }
-        }
-        int j = 0, i = 2;
-        extend_limit = 0;
-        extend_attempts = 0;
-        if (dir < 2 && maxlen >= jump) {
-            // The seed-length jumps of phases 0 and 1: the addresses of the
-            // K = maxlen / jump lookups do not depend on their outcomes, so
-            // they are issued in groups of PREFETCH and checked in order; the
-            // state after the first failing step (or after the K-th) is what
-            // the step-by-step loop leaves (len and the forward starts moved by
-            // the successful steps only).
-            constexpr int PREFETCH = 8;
-            const int64_t K = maxlen / jump;
-            int64_t ok_steps = K;
-            bool done = false;
-            for (int64_t k0 = 1; k0 <= K && !done; k0 += PREFETCH) {
-                uint64_t m0[PREFETCH], m1[PREFETCH];
-                int q0[PREFETCH], q1[PREFETCH];
-                bool in[PREFETCH];
-                const int cnt = (int)((K - k0 + 1) < PREFETCH ? (K - k0 + 1) : PREFETCH);
-MH_PRAGMA_UNROLL
-                for (int u = 0; u < PREFETCH; ++u) {
-                    if (u >= cnt) break;
-                    const int64_t k = k0 + u;
-                    const int64_t ln = len + k * jump;
-                    const int64_t p0 = st[0] > 0 ? st[0] - k * jump : st[0];
-                    const int64_t p1 = st[1] > 0 ? st[1] - k * jump : st[1];
-                    in[u] = lookup(e, 0, p0, ln, st[0], m0[u], q0[u]) && lookup(e, 1, p1, ln, st[1], m1[u], q1[u]);
-                }
-                for (int u = 0; u < cnt; ++u) {
-                    if (++guard > guard_max) return EXT_ERR;
-                    if (budget && guard > budget) return EXT_LONG;
-                    if (!in[u]) return EXT_ERR;
-                    if (m0[u] != m1[u] || q0[u] != q1[u]) {
-                        ok_steps = k0 + u - 1;
-                        done = true;
-                        break;
-                    }
-                }
-            }
-            len += ok_steps * jump;
-            for (int x = 0; x < 2; ++x)
-                if (st[x] > 0) st[x] -= ok_steps * jump;
-            maxlen = 0;   // the loop below does not run
-        }
-        while (maxlen - jump >= 0) {
-            if (++guard > guard_max) return EXT_ERR;
-            if (budget && guard > budget) return EXT_LONG;
-            len += jump;
-            maxlen -= jump;
-            for (j = 0; j < 2; ++j)
-                if (st[j] > 0) {
-                    st[j] -= jump;
-                    if (st[j] <= 0) st[j] += Lg[j];
-                }
-            uint64_t cm, om;
-            int cp, op;
-            if (!lookup(e, 0, st[0], len, st[0], cm, cp)) return EXT_ERR;
-            if (!lookup(e, 1, st[1], len, st[1], om, op)) return EXT_ERR;
-            i = 1;
-            if (cm != om || cp != op) {
-                if (dir < 2) maxlen = 0;
-            } else {
-                i = 2;
-            }
-            extend_attempts += jump;
-            if (i == 2) extend_limit = extend_attempts;
-            if (dir > 1 && extend_attempts == (uint32_t)e.seed_len) break;
-        }
-        if (i < 2) {
-            len -= jump;
-            for (; j > 0; j--)
-                if (st[j - 1] >= 0) st[j - 1] += jump;
-        }
-        if (dir > 1 && extend_attempts > 0) {
-            if (extend_limit > 0) extend_again = true;
-            int unmatched = (int)(extend_attempts - extend_limit);
-            if (i < 2) unmatched -= jump;
-            len -= unmatched;
-            for (j = 0; j < 2; ++j)
-                if (st[j] > 0) {
-                    st[j] += unmatched;
-                    if (st[j] > Lg[j]) st[j] -= Lg[j];
-                }
-        }
-        st[0] = -st[0];
-        st[1] = -st[1];
-        if (dir >= 1) jump = 1;
-        if (dir == 3 && extend_again) {
-            dir = -1;
-            jump = e.seed_len;
-            extend_again = false;
-        }
-    }
-    return EXT_OK;
-}
-
-// The k-genome form of the same walk (the genomes a seed holds; start 0
-// absent): ExtendMatch compares every present genome's window with the first
-// present genome's, and a step matches when all of them do
-// (LM/MatchFinder.h:218-374).  EnvK holds each genome's GetDnaSeedMer by
-// position, list length and sequence length.
 constexpr int EXT_MAXK = 16;
 
-struct ExtEnvK {
-    const uint64_t *kp[EXT_MAXK];
-    uint64_t n[EXT_MAXK];
-    int64_t L[EXT_MAXK];
+#if defined(__HIP__)
+
+// Per genome: the packed sequence and its reverse complement's, or (other
+// patterns) GetDnaSeedMer by position, twice; the length.  mask: the values' top
+// 2 * weight bits; pat: the pattern's characters, the first in bit 0.
+struct WalkEnv {
+    const void *fwd[EXT_MAXK], *rev[EXT_MAXK];
+    uint32_t L[EXT_MAXK];
     int seed_len;
-    uint64_t mer_mask;
+    uint32_t pat;
+    uint64_t mask;
 };
 
-MH_HD inline bool lookup_k(const ExtEnvK &e, int g, int64_t pos1, int64_t len, uint64_t &mer, int &parity)
+constexpr uint32_t WALK_CHUNKS = 16;    // chunks of 32 windows an end before a whole block takes the walk over
+constexpr uint32_t WALK_BLOCK = 1024;
+
+// 32 characters starting at pos (first character in the top two bits)
+__device__ __forceinline__ uint64_t win32(const uint32_t *__restrict__ w, uint64_t pos)
 {
-    int64_t p = pos1;
-    if (p < 0) p = -p + len - e.seed_len;
-    const int64_t idx = p - 1;
-    if (idx < 0 || (uint64_t)idx >= e.n[g]) return false;
-    const uint64_t k = e.kp[g][idx];
-    parity = pos1 < 0 ? (int)(k & 1ull) : (int)!(k & 1ull);
-    mer = k & e.mer_mask;
-    return true;
+    const uint64_t q = pos >> 4;
+    const uint32_t bit = (uint32_t)(pos & 15) * 2;
+    uint64_t m = ((uint64_t)w[q] << 32) | w[q + 1];
+    if (bit) m = (m << bit) | (w[q + 2] >> (32 - bit));
+    return m;
 }
 
-// st[x] is the start in genome gs[x], x < used (the present genomes in genome
-// order).  EXT_ERR if a lookup would leave a list or the walk runs more than
-// 8 (sum of the lengths) steps.
-MH_HD inline int extend_k(const ExtEnvK &e, const int *gs, int used, int64_t *st, int64_t &len)
+// 64 characters starting at pos; words past the last one (whose characters no
+// caller uses) read as the last
+__device__ __forceinline__ void win64(const uint32_t *__restrict__ w, uint32_t pos, uint32_t last, uint64_t *hi,
+                                      uint64_t *lo)
 {
-    int jump = e.seed_len;
-    uint32_t extend_limit = 0, extend_attempts = 0;
-    bool extend_again = false;
-    int64_t guard = 0, guard_max = 64;
-    for (int x = 0; x < used; ++x) guard_max += 8 * e.L[gs[x]];
-    for (int dir = 0; dir < 4; ++dir) {
-        int64_t maxlen = dir >= 2 ? (int64_t)e.seed_len : (int64_t)4294967295ll;
-        for (int x = 0; x < used; ++x) {
-            if (st[x] < 0) {
-                const int64_t rc_len = e.L[gs[x]] - len + st[x] + 1;
-                if (rc_len < maxlen) maxlen = rc_len;
-            } else if (st[x] - 1 < maxlen) {
-                maxlen = st[x] - 1;
-            }
-        }
-        int j = 0, i = used;
-        extend_limit = 0;
-        extend_attempts = 0;
-        while (maxlen - jump >= 0) {
-            if (++guard > guard_max) return EXT_ERR;
-            len += jump;
-            maxlen -= jump;
-            for (j = 0; j < used; ++j)
-                if (st[j] > 0) {
-                    st[j] -= jump;
-                    if (st[j] <= 0) st[j] += e.L[gs[j]];
-                }
-            uint64_t cm;
-            int cp;
-            if (!lookup_k(e, gs[0], st[0], len, cm, cp)) return EXT_ERR;
-            for (i = 1; i < used; ++i) {
-                uint64_t om;
-                int op;
-                if (!lookup_k(e, gs[i], st[i], len, om, op)) return EXT_ERR;
-                if (cm != om || cp != op) {
-                    if (dir < 2) maxlen = 0;
-                    break;
-                }
-            }
-            extend_attempts += jump;
-            if (i == used) extend_limit = extend_attempts;
-            if (dir > 1 && extend_attempts == (uint32_t)e.seed_len) break;
-        }
-        if (i < used) {
-            len -= jump;
-            for (; j > 0; j--)
-                if (st[j - 1] >= 0) st[j - 1] += jump;
-        }
-        if (dir > 1 && extend_attempts > 0) {
-            if (extend_limit > 0) extend_again = true;
-            int unmatched = (int)(extend_attempts - extend_limit);
-            if (i < used) unmatched -= jump;
-            len -= unmatched;
-            for (j = 0; j < used; ++j)
-                if (st[j] > 0) {
-                    st[j] += unmatched;
-                    if (st[j] > e.L[gs[j]]) st[j] -= e.L[gs[j]];
-                }
-        }
-        for (int x = 0; x < used; ++x) st[x] = -st[x];
-        if (dir >= 1) jump = 1;
-        if (dir == 3 && extend_again) {
-            dir = -1;
-            jump = e.seed_len;
-            extend_again = false;
-        }
-    }
-    return EXT_OK;
-}
-
-#if defined(__HIPCC__)
-// extend_k for a seed of at most KMAX present genomes, with the lookups of a
-// step issued together.  The caller passes the present genomes' lists,
-// list sizes and sequence lengths in order (gk, gn, gL: slot x is genome
-// gs[x]; slots from `used` on repeat slot 0 and are never compared), and st
-// with KMAX slots.  A lookup's index is clamped into its list and the miss
-// flagged instead of branching around the load, so a step's loads do not
-// wait on each other; a miss is an error only where the literal loop, which
-// stops at the first genome that differs, would have made that lookup.
-// Same walk, result and errors as extend_k.
-template <int KMAX>
-__device__ inline int extend_kt(const uint64_t *const *gk, const uint32_t *gn, const int64_t *gL, int used,
-                                int seed_len, uint64_t mer_mask, int64_t *st, int64_t &len)
-{
-    int jump = seed_len;
-    uint32_t extend_limit = 0, extend_attempts = 0;
-    bool extend_again = false;
-    int64_t guard = 0, guard_max = 64;
+    uint32_t v[5];
     MH_PRAGMA_UNROLL
-    for (int x = 0; x < KMAX; ++x)
-        if (x < used) guard_max += 8 * gL[x];
-    for (int dir = 0; dir < 4; ++dir) {
-        int64_t maxlen = dir >= 2 ? (int64_t)seed_len : (int64_t)4294967295ll;
+    for (uint32_t u = 0; u < 5; ++u) {
+        const uint32_t q = (pos >> 4) + u;
+        v[u] = w[q < last ? q : last];
+    }
+    const uint32_t bit = (pos & 15) * 2;
+    uint64_t a = (uint64_t)v[0] << 32 | v[1], b = (uint64_t)v[2] << 32 | v[3];
+    if (bit) {
+        a = (a << bit) | (v[2] >> (32 - bit));
+        b = (b << bit) | (v[4] >> (32 - bit));
+    }
+    *hi = a;
+    *lo = b;
+}
+
+// the even bits of hi and lo, the topmost (the first character's) in bit 0
+__device__ __forceinline__ uint64_t char_bits(uint64_t hi, uint64_t lo)
+{
+    uint64_t r[2] = {hi, lo};
+    MH_PRAGMA_UNROLL
+    for (int u = 0; u < 2; ++u) {
+        uint64_t x = r[u] & 0x5555555555555555ull;
+        x = (x | x >> 1) & 0x3333333333333333ull;
+        x = (x | x >> 2) & 0x0F0F0F0F0F0F0F0Full;
+        x = (x | x >> 4) & 0x00FF00FF00FF00FFull;
+        x = (x | x >> 8) & 0x0000FFFF0000FFFFull;
+        r[u] = __brev((uint32_t)(x | x >> 16));
+    }
+    return r[0] | r[1] << 32;
+}
+
+// A seed of up to K genomes: each genome's sequence in its orientation, the
+// window's start there (the first present genome forward); slots past the
+// seed's genomes repeat the first, so that every slot's reads go out together.
+template <int K, bool PAL> struct Walk {
+    const void *b[K];
+    uint32_t p[K], n[K];
+    uint32_t rev;        // bit x: slot x reversed
+    uint32_t S, pat;
+    uint64_t mask;
+
+    // pos: the window's start in genome g's forward coordinates
+    __device__ __forceinline__ void set(int x, const WalkEnv &env, int g, uint32_t pos, bool reversed)
+    {
+        n[x] = env.L[g];
+        b[x] = reversed ? env.rev[g] : env.fwd[g];
+        p[x] = reversed ? n[x] - pos - (uint32_t)env.seed_len : pos;
+        if (reversed) rev |= 1u << x;
+    }
+    __device__ __forceinline__ void fill(int used)
+    {
         MH_PRAGMA_UNROLL
-        for (int x = 0; x < KMAX; ++x) {
-            if (x >= used) continue;
-            if (st[x] < 0) {
-                const int64_t rc_len = gL[x] - len + st[x] + 1;
-                if (rc_len < maxlen) maxlen = rc_len;
-            } else if (st[x] - 1 < maxlen) {
-                maxlen = st[x] - 1;
+        for (int x = 1; x < K; ++x)
+            if (x >= used) {
+                b[x] = b[0];
+                p[x] = p[0];
+                n[x] = n[0];
+            }
+    }
+    __device__ __forceinline__ uint32_t room_left() const
+    {
+        uint32_t r = p[0];
+        MH_PRAGMA_UNROLL
+        for (int x = 1; x < K; ++x) r = p[x] < r ? p[x] : r;
+        return r;
+    }
+    __device__ __forceinline__ uint32_t room_right() const
+    {
+        uint32_t r = n[0] - p[0];
+        MH_PRAGMA_UNROLL
+        for (int x = 1; x < K; ++x) r = n[x] - p[x] < r ? n[x] - p[x] : r;
+        return r - S;
+    }
+    // bit i: the windows c + i characters from the seed's (left or right of it)
+    // match; 0 past the room
+    template <bool RIGHT> __device__ __forceinline__ uint32_t chunk(uint32_t c, uint32_t room) const
+    {
+        if (c > room) return 0;
+        const uint32_t cnt = room - c < 31 ? room - c + 1 : 32;      // windows inside
+        const uint32_t d = RIGHT ? c : 0u - (c + cnt - 1);           // the first by position
+        uint32_t m = 0;
+        if (PAL) {
+            uint64_t fh, fl, dh = 0, dl = 0;
+            win64((const uint32_t *)b[0], p[0] + d, (n[0] + 15) / 16 + 1, &fh, &fl);
+            MH_PRAGMA_UNROLL
+            for (int x = 1; x < K; ++x) {
+                uint64_t h, l;
+                win64((const uint32_t *)b[x], p[x] + d, (n[x] + 15) / 16 + 1, &h, &l);
+                dh |= fh ^ h;
+                dl |= fl ^ l;
+            }
+            const uint64_t diff = char_bits(dh | dh >> 1, dl | dl >> 1);
+            uint32_t bad = 0;
+            for (uint32_t t = pat; t; t &= t - 1) bad |= (uint32_t)(diff >> __builtin_ctz(t));
+            if (rev) {
+                // windows that are their own reverse complement
+                const uint64_t b1 = char_bits(fh >> 1, fl >> 1), b0 = char_bits(fh, fl);
+                uint32_t own = ~0u;
+                for (uint32_t t = pat; t; t &= t - 1) {
+                    const uint32_t a = __builtin_ctz(t), z = S - 1 - a;
+                    if (a > z) break;
+                    own &= (uint32_t)((b1 >> a) ^ (b1 >> z)) & (uint32_t)((b0 >> a) ^ (b0 >> z));
+                }
+                bad |= own;
+            }
+            m = ~bad;
+        } else {
+            for (uint32_t i = 0; i < cnt; ++i) {
+                const uint64_t f = ((const uint64_t *)b[0])[p[0] + d + i];
+                bool ok = true;
+                MH_PRAGMA_UNROLL
+                for (int x = 1; x < K; ++x) {
+                    const uint32_t r = (rev >> x) & 1u, q = p[x] + d + i;
+                    const uint64_t v = f ^ ((const uint64_t *)b[x])[r ? n[x] - q - S : q];
+                    ok = ok && (v & mask) == 0 && (uint32_t)(v & 1ull) == r;
+                }
+                m |= (ok ? 1u : 0u) << i;
             }
         }
-        int i = used;
-        extend_limit = 0;
-        extend_attempts = 0;
-        while (maxlen - jump >= 0) {
-            if (++guard > guard_max) return EXT_ERR;
-            len += jump;
-            maxlen -= jump;
-            MH_PRAGMA_UNROLL
-            for (int x = 0; x < KMAX; ++x)
-                if (x < used && st[x] > 0) {
-                    st[x] -= jump;
-                    if (st[x] <= 0) st[x] += gL[x];
-                }
-            // every slot's window (lookup_k), loads issued together
-            uint64_t kv[KMAX];
-            bool in[KMAX];
-            MH_PRAGMA_UNROLL
-            for (int x = 0; x < KMAX; ++x) {
-                const int64_t p = st[x] < 0 ? -st[x] + len - seed_len : st[x];
-                const int64_t idx = p - 1;
-                in[x] = x >= used || (idx >= 0 && (uint64_t)idx < (uint64_t)gn[x]);
-                kv[x] = gk[x][(x < used && in[x]) ? idx : 0];
+        if (!RIGHT) m = __brev(m) >> (32 - cnt);
+        return cnt < 32 ? m & ((1u << cnt) - 1) : m;
+    }
+};
+
+// the matching windows of m with another within the next S bits of m
+__device__ __forceinline__ uint32_t followed(uint32_t m, uint32_t S)
+{
+    uint32_t a = m >> 1;
+    for (uint32_t have = 1; have < S && have < 31;) {
+        const uint32_t step = have < S - have ? have : S - have;
+        a |= step < 32 ? a >> step : 0;
+        have += step;
+    }
+    return m & a;
+}
+
+// One end by a thread: its distance from the seed's window; false past
+// WALK_CHUNKS chunks.
+template <bool RIGHT, class W> __device__ __forceinline__ bool walk_end(const W &w, uint32_t *end)
+{
+    const uint32_t room = RIGHT ? w.room_right() : w.room_left();
+    uint32_t last = 0;
+    for (uint32_t c = 0; c < 32 * WALK_CHUNKS; c += 32) {
+        const uint32_t m = w.template chunk<RIGHT>(c, room);
+        if (m) {
+            if (c + __builtin_ctz(m) - last > w.S) {
+                *end = last;
+                return true;
             }
-            if (!in[0]) return EXT_ERR;
-            const uint64_t cm = kv[0] & mer_mask;
-            const int cp = st[0] < 0 ? (int)(kv[0] & 1ull) : (int)!(kv[0] & 1ull);
-            i = used;
-            MH_PRAGMA_UNROLL
-            for (int x = 1; x < KMAX; ++x)
-                if (x < used && i == used) {
-                    if (!in[x]) return EXT_ERR;
-                    const int op = st[x] < 0 ? (int)(kv[x] & 1ull) : (int)!(kv[x] & 1ull);
-                    if (cm != (kv[x] & mer_mask) || cp != op) i = x;
-                }
-            if (i < used && dir < 2) maxlen = 0;
-            extend_attempts += jump;
-            if (i == used) extend_limit = extend_attempts;
-            if (dir > 1 && extend_attempts == (uint32_t)seed_len) break;
+            // the first that none follows within S: the chunk's last, or the end
+            const uint32_t lone = m & ~followed(m, w.S);
+            last = c + __builtin_ctz(lone);
+            if (lone & (lone - 1)) {
+                *end = last;
+                return true;
+            }
         }
-        if (i < used) {
-            len -= jump;
-            MH_PRAGMA_UNROLL
-            for (int x = 0; x < KMAX; ++x)
-                if (x < used && st[x] >= 0) st[x] += jump;
-        }
-        if (dir > 1 && extend_attempts > 0) {
-            if (extend_limit > 0) extend_again = true;
-            int unmatched = (int)(extend_attempts - extend_limit);
-            if (i < used) unmatched -= jump;
-            len -= unmatched;
-            MH_PRAGMA_UNROLL
-            for (int x = 0; x < KMAX; ++x)
-                if (x < used && st[x] > 0) {
-                    st[x] += unmatched;
-                    if (st[x] > gL[x]) st[x] -= gL[x];
-                }
-        }
-        MH_PRAGMA_UNROLL
-        for (int x = 0; x < KMAX; ++x)
-            if (x < used) st[x] = -st[x];
-        if (dir >= 1) jump = 1;
-        if (dir == 3 && extend_again) {
-            dir = -1;
-            jump = seed_len;
-            extend_again = false;
+        if (c + 31 >= room || c + 31 - last >= w.S) {
+            *end = last;
+            return true;
         }
     }
-    return EXT_OK;
+    return false;
 }
+
+// The same by WALK_BLOCK threads, a chunk each; the last WALK_AHEAD only show
+// the others whether a match follows within a seed length (of at most 64).
+constexpr uint32_t WALK_AHEAD = 3;
+template <bool RIGHT, class W> __device__ __forceinline__ uint32_t walk_end_block(const W &w, uint32_t *lds)
+{
+    const uint32_t room = RIGHT ? w.room_right() : w.room_left(), t = threadIdx.x;
+    uint32_t *first = lds, *best = lds + WALK_BLOCK;
+    for (uint64_t c0 = 0; c0 <= room; c0 += 32 * (WALK_BLOCK - WALK_AHEAD)) {
+        const uint64_t c = c0 + 32 * t;
+        const uint32_t m = c <= room ? w.template chunk<RIGHT>((uint32_t)c, room) : 0;
+        __syncthreads();
+        first[t] = m ? (uint32_t)__builtin_ctz(m) : 0xFFFFFFFFu;     // in its chunk
+        if (t == 0) *best = 0xFFFFFFFFu;
+        __syncthreads();
+        if (m && t < WALK_BLOCK - WALK_AHEAD) {
+            const uint32_t lone = m & ~followed(m, w.S), at = __builtin_ctz(lone);
+            bool stop = (lone & (lone - 1)) != 0;
+            if (!stop) {
+                uint32_t gap = 0xFFFFFFFFu;      // to the next match
+                MH_PRAGMA_UNROLL
+                for (uint32_t u = WALK_AHEAD; u > 0; --u)
+                    if (first[t + u] != 0xFFFFFFFFu) gap = 32 * u + first[t + u] - at;
+                stop = gap > w.S;
+            }
+            if (stop) atomicMin(best, (uint32_t)c + at);
+        }
+        __syncthreads();
+        if (*best != 0xFFFFFFFFu) return *best;
+    }
+    return 0;      // (not reached: the last matching window stops it)
+}
+
 #endif
 
 }  // namespace mh

@@ -37,7 +37,6 @@ constexpr int JT = 256;              // threads per join/compaction tile
 constexpr int JITEMS = 16;
 constexpr int JTILE = JT * JITEMS;
 constexpr uint32_t MER_REPEAT_LIMIT = 1000;
-constexpr int64_t LONG_WALK = 64;   // steps of a head's walk before it is resolved per diagonal
 
 __device__ __forceinline__ uint64_t lower_bound_m(const uint64_t *__restrict__ ck, uint64_t n, uint64_t m)
 {
@@ -349,94 +348,169 @@ __global__ __launch_bounds__(JT) void compact_kernel(const uint32_t *__restrict_
     }
 }
 
-__global__ void seed_kernel(const uint32_t *__restrict__ pi, const uint32_t *__restrict__ pj, uint64_t ns,
-                            const uint64_t *__restrict__ ck0, const uint32_t *__restrict__ pos0,
-                            const uint64_t *__restrict__ ck1, const uint32_t *__restrict__ pos1, ExtEnv env,
-                            int64_t budget, SeedRec *__restrict__ out, uint32_t *__restrict__ err,
-                            uint32_t *__restrict__ long_flag)
+// ---- walks (extend.hpp): one thread a seed, long ones a block each ----------
+
+// two genomes' seeds, as pairs of sorted-list entries
+template <bool P> struct PairWalks {
+    static constexpr int K = 2;
+    static constexpr bool PAL = P;
+    const uint32_t *heads;
+    const uint32_t *pi, *pj;
+    const uint64_t *ck0, *ck1;
+    const uint32_t *pos0, *pos1;
+    SeedRec *out;
+
+    __device__ __forceinline__ void load(uint64_t h, const WalkEnv &env, Walk<K, P> &w) const
+    {
+        const uint32_t x = heads[h], i = pi[x], j = pj[x];
+        // SetDirection: genome 0 is the reference; genome 1 is flipped if its strand flag differs
+        w.set(0, env, 0, pos0[i], false);
+        w.set(1, env, 1, pos1[j], ((ck0[i] ^ ck1[j]) & 1ull) != 0);
+    }
+    __device__ __forceinline__ void store(uint64_t h, const Walk<K, P> &w, uint32_t left, uint32_t len) const
+    {
+        const uint32_t q = w.p[1] - left;
+        SeedRec r;
+        r.s0 = (int32_t)w.p[0] + 1;
+        r.s1 = w.rev ? -(int32_t)(w.n[1] - w.p[1] - w.S + 1) : (int32_t)w.p[1] + 1;
+        r.e0 = (int32_t)(w.p[0] - left) + 1;
+        r.e1 = w.rev ? -(int32_t)(w.n[1] - q - len + 1) : (int32_t)q + 1;
+        r.elen = len;
+        out[heads[h]] = r;
+    }
+};
+
+template <class SRC>
+__device__ __forceinline__ void walk_setup(const SRC &src, uint64_t x, const WalkEnv &env,
+                                           Walk<SRC::K, SRC::PAL> &w)
 {
-    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= ns) return;
-    const uint32_t i = pi[x], j = pj[x];
-    const int64_t s0 = (int64_t)pos0[i] + 1;
-    int64_t s1 = (int64_t)pos1[j] + 1;
-    // SetDirection: genome 0 is the reference; flip genome 1 if its strand flag differs
-    if ((ck0[i] & 1ull) != (ck1[j] & 1ull)) s1 = -s1;
-    int64_t st[2] = {s0, s1};
-    int64_t len = env.seed_len;
-    const int rc = extend2(env, st, len, budget);
-    if (long_flag) long_flag[x] = rc == EXT_LONG;
-    if (rc == EXT_ERR) atomicAdd(err, 1u);
-    SeedRec r;
-    r.s0 = (int32_t)s0;
-    r.s1 = (int32_t)s1;
-    r.e0 = (int32_t)st[0];
-    r.e1 = (int32_t)st[1];
-    r.elen = (uint32_t)len;
-    out[x] = r;
+    w.rev = 0;
+    w.S = (uint32_t)env.seed_len;
+    w.pat = env.pat;
+    w.mask = env.mask;
+    src.load(x, env, w);
 }
 
-// ---- spaced seeds: one extension per grid chain -----------------------------
-// Two seeds of the same strand relation whose starts differ by the seed length
-// along their diagonal (forward: s0 + L, s1 + L; reverse: s0 + L, |s1| - L)
-// extend to the same match: the later one's seed-length walk to the left steps
-// onto the earlier one's window (a seed, so it matches) and from there repeats
-// the earlier one's walk, with one step less of room; to the right the earlier
-// one steps onto the later one's window the same way; the single-step phases
-// then start from the same match.  So each chain of such seeds is extended once,
-// from its first seed, and the result is copied to the others.
-
-__global__ void grid_key_kernel(const uint32_t *__restrict__ oi, const uint32_t *__restrict__ oj, uint64_t ns,
-                                const uint64_t *__restrict__ ck0, const uint32_t *__restrict__ pos0,
-                                const uint64_t *__restrict__ ck1, const uint32_t *__restrict__ pos1,
-                                uint64_t *__restrict__ key, uint32_t *__restrict__ val, int32_t *__restrict__ t1)
+// The seeds src names; ns: at most this many, or (cnt not null) *count.  cnt[0]:
+// walks left to walk_long_kernel, listed in rest.
+template <class SRC>
+__global__ __launch_bounds__(128) void walk_kernel(SRC src, uint64_t ns, const uint32_t *__restrict__ count,
+                                                   WalkEnv env, uint32_t *__restrict__ rest,
+                                                   uint32_t *__restrict__ cnt)
 {
-    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= ns) return;
-    const uint32_t i = oi[x], j = oj[x];
-    const int32_t s1 = (int32_t)pos1[j] + 1;
-    key[x] = (uint64_t)pos0[i] + 1;
-    val[x] = (uint32_t)x;
-    t1[x] = (ck0[i] & 1ull) != (ck1[j] & 1ull) ? -s1 : s1;   // the seed's signed start in genome 2
+    if (count) ns = *count;
+    for (uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; x < ns; x += (uint64_t)gridDim.x * blockDim.x) {
+        Walk<SRC::K, SRC::PAL> w;
+        walk_setup(src, x, env, w);
+        uint32_t l, r;
+        if (walk_end<false>(w, &l) && walk_end<true>(w, &r)) src.store(x, w, l, l + r + w.S);
+        else rest[atomicAdd(cnt, 1u)] = (uint32_t)x;
+    }
 }
 
-// link[r] = sorted index of the seed one seed length before r on its chain, or
-// r.  Seeds are sorted by their start in genome 1; the predecessor of (s0, t)
-// is (s0 - L, t - L) with t's sign kept (forward: s1 - L; reverse: the start
-// in genome 2 moves right, -(s1 + L)).  At most `scan` seeds sharing a start
-// are looked at: a seed left without its link only extends by itself.
-__global__ void grid_pred_kernel(const uint64_t *__restrict__ sk, const uint32_t *__restrict__ sv,
-                                 const int32_t *__restrict__ t1, uint64_t ns, uint32_t seed_len, int scan,
-                                 uint32_t *__restrict__ link)
+template <class SRC>
+__global__ __launch_bounds__(WALK_BLOCK) void walk_long_kernel(SRC src, WalkEnv env, const uint32_t *__restrict__ rest,
+                                                               const uint32_t *__restrict__ cnt)
 {
-    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= ns) return;
-    const uint64_t k = sk[r];
-    const int32_t t = t1[sv[r]];
-    const int32_t tw = t - (int32_t)seed_len;
-    uint32_t out = (uint32_t)r;
-    if (k > seed_len && (t < 0 || tw > 0)) {
-        const uint64_t want = k - seed_len;
-        uint64_t lo = 0, hi = r;
-        while (lo < hi) {
-            const uint64_t mid = (lo + hi) / 2;
-            if (sk[mid] < want) lo = mid + 1;
-            else hi = mid;
-        }
-        for (int c = 0; c < scan && lo < r && sk[lo] == want; ++c, ++lo)
-            if (t1[sv[lo]] == tw) {
-                out = (uint32_t)lo;
+    __shared__ uint32_t lds[WALK_BLOCK + 1];
+    const uint32_t n = *cnt;
+    for (uint32_t h = blockIdx.x; h < n; h += gridDim.x) {
+        const uint64_t x = rest[h];
+        Walk<SRC::K, SRC::PAL> w;
+        walk_setup(src, x, env, w);
+        const uint32_t l = walk_end_block<false>(w, lds), r = walk_end_block<true>(w, lds);
+        if (threadIdx.x == 0) src.store(x, w, l, l + r + w.S);
+    }
+}
+
+template <class SRC>
+void launch_walks(mh_context *ctx, const SRC &src, uint64_t ns, const uint32_t *count, const WalkEnv &env,
+                  uint32_t *rest, uint32_t *cnt)
+{
+    if (!ns) return;
+    const uint64_t blocks = (ns + 127) / 128;
+    hipLaunchKernelGGL(walk_kernel<SRC>, dim3((unsigned)(count ? std::min<uint64_t>(blocks, 8192) : blocks)), dim3(128),
+                       0, ctx->stream, src, ns, count, env, rest, cnt);
+    hipLaunchKernelGGL(walk_long_kernel<SRC>, dim3(512), dim3(WALK_BLOCK), 0, ctx->stream, src, env, rest, cnt);
+}
+
+// ---- spaced and even seeds: one walk per run of seeds -------------------------
+// Seeds of one strand relation on one diagonal, each at most a seed length from
+// the next, extend to the same match (extend.hpp): the run's first seed (its
+// head) is walked and the others copy its extension.  Runs are found by
+// genome-0 position (a position holds at most one seed, see below): each seed
+// links to the furthest one of its diagonal within a seed length before it, and
+// pointer jumping leads to the heads.  Two such links always span more than a
+// seed length.
+
+__global__ void spaced_link_kernel(const uint2 *__restrict__ pp, uint64_t L0, uint32_t seed_len,
+                                   uint32_t *__restrict__ link)
+{
+    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= L0) return;
+    const uint2 v = pp[p];
+    uint32_t out = (uint32_t)p;
+    if (v.x != 0xFFFFFFFFu) {
+        const bool rev = (v.x >> 31) != 0;
+        const uint32_t q = v.x & 0x7FFFFFFFu;
+        for (uint32_t t = p < seed_len ? (uint32_t)p : seed_len; t > 0; --t) {
+            if (!rev && q < t) continue;
+            if (pp[p - t].x == ((rev ? q + t : q - t) | (v.x & 0x80000000u))) {
+                out = (uint32_t)p - t;
                 break;
             }
+        }
     }
-    link[r] = out;
+    link[p] = out;
 }
 
+// the heads' seed indices, in no order (each walk writes its own seed's result)
+__global__ void spaced_heads_kernel(const uint2 *__restrict__ pp, const uint32_t *__restrict__ root, uint64_t L0,
+                                    uint32_t *__restrict__ heads, uint32_t *__restrict__ count)
+{
+    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint2 v = make_uint2(0xFFFFFFFFu, 0);
+    if (p < L0) v = pp[p];
+    const bool head = v.x != 0xFFFFFFFFu && root[p] == (uint32_t)p;
+    const uint64_t b = __ballot(head);
+    if (!b) return;
+    const int lane = threadIdx.x & 63;
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(count, (uint32_t)__builtin_popcountll(b));
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    if (head) heads[at + __builtin_popcountll(b & ((1ull << lane) - 1))] = v.y;
+}
+
+__global__ void spaced_fill_kernel(const uint2 *__restrict__ pp, const uint32_t *__restrict__ root, uint64_t L0,
+                                   SeedRec *__restrict__ out)
+{
+    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= L0) return;
+    const uint2 v = pp[p];
+    if (v.x == 0xFFFFFFFFu || root[p] == (uint32_t)p) return;
+    const SeedRec h = out[pp[root[p]].y];
+    SeedRec r;
+    r.s0 = (int32_t)p + 1;
+    r.s1 = v.x >> 31 ? -((int32_t)(v.x & 0x7FFFFFFFu) + 1) : (int32_t)v.x + 1;
+    r.e0 = h.e0;
+    r.e1 = h.e1;
+    r.elen = h.elen;
+    out[v.y] = r;
+}
+
+// eight hops a launch, fewer where the chain ends: 200,000 positions take five
+// launches of 3.5 us (one hop, so a doubling, a launch: 19 of 9 us)
 __global__ void grid_jump_kernel(const uint32_t *__restrict__ in, uint32_t *__restrict__ out, uint64_t ns)
 {
     const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= ns) return;
-    out[r] = in[in[r]];
+    uint32_t a = in[r];
+    for (int h = 1; h < 8; ++h) {
+        const uint32_t b = in[a];
+        if (b == a) break;
+        a = b;
+    }
+    out[r] = a;
 }
 
 // flag[r]: sorted seed r heads its chain
@@ -466,220 +540,6 @@ __global__ void grid_head_kernel(const uint32_t *__restrict__ sv, const uint32_t
     head_of[x] = sv[root[r]];
 }
 
-__global__ void grid_gather_kernel(const uint32_t *__restrict__ heads, uint64_t nh, const uint32_t *__restrict__ oi,
-                                   const uint32_t *__restrict__ oj, uint32_t *__restrict__ hoi,
-                                   uint32_t *__restrict__ hoj, uint32_t *__restrict__ headpos)
-{
-    const uint64_t h = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    const uint32_t x = heads[h];
-    hoi[h] = oi[x];
-    hoj[h] = oj[x];
-    headpos[x] = (uint32_t)h;
-}
-
-__global__ void grid_fill_kernel(const uint32_t *__restrict__ oi, const uint32_t *__restrict__ oj, uint64_t ns,
-                                 const uint64_t *__restrict__ ck0, const uint32_t *__restrict__ pos0,
-                                 const uint64_t *__restrict__ ck1, const uint32_t *__restrict__ pos1,
-                                 const uint32_t *__restrict__ head_of, const uint32_t *__restrict__ headpos,
-                                 const SeedRec *__restrict__ hres, SeedRec *__restrict__ out)
-{
-    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= ns) return;
-    const uint32_t i = oi[x], j = oj[x];
-    const int64_t s0 = (int64_t)pos0[i] + 1;
-    int64_t s1 = (int64_t)pos1[j] + 1;
-    if ((ck0[i] & 1ull) != (ck1[j] & 1ull)) s1 = -s1;
-    const SeedRec h = hres[headpos[head_of[x]]];
-    SeedRec r;
-    r.s0 = (int32_t)s0;
-    r.s1 = (int32_t)s1;
-    r.e0 = h.e0;
-    r.e1 = h.e1;
-    r.elen = h.elen;
-    out[x] = r;
-}
-
-// ---- long extensions: both ends resolved per diagonal ----------------------
-// ExtendMatch's two ends move independently.  Within one round the left end
-// takes seed-length jumps while the next window to the left matches, then a
-// single-step phase moves it to the furthest matching window within one seed
-// length (or leaves it); the right end does the same to the right; rounds
-// repeat while either single-step phase moved.  Each end's moves depend only
-// on its own position (the room to the sequence ends and the windows read are
-// functions of it, the diagonal fixed), and an end whose single-step phase
-// found nothing finds nothing again.  So the final left end of a seed is the
-// fixed point of F(p) = J(p) - T(J(p)) from its start, J(p) the last window of
-// p's run of matching windows spaced one seed length apart and T(h) the
-// largest t <= seed length with window h - t matching (0 if none); the right
-// end mirrors it.  For the seeds whose step-by-step walk is long, F is built
-// for every window of a range around them on their diagonal and the fixed
-// points found by pointer jumping.  A window whose value depends on windows
-// beyond a range that was cut short (not by the sequence ends) is flagged, and
-// its diagonal is redone with a wider range.
-
-struct DiagGroup {
-    int64_t lo;        // first window start in genome 1 (1-based) of the range
-    int64_t n;         // windows in the range
-    int64_t base;      // first element of the range in the dense arrays
-    int64_t dconst;    // forward: s1 - s0; reverse: s0 + s1 (window starts pair as p + q)
-    int32_t rev, clip_lo, clip_hi, pad;
-};
-
-struct DiagHead {
-    uint32_t head;     // index into the head results
-    uint32_t group;
-    int32_t s0, t1;    // start in genome 1, signed start in genome 2
-};
-
-constexpr uint32_t DG_ESC = 0x80000000u, DG_IDX = 0x7fffffffu;
-
-__device__ __forceinline__ uint32_t dg_find(const DiagGroup *__restrict__ g, uint32_t ng, uint64_t e)
-{
-    uint32_t lo = 0, hi = ng;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) / 2;
-        if ((uint64_t)g[mid].base <= e) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
-// window e of its range matches (both windows inside the sequences by construction)
-__global__ void dg_match_kernel(const DiagGroup *__restrict__ g, uint32_t ng, uint64_t N, ExtEnv env,
-                                uint8_t *__restrict__ mg)
-{
-    const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= N) return;
-    const DiagGroup d = g[dg_find(g, ng, e)];
-    const int64_t p = d.lo + (int64_t)(e - (uint64_t)d.base);
-    const int64_t q = d.rev ? d.dconst - p : p + d.dconst;
-    const uint64_t k0 = env.kp0[p - 1], k1 = env.kp1[q - 1];
-    mg[e] = ((k0 ^ k1) & env.mer_mask) == 0 && ((k0 ^ k1) & 1ull) == (uint64_t)d.rev;
-}
-
-// one seed-length step of the jump runs, left and right
-__global__ void dg_link_kernel(const DiagGroup *__restrict__ g, uint32_t ng, uint64_t N, int L,
-                               const uint8_t *__restrict__ mg, uint32_t *__restrict__ cl, uint32_t *__restrict__ cr)
-{
-    const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= N) return;
-    const DiagGroup d = g[dg_find(g, ng, e)];
-    const int64_t off = (int64_t)(e - (uint64_t)d.base);
-    uint32_t l = (uint32_t)e, r = (uint32_t)e;
-    if (off >= L) {
-        if (mg[e - L]) l = (uint32_t)(e - L);
-    } else if (d.clip_lo) {
-        l |= DG_ESC;
-    }
-    if (off + L < d.n) {
-        if (mg[e + L]) r = (uint32_t)(e + L);
-    } else if (d.clip_hi) {
-        r |= DG_ESC;
-    }
-    cl[e] = l;
-    cr[e] = r;
-}
-
-// pointer jumping; a root keeps its own flag, which the others take with it
-__global__ void dg_jump_kernel(uint64_t N, const uint32_t *__restrict__ il, const uint32_t *__restrict__ ir,
-                               uint32_t *__restrict__ ol, uint32_t *__restrict__ orr)
-{
-    const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= N) return;
-    ol[e] = il[il[e] & DG_IDX];
-    orr[e] = ir[ir[e] & DG_IDX];
-}
-
-// F (left) and its mirror (right) from the jump-run ends hl, hr
-__global__ void dg_step_kernel(const DiagGroup *__restrict__ g, uint32_t ng, uint64_t N, int L,
-                               const uint8_t *__restrict__ mg, const uint32_t *__restrict__ hl,
-                               const uint32_t *__restrict__ hr, uint32_t *__restrict__ fl, uint32_t *__restrict__ fr)
-{
-    const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= N) return;
-    const DiagGroup d = g[dg_find(g, ng, e)];
-    uint32_t h = hl[e], esc = h & DG_ESC;
-    h &= DG_IDX;
-    int64_t ho = (int64_t)h - d.base;
-    int T = 0;
-    for (int t = 1; t <= L; ++t) {
-        if (ho - t < 0) {
-            if (d.clip_lo) esc = DG_ESC;
-            break;
-        }
-        if (mg[h - t]) T = t;
-    }
-    fl[e] = (h - (uint32_t)T) | esc;
-    h = hr[e];
-    esc = h & DG_ESC;
-    h &= DG_IDX;
-    ho = (int64_t)h - d.base;
-    T = 0;
-    for (int t = 1; t <= L; ++t) {
-        if (ho + t >= d.n) {
-            if (d.clip_hi) esc = DG_ESC;
-            break;
-        }
-        if (mg[h + t]) T = t;
-    }
-    fr[e] = (h + (uint32_t)T) | esc;
-}
-
-// pointer jumping that collects the flags along the path
-__global__ void dg_jump_or_kernel(uint64_t N, const uint32_t *__restrict__ il, const uint32_t *__restrict__ ir,
-                                  uint32_t *__restrict__ ol, uint32_t *__restrict__ orr)
-{
-    const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= N) return;
-    uint32_t a = il[e], b = il[a & DG_IDX];
-    ol[e] = (b & DG_IDX) | ((a | b) & DG_ESC);
-    a = ir[e];
-    b = ir[a & DG_IDX];
-    orr[e] = (b & DG_IDX) | ((a | b) & DG_ESC);
-}
-
-__global__ void dg_heads_kernel(const uint32_t *__restrict__ long_idx, uint64_t nl, const uint32_t *__restrict__ hoi,
-                                const uint32_t *__restrict__ hoj, const uint64_t *__restrict__ ck0,
-                                const uint32_t *__restrict__ pos0, const uint64_t *__restrict__ ck1,
-                                const uint32_t *__restrict__ pos1, DiagHead *__restrict__ out)
-{
-    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= nl) return;
-    const uint32_t h = long_idx[x], i = hoi[h], j = hoj[h];
-    const int32_t s1 = (int32_t)pos1[j] + 1;
-    DiagHead r;
-    r.head = h;
-    r.group = 0;
-    r.s0 = (int32_t)pos0[i] + 1;
-    r.t1 = (ck0[i] & 1ull) != (ck1[j] & 1ull) ? -s1 : s1;
-    out[x] = r;
-}
-
-__global__ void dg_result_kernel(const DiagHead *__restrict__ hd, uint64_t nh, const DiagGroup *__restrict__ g,
-                                 const uint32_t *__restrict__ fl, const uint32_t *__restrict__ fr, int L,
-                                 SeedRec *__restrict__ res, uint8_t *__restrict__ esc)
-{
-    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= nh) return;
-    const DiagHead h = hd[x];
-    const DiagGroup d = g[h.group];
-    const uint64_t e = (uint64_t)d.base + (uint64_t)(h.s0 - d.lo);
-    const uint32_t a = fl[e], b = fr[e];
-    esc[x] = ((a | b) & DG_ESC) != 0;
-    const int64_t left = d.lo + ((int64_t)(a & DG_IDX) - d.base);
-    const int64_t last = d.lo + ((int64_t)(b & DG_IDX) - d.base);   // start of the rightmost window
-    const int64_t len = last - left + L;
-    const int64_t s0 = h.s0, s1 = h.t1 < 0 ? -(int64_t)h.t1 : h.t1;
-    SeedRec r;
-    r.s0 = h.s0;
-    r.s1 = h.t1;
-    r.e0 = (int32_t)left;
-    r.e1 = (int32_t)(d.rev ? -(s0 + s1 + L - left - len) : left + (s1 - s0));
-    r.elen = (uint32_t)len;
-    res[h.head] = r;
-}
-
 // ---- solid odd-length seeds ----------------------------------------------
 // With a solid seed of odd length k, a window and its reverse complement are
 // never equal, so comparing canonical keys plus strand parity (ExtendMatch's
@@ -688,16 +548,6 @@ __global__ void dg_result_kernel(const DiagHead *__restrict__ hd, uint64_t nh, c
 // extension then stops at the first mismatching character on each side, or at
 // a sequence end: the result is the maximal exact match through the seed.
 // It is computed here 32 characters per 64-bit XOR of packed words.
-
-__device__ __forceinline__ uint64_t win32(const uint32_t *__restrict__ w, uint64_t pos)
-{
-    // 32 characters starting at pos (first character in the top two bits)
-    const uint64_t q = pos >> 4;
-    const uint32_t bit = (uint32_t)(pos & 15) * 2;
-    uint64_t m = ((uint64_t)w[q] << 32) | w[q + 1];
-    if (bit) m = (m << bit) | (w[q + 2] >> (32 - bit));
-    return m;
-}
 
 // number of equal characters going right from (pa, pb), at most lim
 __device__ __forceinline__ int64_t match_right(const uint32_t *__restrict__ wa, int64_t pa,
@@ -737,14 +587,18 @@ __global__ void rc_pack_kernel(const uint32_t *__restrict__ w, uint64_t len, uin
     // packed reverse complement: character q of the output is 3 - char(len-1-q)
     const uint64_t ow = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (ow >= n_words) return;
+    // the output's 16 characters are the input's [s, s + 16) turned round
+    const int64_t s = (int64_t)len - 16 * ((int64_t)ow + 1);
     uint32_t v = 0;
-    for (int k = 0; k < 16; ++k) {
-        const uint64_t q = ow * 16 + k;
-        if (q < len) {
-            const uint64_t src = len - 1 - q;
-            const uint32_t c = (w[src >> 4] >> (30 - 2 * (src & 15))) & 3u;
-            v |= (3u - c) << (30 - 2 * k);
-        }
+    if (s > -16) {
+        const uint64_t q = s < 0 ? 0 : (uint64_t)s >> 4;
+        const uint32_t bit = s < 0 ? 0 : 2 * (uint32_t)(s & 15);
+        v = w[q] << bit;
+        if (bit) v |= w[q + 1] >> (32 - bit);
+        if (s < 0) v >>= 2 * (uint32_t)(-s);
+        v = __brev(~v);
+        v = ((v >> 1) & 0x55555555u) | ((v & 0x55555555u) << 1);
+        if (s < 0) v &= ~0u << (2 * (uint32_t)(-s));
     }
     out[ow] = v;
 }
@@ -1141,215 +995,71 @@ __global__ void gather_dirty_kernel(const uint32_t *__restrict__ idx, uint64_t m
 static int compact_flags(mh_context *ctx, const uint32_t *flag, uint64_t n, uint32_t *out_idx, uint32_t *tiles,
                          uint32_t *d_count, uint64_t *count);
 
-// The long walks of the heads in long_idx, per diagonal (the kernels above).
-static int resolve_long(mh_context *ctx, const mh_sml *a, const mh_sml *b, const ExtEnv &env,
-                        const uint32_t *long_idx, uint64_t nl, const uint32_t *hoi, const uint32_t *hoj,
-                        SeedRec *hres)
+// the genomes' operands of a walk: under a palindromic pattern of at most 32
+// characters the packed sequences (rc: their reverse complements, filled in
+// here where null is not given), else the values by position
+static bool walk_env(mh_context *ctx, const mh_sml *const *smls, int k, DevBuf *const *rc_bufs, WalkEnv *env, int *rc)
 {
-    DevBuf *g = ctx->diag_scratch;
-    int rc;
-    if ((rc = g[0].ensure(nl * sizeof(DiagHead) + 64)) != MH_OK) return rc;
-    DiagHead *d_heads = g[0].as<DiagHead>();
-    const dim3 blk(256);
-    hipLaunchKernelGGL(dg_heads_kernel, dim3((unsigned)((nl + 255) / 256)), blk, 0, ctx->stream, long_idx, nl, hoi,
-                       hoj, a->d_keys, a->d_pos, b->d_keys, b->d_pos, d_heads);
-    MH_HIP(hipGetLastError());
-    std::vector<DiagHead> hh(nl);
-    MH_HIP(hipMemcpyAsync(hh.data(), d_heads, nl * sizeof(DiagHead), hipMemcpyDeviceToHost, ctx->stream));
-    MH_HIP(hipStreamSynchronize(ctx->stream));
-    const int64_t L = env.seed_len;
-    const int64_t last0 = env.L0 - L + 1, last1 = env.L1 - L + 1;   // last window starts
-    auto key = [](const DiagHead &h) {
-        const int64_t s1 = h.t1 < 0 ? -(int64_t)h.t1 : h.t1;
-        return h.t1 < 0 ? std::make_pair(1, h.s0 + s1) : std::make_pair(0, s1 - h.s0);
-    };
-    std::sort(hh.begin(), hh.end(), [&](const DiagHead &x, const DiagHead &y) {
-        const auto kx = key(x), ky = key(y);
-        return kx != ky ? kx < ky : x.s0 < y.s0;
-    });
-    struct Diag {
-        int rev;
-        int64_t dconst, glo, ghi, smin, smax, reach;
-        size_t h0, h1;
-        bool done;
-    };
-    std::vector<Diag> diags;
-    for (size_t i = 0; i < nl;) {
-        size_t j = i + 1;
-        while (j < nl && key(hh[j]) == key(hh[i])) ++j;
-        Diag d;
-        d.rev = key(hh[i]).first;
-        d.dconst = key(hh[i]).second;
-        // window starts p of genome 1 whose partner q is a window start of genome 2
-        if (d.rev) {
-            d.glo = std::max<int64_t>(1, d.dconst - last1);
-            d.ghi = std::min<int64_t>(last0, d.dconst - 1);
-        } else {
-            d.glo = std::max<int64_t>(1, 1 - d.dconst);
-            d.ghi = std::min<int64_t>(last0, last1 - d.dconst);
-        }
-        d.smin = hh[i].s0;
-        d.smax = hh[j - 1].s0;
-        MH_CHECK(d.glo <= d.smin && d.smax <= d.ghi, MH_ERR_DEVICE, "seed window outside its sequences");
-        d.reach = 16384;
-        d.h0 = i;
-        d.h1 = j;
-        d.done = false;
-        diags.push_back(d);
-        i = j;
+    std::memset(env, 0, sizeof(*env));
+    const int S = smls[0]->seed_length, w = smls[0]->seed_weight;
+    const uint64_t seed = smls[0]->seed >> __builtin_ctzll(smls[0]->seed);
+    bool pal = S <= 32;
+    for (int q = 0; q < S && pal; ++q) pal = ((seed >> q) & 1ull) == ((seed >> (S - 1 - q)) & 1ull);
+    env->seed_len = S;
+    env->pat = (uint32_t)seed;
+    env->mask = w >= 32 ? ~0ull : (~0ull << (64 - 2 * w));
+    *rc = MH_OK;
+    for (int g = 0; g < k; ++g) {
+        const mh_sml *s = smls[g];
+        env->L[g] = (uint32_t)s->len;
+        env->fwd[g] = env->rev[g] = pal ? (const void *)s->d_words : (const void *)s->d_keys_pos;
+        if (!pal || !rc_bufs[g]) continue;
+        if ((*rc = rc_bufs[g]->ensure(s->n_words * 4 + 64)) != MH_OK) return pal;
+        env->rev[g] = rc_bufs[g]->ptr;
+        hipLaunchKernelGGL(rc_pack_kernel, dim3((unsigned)((s->n_words + 255) / 256)), dim3(256), 0, ctx->stream,
+                           s->d_words, s->len, s->n_words, rc_bufs[g]->as<uint32_t>());
     }
-    std::vector<DiagGroup> tab;
-    std::vector<DiagHead> hp;
-    std::vector<size_t> owner;
-    std::vector<uint8_t> esc;
-    for (int iter = 0;; ++iter) {
-        MH_CHECK(iter < 16, MH_ERR_DEVICE, "long seed extensions did not settle");
-        tab.clear();
-        hp.clear();
-        owner.clear();
-        int64_t N = 0, max_n = 1;
-        for (size_t k = 0; k < diags.size(); ++k) {
-            Diag &d = diags[k];
-            if (d.done) continue;
-            DiagGroup t;
-            t.lo = std::max(d.glo, d.smin - d.reach);
-            const int64_t hi = std::min(d.ghi, d.smax + d.reach);
-            t.n = hi - t.lo + 1;
-            t.base = N;
-            t.dconst = d.dconst;
-            t.rev = d.rev;
-            t.clip_lo = t.lo > d.glo;
-            t.clip_hi = hi < d.ghi;
-            t.pad = 0;
-            N += t.n;
-            max_n = std::max(max_n, t.n);
-            for (size_t i = d.h0; i < d.h1; ++i) {
-                DiagHead h = hh[i];
-                h.group = (uint32_t)tab.size();
-                hp.push_back(h);
-            }
-            owner.push_back(k);
-            tab.push_back(t);
-        }
-        if (tab.empty()) break;
-        MH_CHECK(N < (int64_t)DG_IDX, MH_ERR_UNSUPPORTED, "long seed extensions span too many windows");
-        const uint64_t nh = hp.size(), ng = tab.size();
-        if ((rc = g[1].ensure(ng * sizeof(DiagGroup) + 64)) != MH_OK) return rc;
-        if ((rc = g[0].ensure(nh * sizeof(DiagHead) + 64)) != MH_OK) return rc;
-        if ((rc = g[2].ensure((uint64_t)N + 64)) != MH_OK) return rc;
-        for (int q = 3; q < 7; ++q)
-            if ((rc = g[q].ensure((uint64_t)N * 4 + 64)) != MH_OK) return rc;
-        if ((rc = g[7].ensure(nh + 64)) != MH_OK) return rc;
-        DiagGroup *d_tab = g[1].as<DiagGroup>();
-        DiagHead *d_hp = g[0].as<DiagHead>();
-        uint8_t *mg = g[2].as<uint8_t>(), *d_esc = g[7].as<uint8_t>();
-        uint32_t *l0 = g[3].as<uint32_t>(), *r0 = g[4].as<uint32_t>(), *l1 = g[5].as<uint32_t>(),
-                 *r1 = g[6].as<uint32_t>();
-        MH_HIP(hipMemcpyAsync(d_tab, tab.data(), ng * sizeof(DiagGroup), hipMemcpyHostToDevice, ctx->stream));
-        MH_HIP(hipMemcpyAsync(d_hp, hp.data(), nh * sizeof(DiagHead), hipMemcpyHostToDevice, ctx->stream));
-        const dim3 grid((unsigned)((N + 255) / 256));
-        int rounds = 1;
-        while ((1ll << (rounds - 1)) < max_n) ++rounds;
-        hipLaunchKernelGGL(dg_match_kernel, grid, blk, 0, ctx->stream, d_tab, (uint32_t)ng, (uint64_t)N, env, mg);
-        hipLaunchKernelGGL(dg_link_kernel, grid, blk, 0, ctx->stream, d_tab, (uint32_t)ng, (uint64_t)N, (int)L, mg,
-                           l0, r0);
-        for (int r = 0; r < rounds; ++r) {
-            hipLaunchKernelGGL(dg_jump_kernel, grid, blk, 0, ctx->stream, (uint64_t)N, l0, r0, l1, r1);
-            std::swap(l0, l1);
-            std::swap(r0, r1);
-        }
-        hipLaunchKernelGGL(dg_step_kernel, grid, blk, 0, ctx->stream, d_tab, (uint32_t)ng, (uint64_t)N, (int)L, mg,
-                           l0, r0, l1, r1);
-        std::swap(l0, l1);
-        std::swap(r0, r1);
-        for (int r = 0; r < rounds; ++r) {
-            hipLaunchKernelGGL(dg_jump_or_kernel, grid, blk, 0, ctx->stream, (uint64_t)N, l0, r0, l1, r1);
-            std::swap(l0, l1);
-            std::swap(r0, r1);
-        }
-        hipLaunchKernelGGL(dg_result_kernel, dim3((unsigned)((nh + 255) / 256)), blk, 0, ctx->stream, d_hp, nh,
-                           d_tab, l0, r0, (int)L, hres, d_esc);
-        MH_HIP(hipGetLastError());
-        esc.resize(nh);
-        MH_HIP(hipMemcpyAsync(esc.data(), d_esc, nh, hipMemcpyDeviceToHost, ctx->stream));
-        MH_HIP(hipStreamSynchronize(ctx->stream));
-        std::vector<uint8_t> redo(ng, 0);
-        for (uint64_t i = 0; i < nh; ++i)
-            if (esc[i]) redo[hp[i].group] = 1;
-        for (uint64_t k = 0; k < ng; ++k) {
-            Diag &d = diags[owner[k]];
-            if (redo[k]) d.reach *= 8;
-            else d.done = true;
-        }
-    }
-    return MH_OK;
+    return pal;
 }
 
-// Spaced-seed extension with one ExtendMatch per grid chain (see the kernels
-// above): sort the seeds by (diagonal, start), link each to its chain
-// predecessor, find chain heads by pointer jumping, extend the heads, copy.
-static int extend_by_chains(mh_context *ctx, const mh_sml *a, const mh_sml *b, const uint32_t *oi,
-                            const uint32_t *oj, uint64_t ns, const ExtEnv &env, SeedRec *d_seeds, uint32_t *cnt)
+// Seeds of a pair, other than odd solid ones, in HashMatch order with their
+// extensions (the kernels above).  cnt[0, 2): cleared; heads, long walks.
+static int extend_by_runs(mh_context *ctx, const mh_sml *a, const mh_sml *b, const uint32_t *oi, const uint32_t *oj,
+                          uint64_t ns, SeedRec *d_seeds, uint32_t *cnt)
 {
-    DevBuf *g = ctx->grid_scratch;
+    const uint64_t L0 = a->len, S = (uint64_t)a->seed_length;
+    DevBuf *rs = ctx->run_scratch;
     int rc;
-    for (int q = 0; q < 2; ++q)
-        if ((rc = g[q].ensure(ns * 8 + 64)) != MH_OK) return rc;            // keys
-    for (int q = 2; q < 8; ++q)
-        if ((rc = g[q].ensure(ns * 4 + 64)) != MH_OK) return rc;            // u32 arrays
-    if ((rc = g[8].ensure(((ns + JTILE - 1) / JTILE) * 4 + 64)) != MH_OK) return rc;
-    if ((rc = g[9].ensure(ns * sizeof(SeedRec) + 64)) != MH_OK) return rc;
-    if ((rc = g[10].ensure(ns * 4 + 64)) != MH_OK) return rc;
-    int bits = 1;
-    while (bits < 32 && (1ull << bits) - 1 < a->len) ++bits;
-    const dim3 grid((unsigned)((ns + 255) / 256)), blk(256);
-    uint64_t *k0 = g[0].as<uint64_t>(), *k1 = g[1].as<uint64_t>();
-    uint32_t *v0 = g[2].as<uint32_t>(), *v1 = g[3].as<uint32_t>();
-    int32_t *t1 = g[10].as<int32_t>();
-    hipLaunchKernelGGL(grid_key_kernel, grid, blk, 0, ctx->stream, oi, oj, ns, a->d_keys, a->d_pos, b->d_keys,
-                       b->d_pos, k0, v0, t1);
-    uint64_t *sk = nullptr;
-    uint32_t *sv = nullptr;
-    if ((rc = radix_sort_kv(ctx, k0, v0, k1, v1, ns, bits, &sk, &sv)) != MH_OK) return rc;
-    // the sort's spare value array holds the links, g[4] their jumps
-    uint32_t *la = sv == v0 ? v1 : v0, *lb = g[4].as<uint32_t>();
-    hipLaunchKernelGGL(grid_pred_kernel, grid, blk, 0, ctx->stream, sk, sv, t1, ns, (uint32_t)env.seed_len, 64, la);
-    // links point to earlier sorted entries, so a chain has at most ns seeds and
-    // this many doublings reach every head without a check in between
-    int rounds = 1;
-    while ((1ull << (rounds - 1)) < ns) ++rounds;
-    for (int round = 0; round < rounds; ++round) {
-        hipLaunchKernelGGL(grid_jump_kernel, grid, blk, 0, ctx->stream, la, lb, ns);
+    if ((rc = rs[0].ensure(L0 * 4 * 4 + 64)) != MH_OK) return rc;
+    if ((rc = ctx->grid_scratch[7].ensure(ns * 4 + 64)) != MH_OK) return rc;
+    if ((rc = ctx->grid_scratch[6].ensure(ns * 4 + 64)) != MH_OK) return rc;
+    uint2 *pp = rs[0].as<uint2>();
+    uint32_t *la = (uint32_t *)(pp + L0), *lb = la + L0;
+    uint32_t *heads = ctx->grid_scratch[7].as<uint32_t>(), *rest = ctx->grid_scratch[6].as<uint32_t>();
+    const mh_sml *smls[2] = {a, b};
+    DevBuf *bufs[2] = {nullptr, &ctx->mf_scratch[7]};
+    WalkEnv env;
+    const bool pal = walk_env(ctx, smls, 2, bufs, &env, &rc);
+    if (rc != MH_OK) return rc;
+    const dim3 gs((unsigned)((ns + 255) / 256)), gp((unsigned)((L0 + 255) / 256)), blk(256);
+    MH_HIP(hipMemsetAsync(pp, 0xFF, L0 * 8, ctx->stream));
+    hipLaunchKernelGGL(run_scatter_kernel, gs, blk, 0, ctx->stream, oi, oj, ns, a->d_keys, a->d_pos, b->d_keys,
+                       b->d_pos, pp);
+    hipLaunchKernelGGL(spaced_link_kernel, gp, blk, 0, ctx->stream, pp, L0, (uint32_t)S, la);
+    // so many launches reach every head, without a check in between
+    const uint64_t longest = std::min<uint64_t>(ns, 2 * (L0 / S) + 2);
+    for (uint64_t reach = 1; reach < longest; reach *= 8) {
+        hipLaunchKernelGGL(grid_jump_kernel, gp, blk, 0, ctx->stream, la, lb, L0);
         std::swap(la, lb);
     }
-    uint32_t *is_head = g[5].as<uint32_t>(), *head_of = g[6].as<uint32_t>();
-    hipLaunchKernelGGL(grid_head_kernel, grid, blk, 0, ctx->stream, sv, la, ns, is_head, head_of);
-    // the heads in genome-1 order, so that neighbouring threads walk
-    // neighbouring stretches and share cache lines
-    uint32_t *heads = g[7].as<uint32_t>();
-    hipLaunchKernelGGL(chain_root_flag_kernel, grid, blk, 0, ctx->stream, la, ns, lb);
-    uint64_t nh = 0;
-    if ((rc = compact_flags(ctx, lb, ns, heads, g[8].as<uint32_t>(), cnt + 3, &nh)) != MH_OK) return rc;
-    if (nh)
-        hipLaunchKernelGGL(chain_gather_kernel, dim3((unsigned)((nh + 255) / 256)), blk, 0, ctx->stream, sv, nh,
-                           heads);
-    // head operands reuse the key buffer the sort left spare (8 ns + 64 bytes)
-    uint32_t *hoi = reinterpret_cast<uint32_t *>(sk == k0 ? k1 : k0), *hoj = hoi + ns + 16;
-    uint32_t *headpos = lb;
-    SeedRec *hres = g[9].as<SeedRec>();
-    const dim3 hgrid((unsigned)((nh + 255) / 256));
-    hipLaunchKernelGGL(grid_gather_kernel, hgrid, blk, 0, ctx->stream, heads, nh, oi, oj, hoi, hoj, headpos);
-    // heads: the step-by-step walk up to a budget, the longer ones per diagonal
-    uint32_t *long_flag = is_head, *long_idx = heads;   // both free by now
-    hipLaunchKernelGGL(seed_kernel, hgrid, blk, 0, ctx->stream, hoi, hoj, nh, a->d_keys, a->d_pos, b->d_keys,
-                       b->d_pos, env, (int64_t)LONG_WALK, hres, cnt + 2, long_flag);
-    uint64_t nl = 0;
-    if ((rc = compact_flags(ctx, long_flag, nh, long_idx, g[8].as<uint32_t>(), cnt + 3, &nl)) != MH_OK) return rc;
-    if (nl && (rc = resolve_long(ctx, a, b, env, long_idx, nl, hoi, hoj, hres)) != MH_OK) return rc;
-    ctx->last_walks = nh;
-    ctx->last_long_walks = nl;
-    hipLaunchKernelGGL(grid_fill_kernel, grid, blk, 0, ctx->stream, oi, oj, ns, a->d_keys, a->d_pos, b->d_keys,
-                       b->d_pos, head_of, headpos, hres, d_seeds);
+    hipLaunchKernelGGL(spaced_heads_kernel, gp, blk, 0, ctx->stream, pp, la, L0, heads, cnt);
+    if (pal)
+        launch_walks(ctx, PairWalks<true>{heads, oi, oj, a->d_keys, b->d_keys, a->d_pos, b->d_pos, d_seeds}, ns, cnt,
+                     env, rest, cnt + 1);
+    else
+        launch_walks(ctx, PairWalks<false>{heads, oi, oj, a->d_keys, b->d_keys, a->d_pos, b->d_pos, d_seeds}, ns, cnt,
+                     env, rest, cnt + 1);
+    hipLaunchKernelGGL(spaced_fill_kernel, gp, blk, 0, ctx->stream, pp, la, L0, d_seeds);
     MH_HIP(hipGetLastError());
     return MH_OK;
 }
@@ -1543,7 +1253,7 @@ int join_and_extend(mh_context *ctx, const mh_sml *a, const mh_sml *b, const Liv
     uint32_t *flag = ctx->mf_scratch[0].as<uint32_t>();
     uint32_t *partner = ctx->mf_scratch[1].as<uint32_t>();
     uint32_t *tiles = ctx->mf_scratch[2].as<uint32_t>();
-    uint32_t *cnt = ctx->mf_scratch[3].as<uint32_t>();   // [1] total seeds, [2] ext errors
+    uint32_t *cnt = ctx->mf_scratch[3].as<uint32_t>();   // [1] total seeds, [4], [5] walk_kernel's
     // live ranges other than the whole list go to the device
     LivePair lp;
     std::memset(&lp, 0, sizeof(lp));
@@ -1573,7 +1283,7 @@ int join_and_extend(mh_context *ctx, const mh_sml *a, const mh_sml *b, const Liv
         // a list that reads nothing gives no seeds
         if ((cut_a && ca == 0) || (cut_b && cb == 0)) return MH_OK;
     }
-    MH_HIP(hipMemsetAsync(cnt, 0, 16, ctx->stream));
+    MH_HIP(hipMemsetAsync(cnt, 0, 32, ctx->stream));
     const bool tiled = !cut_a && !cut_b;
     const uint64_t ntj = (n0 + TJ_I - 1) / TJ_I;
     if (tiled) {
@@ -1619,15 +1329,6 @@ int join_and_extend(mh_context *ctx, const mh_sml *a, const mh_sml *b, const Liv
         hipLaunchKernelGGL(compact_kernel, dim3((unsigned)ntiles), dim3(JT), 0, ctx->stream, flag, partner, n0, tiles,
                            oi, oj);
     }
-    ExtEnv env;
-    env.kp0 = a->d_keys_pos;
-    env.kp1 = b->d_keys_pos;
-    env.n0 = n0;
-    env.n1 = n1;
-    env.L0 = (int64_t)a->len;
-    env.L1 = (int64_t)b->len;
-    env.seed_len = a->seed_length;
-    env.mer_mask = a->seed_weight >= 32 ? ~0ull : (~0ull << (64 - 2 * a->seed_weight));
     const bool solid_odd = a->seed_length == a->seed_weight && (a->seed_length & 1);
     if (solid_odd) {
         if ((rc = ctx->mf_scratch[7].ensure(b->n_words * 4 + 64)) != MH_OK) return rc;
@@ -1658,26 +1359,19 @@ int join_and_extend(mh_context *ctx, const mh_sml *a, const mh_sml *b, const Liv
         hipLaunchKernelGGL(run_final_kernel, dim3((unsigned)nb), dim3(RS_T), 0, ctx->stream, fl, pp, L0, chead,
                            ctail, lft, rgt, (int64_t)b->len, a->seed_length, d_seeds);
         MH_HIP(hipGetLastError());
-        ctx->last_walks = ns;
-    } else if (a->len < (1ull << 30) && b->len < (1ull << 30)) {
-        TimedLaunch tl(ctx, "extend");
-        if ((rc = extend_by_chains(ctx, a, b, oi, oj, ns, env, d_seeds, cnt)) != MH_OK) return rc;
     } else {
         TimedLaunch tl(ctx, "extend");
-        hipLaunchKernelGGL(seed_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, ctx->stream, oi, oj, ns,
-                           a->d_keys, a->d_pos, b->d_keys, b->d_pos, env, (int64_t)0, d_seeds, cnt + 2,
-                           (uint32_t *)nullptr);
-        MH_HIP(hipGetLastError());
-        ctx->last_walks = ns;
+        if ((rc = extend_by_runs(ctx, a, b, oi, oj, ns, d_seeds, cnt + 4)) != MH_OK) return rc;
     }
-    uint32_t ext_err = 0;
-    MH_HIP(hipMemcpyAsync(&ext_err, cnt + 2, 4, hipMemcpyDeviceToHost, ctx->stream));
+    uint32_t walked[2] = {(uint32_t)ns, 0};
+    if (!solid_odd) MH_HIP(hipMemcpyAsync(walked, cnt + 4, 8, hipMemcpyDeviceToHost, ctx->stream));
     const double t0 = now_ms();
     MH_HIP(hipStreamSynchronize(ctx->stream));
     host_time(ctx, "host_wait_seeds", now_ms() - t0);
+    ctx->last_walks = walked[0];
+    ctx->last_long_walks = walked[1];
     *seeds_out = d_seeds;
     *ns_out = ns;
-    MH_CHECK(ext_err == 0, MH_ERR_UNSUPPORTED, "seed extension left the sorted mer lists");
     return MH_OK;
 }
 
@@ -1801,6 +1495,7 @@ struct UqLists {
     const uint32_t *w[EXT_MAXK];      // packed sequence
     const uint32_t *wrc[EXT_MAXK];    // packed reverse complement
     uint64_t off[EXT_MAXK];           // each list's first entry in the merged numbering
+    int64_t L[EXT_MAXK];
 };
 
 __global__ void uq_gather_kernel(const uint64_t *__restrict__ ck, uint64_t lo, uint64_t cnt, uint64_t tag,
@@ -1837,14 +1532,12 @@ __global__ void uq_leader_kernel(const uint64_t *__restrict__ key, const uint32_
 
 __global__ void uq_seed_kernel(const uint64_t *__restrict__ key, const uint32_t *__restrict__ val,
                                const uint32_t *__restrict__ U, uint64_t m, const uint32_t *__restrict__ lead,
-                               uint64_t ns, UqLists ls, ExtEnvK env, int k, int solid_odd, int walk,
-                               int32_t *__restrict__ seed_st, int32_t *__restrict__ ext_st,
-                               uint32_t *__restrict__ ext_len, int64_t *__restrict__ offset,
-                               uint32_t *__restrict__ err)
+                               uint64_t ns, UqLists ls, int sl, int k, int solid_odd, int32_t *__restrict__ seed_st,
+                               int32_t *__restrict__ ext_st, uint32_t *__restrict__ ext_len,
+                               int64_t *__restrict__ offset)
 {
     const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= ns) return;
-    const int sl = env.seed_len;
     int gs[EXT_MAXK];
     int64_t st[EXT_MAXK], p[EXT_MAXK];
     int used = 0, fstrand = 0;
@@ -1875,13 +1568,13 @@ __global__ void uq_seed_kernel(const uint64_t *__restrict__ key, const uint32_t 
     if (solid_odd) {
         // the shortest of the pairwise maximal exact matches with the first genome
         const int f = gs[0];
-        const int64_t pf = p[0], Lf = env.L[f];
+        const int64_t pf = p[0], Lf = ls.L[f];
         int64_t left = pf, right = Lf - (pf + sl);
         int64_t q1[EXT_MAXK];
         for (int x = 1; x < used; ++x) {
             const int g = gs[x];
             const bool rev = st[x] < 0;
-            const int64_t Lg = env.L[g];
+            const int64_t Lg = ls.L[g];
             q1[x] = rev ? Lg - p[x] - sl : p[x];
             const uint32_t *wg = rev ? ls.wrc[g] : ls.w[g];
             const int64_t lim_l = left < q1[x] ? left : q1[x];
@@ -1895,11 +1588,9 @@ __global__ void uq_seed_kernel(const uint64_t *__restrict__ key, const uint32_t 
         len = sl + left + right;
         ex[0] = pf - left + 1;
         for (int x = 1; x < used; ++x)
-            ex[x] = st[x] > 0 ? q1[x] - left + 1 : -(env.L[gs[x]] - (q1[x] - left + len) + 1);
+            ex[x] = st[x] > 0 ? q1[x] - left + 1 : -(ls.L[gs[x]] - (q1[x] - left + len) + 1);
     } else {
-        if (!walk) return;   // extended by chains (uq_chain_*)
-        for (int x = 0; x < used; ++x) ex[x] = st[x];
-        if (extend_k(env, gs, used, ex, len) != EXT_OK) atomicOr(err, 1u);
+        return;   // extended by walks (uq_extend_by_chains)
     }
     for (int g = 0; g < k; ++g) ext_st[s * k + g] = 0;
     for (int x = 0; x < used; ++x) ext_st[s * k + gs[x]] = (int32_t)ex[x];
@@ -1908,13 +1599,10 @@ __global__ void uq_seed_kernel(const uint64_t *__restrict__ key, const uint32_t 
 
 // ---- spaced seeds: one k-genome walk per chain ---------------------------
 // As for two genomes (grid_* kernels): seed B and seed A with the same
-// genomes, where every start of A is B's minus the seed length L (forward:
-// the window L to the left; reversed: -(q + 1) - L, the window L to the right
-// in that genome's forward coordinates), extend to the same match.  B's first
-// seed-length step to the left lands on A's windows, which match (A is a
-// seed), and from there its walk is A's; A's first step to the right lands
-// on B's windows the same way.  Each chain is walked once, from its first
-// seed (its head), and the others copy the head's extension.
+// genomes, where every start of A is B's minus one distance of at most a seed
+// length (reversed: the window as far to the right in that genome's forward
+// coordinates), extend to the same match.  Each chain of such seeds is walked
+// once, from its first seed (its head), and the others copy the head's extension.
 
 // key: the first present genome and its (positive) start; a genome position
 // holds one mer, so no two seeds share a key
@@ -1929,7 +1617,7 @@ __global__ void uq_chain_key_kernel(const int32_t *__restrict__ seed_st, uint64_
     val[s] = (uint32_t)s;
 }
 
-// link[r] = the sorted index of seed r's chain predecessor, or r
+// link[r] = the sorted index of the nearest seed before r on its chain, or r
 __global__ void uq_chain_pred_kernel(const uint64_t *__restrict__ sk, const uint32_t *__restrict__ sv, uint64_t ns,
                                      const int32_t *__restrict__ seed_st, int k, uint32_t seed_len,
                                      uint32_t *__restrict__ link)
@@ -1937,70 +1625,76 @@ __global__ void uq_chain_pred_kernel(const uint64_t *__restrict__ sk, const uint
     const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= ns) return;
     const uint64_t key = sk[r];
+    const int32_t *b = seed_st + (uint64_t)sv[r] * k;
     uint32_t out = (uint32_t)r;
-    if ((key & 0xFFFFFFFFull) > seed_len) {
-        const uint64_t want = key - seed_len;
-        uint64_t lo = 0, hi = r;
-        while (lo < hi) {
-            const uint64_t mid = (lo + hi) / 2;
-            if (sk[mid] < want) lo = mid + 1;
-            else hi = mid;
-        }
-        if (lo < r && sk[lo] == want) {
-            const int32_t *b = seed_st + (uint64_t)sv[r] * k, *a = seed_st + (uint64_t)sv[lo] * k;
-            bool same = true;
-            for (int g = 0; g < k && same; ++g)
-                same = b[g] == 0 ? a[g] == 0 : (a[g] == b[g] - (int32_t)seed_len && (b[g] < 0 || a[g] > 0));
-            if (same) out = (uint32_t)lo;
+    for (uint64_t x = r; x > 0; --x) {
+        const uint64_t d = key - sk[x - 1];       // (another genome's: 2^32 less a start or more)
+        if (d > seed_len) break;
+        const int32_t *a = seed_st + (uint64_t)sv[x - 1] * k;
+        bool same = true;
+        for (int g = 0; g < k && same; ++g)
+            same = b[g] == 0 ? a[g] == 0 : (a[g] == b[g] - (int32_t)d && (b[g] < 0 || a[g] > 0));
+        if (same) {
+            out = (uint32_t)(x - 1);
+            break;
         }
     }
     link[r] = out;
 }
 
-// the heads' walks (extend_kt: a seed holds at most KMAX genomes)
-template <int KMAX>
-__global__ __launch_bounds__(128) void uq_chain_walk_kernel(const uint32_t *__restrict__ heads, uint64_t nh, ExtEnvK env, int k,
-                                     const int32_t *__restrict__ seed_st, int32_t *__restrict__ ext_st,
-                                     uint32_t *__restrict__ ext_len, uint32_t *__restrict__ err)
-{
-    const uint64_t h = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nh) return;
-    const uint64_t s = heads[h];
-    const uint64_t *gk[KMAX];
-    uint32_t gn[KMAX];
-    int64_t gL[KMAX], ex[KMAX];
-    int gsl[KMAX];
-    int used = 0;
-    for (int g = 0; g < k; ++g) {
-        const int32_t v = seed_st[s * k + g];
-        if (v == 0) continue;
-#pragma unroll
-        for (int x = 0; x < KMAX; ++x)
-            if (x == used) {
-                gk[x] = env.kp[g];
-                gn[x] = (uint32_t)env.n[g];
-                gL[x] = env.L[g];
-                ex[x] = v;
-                gsl[x] = g;
-            }
-        ++used;
-    }
-#pragma unroll
-    for (int x = 1; x < KMAX; ++x)
-        if (x >= used) {
-            gk[x] = gk[0];
-            gn[x] = gn[0];
-            gL[x] = 0;
-            ex[x] = 0;
-            gsl[x] = 0;
+// the seeds heads (null: all) as walks, of at most MK genomes
+template <int MK, bool P> struct UqWalks {
+    static constexpr int K = MK;
+    static constexpr bool PAL = P;
+    const uint32_t *heads;
+    int k;
+    const int32_t *seed_st;
+    int32_t *ext_st;
+    uint32_t *ext_len;
+
+    __device__ __forceinline__ void load(uint64_t x, const WalkEnv &env, Walk<K, P> &w) const
+    {
+        const uint64_t s = heads ? heads[x] : x;
+        int used = 0;
+        for (int g = 0; g < k; ++g) {
+            const int32_t v = seed_st[s * k + g];
+            if (v == 0) continue;
+MH_PRAGMA_UNROLL
+            for (int t = 0; t < K; ++t)
+                if (t == used) w.set(t, env, g, (uint32_t)(v < 0 ? -v : v) - 1, v < 0);
+            ++used;
         }
-    int64_t len = env.seed_len;
-    if (extend_kt<KMAX>(gk, gn, gL, used, env.seed_len, env.mer_mask, ex, len) != EXT_OK) atomicOr(err, 1u);
-    for (int g = 0; g < k; ++g) ext_st[s * k + g] = 0;
-#pragma unroll
-    for (int x = 0; x < KMAX; ++x)
-        if (x < used) ext_st[s * k + gsl[x]] = (int32_t)ex[x];
-    ext_len[s] = (uint32_t)len;
+        w.fill(used);
+    }
+    __device__ __forceinline__ void store(uint64_t x, const Walk<K, P> &w, uint32_t left, uint32_t len) const
+    {
+        const uint64_t s = heads ? heads[x] : x;
+        int used = 0;
+        for (int g = 0; g < k; ++g) {
+            const int32_t v = seed_st[s * k + g];
+            int32_t e = 0;
+            if (v != 0) {
+MH_PRAGMA_UNROLL
+                for (int t = 0; t < K; ++t)
+                    if (t == used) {
+                        const uint32_t q = w.p[t] - left;
+                        e = v < 0 ? -(int32_t)(w.n[t] - q - len + 1) : (int32_t)q + 1;
+                    }
+                ++used;
+            }
+            ext_st[s * k + g] = e;
+        }
+        ext_len[s] = len;
+    }
+};
+
+template <bool P>
+void uq_launch_walks(mh_context *ctx, const uint32_t *heads, uint64_t nh, const WalkEnv &env, int k,
+                     const int32_t *d_sst, int32_t *d_est, uint32_t *d_len, uint32_t *rest, uint32_t *cnt)
+{
+    if (k <= 4) launch_walks(ctx, UqWalks<4, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt);
+    else if (k <= 8) launch_walks(ctx, UqWalks<8, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt);
+    else launch_walks(ctx, UqWalks<16, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt);
 }
 
 // every other seed copies its head's extension
@@ -2443,10 +2137,12 @@ __global__ void uq_emit_kernel(UqSeeds q, const uint32_t *__restrict__ bstart, c
 // Spaced-seed extension of the k-genome seeds with one walk per chain (the
 // uq_chain_* kernels): sort the seeds by (first genome, start), link each to
 // its chain predecessor, find the heads by pointer jumping, walk the heads,
-// copy.  ext_st / ext_len as uq_seed_kernel writes them; *err set by a walk
-// that left a list; *walks the heads walked.
-static int uq_extend_by_chains(mh_context *ctx, const int32_t *d_sst, uint64_t S, int k, const ExtEnvK &env,
-                               int32_t *d_est, uint32_t *d_len, uint32_t *err, uint64_t *walks)
+// copy.  ext_st / ext_len as uq_seed_kernel writes them; *walks the heads
+// walked.  Without chains every seed walks.  max_len: the longest genome's; cnt
+// cleared.
+static int uq_extend_by_chains(mh_context *ctx, const int32_t *d_sst, uint64_t S, int k, const WalkEnv &env, bool pal,
+                               bool chains, uint64_t max_len, int32_t *d_est, uint32_t *d_len, uint32_t *cnt,
+                               uint64_t *walks)
 {
     DevBuf *g = ctx->grid_scratch;
     int rc;
@@ -2456,6 +2152,16 @@ static int uq_extend_by_chains(mh_context *ctx, const int32_t *d_sst, uint64_t S
         if ((rc = g[q].ensure(S * 4 + 64)) != MH_OK) return rc;            // u32 arrays
     if ((rc = g[8].ensure(((S + JTILE - 1) / JTILE) * 4 + 64)) != MH_OK) return rc;
     if ((rc = g[10].ensure(64)) != MH_OK) return rc;
+    auto walk = [&](const uint32_t *heads, uint64_t nh, uint32_t *rest) {
+        if (pal) uq_launch_walks<true>(ctx, heads, nh, env, k, d_sst, d_est, d_len, rest, cnt);
+        else uq_launch_walks<false>(ctx, heads, nh, env, k, d_sst, d_est, d_len, rest, cnt);
+    };
+    if (!chains) {
+        walk(nullptr, S, g[7].as<uint32_t>());
+        MH_HIP(hipGetLastError());
+        *walks = S;
+        return MH_OK;
+    }
     const dim3 grid((unsigned)((S + 255) / 256)), blk(256);
     uint64_t *k0 = g[0].as<uint64_t>(), *k1 = g[1].as<uint64_t>();
     uint32_t *v0 = g[2].as<uint32_t>(), *v1 = g[3].as<uint32_t>();
@@ -2466,10 +2172,8 @@ static int uq_extend_by_chains(mh_context *ctx, const int32_t *d_sst, uint64_t S
     uint32_t *la = sv == v0 ? v1 : v0, *lb = g[4].as<uint32_t>();
     hipLaunchKernelGGL(uq_chain_pred_kernel, grid, blk, 0, ctx->stream, sk, sv, S, d_sst, k, (uint32_t)env.seed_len,
                        la);
-    // links point to earlier sorted entries: this many doublings reach every head
-    int rounds = 1;
-    while ((1ull << (rounds - 1)) < S) ++rounds;
-    for (int round = 0; round < rounds; ++round) {
+    // links point to earlier starts in one genome: so many launches reach every head
+    for (uint64_t reach = 1; reach < std::min(S, max_len); reach *= 8) {
         hipLaunchKernelGGL(grid_jump_kernel, grid, blk, 0, ctx->stream, la, lb, S);
         std::swap(la, lb);
     }
@@ -2485,16 +2189,7 @@ static int uq_extend_by_chains(mh_context *ctx, const int32_t *d_sst, uint64_t S
     if (nh) {
         hipLaunchKernelGGL(chain_gather_kernel, dim3((unsigned)((nh + 255) / 256)), blk, 0, ctx->stream, sv, nh,
                            heads);
-        const dim3 hg((unsigned)((nh + 127) / 128)), hb(128);
-        if (k <= 4)
-            hipLaunchKernelGGL(uq_chain_walk_kernel<4>, hg, hb, 0, ctx->stream, heads, nh, env, k, d_sst, d_est, d_len,
-                               err);
-        else if (k <= 8)
-            hipLaunchKernelGGL(uq_chain_walk_kernel<8>, hg, hb, 0, ctx->stream, heads, nh, env, k, d_sst, d_est, d_len,
-                               err);
-        else
-            hipLaunchKernelGGL(uq_chain_walk_kernel<16>, hg, hb, 0, ctx->stream, heads, nh, env, k, d_sst, d_est,
-                               d_len, err);
+        walk(heads, nh, sflag);
     }
     hipLaunchKernelGGL(uq_chain_fill_kernel, grid, blk, 0, ctx->stream, is_head, head_of, S, k, d_est, d_len);
     MH_HIP(hipGetLastError());
@@ -2573,16 +2268,10 @@ int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRa
     out->walks = S;
     if (S == 0) return MH_OK;
     const bool solid_odd = smls[0]->seed_length == smls[0]->seed_weight && (smls[0]->seed_length & 1);
-    ExtEnvK env;
-    std::memset(&env, 0, sizeof(env));
-    env.seed_len = sl;
-    env.mer_mask = w >= 32 ? ~0ull : (~0ull << (64 - 2 * w));
     uint64_t longest = 0;
     for (int g = 0; g < k; ++g) {
         longest = std::max<uint64_t>(longest, smls[g]->len);
-        env.kp[g] = smls[g]->d_keys_pos;
-        env.n[g] = smls[g]->n;
-        env.L[g] = (int64_t)smls[g]->len;
+        ls.L[g] = (int64_t)smls[g]->len;
         MH_CHECK(smls[g]->len < (1ull << 31), MH_ERR_UNSUPPORTED, "genomes of 2^31 bases or more");
     }
     if (solid_odd) {
@@ -2598,23 +2287,27 @@ int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRa
     int32_t *d_est = d_sst + S * k;
     uint32_t *d_len = reinterpret_cast<uint32_t *>(d_est + S * k);
     int64_t *d_off = reinterpret_cast<int64_t *>((reinterpret_cast<uintptr_t>(d_len + S) + 7) & ~(uintptr_t)7);
-    MH_HIP(hipMemsetAsync(d_cnt, 0, 4, ctx->stream));
+    MH_HIP(hipMemsetAsync(d_cnt, 0, 8, ctx->stream));
     {
         TimedLaunch tl(ctx, "extend");
         // spaced seeds: starts and offsets here, one walk per chain below
         // (MH_UQ_CHAINS=0 walks every seed)
         const char *ce = getenv("MH_UQ_CHAINS");
-        const bool chains = !solid_odd && !(ce && ce[0] == '0');
+        const bool chains = !(ce && ce[0] == '0');
         hipLaunchKernelGGL(uq_seed_kernel, dim3((unsigned)((S + 127) / 128)), dim3(128), 0, ctx->stream, sk, sv, U, M,
-                           lead, S, ls, env, k, solid_odd ? 1 : 0, chains ? 0 : 1, d_sst, d_est, d_len, d_off, d_cnt);
+                           lead, S, ls, sl, k, solid_odd ? 1 : 0, d_sst, d_est, d_len, d_off);
         MH_HIP(hipGetLastError());
-        if (chains && (rc = uq_extend_by_chains(ctx, d_sst, S, k, env, d_est, d_len, d_cnt, &out->walks)) != MH_OK)
-            return rc;
+        if (!solid_odd) {
+            DevBuf *bufs[EXT_MAXK];
+            for (int g = 0; g < k; ++g) bufs[g] = &ctx->uq_rc[g];
+            WalkEnv env;
+            const bool pal = walk_env(ctx, smls, k, bufs, &env, &rc);
+            if (rc != MH_OK) return rc;
+            if ((rc = uq_extend_by_chains(ctx, d_sst, S, k, env, pal, chains, longest, d_est, d_len, d_cnt,
+                                          &out->walks)) != MH_OK)
+                return rc;
+        }
     }
-    uint32_t err = 0;
-    MH_HIP(hipMemcpyAsync(&err, d_cnt, 4, hipMemcpyDeviceToHost, ctx->stream));
-    MH_HIP(hipStreamSynchronize(ctx->stream));
-    MH_CHECK(err == 0, MH_ERR_UNSUPPORTED, "seed extension left the sorted mer lists");
     // AddHashEntry, bucket by bucket: seeds ordered by bucket (stable), bucket
     // starts, one wavefront per bucket, the list in bucket order
     const double t0 = now_ms();

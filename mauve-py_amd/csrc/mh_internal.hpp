@@ -117,11 +117,10 @@ struct mh_context {
     mh::DevBuf ml_jobs, ml_y;   // learned band: job table, network outputs + bands
     // seed-matching scratch
     mh::DevBuf mf_scratch[16];
-    mh::DevBuf grid_scratch[11];   // spaced-seed extension by chains
-    mh::DevBuf diag_scratch[8];    // long extensions resolved per diagonal
+    mh::DevBuf grid_scratch[11];   // seed extension by runs and chains
     mh::DevBuf multi_scratch[11];  // the seeds of every genome pair, merged and filtered
     mh::DevBuf heavy_buf, live_buf; // masked mers above the repeat limit; live ranges of a join
-    mh::DevBuf run_scratch[4];      // odd solid seeds extended by runs
+    mh::DevBuf run_scratch[4];      // seeds extended by runs
     mh::DevBuf uq_scratch[8];       // UniqueMatchFinder: merged lists, runs, seeds
     mh::DevBuf uq_rc[16];           // UniqueMatchFinder: packed reverse complements
     uint64_t last_walks = 0, last_long_walks = 0;   // of the last seed extension

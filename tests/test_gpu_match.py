@@ -199,3 +199,23 @@ def test_match_repeat_restart_multi(ctx, ng, seed):
     assert len(gl) == len(ol) > 50
     assert np.array_equal(gs, os_)
     assert np.array_equal(gl, ol)
+
+
+@pytest.mark.parametrize("seed", [po.get_seed(15, 0), 0xFFF, 0x3FFFF, 0b1101011101110111011])
+def test_match_walk_ends(ctx, seed):
+    """The walk's two ends: jumps past a thread's and past a block's number,
+    ends at both sequence ends with less room than a window, single steps up to
+    a seed length behind a difference, windows that are their own reverse
+    complement, on both strands; a palindromic spaced pattern, two solid
+    ones of even length and one that is not palindromic."""
+    rng = np.random.default_rng(seed & 0xFFFF)
+    a = synth.BASES[rng.integers(0, 4, 40_000)]
+    a[12_000:12_040] = np.frombuffer(b"AT" * 20, dtype=np.uint8)
+    a[30_000:30_060] = np.frombuffer(b"ACGT" * 15, dtype=np.uint8)
+    b = a.copy()
+    for p in list(range(22_000, 23_000, 17)) + list(range(25_000, 25_600, 23)) + [11, 39_980]:
+        b[p] = synth.BASES[(int(np.searchsorted(synth.BASES, b[p])) + 1) % 4]
+    b[24_000:33_000] = synth.revcomp(b[24_000:33_000])
+    n = _compare(ctx, a.tobytes(), b.tobytes(), seed)
+    assert n >= 2
+    _compare(ctx, a[:35].tobytes(), synth.revcomp(a[:35].copy()).tobytes(), seed)

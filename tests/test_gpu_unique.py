@@ -147,3 +147,20 @@ def test_unique_many_entries_of_one_bucket(ctx, ng, n):
         seqs.append("".join("ACGT"[x] for x in t))
     st = _check(ctx, seqs, (1 << 13) - 1)
     assert st.matches > n // 40
+
+
+@pytest.mark.parametrize("ng,seed", [(3, 0x16DF6D), (6, 0xFFF), (9, 0x7B974EF), (3, 0b1101011101110111011)])
+def test_unique_long_identical_stretches(ctx, ng, seed):
+    """Walks of more jumps than a thread's number, over up to four, eight and
+    sixteen genomes, on both strands, to the sequences' ends; the last pattern
+    is not palindromic."""
+    rng = np.random.default_rng(ng)
+    base = "".join("ACGT"[x] for x in rng.integers(0, 4, 9000))
+    seqs = []
+    for g in range(ng):
+        t = list(base)
+        for p in range(4000 + 7 * g, 5200, 53 + g):
+            t[p] = "ACGT"[("ACGT".index(t[p]) + 1 + g % 3) % 4]
+        t = "".join(t)
+        seqs.append(t[::-1].translate(COMP) if g % 3 == 1 else t[g:])
+    _check(ctx, seqs, seed)
