@@ -24,9 +24,7 @@
 namespace mh {
 namespace {
 
-constexpr int SORT_THREADS = 256;
-constexpr int SORT_ITEMS = 16;
-constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;   // 4096 entries per tile
+constexpr int SORT_THREADS = 1024;
 
 struct SeedPattern {
     int sl, sw, spaced;
@@ -119,7 +117,7 @@ __global__ void keys_kernel(const uint32_t *__restrict__ words, uint64_t n, Seed
 // the keys (per-workgroup LDS histograms, reduced and scanned by a second
 // small kernel into each pass's digit starts).  Then one kernel per pass:
 // each workgroup takes the next tile ticket (tiles in ticket order, so a
-// tile's predecessors are already running), ranks its 4096 keys stably in LDS,
+// tile's predecessors are already running), ranks its keys stably in LDS,
 // publishes its digit counts, and finds each digit's offset among the
 // preceding tiles by decoupled look-back over their published counts: a
 // predecessor's word carries either its own count (aggregate) or the sum over
@@ -134,9 +132,14 @@ constexpr int OS_MAX_BITS = 10;                       // widest digit (radix 102
 constexpr int OS_MAX_RADIX = 1 << OS_MAX_BITS;
 constexpr int OS_MAX_PASSES = 8;                      // 64-bit keys
 constexpr int OS_HIST_WGS = 256;                      // workgroups of the histogram
-constexpr int OS_HIST_THREADS = 256;
+constexpr int OS_HIST_THREADS = 1024;
+constexpr int OS_START_THREADS = 1024;
 constexpr int OS_HIST_LDS = 7 * OS_MAX_RADIX;          // passes x radix at most (64-bit keys: 7 x 1024)
 constexpr uint32_t OS_SPIN_MAX = 1u << 22;
+// Below these, tiles of two and four rounds fill more CUs with shorter chains:
+// 20,000 keys 7.7 us a pass (8.7 in four rounds, 11.6 in eight), 200,000 13.4
+// (13.4, 16.2), a million 24.7, 19.9 and 20.4, 4.6 million 85, 57 and 53.
+constexpr uint64_t OS_SMALL = 1u << 18, OS_MIDDLE = 1u << 21;
 constexpr uint64_t OS_FLAG_A = 1, OS_FLAG_P = 2;
 constexpr uint64_t OS_VALUE_MASK = (1ull << 38) - 1;
 
@@ -145,8 +148,10 @@ __device__ __forceinline__ uint64_t os_word(uint32_t epoch, uint64_t flag, uint6
     return ((uint64_t)epoch << 40) | (flag << 38) | v;
 }
 
-// Per-workgroup digit counts of every pass (digits of db bits); workgroup 0
-// also zeroes the passes' tile tickets (the passes run after this kernel on
+// Per-workgroup digit counts of every pass (digits of db bits), bound by the LDS
+// atomics' latency: 16 waves a CU take 18 us over 4.6 million keys, 4 took 24.
+// Workgroup 0
+// also zeroes the passes' tile tickets and os_start_kernel's counts (run after this kernel on
 // the stream).
 __global__ __launch_bounds__(OS_HIST_THREADS) void os_hist_kernel(const uint64_t *__restrict__ keys, uint64_t n,
                                                                  int db, int passes, uint32_t *__restrict__ part,
@@ -156,12 +161,12 @@ __global__ __launch_bounds__(OS_HIST_THREADS) void os_hist_kernel(const uint64_t
     const int t = threadIdx.x, radix = 1 << db;
     const uint32_t mask = (uint32_t)radix - 1u;
     for (int i = t; i < passes * radix; i += OS_HIST_THREADS) h[i] = 0;
-    if (blockIdx.x == 0 && t < OS_MAX_PASSES) tickets[t] = 0;
+    if (blockIdx.x == 0 && t < 2 * OS_MAX_PASSES) tickets[t] = 0;
     __syncthreads();
-    // a contiguous chunk per workgroup, eight keys a thread loaded at once
+    // a contiguous chunk per workgroup, four keys a thread loaded at once
     const uint64_t chunk = (n + gridDim.x - 1) / gridDim.x;
     const uint64_t lo = (uint64_t)blockIdx.x * chunk, hi = min<uint64_t>(n, lo + chunk);
-    constexpr int U = 8;
+    constexpr int U = 4;
     for (uint64_t x0 = lo + t; x0 < hi; x0 += (uint64_t)U * OS_HIST_THREADS) {
         uint64_t k[U];
 #pragma unroll
@@ -180,35 +185,68 @@ __global__ __launch_bounds__(OS_HIST_THREADS) void os_hist_kernel(const uint64_t
     for (int i = t; i < passes * radix; i += OS_HIST_THREADS) out[i] = h[i];
 }
 
-// Pass q = blockIdx.x, digit d = threadIdx.x (blockDim = radix): the digit's
-// total over the histogram workgroups, then the exclusive scan of the totals
-// (the first output position of each digit).
-__global__ __launch_bounds__(OS_MAX_RADIX) void os_start_kernel(const uint32_t *__restrict__ part, int nparts,
-                                                               int passes, uint32_t *__restrict__ start)
+// Pass q = blockIdx.y, 64 digits a workgroup: the digits' totals over the
+// histogram workgroups, a sixteenth of these a wave; the pass's last workgroup
+// scans all totals (the first output position of each digit).  One workgroup a
+// pass pulled half a megabyte through one CU: 11 us for 256 histograms, 5 here.
+__global__ __launch_bounds__(OS_START_THREADS) void os_start_kernel(const uint32_t *__restrict__ part, int nparts,
+                                                                   int passes, int radix, uint32_t *__restrict__ total,
+                                                                   uint32_t *__restrict__ done,
+                                                                   uint32_t *__restrict__ start)
 {
-    __shared__ uint32_t s[OS_MAX_RADIX];
-    const int d = threadIdx.x, q = blockIdx.x, radix = blockDim.x;
-    uint32_t sum = 0;
-#pragma unroll 16
-    for (int w = 0; w < nparts; ++w) sum += part[((uint64_t)w * passes + q) * radix + d];
-    s[d] = sum;
-    __syncthreads();
-    for (int off = 1; off < radix; off <<= 1) {
-        const uint32_t v = d >= off ? s[d - off] : 0u;
-        __syncthreads();
-        s[d] += v;
-        __syncthreads();
+    constexpr int W = OS_START_THREADS / 64;
+    __shared__ uint32_t s[W][64];
+    __shared__ int last;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, q = blockIdx.y, d = blockIdx.x * 64 + lane;
+    uint32_t v[OS_HIST_WGS / W], sum = 0;
+#pragma unroll
+    for (int u = 0; u < OS_HIST_WGS / W; ++u) {
+        const int w = u * W + wv;
+        v[u] = w < nparts ? part[((uint64_t)w * passes + q) * radix + d] : 0u;
     }
-    start[q * radix + d] = s[d] - sum;
+#pragma unroll
+    for (int u = 0; u < OS_HIST_WGS / W; ++u) sum += v[u];
+    s[wv][lane] = sum;
+    __syncthreads();
+    if (wv == 0) {
+        for (int w = 1; w < W; ++w) sum += s[w][lane];
+        __hip_atomic_store(&total[q * radix + d], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __threadfence();
+        if (lane == 0)
+            last = __hip_atomic_fetch_add(&done[q], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    const int t = threadIdx.x;
+    uint32_t c = t < radix ? __hip_atomic_load(&total[q * radix + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    uint32_t run = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t x = __shfl_up(run, off);
+        if (lane >= off) run += x;
+    }
+    if (lane == 63) s[0][wv] = run;
+    __syncthreads();
+    for (int w = 0; w < wv; ++w) run += s[0][w];
+    if (t < radix) start[q * radix + t] = run - c;
 }
 
 // One pass over the DB-bit digit (key >> shift) & (2^DB - 1).  Wave w ranks
-// its own contiguous quarter of the tile (16 rounds of 64 keys): per round,
+// its own contiguous part of the tile (ITEMS rounds of 64 keys): per round,
 // lanes with the same digit find each other with DB ballots, read the wave's
 // running count of that digit from LDS and the round's leader advances it
-// (LDS operations of one wave complete in order).  Thread t owns digits t,
-// t + 256, ... for the tile's counts, the look-back and the global bases.
-template <int DB>
+// (LDS operations of one wave complete in order).  Thread t < 2^DB owns digit t
+// for the tile's counts, the look-back and the global base.
+//
+// A pass moves 24 bytes a key; what it spends beyond that is the tile's own
+// chain (load, rank, publish, look back, place) and the writes, which leave in
+// runs of the tile's keys of one digit.  So a tile is large, 8,192 keys for 16
+// waves, the waves' rounds few, and the values are placed in the keys' LDS after
+// these have left.  40 million keys, nine bits: 221 us a pass, 4.3 TB/s (4 waves
+// of 16 rounds with 4,096 keys, each with LDS for both: 319); 7 million, ten
+// bits: 63 (99); 4.6 million, nine: 53 (72).  Eight predecessors read at once in
+// the look-back: no gain.
+template <int DB, int ITEMS>
 __global__ __launch_bounds__(SORT_THREADS) void os_pass_kernel(const uint64_t *__restrict__ kin,
                                                               const uint32_t *__restrict__ vin,
                                                               uint64_t *__restrict__ kout,
@@ -218,35 +256,32 @@ __global__ __launch_bounds__(SORT_THREADS) void os_pass_kernel(const uint64_t *_
                                                               uint32_t *__restrict__ ticket, uint32_t epoch,
                                                               int *__restrict__ err)
 {
-    constexpr int NWAVES = SORT_THREADS / 64;
-    constexpr int R = 1 << DB, E = R / SORT_THREADS;   // digits a thread owns
+    constexpr int NWAVES = SORT_THREADS / 64, TILE = SORT_THREADS * ITEMS;
+    constexpr int R = 1 << DB;
     constexpr uint32_t MASK = (uint32_t)R - 1u;
-    __shared__ uint64_t sk[SORT_TILE];
-    __shared__ uint32_t sv[SORT_TILE];
-    __shared__ uint16_t wcnt[NWAVES][R];   // per wave and digit: counts, then offsets (<= 4096)
-    __shared__ uint16_t start[R];          // the tile's digit counts, then its digit run starts
-    __shared__ uint32_t tile_s;
-    // the key tile's LDS is free until the keys are placed: the scan's sums
+    static_assert(R <= SORT_THREADS && TILE <= 65535, "a digit a thread, 16-bit offsets");
+    __shared__ uint64_t sk[TILE];
+    __shared__ uint16_t wcnt[NWAVES][R];   // per wave and digit: counts, then offsets in the tile
+    // the key tile's LDS is free until the keys are placed: the ticket and the scan's sums
     uint32_t *part = reinterpret_cast<uint32_t *>(sk);
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    if (t == 0) tile_s = atomicAdd(ticket, 1u);
-    for (int w = 0; w < NWAVES; ++w)
-        for (int e = 0; e < E; ++e) wcnt[w][t + e * SORT_THREADS] = 0;
+    if (t == 0) part[0] = atomicAdd(ticket, 1u);
+    for (int i = t; i < NWAVES * R / 2; i += SORT_THREADS) reinterpret_cast<uint32_t *>(&wcnt[0][0])[i] = 0;
     __syncthreads();
-    const uint32_t tile = tile_s;
-    const uint64_t base = (uint64_t)tile * SORT_TILE;
-    const uint64_t wbase = base + (uint64_t)wv * (SORT_ITEMS * 64);
+    const uint32_t tile = part[0];
+    const uint64_t base = (uint64_t)tile * TILE;
+    const uint64_t wbase = base + (uint64_t)wv * (ITEMS * 64);
     const uint64_t lane_lt = (1ull << lane) - 1ull;
-    uint64_t key[SORT_ITEMS];
-    uint32_t val[SORT_ITEMS], rank[SORT_ITEMS];
+    uint64_t key[ITEMS];
+    uint32_t val[ITEMS], rank[ITEMS];
 #pragma unroll
-    for (int r = 0; r < SORT_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const uint64_t x = wbase + (uint64_t)r * 64 + lane;
         key[r] = x < n ? kin[x] : 0ull;
         val[r] = x < n ? vin[x] : 0u;
     }
 #pragma unroll
-    for (int r = 0; r < SORT_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const bool valid = wbase + (uint64_t)r * 64 + lane < n;
         const uint32_t d = (uint32_t)(key[r] >> shift) & MASK;
         uint64_t peers = __ballot(valid);
@@ -263,34 +298,42 @@ __global__ __launch_bounds__(SORT_THREADS) void os_pass_kernel(const uint64_t *_
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
-    // owned digits: wave offsets within the tile and the tile's counts, which
-    // are published at once (tile 0: its count is its inclusive prefix)
-    uint32_t cnt[E];
+    // the owned digit's count, published at once (tile 0: it is the inclusive prefix)
+    uint32_t cnt = 0, gb = 0;
     uint64_t *st = status + (uint64_t)tile * R;
+    if (t < R) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int d = t + e * SORT_THREADS;
-        uint32_t c = 0;
-        for (int w = 0; w < NWAVES; ++w) {
-            const uint32_t x = wcnt[w][d];
-            wcnt[w][d] = (uint16_t)c;
-            c += x;
-        }
-        cnt[e] = c;
-        __hip_atomic_store(&st[d], os_word(epoch, tile == 0 ? OS_FLAG_P : OS_FLAG_A, c), __ATOMIC_RELAXED,
+        for (int w = 0; w < NWAVES; ++w) cnt += wcnt[w][t];
+        __hip_atomic_store(&st[t], os_word(epoch, tile == 0 ? OS_FLAG_P : OS_FLAG_A, cnt), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     }
-    // look-back: each owned digit's count over every preceding tile
-    uint32_t gb[E];
+    // exclusive scan of the tile's digit counts: the start of each digit's run
+    uint32_t run = cnt;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int d = t + e * SORT_THREADS;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t v = __shfl_up(run, off);
+        if (lane >= off) run += v;
+    }
+    if (lane == 63) part[wv] = run;
+    __syncthreads();
+    uint32_t before_wave = 0;
+    for (int w = 0; w < wv; ++w) before_wave += part[w];
+    run += before_wave - cnt;
+    if (t < R) {
+        uint32_t c = run;
+#pragma unroll
+        for (int w = 0; w < NWAVES; ++w) {
+            const uint32_t x = wcnt[w][t];
+            wcnt[w][t] = (uint16_t)c;
+            c += x;
+        }
+        // look-back: the digit's count over every preceding tile
         uint64_t before = 0;
         if (tile > 0) {
             int64_t j = (int64_t)tile - 1;
             uint32_t spins = 0;
             for (;;) {
-                const uint64_t w = __hip_atomic_load(&status[(uint64_t)j * R + d], __ATOMIC_RELAXED,
+                const uint64_t w = __hip_atomic_load(&status[(uint64_t)j * R + t], __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT);
                 const uint64_t flag = (w >> 38) & 3u;
                 if ((uint32_t)(w >> 40) == epoch && flag != 0) {
@@ -304,63 +347,44 @@ __global__ __launch_bounds__(SORT_THREADS) void os_pass_kernel(const uint64_t *_
                 }
                 __builtin_amdgcn_s_sleep(1);
             }
-            __hip_atomic_store(&st[d], os_word(epoch, OS_FLAG_P, (before + cnt[e]) & OS_VALUE_MASK),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&st[t], os_word(epoch, OS_FLAG_P, (before + cnt) & OS_VALUE_MASK), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
         }
-        gb[e] = dstart[d] + (uint32_t)before;
-        start[d] = (uint16_t)cnt[e];
-    }
-    __syncthreads();
-    // exclusive scan of the tile's digit counts (the start of each digit run):
-    // thread t sums digits [t*E, t*E + E), the 256 sums are scanned, then each
-    // thread writes its digits' starts
-    uint32_t loc[E], tot = 0;
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        loc[e] = start[t * E + e];
-        tot += loc[e];
-    }
-    part[t] = tot;
-    __syncthreads();
-    for (int off = 1; off < SORT_THREADS; off <<= 1) {
-        const uint32_t v = t >= off ? part[t - off] : 0u;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    uint32_t run = part[t] - tot;
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        start[t * E + e] = (uint16_t)run;
-        run += loc[e];
+        gb = dstart[t] + (uint32_t)before;
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < SORT_ITEMS; ++r) {
-        if (wbase + (uint64_t)r * 64 + lane < n) {
-            const uint32_t d = (uint32_t)(key[r] >> shift) & MASK;
-            const uint32_t p = start[d] + wcnt[wv][d] + rank[r];
-            sk[p] = key[r];
-            sv[p] = val[r];
-        }
+    for (int r = 0; r < ITEMS; ++r) {
+        rank[r] += wcnt[wv][(uint32_t)(key[r] >> shift) & MASK];
+        if (wbase + (uint64_t)r * 64 + lane < n) sk[rank[r]] = key[r];
     }
     __syncthreads();
     // the wave counts' LDS (no longer read) takes each digit's offset from a
     // tile slot to its output position
     uint32_t *off = reinterpret_cast<uint32_t *>(&wcnt[0][0]);
+    if (t < R) off[t] = gb - run;
+    __syncthreads();
+    const uint32_t tile_n = (uint32_t)min<uint64_t>(TILE, n - base);
+    uint32_t g[ITEMS];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int d = t + e * SORT_THREADS;
-        off[d] = gb[e] - (uint32_t)start[d];
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t p = (uint32_t)(r * SORT_THREADS + t);
+        if (p < tile_n) {
+            const uint64_t k = sk[p];
+            g[r] = off[(uint32_t)(k >> shift) & MASK] + p;   // below n < 2^32, so exact mod 2^32
+            kout[g[r]] = k;
+        }
     }
     __syncthreads();
-    const uint32_t tile_n = (uint32_t)min<uint64_t>(SORT_TILE, n - base);
-    for (uint32_t p = t; p < tile_n; p += SORT_THREADS) {
-        const uint64_t k = sk[p];
-        const uint32_t d = (uint32_t)(k >> shift) & MASK;
-        const uint64_t g = (uint32_t)(off[d] + p);   // below n < 2^32, so exact mod 2^32
-        kout[g] = k;
-        vout[g] = sv[p];
+    uint32_t *sv = reinterpret_cast<uint32_t *>(sk);
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+        if (wbase + (uint64_t)r * 64 + lane < n) sv[rank[r]] = val[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t p = (uint32_t)(r * SORT_THREADS + t);
+        if (p < tile_n) vout[g[r]] = sv[p];
     }
 }
 
@@ -579,7 +603,9 @@ int radix_sort_kv(mh_context *ctx, uint64_t *k0, uint32_t *v0, uint64_t *k1, uin
     if (n == 0) return MH_OK;
     MH_CHECK(bits > 0 && bits <= 64, MH_ERR_INVALID, "radix sort: key bits out of range");
     MH_CHECK(n < (1ull << 32), MH_ERR_UNSUPPORTED, "radix sort: more than 2^32 - 1 keys");
-    const uint32_t ntiles = (uint32_t)((n + SORT_TILE - 1) / SORT_TILE);
+    const int items = n <= OS_SMALL ? 2 : n <= OS_MIDDLE ? 4 : 8;
+    const uint64_t tile = (uint64_t)items * SORT_THREADS;
+    const uint32_t ntiles = (uint32_t)((n + tile - 1) / tile);
     // the fewest passes of digits up to 10 bits, then the narrowest digit
     // (8 at least) that covers the key in that many passes
     int max_bits = OS_MAX_BITS;
@@ -591,11 +617,12 @@ int radix_sort_kv(mh_context *ctx, uint64_t *k0, uint32_t *v0, uint64_t *k1, uin
     const uint32_t nparts = std::min<uint32_t>(OS_HIST_WGS, ntiles);
     const uint64_t part_n = (uint64_t)nparts * passes * radix;
     int rc;
-    if ((rc = ctx->sort_tmp[2].ensure((part_n + (uint64_t)passes * radix + OS_MAX_PASSES) * 4 + 64)) != MH_OK)
+    if ((rc = ctx->sort_tmp[2].ensure((part_n + (uint64_t)passes * radix * 2 + 2 * OS_MAX_PASSES) * 4 + 64)) != MH_OK)
         return rc;
     uint32_t *part = ctx->sort_tmp[2].as<uint32_t>();
     uint32_t *dstart = part + part_n;
-    uint32_t *tickets = dstart + (uint64_t)passes * radix;
+    uint32_t *total = dstart + (uint64_t)passes * radix;
+    uint32_t *tickets = total + (uint64_t)passes * radix;
     // the look-back's status words (and the error word in front of them):
     // zeroed when (re)allocated, then never cleared -- each pass has an epoch
     const uint64_t status_bytes = 256 + (uint64_t)ntiles * radix * 8;
@@ -609,7 +636,8 @@ int radix_sort_kv(mh_context *ctx, uint64_t *k0, uint32_t *v0, uint64_t *k1, uin
     uint64_t *status = reinterpret_cast<uint64_t *>(ctx->sort_status.as<uint8_t>() + 256);
     hipLaunchKernelGGL(os_hist_kernel, dim3(nparts), dim3(OS_HIST_THREADS), 0, ctx->stream, k0, n, db, passes, part,
                        tickets);
-    hipLaunchKernelGGL(os_start_kernel, dim3(passes), dim3(radix), 0, ctx->stream, part, (int)nparts, passes, dstart);
+    hipLaunchKernelGGL(os_start_kernel, dim3(radix / 64, passes), dim3(OS_START_THREADS), 0, ctx->stream, part,
+                       (int)nparts, passes, radix, total, tickets + OS_MAX_PASSES, dstart);
     for (int pass = 0; pass < passes; ++pass) {
         if (++ctx->sort_epoch >= (1u << 24)) {
             MH_HIP(hipMemsetAsync(ctx->sort_status.ptr, 0, ctx->sort_status.bytes, ctx->stream));
@@ -617,15 +645,13 @@ int radix_sort_kv(mh_context *ctx, uint64_t *k0, uint32_t *v0, uint64_t *k1, uin
         }
         const uint32_t *ds = dstart + (uint64_t)pass * radix;
         const int shift = db * pass;
-        if (db == 8)
-            hipLaunchKernelGGL(os_pass_kernel<8>, dim3(ntiles), dim3(SORT_THREADS), 0, ctx->stream, k0, v0, k1, v1, n,
-                               shift, ds, status, tickets + pass, ctx->sort_epoch, err);
-        else if (db == 9)
-            hipLaunchKernelGGL(os_pass_kernel<9>, dim3(ntiles), dim3(SORT_THREADS), 0, ctx->stream, k0, v0, k1, v1, n,
-                               shift, ds, status, tickets + pass, ctx->sort_epoch, err);
-        else
-            hipLaunchKernelGGL(os_pass_kernel<10>, dim3(ntiles), dim3(SORT_THREADS), 0, ctx->stream, k0, v0, k1, v1,
-                               n, shift, ds, status, tickets + pass, ctx->sort_epoch, err);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(ntiles), dim3(SORT_THREADS), 0, ctx->stream, k0, v0, k1, v1, n, shift, ds,
+                               status, tickets + pass, ctx->sort_epoch, err);
+        };
+        if (items == 2) go(db == 8 ? os_pass_kernel<8, 2> : db == 9 ? os_pass_kernel<9, 2> : os_pass_kernel<10, 2>);
+        else if (items == 4) go(db == 8 ? os_pass_kernel<8, 4> : db == 9 ? os_pass_kernel<9, 4> : os_pass_kernel<10, 4>);
+        else go(db == 8 ? os_pass_kernel<8, 8> : db == 9 ? os_pass_kernel<9, 8> : os_pass_kernel<10, 8>);
         std::swap(k0, k1);
         std::swap(v0, v1);
     }

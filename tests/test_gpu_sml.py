@@ -100,3 +100,15 @@ def test_sml_full_size(ctx, which):
         seed = po.get_seed(17, 3)
     for g in (ref, mut):
         _check_sml(ctx, g.tobytes(), seed)
+
+
+@pytest.mark.parametrize("n", [2047, 2049, (1 << 18) - 1, (1 << 18) + 1, (1 << 21) - 4095, (1 << 21) + 1])
+@pytest.mark.parametrize("seed", [po.get_seed(9, 3), po.get_seed(13, 3), po.get_seed(17, 3)])
+def test_sml_sort_tile_edges(ctx, n, seed):
+    """Keys at the edges of the sort's tiles and of the sizes each tile is for,
+    with digits of ten and nine bits, half of the keys equal (stable order)."""
+    rng = np.random.default_rng(n)
+    L = n + po.seed_length(seed) - 1
+    seq = synth.BASES[rng.integers(0, 4, size=L)]
+    seq[L // 3:L // 3 + L // 2] = ord("A")
+    _check_sml(ctx, seq.tobytes(), seed)
