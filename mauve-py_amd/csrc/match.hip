@@ -2391,11 +2391,11 @@ int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRa
     uint64_t *d_olen = reinterpret_cast<uint64_t *>(d_ost + nm * k);
     hipLaunchKernelGGL(uq_emit_kernel, dim3(NB), dim3(64), 0, ctx->stream, qs, bst, vec, nent, outpos, d_ost, d_olen);
     MH_HIP(hipGetLastError());
-    out->starts.resize(nm * k);
-    out->lengths.resize(nm);
+    if ((rc = out->starts.make(nm * k)) != MH_OK) return rc;
+    if ((rc = out->lengths.make(nm)) != MH_OK) return rc;
     if (nm) {
-        MH_HIP(hipMemcpyAsync(out->starts.data(), d_ost, nm * k * 8, hipMemcpyDeviceToHost, ctx->stream));
-        MH_HIP(hipMemcpyAsync(out->lengths.data(), d_olen, nm * 8, hipMemcpyDeviceToHost, ctx->stream));
+        if ((rc = copy_to_host(ctx, out->starts.data(), d_ost, nm * k * 8)) != MH_OK) return rc;
+        if ((rc = copy_to_host(ctx, out->lengths.data(), d_olen, nm * 8)) != MH_OK) return rc;
     }
     MH_HIP(hipStreamSynchronize(ctx->stream));
     out->collisions = (int64_t)coll;

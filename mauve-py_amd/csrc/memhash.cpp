@@ -394,8 +394,8 @@ int find_matches_pairwise(mh_context *ctx, const mh_sml *const *smls, int k, std
 // ranges, then the seeds, their extensions and the bucket insertion on the
 // device (unique_seeds); the list comes out bucket by bucket
 // (LM/MemHash.h:182-203).
-int find_matches_unique(mh_context *ctx, const mh_sml *const *smls, int k, std::vector<int64_t> &starts,
-                        std::vector<uint64_t> &lengths, mh_match_stats *st)
+int find_matches_unique(mh_context *ctx, const mh_sml *const *smls, int k, HostArray<int64_t> &starts,
+                        HostArray<uint64_t> &lengths, mh_match_stats *st)
 {
     MH_CHECK(k >= 2 && k <= 16, MH_ERR_UNSUPPORTED, "UniqueMatchFinder takes 2 to 16 genomes");
     for (int i = 0; i < k; ++i) {
@@ -407,8 +407,8 @@ int find_matches_unique(mh_context *ctx, const mh_sml *const *smls, int k, std::
     if ((rc = search_live_ranges(ctx, smls, k, &live)) != MH_OK) return rc;
     UniqueSeeds us;
     if ((rc = unique_seeds(ctx, smls, k, live, &us)) != MH_OK) return rc;
-    starts.swap(us.starts);
-    lengths.swap(us.lengths);
+    starts = std::move(us.starts);
+    lengths = std::move(us.lengths);
     if (st) {
         std::memset(st, 0, sizeof(*st));
         st->seed_tuples = (int64_t)us.n;
@@ -618,8 +618,8 @@ int mh_find_matches_pairwise_list(mh_context *ctx, const mh_sml *const *smls, in
 
 struct mh_match_k_list {
     int k = 0;
-    std::vector<int64_t> starts;
-    std::vector<uint64_t> lengths;
+    HostArray<int64_t> starts;
+    HostArray<uint64_t> lengths;
 };
 
 int mh_find_matches_unique(mh_context *ctx, const mh_sml *const *smls, int k, mh_match_k_list **out,

@@ -6,6 +6,8 @@
 #include <cstddef>
 #include <string>
 #include <vector>
+#include <memory>
+#include <new>
 #include <set>
 #include <map>
 #include "mauvehip.h"
@@ -183,6 +185,7 @@ void host_parallel(size_t n, const std::function<void(size_t)> &f);
 unsigned host_threads();
 // Pinned host staging buffer of at least `bytes` (owned by the context).
 int pinned(mh_context *ctx, size_t bytes, void **out);
+int copy_to_host(mh_context *ctx, void *dst, const void *src, size_t bytes);   // waits
 int pinned_jobs(mh_context *ctx, size_t bytes, void **out);   // a second pinned buffer, for DP job tables
 
 // Launchers (return MH_OK or an error code); all run on ctx->stream.
@@ -333,13 +336,30 @@ int search_live_ranges(mh_context *ctx, const mh_sml *const *smls, int k, LiveRa
 // HashMatch order), the collisions AddHashEntry counts, and the match list in
 // GetMatchList order (starts k a match, 1-based, negative = reverse, 0 =
 // absent; lengths).  match.hip.
+// A host array that is not filled when it is made.
+template <class T> struct HostArray {
+    std::unique_ptr<T[]> p;
+    size_t n = 0;
+
+    int make(size_t count)
+    {
+        p.reset(count ? new (std::nothrow) T[count] : nullptr);
+        n = p ? count : 0;
+        MH_CHECK(n == count, MH_ERR_NOMEM, "host allocation failed");
+        return MH_OK;
+    }
+    T *data() const { return p.get(); }
+    size_t size() const { return n; }
+    bool empty() const { return n == 0; }
+};
+
 struct UniqueSeeds {
     int k = 0;
     uint64_t n = 0;
     uint64_t walks = 0;        // ExtendMatch walks run (spaced seeds: one a chain)
     int64_t collisions = 0;
-    std::vector<int64_t> starts;
-    std::vector<uint64_t> lengths;
+    HostArray<int64_t> starts;
+    HostArray<uint64_t> lengths;
 };
 int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRanges &live, UniqueSeeds *out);
 
