@@ -873,51 +873,79 @@ __device__ __forceinline__ uint32_t bucket_of(int64_t off)
     return (uint32_t)(((off % (int64_t)TABLE_SIZE) + TABLE_SIZE) % TABLE_SIZE);
 }
 
-__global__ void bucket_key_kernel(const SeedRec *__restrict__ seeds, uint64_t ns, int k, uint64_t *__restrict__ key,
-                                  uint32_t *__restrict__ val)
+// What the kernels after the bucket sort need of a seed travels above its key's
+// 16 sorted bits where it fits: the extended start (eb bits) and the line (its
+// offset's quotient by the table's size and the strand).  Reading the records in
+// bucket order instead is one scattered read a seed and kernel: key2_kernel 73 us
+// and bucket_dirty_kernel 64 over 4.5 million seeds, 15 and 6 here.  Genomes
+// whose starts and lines need more bits take that way.
+struct BucketKey {
+    int eb;          // bits of a start
+    int packed;
+    int64_t bias;    // makes the quotient positive
+};
+
+// the seed's line: its offset and strand
+__device__ __forceinline__ uint64_t seed_line(const SeedRec &r, int k)
+{
+    return (uint64_t)(seed_offset(r, k) * 2 + (r.s1 < 0 ? 1 : 0));
+}
+
+__device__ __forceinline__ uint64_t line_of(const BucketKey &bk, uint64_t key, const SeedRec *__restrict__ seeds,
+                                            uint32_t x, int k)
+{
+    return bk.packed ? key >> (16 + bk.eb) : seed_line(seeds[x], k);
+}
+
+__global__ void bucket_key_kernel(const SeedRec *__restrict__ seeds, uint64_t ns, int k, BucketKey bk,
+                                  uint64_t *__restrict__ key, uint32_t *__restrict__ val)
 {
     const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= ns) return;
-    key[x] = bucket_of(seed_offset(seeds[x], k));
+    const SeedRec r = seeds[x];
+    const int64_t off = seed_offset(r, k);
+    uint64_t v = bucket_of(off);
+    if (bk.packed) {
+        const uint64_t m = (uint64_t)((off - (int64_t)v) / (int64_t)TABLE_SIZE + bk.bias);
+        v |= ((m * 2 + (r.s1 < 0 ? 1 : 0)) << (16 + bk.eb)) | ((uint64_t)(uint32_t)r.e0 << 16);
+    }
+    key[x] = v;
     val[x] = (uint32_t)x;
 }
 
-// the seed's line: its offset and strand
-__device__ __forceinline__ int64_t seed_line(const SeedRec &r, int k)
-{
-    return seed_offset(r, k) * 2 + (r.s1 < 0 ? 1 : 0);
-}
-
 __global__ void bucket_first_kernel(const uint64_t *__restrict__ skey, const uint32_t *__restrict__ sval,
-                                    const SeedRec *__restrict__ seeds, uint64_t ns, int k,
-                                    int64_t *__restrict__ first_line)
+                                    const SeedRec *__restrict__ seeds, uint64_t ns, int k, BucketKey bk,
+                                    uint64_t *__restrict__ first_line)
 {
     const uint64_t y = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (y >= ns) return;
-    const uint64_t b = skey[y];
-    if (y == 0 || skey[y - 1] != b) first_line[b] = seed_line(seeds[sval[y]], k);
+    const uint32_t b = (uint16_t)skey[y];
+    if (y == 0 || (uint16_t)skey[y - 1] != b) first_line[b] = line_of(bk, skey[y], seeds, sval[y], k);
 }
 
 __global__ void bucket_dirty_kernel(const uint64_t *__restrict__ skey, const uint32_t *__restrict__ sval,
-                                    const SeedRec *__restrict__ seeds, uint64_t ns, int k, int solid_odd,
-                                    const int64_t *__restrict__ first_line, uint32_t *__restrict__ dirty)
+                                    const SeedRec *__restrict__ seeds, uint64_t ns, int k, BucketKey bk, int solid_odd,
+                                    const uint64_t *__restrict__ first_line, uint32_t *__restrict__ dirty)
 {
     const uint64_t y = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (y >= ns) return;
-    const uint64_t b = skey[y];
-    if (!solid_odd || seed_line(seeds[sval[y]], k) != first_line[b]) dirty[b] = 1u;
+    const uint64_t key = skey[y];
+    const uint32_t b = (uint16_t)key;
+    if (!solid_odd || line_of(bk, key, seeds, sval[y], k) != first_line[b]) dirty[b] = 1u;
 }
 
 __global__ void key2_kernel(const uint64_t *__restrict__ skey, const uint32_t *__restrict__ sval,
-                            const SeedRec *__restrict__ seeds, uint64_t ns, int eb, const uint32_t *__restrict__ dirty,
-                            uint64_t *__restrict__ key2, uint32_t *__restrict__ val2, uint32_t *__restrict__ flag_dirty)
+                            const SeedRec *__restrict__ seeds, uint64_t ns, BucketKey bk,
+                            const uint32_t *__restrict__ dirty, uint64_t *__restrict__ key2,
+                            uint32_t *__restrict__ val2, uint32_t *__restrict__ flag_dirty)
 {
     const uint64_t y = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (y >= ns) return;
-    const uint64_t b = skey[y];
-    const uint32_t v = sval[y];
+    const uint64_t key = skey[y], ones = (1ull << bk.eb) - 1;
+    const uint32_t v = sval[y], b = (uint16_t)key;
     const bool d = dirty[b] != 0;
-    key2[y] = (b << eb) | (d ? ((1ull << eb) - 1) : (uint64_t)(uint32_t)seeds[v].e0);
+    const uint64_t e0 = bk.packed ? (key >> 16) & ones : (uint64_t)(uint32_t)seeds[v].e0;
+    key2[y] = ((uint64_t)b << bk.eb) | (d ? ones : e0);
     val2[y] = v;
     flag_dirty[y] = d ? 1u : 0u;
 }
@@ -984,7 +1012,7 @@ __global__ void gather_dirty_kernel(const uint32_t *__restrict__ idx, uint64_t m
     if (x >= m) return;
     const uint32_t y = idx[x];
     DirtySeed d;
-    d.bucket = (uint32_t)skey[y];
+    d.bucket = (uint16_t)skey[y];
     d.r = seeds[sval[y]];
     out[x] = d;
 }
@@ -1393,12 +1421,21 @@ static int compact_flags(mh_context *ctx, const uint32_t *flag, uint64_t n, uint
 }
 
 int partition_seeds(mh_context *ctx, const SeedRec *d_seeds, uint64_t ns, int k, bool solid_odd, uint64_t len_a,
+                    uint64_t len_b,
                     std::vector<CleanEnt> &clean, std::vector<DirtySeed> &dirty, uint64_t *n_clean_seeds)
 {
     // the second sort key is (bucket << eb) | extended start, eb bits holding
     // every start (1-based, <= len_a) and the all-ones mark of other buckets
     int eb = 1;
     while (eb < 32 && (1ull << eb) - 1 <= len_a) ++eb;
+    // the offsets lie in [-(len_a + len_b + k), len_b]
+    BucketKey bk;
+    bk.eb = eb;
+    bk.bias = (int64_t)((len_a + len_b + (uint64_t)k) / TABLE_SIZE) + 1;
+    const uint64_t lines = 2 * ((uint64_t)bk.bias + len_b / TABLE_SIZE + 2);
+    int lbits = 1;
+    while ((1ull << lbits) < lines) ++lbits;
+    bk.packed = 16 + eb + lbits <= 64;
     clean.clear();
     dirty.clear();
     *n_clean_seeds = 0;
@@ -1417,7 +1454,7 @@ int partition_seeds(mh_context *ctx, const SeedRec *d_seeds, uint64_t ns, int k,
     if ((rc = m[15].ensure(((ns + JTILE - 1) / JTILE) * 4 + 64 + ns * (sizeof(DirtySeed) + 16))) != MH_OK) return rc;
     uint64_t *kA = m[8].as<uint64_t>(), *kB = m[9].as<uint64_t>();
     uint32_t *vA = m[10].as<uint32_t>(), *vB = m[11].as<uint32_t>();
-    int64_t *first_off = m[12].as<int64_t>();
+    uint64_t *first_off = m[12].as<uint64_t>();
     uint32_t *dirty_b = reinterpret_cast<uint32_t *>(first_off + TABLE_SIZE);
     uint32_t *flag = m[13].as<uint32_t>(), *idx = m[14].as<uint32_t>();
     uint32_t *tiles = m[15].as<uint32_t>();
@@ -1429,16 +1466,16 @@ int partition_seeds(mh_context *ctx, const SeedRec *d_seeds, uint64_t ns, int k,
     uint32_t *sv = nullptr, *v2 = nullptr;
     {
         TimedLaunch tl(ctx, "partition");
-        hipLaunchKernelGGL(bucket_key_kernel, dim3(grid), dim3(256), 0, ctx->stream, d_seeds, ns, k, kA, vA);
+        hipLaunchKernelGGL(bucket_key_kernel, dim3(grid), dim3(256), 0, ctx->stream, d_seeds, ns, k, bk, kA, vA);
         if ((rc = radix_sort_kv(ctx, kA, vA, kB, vB, ns, 16, &sk, &sv)) != MH_OK) return rc;
-        hipLaunchKernelGGL(bucket_first_kernel, dim3(grid), dim3(256), 0, ctx->stream, sk, sv, d_seeds, ns, k,
+        hipLaunchKernelGGL(bucket_first_kernel, dim3(grid), dim3(256), 0, ctx->stream, sk, sv, d_seeds, ns, k, bk,
                            first_off);
-        hipLaunchKernelGGL(bucket_dirty_kernel, dim3(grid), dim3(256), 0, ctx->stream, sk, sv, d_seeds, ns, k,
+        hipLaunchKernelGGL(bucket_dirty_kernel, dim3(grid), dim3(256), 0, ctx->stream, sk, sv, d_seeds, ns, k, bk,
                            solid_odd ? 1 : 0, first_off, dirty_b);
         // (sk, sv) now hold the bucket order; the other pair is free for the second sort
         uint64_t *k2a = (sk == kA) ? kB : kA;
         uint32_t *v2a = (sv == vA) ? vB : vA;
-        hipLaunchKernelGGL(key2_kernel, dim3(grid), dim3(256), 0, ctx->stream, sk, sv, d_seeds, ns, eb, dirty_b, k2a,
+        hipLaunchKernelGGL(key2_kernel, dim3(grid), dim3(256), 0, ctx->stream, sk, sv, d_seeds, ns, bk, dirty_b, k2a,
                            v2a, flag);
         MH_HIP(hipGetLastError());
         // dirty seeds in (bucket, call) order

@@ -145,7 +145,7 @@ int find_matches_multi(mh_context *ctx, const mh_sml *const *smls, int k, std::v
                 // the pair's buckets that the two-genome closed form settles
                 std::vector<DirtySeed> dirty_p;
                 uint64_t ncs = 0;
-                if ((rc = partition_seeds(ctx, d_seeds, ns, (int)sl, solid_odd, smls[a]->len, clean_p[np], dirty_p,
+                if ((rc = partition_seeds(ctx, d_seeds, ns, (int)sl, solid_odd, smls[a]->len, smls[b]->len, clean_p[np], dirty_p,
                                           &ncs)) != MH_OK)
                     return rc;
                 for (const DirtySeed &d : dirty_p) replay_bucket[d.bucket] = 1;
@@ -309,7 +309,7 @@ int find_matches_pairwise(mh_context *ctx, const mh_sml *const *smls, int k, std
     std::vector<CleanEnt> clean;
     std::vector<DirtySeed> dirty;
     uint64_t n_clean_seeds = 0;
-    if ((rc = partition_seeds(ctx, d_seeds, nseeds, (int)sl, solid_odd, a->len, clean, dirty, &n_clean_seeds)) != MH_OK)
+    if ((rc = partition_seeds(ctx, d_seeds, nseeds, (int)sl, solid_odd, a->len, b->len, clean, dirty, &n_clean_seeds)) != MH_OK)
         return rc;
     const double tg1 = now_ms();
     // the remaining buckets: runs of equal bucket in the dirty list, each in HashMatch order
