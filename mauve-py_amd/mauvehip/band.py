@@ -34,7 +34,8 @@ def est_cells(la, lb, w):
 
 
 # Time model of a banded run on one MI355X (seconds), from measurements of the
-# DP kernels: each pass of the fallback costs its cells at the batch rate
+# DP kernels the committed model was calibrated on (they have become faster; the
+# constants stay, since they decide delta): each pass of the fallback costs its cells at the batch rate
 # (~950 GCUPS of region cells) or its largest job at the rate of one
 # wavefront (a job runs on one wavefront: ~1.7 GCUPS), whichever is longer;
 # then the trace-back, whose longest walk takes ~0.6 us per step; plus a
