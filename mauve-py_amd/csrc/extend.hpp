@@ -51,6 +51,25 @@ namespace mh {
 
 constexpr int EXT_MAXK = 16;
 
+// Seeds of two genomes by genome-0 position: a word holds the partner's forward
+// position in genome 1 (31 bits) with the strand relation in bit 31, or this.
+// It is also what a reversed partner at position 2^31 - 1 would give, which is
+// past the last window of the longest genomes (2^31 - 1 bases).
+constexpr uint32_t NO_SEED = 0xFFFFFFFFu;
+
+// The furthest seed of position p's diagonal within a seed length S before it,
+// or p: word(x) is the table's word of position x, word(p) a seed's.
+template <class W> MH_HD inline uint32_t spaced_link(uint32_t p, uint32_t S, W word)
+{
+    const uint32_t v = word(p), rev = v & 0x80000000u, q = v & 0x7FFFFFFFu;
+    for (uint32_t t = p < S ? p : S; t > 0; --t) {
+        if (!rev && q < t) continue;
+        const uint32_t want = (rev ? q + t : q - t) | rev;
+        if (want != NO_SEED && word(p - t) == want) return p - t;
+    }
+    return p;
+}
+
 #if defined(__HIP__)
 
 // Per genome: the packed sequence and its reverse complement's, or (other

@@ -450,17 +450,7 @@ __global__ void spaced_link_kernel(const uint2 *__restrict__ pp, uint64_t L0, ui
     if (p >= L0) return;
     const uint2 v = pp[p];
     uint32_t out = (uint32_t)p;
-    if (v.x != 0xFFFFFFFFu) {
-        const bool rev = (v.x >> 31) != 0;
-        const uint32_t q = v.x & 0x7FFFFFFFu;
-        for (uint32_t t = p < seed_len ? (uint32_t)p : seed_len; t > 0; --t) {
-            if (!rev && q < t) continue;
-            if (pp[p - t].x == ((rev ? q + t : q - t) | (v.x & 0x80000000u))) {
-                out = (uint32_t)p - t;
-                break;
-            }
-        }
-    }
+    if (v.x != NO_SEED) out = spaced_link((uint32_t)p, seed_len, [&](uint32_t x) { return pp[x].x; });
     link[p] = out;
 }
 
@@ -469,9 +459,9 @@ __global__ void spaced_heads_kernel(const uint2 *__restrict__ pp, const uint32_t
                                     uint32_t *__restrict__ heads, uint32_t *__restrict__ count)
 {
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint2 v = make_uint2(0xFFFFFFFFu, 0);
+    uint2 v = make_uint2(NO_SEED, 0);
     if (p < L0) v = pp[p];
-    const bool head = v.x != 0xFFFFFFFFu && root[p] == (uint32_t)p;
+    const bool head = v.x != NO_SEED && root[p] == (uint32_t)p;
     const uint64_t b = __ballot(head);
     if (!b) return;
     const int lane = threadIdx.x & 63;
@@ -487,7 +477,7 @@ __global__ void spaced_fill_kernel(const uint2 *__restrict__ pp, const uint32_t 
     const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= L0) return;
     const uint2 v = pp[p];
-    if (v.x == 0xFFFFFFFFu || root[p] == (uint32_t)p) return;
+    if (v.x == NO_SEED || root[p] == (uint32_t)p) return;
     const SeedRec h = out[pp[root[p]].y];
     SeedRec r;
     r.s0 = (int32_t)p + 1;
@@ -614,7 +604,6 @@ __global__ void rc_pack_kernel(const uint32_t *__restrict__ w, uint64_t len, uin
 // last seed of the run at each position come from a segmented scan over the
 // positions (the nearest head at or before, the nearest tail at or after).
 
-constexpr uint32_t NO_SEED = 0xFFFFFFFFu;
 constexpr int RS_T = 256, RS_ITEMS = 16, RS_P = RS_T * RS_ITEMS;   // positions per scan block
 constexpr uint8_t RF_SEED = 4, RF_FOLLOW = 1, RF_NEXT = 2;       // position flags
 
