@@ -1830,7 +1830,7 @@ static int dp_launch_round(mh_context *ctx, int v, bool graph, unsigned grid, Ro
     return MH_OK;
 }
 
-// ints of the boundary columns of an item's job (rounded up: two values a row)
+// ints of the boundary columns of an item's job: 3 a row, for a pipelined job 12
 static uint64_t item_bnd_ints(const DpItem &it, const mh_dp_job *jobs)
 {
     // one-lane and window jobs hand no column over; a job of 16-lane
@@ -1838,7 +1838,16 @@ static uint64_t item_bnd_ints(const DpItem &it, const mh_dp_job *jobs)
     if (it.cols == TINY_COLS_TAG || it.cols >= WINDOW_TAG) return 0ull;
     const uint64_t sw = it.cols > GROUP_TAG ? 16ull * (it.cols - GROUP_TAG) : 64ull * it.cols;
     const uint64_t ns = (jobs[it.job].b_len + sw - 1) / sw;
-    return ns > 1 ? 3ull * ((jobs[it.job].a_len + 63) & ~63ull) : 0ull;
+    return ns > 1 ? (it.parts ? 12ull : 3ull) * ((jobs[it.job].a_len + 63) & ~63ull) : 0ull;
+}
+
+// bytes of the arena of a round with tbb bytes of trace and bi boundary ints
+static uint64_t arena_bytes(uint64_t tbb, uint64_t bi) { return align256(bi * 4) + tbb; }
+
+// an item's part of them (boundary columns are whole multiples of 256 bytes)
+static uint64_t item_bytes(const DpItem &it, const mh_dp_job *jobs)
+{
+    return arena_bytes((it.tb_bytes + 15) & ~15ull, item_bnd_ints(it, jobs));
 }
 
 // footprint in a fixed scratch of a round of `cnt` jobs with trace bytes
@@ -1866,6 +1875,10 @@ static uint64_t fixed_need(uint64_t cnt, uint64_t tbb, uint64_t bi)
 // shape), longest first; other: its remaining wavefronts.  MH_DP_PIPE = P (p_env)
 // instead gives P wavefronts to the first 64-lane jobs with at least P stripes,
 // as many as the idle slots hold.
+// A pipelined job's boundary takes four times the memory, and a byte a column
+// holds half a byte where a lane has one: spare is what the round's bytes may
+// still grow by (item_bytes), and the jobs that would pass it, the longest
+// first, keep one wavefront.
 //
 // Measured, with the parts' priorities (dp_job): 4,000 jobs of 10-20,000 columns
 // (at most 8 parts a job, all the round's wavefronts fitting the slots together,
@@ -1874,7 +1887,7 @@ static uint64_t fixed_need(uint64_t cnt, uint64_t tbb, uint64_t bi)
 // instead of four, and a banded job's stripes wait for each other (9 ms for 20,000
 // columns).
 static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_t other, uint64_t simds, int wpe,
-                       int p_env)
+                       int p_env, uint64_t spare)
 {
     auto group = [](const DpItem &it) { return it.cols > GROUP_TAG; };
     auto cols_of = [&](const DpItem &it) { return group(it) ? it.cols - GROUP_TAG : it.cols; };
@@ -1887,6 +1900,20 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
     const bool tagged = wpe < 0;     // (only these cells have the one- and two-column lanes)
     if (tagged) wpe = FWD_VARIANTS[dp_variant_for(wide)].wpe;
     const double slots = std::max(1.0, (double)(simds * (uint64_t)wpe) - (double)other);
+    // p wavefronts for it (over all lanes, if it is of 16-lane stripes), while the memory lasts
+    auto give = [&](DpItem &it, uint32_t p) {
+        DpItem w = it;
+        w.parts = p;
+        if (group(it)) {
+            w.cols = cols_of(it) / 4;
+            w.tb_bytes = dp_steps(jobs[it.job].a_len, jobs[it.job].b_len, it.band, w.cols, 64) * 64 * lane_bytes_of(w.cols);
+        }
+        const uint64_t had = item_bytes(it, jobs), has = item_bytes(w, jobs);
+        if (has > had && has - had > spare) return false;
+        spare -= has - had;     // (back to spare where a shape takes less)
+        it = w;
+        return true;
+    };
     if (p_env > 1) {
         if (est >= slots) return;
         double used = est;
@@ -1894,8 +1921,7 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
             DpItem &it = items[x];
             const uint64_t ns = (jobs[it.job].b_len + 64ull * it.cols - 1) / (64ull * it.cols);
             if (group(it) || ns < (uint64_t)p_env || used + p_env - 1 > slots) continue;
-            it.parts = (uint32_t)p_env;
-            used += p_env - 1;
+            if (give(it, (uint32_t)p_env)) used += p_env - 1;
         }
         return;
     }
@@ -1946,12 +1972,7 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
     for (uint64_t x = 0; x < n; ++x) {
         DpItem &it = items[x];
         const uint32_t p = parts_of(opt[x], up);
-        if (!p || (p == 1 && !group(it))) continue;
-        it.parts = p;
-        if (group(it)) {
-            it.cols = (it.cols - GROUP_TAG) / 4;
-            it.tb_bytes = dp_steps(jobs[it.job].a_len, jobs[it.job].b_len, it.band, it.cols, 64) * 64 * lane_bytes_of(it.cols);
-        }
+        if (p && (p > 1 || group(it))) give(it, p);
     }
 }
 
@@ -1999,21 +2020,10 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
     if (!fx) {
         size_t free_b = 0, total_b = 0;
         MH_HIP(hipMemGetInfo(&free_b, &total_b));
-        budget = (uint64_t)((free_b + ctx->dp_tb.bytes + ctx->dp_bnd.bytes) * 0.7);
+        budget = (uint64_t)((free_b + ctx->dp_tb.bytes) * 0.7);
         const uint64_t cap = 192ull << 30;
         if (budget > cap) budget = cap;
         if (const char *e = getenv("MH_DP_TB_BUDGET_GB")) budget = (uint64_t)(atof(e) * (1ull << 30));
-    }
-    if (!fx) {
-        // size the arena once for the whole call: the largest round fits the budget
-        uint64_t need = 0;
-        for (const DpItem &it : items) need += it.tb_bytes + bnd_ints(it) * 4;
-        if (need > budget) need = budget;
-        int rc0;
-        if (ctx->dp_tb.bytes < need) {
-            ctx->dp_bnd.release();
-            if ((rc0 = ctx->dp_tb.ensure(need + 256)) != MH_OK) return rc0;
-        }
     }
     RoundArgs ra;
     packed_rows(ra.sc);
@@ -2026,21 +2036,21 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
     if (!fx && pipe_env != 0 && pipe_env != 1)
         MH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
 
-    uint64_t first = 0;
-    std::vector<DpItem> shaped;
-    while (first < nitems) {
+    // the rounds, and each one's pipelined jobs
+    struct Round {
+        uint64_t last, nbig, nstripe;   // end of the items; how many are not one-lane jobs; stripe jobs
+    };
+    std::vector<Round> rounds;
+    uint64_t arena = 0;
+    for (uint64_t first = 0; first < nitems;) {
         // one round: as many jobs (in schedule order) as fit the trace budget
         uint64_t tbb = 0, bi = 0, last = first;
         while (last < nitems) {
-            const uint64_t w = items[last].tb_bytes, b = bnd_ints(items[last]);
-            if (fx) {
-                const uint64_t w16 = (w + 15) & ~15ull;
-                if (last > first && fixed_need(last - first + 1, tbb + w16, bi + b) > fx->bytes) break;
-                tbb += w16;
-            } else {
-                if (last > first && tbb + w + (bi + b) * 4 > budget) break;
-                tbb += w;
-            }
+            const uint64_t w = (items[last].tb_bytes + 15) & ~15ull, b = bnd_ints(items[last]);
+            if (last > first && (fx ? fixed_need(last - first + 1, tbb + w, bi + b) > fx->bytes
+                                    : arena_bytes(tbb + w, bi + b) > budget))
+                break;
+            tbb += w;
             bi += b;
             ++last;
         }
@@ -2054,9 +2064,32 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
                               [](const DpItem &it) { return it.cols < WINDOW_TAG; });
         uint64_t nstripe = 0;
         while (nstripe < nbig && items[first + nstripe].cols < WINDOW_TAG) ++nstripe;
-        if (!fx && ncu > 0)
+        if (!fx && ncu > 0) {
+            const uint64_t bytes = arena_bytes(tbb, bi);
             plan_parts(jobs, items.data() + first, nstripe, (nbig - nstripe) + (n - nbig + 63) / 64,
-                       (uint64_t)ncu * 4, form == DpCells::TAGGED ? -1 : FWD_VARIANTS[VARIANT_FLOAT].wpe, pipe_env);
+                       (uint64_t)ncu * 4, form == DpCells::TAGGED ? -1 : FWD_VARIANTS[VARIANT_FLOAT].wpe, pipe_env,
+                       bytes < budget ? budget - bytes : 0);
+        }
+        uint64_t tw = 0, bo = 0;
+        for (uint64_t x = first; x < last; ++x) {
+            tw += (items[x].tb_bytes + 15) & ~15ull;
+            bo += bnd_ints(items[x]);
+        }
+        arena = std::max(arena, arena_bytes(tw, bo));
+        rounds.push_back({last, nbig, nstripe});
+        first = last;
+    }
+    if (!fx) {
+        // the arena, once for the whole call
+        const int rc = ctx->dp_tb.ensure(arena + 256);
+        if (rc != MH_OK) return rc;
+        // (a count under the timers' names: its bytes)
+        host_time(ctx, "dp_arena_bytes", (double)arena);
+    }
+    std::vector<DpItem> shaped;
+    uint64_t first = 0;
+    for (const Round &rd : rounds) {
+        const uint64_t last = rd.last, n = last - first, nbig = rd.nbig, nstripe = rd.nstripe;
         // wavefront stripes (the pipelined ones first, most parts first), then
         // the row-packed jobs by shape (16, 14, ..., 4 columns a lane), each in
         // order: a stable bucket pass
@@ -2143,11 +2176,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             d.pad_ = 0;
             tw += (it.tb_bytes + 15) & ~15ull;
             bo += bnd_ints(it);
-            if (x < npipe) {
-                // tagged 64-bit words, in two buffers (stripes alternate by parity)
-                bo += 3 * bnd_ints(it);
-                bo_pipe = bo;
-            }
+            if (x < npipe) bo_pipe = bo;
             if (cells) *cells += it.cells;
         }
         DevJob *d_jobs;
@@ -2169,14 +2198,12 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             MH_CHECK((uint64_t)(q - fx->ptr) + tw <= fx->bytes, MH_ERR_INVALID, "DP round exceeds the scratch");
         } else {
             int rc;
-            if ((rc = ctx->dp_tb.ensure(tw + 256)) != MH_OK) return rc;
-            if ((rc = ctx->dp_bnd.ensure(bo * 4 + 256)) != MH_OK) return rc;
             if ((rc = ctx->dp_jobs.ensure(n * (sizeof(DevJob) + sizeof(DpOut) + 4) + 256)) != MH_OK) return rc;
             if ((rc = ctx->dp_round.ensure(DP_ROUND_BYTES)) != MH_OK) return rc;
             d_jobs = ctx->dp_jobs.as<DevJob>();
             d_outs = reinterpret_cast<DpOut *>(d_jobs + n);
-            d_tb = ctx->dp_tb.as<uint8_t>();
-            d_bnd = ctx->dp_bnd.as<int>();
+            d_bnd = ctx->dp_tb.as<int>();
+            d_tb = ctx->dp_tb.as<uint8_t>() + align256(bo * 4);
             d_round = ctx->dp_round.as<DpRound>();
         }
         MH_HIP(hipMemcpyAsync(d_jobs, dj, n * sizeof(DevJob), hipMemcpyHostToDevice, ctx->stream));

@@ -105,7 +105,7 @@ struct mh_context {
     std::vector<std::pair<std::string, std::pair<hipEvent_t, hipEvent_t>>> pending;
     std::vector<hipEvent_t> event_pool;
     // DP scratch
-    mh::DevBuf dp_tb, dp_bnd, dp_jobs, dp_a, dp_b, dp_paths, dp_res, dp_dev;
+    mh::DevBuf dp_tb, dp_jobs, dp_a, dp_b, dp_paths, dp_res, dp_dev;
     mh::DevBuf dp_wild;   // operand scan
     // DP rounds: the descriptor and queue cursors (fixed address), its pinned
     // host copy, the launches captured as graphs per forward variant, and the

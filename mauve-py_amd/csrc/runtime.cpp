@@ -384,7 +384,6 @@ void mh_destroy(mh_context *ctx)
     if (ctx->dp_round_host) (void)hipHostFree(ctx->dp_round_host);
     ctx->dp_round.release();
     ctx->dp_tb.release();
-    ctx->dp_bnd.release();
     ctx->dp_jobs.release();
     ctx->dp_a.release();
     ctx->dp_b.release();

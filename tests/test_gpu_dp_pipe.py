@@ -161,6 +161,44 @@ def test_narrow_banded_stripes_over_all_lanes(ctx, dp_env):
     assert got["1"] == got["auto"]
 
 
+@pytest.mark.parametrize("budget_gb", ["0.002", "0.004", "0.02"])
+def test_rounds_of_spread_banded_jobs_stay_within_the_budget(ctx, dp_env, monkeypatch, budget_gb):
+    """A job spread over wavefronts takes more memory (a boundary four times as
+    large, a byte a column where a lane has one): a round's trace and boundary
+    columns stay within the budget with it, and paths, scores and deviations
+    are those of one wavefront a job."""
+    rng = np.random.default_rng(740)
+    shapes = [(2100, 1000), (1600, 1500), (1000, 2300), (900, 640)] * 15
+    pairs = [_related(rng, la, lb, 0.05) for la, lb in shapes]
+    bands = rng.choice([2, 9, 40], size=len(pairs)).astype(np.uint32)
+    A, B, jobs = _batch(pairs)
+    os.environ.pop("MH_DP_COLS", None)
+    os.environ["MH_DP_BAND_KIND"] = "stripes"
+
+    def run():
+        ctx.set_timing(True)
+        ctx.reset_kernel_times()
+        paths, res, dev, st = mauvehip.global_align_banded(ctx, A, B, jobs, bands, flags=mauvehip.BAND_NO_FALLBACK)
+        arena, piped = ctx.kernel_time("dp_arena_bytes")[0], _pipe_parts(ctx)
+        ctx.set_timing(False)
+        return [(mauvehip.path_of(paths, res, k), int(res[k]["score"]), int(dev[k]), int(res[k]["path_len"]))
+                for k in range(len(pairs))], arena, piped
+
+    os.environ["MH_DP_PIPE"] = "1"
+    want, one, piped = run()
+    assert piped == 0
+    os.environ.pop("MH_DP_PIPE")
+    free, most, piped = run()
+    assert piped > 0 and most > one and free == want
+    monkeypatch.setenv("MH_DP_TB_BUDGET_GB", budget_gb)
+    got, arena, piped = run()
+    budget = float(budget_gb) * (1 << 30)
+    assert 0 < arena <= budget
+    if budget > most:
+        assert arena == most
+    assert got == want
+
+
 def test_pipelined_prefix_with_many_small_jobs(ctx, dp_env):
     """A round whose work items nearly fill the slots pipes only a prefix of
     its stripe jobs; the output equals the unpipelined one."""
