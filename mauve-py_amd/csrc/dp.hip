@@ -29,6 +29,7 @@
 #include "dp_tune_table.h"
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <numeric>
 #include <cstdlib>
 #include <utility>
@@ -702,13 +703,17 @@ constexpr uint32_t DP_PIPE_MAX = 32;
 constexpr int DPQ_MAXB = 72;
 constexpr int DPQ_CURSORS = DPQ_MAXB;
 
-// (Behind it in device memory: DPQ_CURSORS cursors, zeroed at the start of every
-// round, the last of them the round's wait-bound error flag.)
+struct alignas(16) DpBin {
+    uint32_t kind, first, count;
+    uint32_t item0;     // the bin's first item in queue order (prefix sums)
+};
+
+// (Behind its bins in device memory: DPQ_CURSORS cursors, zeroed at the start of
+// every round, the last of them the round's wait-bound error flag.)
 struct DpRound {
     uint32_t nbins;
     float table[DP_NCLASS * DP_NCLASS];   // match scores of cells without a tag
-    uint32_t kind[DPQ_MAXB], first[DPQ_MAXB], count[DPQ_MAXB];
-    uint32_t item0[DPQ_MAXB + 1];   // the bins' first items in queue order (prefix sums)
+    DpBin bin[DPQ_MAXB + 1];              // the last one's item0: the items
 };
 
 __device__ __forceinline__ uint32_t qk_per_item(uint32_t kind)
@@ -1330,22 +1335,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     const uint32_t nb = rd->nbins;
     if constexpr (!PERSIST) {
         const uint32_t w = blockIdx.x;
-        if (nb == 0 || w >= rd->item0[nb]) return;
+        if (nb == 0 || w >= rd->bin[nb].item0) return;
         uint32_t b = 0;    // the last bin that starts at or before item w
         for (uint32_t len = nb; len > 1;) {
             const uint32_t half = len >> 1;
-            if (rd->item0[b + half] <= w) { b += half; len -= half; }
+            if (rd->bin[b + half].item0 <= w) { b += half; len -= half; }
             else len = half;
         }
-        uint32_t item = w - rd->item0[b];
-        if (rd->kind[b] >= QK_PIPE) {
+        uint32_t item = w - rd->bin[b].item0;
+        if (rd->bin[b].kind >= QK_PIPE) {
             // a ticket, so that the parts of a job are taken in order by
             // running wavefronts (a part waits only on parts taken before it)
             uint32_t v = 0;
             if (threadIdx.x == 0) v = atomicAdd(&cursor[b], 1u);
             item = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
         }
-        run_item<CELL, MAXC>(DP_FWD_ARGS, table, rd->kind[b], rd->first[b], rd->count[b], item, lds);
+        run_item<CELL, MAXC>(DP_FWD_ARGS, table, rd->bin[b].kind, rd->bin[b].first, rd->bin[b].count, item, lds);
     } else {
         uint32_t b = 0;
         for (;;) {
@@ -1355,10 +1360,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                 uint32_t v = 0;
                 if (threadIdx.x == 0) v = atomicAdd(&cursor[b], 1u);
                 item = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
-                if ((uint64_t)item * qk_per_item(rd->kind[b]) < rd->count[b]) break;
+                if ((uint64_t)item * qk_per_item(rd->bin[b].kind) < rd->bin[b].count) break;
             }
             if (b >= nb) return;
-            run_item<CELL, MAXC>(DP_FWD_ARGS, table, rd->kind[b], rd->first[b], rd->count[b], item, lds);
+            run_item<CELL, MAXC>(DP_FWD_ARGS, table, rd->bin[b].kind, rd->bin[b].first, rd->bin[b].count, item, lds);
         }
     }
 }
@@ -1606,8 +1611,15 @@ uint32_t dp_effective_band(uint32_t la, uint32_t lb, uint32_t band, uint32_t col
 
 static inline uint64_t align256(uint64_t v) { return (v + 255) & ~255ull; }
 
-// device bytes of a round's descriptor and its queue cursors
-constexpr uint64_t DP_ROUND_BYTES = (sizeof(DpRound) + DPQ_CURSORS * 4 + 255) & ~255ull;
+// device bytes of a round's descriptor with room for `bins` bins, and its queue cursors
+static constexpr uint64_t dp_cursor_at(uint32_t bins) { return offsetof(DpRound, bin) + (bins + 1) * sizeof(DpBin); }
+static constexpr uint64_t dp_round_bytes(uint32_t bins) { return (dp_cursor_at(bins) + DPQ_CURSORS * 4 + 255) & ~255ull; }
+
+// The fixed scratch's rounds hold no pipelined jobs, so fewer bins.  A job there
+// is refused by its trace, its boundary at 12 bytes a row and 1,792 bytes, which
+// the layout must not exceed.
+constexpr uint32_t DPQ_FIXED_MAXB = 48;
+static_assert(dp_round_bytes(DPQ_FIXED_MAXB) <= 1280, "the fixed scratch's limit");
 
 // The forward kernel's variants: the widest shape each holds, its
 // wavefronts a SIMD, and whether its wavefronts persist.  Rounds with a shape
@@ -1830,7 +1842,8 @@ static int dp_launch_round(mh_context *ctx, int v, bool graph, unsigned grid, Ro
     return MH_OK;
 }
 
-// ints of the boundary columns of an item's job: 3 a row, for a pipelined job 12
+// ints of the boundary columns of an item's job: two values a row, for a
+// pipelined job two 64-bit words in each of two buffers
 static uint64_t item_bnd_ints(const DpItem &it, const mh_dp_job *jobs)
 {
     // one-lane and window jobs hand no column over; a job of 16-lane
@@ -1838,7 +1851,7 @@ static uint64_t item_bnd_ints(const DpItem &it, const mh_dp_job *jobs)
     if (it.cols == TINY_COLS_TAG || it.cols >= WINDOW_TAG) return 0ull;
     const uint64_t sw = it.cols > GROUP_TAG ? 16ull * (it.cols - GROUP_TAG) : 64ull * it.cols;
     const uint64_t ns = (jobs[it.job].b_len + sw - 1) / sw;
-    return ns > 1 ? (it.parts ? 12ull : 3ull) * ((jobs[it.job].a_len + 63) & ~63ull) : 0ull;
+    return ns > 1 ? (it.parts ? 8ull : 2ull) * ((jobs[it.job].a_len + 63) & ~63ull) : 0ull;
 }
 
 // bytes of the arena of a round with tbb bytes of trace and bi boundary ints
@@ -1854,7 +1867,14 @@ static uint64_t item_bytes(const DpItem &it, const mh_dp_job *jobs)
 // tbb (each rounded up to 16) and bi boundary ints
 static uint64_t fixed_need(uint64_t cnt, uint64_t tbb, uint64_t bi)
 {
-    return DP_ROUND_BYTES + align256(cnt * (sizeof(DevJob) + sizeof(DpOut) + 4)) + align256(bi * 4) + tbb + 256;
+    return dp_round_bytes(DPQ_FIXED_MAXB) + align256(cnt * (sizeof(DevJob) + sizeof(DpOut) + 4)) + align256(bi * 4) +
+           tbb + 256;
+}
+
+// does the fixed scratch take the job (see DPQ_FIXED_MAXB)
+static bool fixed_takes(const DpItem &it, const mh_dp_job *jobs, const FixedScratch *fx)
+{
+    return fixed_need(1, (it.tb_bytes + 15) & ~15ull, item_bnd_ints(it, jobs) / 2 * 3) <= fx->bytes;
 }
 
 // Pipelined stripe jobs.  Where the longest job takes longer on its own wavefront
@@ -2009,7 +2029,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
     auto bnd_ints = [&](const DpItem &it) { return item_bnd_ints(it, jobs); };
     if (fx) {
         for (const DpItem &it : items)
-            MH_CHECK(fixed_need(1, (it.tb_bytes + 15) & ~15ull, bnd_ints(it)) <= fx->bytes, MH_ERR_INVALID,
+            MH_CHECK(fixed_takes(it, jobs, fx), MH_ERR_INVALID,
                      "DP job " + std::to_string(it.job) + " (" + std::to_string(jobs[it.job].a_len) + " x " +
                          std::to_string(jobs[it.job].b_len) + ") needs more than the " +
                          std::to_string(fx->bytes >> 20) + " MiB scratch of the no-allocation entry point");
@@ -2188,7 +2208,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             // [round descriptor + cursors] [jobs | results] [boundary ints] [trace]
             uint8_t *q = fx->ptr;
             d_round = reinterpret_cast<DpRound *>(q);
-            q += DP_ROUND_BYTES;
+            q += dp_round_bytes(DPQ_FIXED_MAXB);
             d_jobs = reinterpret_cast<DevJob *>(q);
             d_outs = reinterpret_cast<DpOut *>(d_jobs + n);
             q += align256(n * (sizeof(DevJob) + sizeof(DpOut) + 4));
@@ -2199,7 +2219,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
         } else {
             int rc;
             if ((rc = ctx->dp_jobs.ensure(n * (sizeof(DevJob) + sizeof(DpOut) + 4) + 256)) != MH_OK) return rc;
-            if ((rc = ctx->dp_round.ensure(DP_ROUND_BYTES)) != MH_OK) return rc;
+            if ((rc = ctx->dp_round.ensure(dp_round_bytes(DPQ_MAXB))) != MH_OK) return rc;
             d_jobs = ctx->dp_jobs.as<DevJob>();
             d_outs = reinterpret_cast<DpOut *>(d_jobs + n);
             d_bnd = ctx->dp_tb.as<int>();
@@ -2212,13 +2232,11 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
         // the round's descriptor: the queue's bins
         DpRound hr;
         std::memset(&hr, 0, sizeof(hr));
+        const uint32_t max_bins = fx ? DPQ_FIXED_MAXB : DPQ_MAXB;
         if (form != DpCells::TAGGED) dp_score6(hr.table);
         auto add_bin = [&](uint32_t kind, uint64_t b0, uint64_t cnt) {
             if (cnt == 0) return;
-            hr.kind[hr.nbins] = kind;
-            hr.first[hr.nbins] = (uint32_t)b0;
-            hr.count[hr.nbins] = (uint32_t)cnt;
-            ++hr.nbins;
+            hr.bin[hr.nbins++] = {kind, (uint32_t)b0, (uint32_t)cnt, 0};
         };
         {
             // stripe jobs: a new bin where the trace size falls below the next power of 4
@@ -2237,7 +2255,7 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
                 while (y < n64 && cls(items[first + y].tb_bytes) == c0) ++y;
                 // keep ROW_SHAPES + 2 bins for the row, window and one-lane
                 // jobs, and the last cursor for the wait-bound error flag
-                if (hr.nbins + 1 >= (uint32_t)(DPQ_MAXB - ROW_SHAPES - 3)) y = n64;
+                if (hr.nbins + 1 >= max_bins - ROW_SHAPES - 3) y = n64;
                 add_bin(QK_STRIPE, x, y - x);
                 x = y;
             }
@@ -2245,16 +2263,17 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             add_bin(QK_WINDOW, nstripe, nbig - nstripe);
             add_bin(QK_TINY, nbig, n - nbig);
         }
-        MH_CHECK(hr.nbins < (uint32_t)DPQ_CURSORS, MH_ERR_INVALID, "DP round: too many queue bins");
+        MH_CHECK(hr.nbins < max_bins, MH_ERR_INVALID, "DP round: too many queue bins");
         uint64_t nitems_q = 0;
         for (uint32_t q = 0; q < hr.nbins; ++q) {
+            const uint32_t kind = hr.bin[q].kind;
             const uint32_t per =
-                hr.kind[q] == QK_STRIPE || hr.kind[q] == QK_WINDOW || hr.kind[q] >= QK_PIPE ? 1u
-                                                                                          : (hr.kind[q] == QK_TINY ? 64u : 4u);
-            hr.item0[q] = (uint32_t)nitems_q;
-            nitems_q += (hr.count[q] + per - 1) / per;
+                kind == QK_STRIPE || kind == QK_WINDOW || kind >= QK_PIPE ? 1u : (kind == QK_TINY ? 64u : 4u);
+            hr.bin[q].item0 = (uint32_t)nitems_q;
+            nitems_q += (hr.bin[q].count + per - 1) / per;
         }
-        hr.item0[hr.nbins] = (uint32_t)nitems_q;
+        hr.bin[hr.nbins].item0 = (uint32_t)nitems_q;
+        const uint64_t hr_bytes = offsetof(DpRound, bin) + (hr.nbins + 1) * sizeof(DpBin);
         unsigned grid = 0;
         {
             int rc;
@@ -2267,20 +2286,20 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
         ra.tb = d_tb;
         ra.bnd = d_bnd;
         ra.rd = d_round;
-        ra.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(d_round) + sizeof(DpRound));
+        ra.cursor = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(d_round) + dp_cursor_at(max_bins));
         ra.paths = d_paths;
         ra.res = d_results;
         ra.dev = d_dev;
         ra.npipe = (uint32_t)npipe;
         if (fx) {
-            MH_HIP(hipMemcpyAsync(d_round, &hr, sizeof(hr), hipMemcpyHostToDevice, ctx->stream));
+            MH_HIP(hipMemcpyAsync(d_round, &hr, hr_bytes, hipMemcpyHostToDevice, ctx->stream));
             int rc;
             if ((rc = dp_launch_round(ctx, variant, false, grid, ra)) != MH_OK) return rc;
         } else {
             int rc;
             if ((rc = dp_round_staging(ctx)) != MH_OK) return rc;
-            std::memcpy(ctx->dp_round_host, &hr, sizeof(hr));
-            MH_HIP(hipMemcpyAsync(d_round, ctx->dp_round_host, sizeof(hr), hipMemcpyHostToDevice, ctx->stream));
+            std::memcpy(ctx->dp_round_host, &hr, hr_bytes);
+            MH_HIP(hipMemcpyAsync(d_round, ctx->dp_round_host, hr_bytes, hipMemcpyHostToDevice, ctx->stream));
             if ((rc = dp_launch_round(ctx, variant, dp_use_graph(), grid, ra)) != MH_OK) return rc;
         }
         // the host job table is reused by the next round
@@ -2452,7 +2471,7 @@ static int dp_run_wild(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, 
         if (fx && (rc = dp_float_fits(jobs, j, fx)) != MH_OK) return rc;
         DpItem it = make_item(jobs[j], j, 0, force, false, false);
         it.cells = (uint64_t)jobs[j].a_len * jobs[j].b_len;
-        if (fx && fixed_need(1, (it.tb_bytes + 15) & ~15ull, item_bnd_ints(it, jobs)) > fx->bytes) thin.push_back(j);
+        if (fx && !fixed_takes(it, jobs, fx)) thin.push_back(j);
         else items.push_back(it);
     }
     if ((rc = dp_run_items(ctx, d_a, d_b, jobs, slot, items, d_paths, d_results, d_dev, cells, fx, DpCells::FLOAT)) !=

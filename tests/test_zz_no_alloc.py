@@ -82,3 +82,30 @@ def test_noalloc_refuses_a_job_above_the_scratch(ctx, jobset):
     finally:
         ctx.free(dA)
         ctx.free(dB)
+
+
+@pytest.mark.parametrize("la,lb", [(262074, 400), (43288, 3000)])
+def test_noalloc_takes_jobs_up_to_its_limit(ctx, la, lb):
+    """The largest job of a shape: trace, 12 bytes a row of boundary (none
+    for one stripe) and 1,792 bytes are exactly 64 MiB; a row more is
+    refused."""
+    stripe, lane_bytes = (512, 4) if lb <= 512 else (1024, 8)
+    ns = -(-lb // stripe)
+    bnd = 12 * ((la + 63) // 64 * 64) if ns > 1 else 0
+    assert (la + 63) * ns * 64 * lane_bytes + (bnd + 255) // 256 * 256 + 1792 == 64 << 20
+    rng = np.random.default_rng(la)
+    A = rng.integers(0, 4, la + 1, dtype=np.uint8)
+    B = A[1000:1000 + lb].copy()
+    B[::9] = rng.integers(0, 4, len(B[::9]), dtype=np.uint8)
+    dA, dB = ctx.alloc(len(A) + 16), ctx.alloc(len(B) + 16)
+    try:
+        ctx.h2d(dA, A)
+        ctx.h2d(dB, B)
+        jobs = mauvehip.make_jobs(np.array([0]), np.array([la]), np.array([0]), np.array([lb]))
+        _same(*_call(ctx, "mh_dp_align_device", dA, dB, jobs), *_call(ctx, "mh_dp_align_device_noalloc", dA, dB, jobs))
+        jobs["a_len"] = la + 1
+        with pytest.raises(mauvehip.MhError, match="64 MiB"):
+            _call(ctx, "mh_dp_align_device_noalloc", dA, dB, jobs)
+    finally:
+        ctx.free(dA)
+        ctx.free(dB)
