@@ -410,6 +410,16 @@ template <class T> struct CmpCell {
 // score and edge are then the final pick in every lane of the group.
 constexpr uint32_t DP_SPIN_MAX = 1u << 22;
 
+// Between one lane's write to LDS and another lane's access to the same slot
+// (the lanes of a wavefront): its LDS operations complete in order, and the
+// compiler moves none across this.
+__device__ __forceinline__ void lanes_ordered()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // LDS of one wavefront: the rows a group's first lane takes in, and the
 // boundary column its last lane hands on
 struct DpLds {
@@ -594,7 +604,9 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
                 }
                 int lo, hi;
                 CELL::operand(sc, nA, lo, hi);
+                lanes_ordered();     // (the chunk before has been read)
                 if (CH == G || lane < CH) lds.in[gb + lane] = make_int4(nH, nF, lo, hi);
+                lanes_ordered();
                 left_in(t + CH + lane, nH, nF, nA);
                 ahead = lds.in[gb];
             }
@@ -616,6 +628,7 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
             out_slot[q * out_next] = make_int2(outH, outF);
             if ((q == CH - 1 || t == nsteps - 1) && !last_stripe && (CH == G || lane < CH)) {
                 // the rows of the stripe's last column that this chunk finished
+                lanes_ordered();
                 const int x = t - q - (G - 1) + lane;
                 if (x >= 0 && x < nrows) {
                     const int r = r0 - 1 + x;
@@ -630,6 +643,7 @@ __device__ __forceinline__ bool dp_job(const DevJob &jb, const uint8_t *__restri
                         bF[r] = v.y;
                     }
                 }
+                lanes_ordered();     // (before the next chunk's writes)
             }
         }
         if constexpr (PIPE) __builtin_amdgcn_s_setprio(0);
