@@ -867,7 +867,8 @@ __device__ __forceinline__ uint32_t bucket_of(int64_t off)
 // offset's quotient by the table's size and the strand).  Reading the records in
 // bucket order instead is one scattered read a seed and kernel: key2_kernel 73 us
 // and bucket_dirty_kernel 64 over 4.5 million seeds, 15 and 6 here.  Genomes
-// whose starts and lines need more bits take that way.
+// whose starts and lines need more bits take that way (a gigabase or so;
+// MH_BUCKET_KEY=records: any).
 struct BucketKey {
     int eb;          // bits of a start
     int packed;
@@ -1424,7 +1425,8 @@ int partition_seeds(mh_context *ctx, const SeedRec *d_seeds, uint64_t ns, int k,
     const uint64_t lines = 2 * ((uint64_t)bk.bias + len_b / TABLE_SIZE + 2);
     int lbits = 1;
     while ((1ull << lbits) < lines) ++lbits;
-    bk.packed = 16 + eb + lbits <= 64;
+    const char *ke = getenv("MH_BUCKET_KEY");
+    bk.packed = 16 + eb + lbits <= 64 && !(ke && !strcmp(ke, "records"));
     clean.clear();
     dirty.clear();
     *n_clean_seeds = 0;
@@ -2387,7 +2389,9 @@ int unique_seeds(mh_context *ctx, const mh_sml *const *smls, int k, const LiveRa
                 hipLaunchKernelGGL(kern, dim3(hi - lo), dim3(64), 0, ctx->stream, qs, blist + lo, order, bst, vec, nent,
                                    resume, d_coll);
         };
-        if (longest >= (1u << 29)) {     // (uq_cmp's differences past 32 bits)
+        // past 32 bits of uq_cmp's differences (or where MH_UQ_REPLAY=memory asks) nothing from LDS
+        const char *re = getenv("MH_UQ_REPLAY");
+        if (longest >= (1u << 29) || (re && !strcmp(re, "memory"))) {
             MH_HIP(hipMemcpyAsync(resume, bst, NB * 4, hipMemcpyDeviceToDevice, ctx->stream));
             bin(uq_replay_rest_kernel<EntU>, 0, n_some);
         } else if (k <= 8) {

@@ -76,8 +76,8 @@ def test_match_recoded_4_6Mb(ctx):
 @pytest.mark.parametrize("seed", [po.get_seed(15, 0), po.get_seed(11, 0)])
 def test_match_spaced_long_walks(ctx, seed):
     """Spaced seeds over long identical and near-identical stretches, forward
-    and inverted: the seeds of one chain (one seed length apart on a diagonal)
-    share one walk, and walks past the step budget finish per diagonal."""
+    and inverted: the seeds of one run (each within a seed length of the next
+    on a diagonal) share one walk, and a whole block finishes a long walk."""
     rng = np.random.default_rng(seed & 0xFFFF)
     a = synth.BASES[rng.integers(0, 4, 120_000)]
     b = a.copy()
@@ -141,6 +141,32 @@ def test_match_three_and_four_genomes(ctx, ng, seed):
     assert np.array_equal(gs, os_)
     assert np.array_equal(gl, ol)
     assert (gs != 0).sum(axis=1).max() == 2      # pairwise matches: two genomes each
+
+
+@pytest.mark.parametrize("ng,seed", [(2, po.get_seed(17, 3)), (2, po.get_seed(15, 0)), (2, 0xFFF),
+                                     (3, po.get_seed(15, 3)), (4, po.get_seed(15, 0))])
+def test_match_bucket_keys_without_starts_and_lines(ctx, monkeypatch, ng, seed):
+    """Genomes whose starts and lines do not fit the bucket sort's key have the
+    seed records read instead (MH_BUCKET_KEY=records asks for that at any
+    size): the oracle's lists and counts, and those of the packed keys; half
+    of each genome lies a whole table further on, so lines share buckets."""
+    rng = np.random.default_rng(ng * 100 + (seed & 0xFF))
+    seqs = _relatives(rng, synth.BASES[rng.integers(0, 4, 60_000)], ng, 0.02, 6000)
+    seqs = [s if g == 0 else np.concatenate([s[:30_000], synth.BASES[rng.integers(0, 4, 40_000)], s[30_000:]])
+            for g, s in enumerate(seqs)]
+    seqs = [s.tobytes() for s in seqs]
+    smls = [mauvehip.SortedMerList(ctx, s, seed) for s in seqs]
+    packed = mauvehip.find_matches(ctx, smls)
+    monkeypatch.setenv("MH_BUCKET_KEY", "records")
+    gs, gl, gst = mauvehip.find_matches(ctx, smls)
+    os_, ol, ost = po.find_matches(seqs, seed)
+    assert gst.seed_tuples == ost.hash_calls and gst.collisions == ost.collisions
+    # (spaced seeds step over single substitutions: at least a match a piece
+    # between the insert, the inversion and the deletion)
+    assert len(gl) == len(ol) > 5
+    for st, ln in ((gs, gl), packed[:2]):
+        assert np.array_equal(st, os_)
+        assert np.array_equal(ln, ol)
 
 
 def _tandem(unit, copies):

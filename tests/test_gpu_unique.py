@@ -116,8 +116,8 @@ def test_unique_eight_genome_tree_family(ctx):
 
 @pytest.mark.parametrize("seed", [0xFFF, 0x7B974EF])
 def test_unique_chain_walks_equal_every_seed_walk(ctx, monkeypatch, seed):
-    """Spaced (and even solid) seeds walk once per chain of seeds one seed
-    length apart on their diagonal: the lists equal those of a walk from every
+    """Spaced (and even solid) seeds walk once per chain of seeds within a seed
+    length of each other on their diagonal: the lists equal those of a walk from every
     seed, with fewer walks."""
     rng = np.random.default_rng(66)
     seqs = _family(rng, 20000, 6)
@@ -164,3 +164,52 @@ def test_unique_long_identical_stretches(ctx, ng, seed):
         t = "".join(t)
         seqs.append(t[::-1].translate(COMP) if g % 3 == 1 else t[g:])
     _check(ctx, seqs, seed)
+
+
+@pytest.mark.parametrize("ng,seed", [(3, 0x1FFF), (8, 0x7B974EF), (9, 0xFFF), (16, 0x7FFF)])
+def test_unique_replay_from_memory(ctx, monkeypatch, ng, seed):
+    """Genomes of 2^29 bases and more have every bucket replayed from device
+    memory from its first seed (MH_UQ_REPLAY=memory asks for that at any
+    size): the oracle's lists and collisions, buckets of one and of thousands
+    of seeds among them."""
+    rng = np.random.default_rng(500 + ng)
+    seqs = _family(rng, 12000, ng)
+    monkeypatch.setenv("MH_UQ_REPLAY", "memory")
+    st = _check(ctx, seqs, seed)
+    assert st.matches > 50 and st.collisions > 0
+    base = rng.integers(0, 4, 8000)
+    same = []
+    for g in range(ng):
+        t = base.copy()
+        hit = rng.random(len(t)) < 0.03
+        t[hit] = (t[hit] + 1) % 4
+        same.append("".join("ACGT"[x] for x in t))
+    _check(ctx, same, seed)
+
+
+def test_unique_list_of_several_pinned_pieces(ctx):
+    """A list of more than two pieces of the pinned copy to the host (8 MB
+    each, the last one short): that of the pairwise matcher, whose list comes
+    another way."""
+    rng = np.random.default_rng(31)
+    block = 997
+    n = 60_000 * block
+    bases = np.frombuffer(b"ACGT", dtype=np.uint8)
+    a = bases[rng.integers(0, 4, n, dtype=np.uint8)]
+    # (blocks in another order: the matches' offsets fill the buckets evenly)
+    b = a.reshape(-1, block)[rng.permutation(n // block)].ravel()
+    hit = np.flatnonzero(rng.random(n, dtype=np.float32) < 0.055)
+    b[hit] = bases[(np.searchsorted(bases, b[hit]) + 1) % 4]
+    seed = (1 << 17) - 1
+    smls = [mauvehip.SortedMerList(ctx, s.tobytes(), seed) for s in (a, b)]
+    try:
+        gs, gl, gst = mauvehip.find_matches_unique(ctx, smls)
+        pm, pst = mauvehip.find_matches_raw(ctx, smls)
+    finally:
+        for x in smls:
+            x.free()
+    assert gs.nbytes > 17 << 20 and gs.nbytes % (8 << 20) != 0
+    assert gl.nbytes > 8 << 20
+    assert np.array_equal(gs, pm["start"][:, :2])
+    assert np.array_equal(gl, pm["length"])
+    assert gst.collisions == pst.collisions
