@@ -443,11 +443,20 @@ void launch_walks(mh_context *ctx, const SRC &src, uint64_t ns, const uint32_t *
 // pointer jumping leads to the heads.  Two such links always span more than a
 // seed length.
 
-__global__ void spaced_link_kernel(const uint2 *__restrict__ pp, uint64_t L0, uint32_t seed_len,
+// The positions these kernels look at, a thread each: all of them, or only the
+// seeds' (pi not null), which lie in no order but are far fewer.
+struct RunPos {
+    uint64_t n;
+    const uint32_t *pi, *pos0;
+    __device__ __forceinline__ uint64_t at(uint64_t x) const { return pi ? (uint64_t)pos0[pi[x]] : x; }
+};
+
+__global__ void spaced_link_kernel(RunPos rp, const uint2 *__restrict__ pp, uint32_t seed_len,
                                    uint32_t *__restrict__ link)
 {
-    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= L0) return;
+    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= rp.n) return;
+    const uint64_t p = rp.at(x);
     const uint2 v = pp[p];
     uint32_t out = (uint32_t)p;
     if (v.x != NO_SEED) out = spaced_link((uint32_t)p, seed_len, [&](uint32_t x) { return pp[x].x; });
@@ -455,12 +464,13 @@ __global__ void spaced_link_kernel(const uint2 *__restrict__ pp, uint64_t L0, ui
 }
 
 // the heads' seed indices, in no order (each walk writes its own seed's result)
-__global__ void spaced_heads_kernel(const uint2 *__restrict__ pp, const uint32_t *__restrict__ root, uint64_t L0,
+__global__ void spaced_heads_kernel(RunPos rp, const uint2 *__restrict__ pp, const uint32_t *__restrict__ root,
                                     uint32_t *__restrict__ heads, uint32_t *__restrict__ count)
 {
-    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t p = x < rp.n ? rp.at(x) : 0;
     uint2 v = make_uint2(NO_SEED, 0);
-    if (p < L0) v = pp[p];
+    if (x < rp.n) v = pp[p];
     const bool head = v.x != NO_SEED && root[p] == (uint32_t)p;
     const uint64_t b = __ballot(head);
     if (!b) return;
@@ -471,11 +481,12 @@ __global__ void spaced_heads_kernel(const uint2 *__restrict__ pp, const uint32_t
     if (head) heads[at + __builtin_popcountll(b & ((1ull << lane) - 1))] = v.y;
 }
 
-__global__ void spaced_fill_kernel(const uint2 *__restrict__ pp, const uint32_t *__restrict__ root, uint64_t L0,
+__global__ void spaced_fill_kernel(RunPos rp, const uint2 *__restrict__ pp, const uint32_t *__restrict__ root,
                                    SeedRec *__restrict__ out)
 {
-    const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= L0) return;
+    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= rp.n) return;
+    const uint64_t p = rp.at(x);
     const uint2 v = pp[p];
     if (v.x == NO_SEED || root[p] == (uint32_t)p) return;
     const SeedRec h = out[pp[root[p]].y];
@@ -490,17 +501,29 @@ __global__ void spaced_fill_kernel(const uint2 *__restrict__ pp, const uint32_t 
 
 // eight hops a launch, fewer where the chain ends: 200,000 positions take five
 // launches of 3.5 us (one hop, so a doubling, a launch: 19 of 9 us)
-__global__ void grid_jump_kernel(const uint32_t *__restrict__ in, uint32_t *__restrict__ out, uint64_t ns)
+__device__ __forceinline__ uint32_t hop8(const uint32_t *__restrict__ in, uint64_t r)
 {
-    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= ns) return;
     uint32_t a = in[r];
     for (int h = 1; h < 8; ++h) {
         const uint32_t b = in[a];
         if (b == a) break;
         a = b;
     }
-    out[r] = a;
+    return a;
+}
+
+__global__ void grid_jump_kernel(const uint32_t *__restrict__ in, uint32_t *__restrict__ out, uint64_t ns)
+{
+    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < ns) out[r] = hop8(in, r);
+}
+
+__global__ void spaced_jump_kernel(RunPos rp, const uint32_t *__restrict__ in, uint32_t *__restrict__ out)
+{
+    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= rp.n) return;
+    const uint64_t p = rp.at(x);
+    out[p] = hop8(in, p);
 }
 
 // flag[r]: sorted seed r heads its chain
@@ -1040,6 +1063,11 @@ static bool walk_env(mh_context *ctx, const mh_sml *const *smls, int k, DevBuf *
     return pal;
 }
 
+// Fewer than a seed in so many positions: by seed.  100 million positions with
+// 5 thousand seeds, by seed 185 us, by position 1,892; with 400 thousand 487 and
+// 2,482, 3.2 million 2,604 and 3,092, 6.1 million 4,728 and 3,401.
+constexpr uint64_t SEEDS_FEW = 32;
+
 // Seeds of a pair, other than odd solid ones, in HashMatch order with their
 // extensions (the kernels above).  cnt[0, 2): cleared; heads, long walks.
 static int extend_by_runs(mh_context *ctx, const mh_sml *a, const mh_sml *b, const uint32_t *oi, const uint32_t *oj,
@@ -1059,25 +1087,27 @@ static int extend_by_runs(mh_context *ctx, const mh_sml *a, const mh_sml *b, con
     WalkEnv env;
     const bool pal = walk_env(ctx, smls, 2, bufs, &env, &rc);
     if (rc != MH_OK) return rc;
-    const dim3 gs((unsigned)((ns + 255) / 256)), gp((unsigned)((L0 + 255) / 256)), blk(256);
+    RunPos rp{L0, nullptr, nullptr};
+    if (ns < L0 / SEEDS_FEW) rp = {ns, oi, a->d_pos};
+    const dim3 gs((unsigned)((ns + 255) / 256)), gp((unsigned)((rp.n + 255) / 256)), blk(256);
     MH_HIP(hipMemsetAsync(pp, 0xFF, L0 * 8, ctx->stream));
     hipLaunchKernelGGL(run_scatter_kernel, gs, blk, 0, ctx->stream, oi, oj, ns, a->d_keys, a->d_pos, b->d_keys,
                        b->d_pos, pp);
-    hipLaunchKernelGGL(spaced_link_kernel, gp, blk, 0, ctx->stream, pp, L0, (uint32_t)S, la);
+    hipLaunchKernelGGL(spaced_link_kernel, gp, blk, 0, ctx->stream, rp, pp, (uint32_t)S, la);
     // so many launches reach every head, without a check in between
     const uint64_t longest = std::min<uint64_t>(ns, 2 * (L0 / S) + 2);
     for (uint64_t reach = 1; reach < longest; reach *= 8) {
-        hipLaunchKernelGGL(grid_jump_kernel, gp, blk, 0, ctx->stream, la, lb, L0);
+        hipLaunchKernelGGL(spaced_jump_kernel, gp, blk, 0, ctx->stream, rp, la, lb);
         std::swap(la, lb);
     }
-    hipLaunchKernelGGL(spaced_heads_kernel, gp, blk, 0, ctx->stream, pp, la, L0, heads, cnt);
+    hipLaunchKernelGGL(spaced_heads_kernel, gp, blk, 0, ctx->stream, rp, pp, la, heads, cnt);
     if (pal)
         launch_walks(ctx, PairWalks<true>{heads, oi, oj, a->d_keys, b->d_keys, a->d_pos, b->d_pos, d_seeds}, ns, cnt,
                      env, rest, cnt + 1);
     else
         launch_walks(ctx, PairWalks<false>{heads, oi, oj, a->d_keys, b->d_keys, a->d_pos, b->d_pos, d_seeds}, ns, cnt,
                      env, rest, cnt + 1);
-    hipLaunchKernelGGL(spaced_fill_kernel, gp, blk, 0, ctx->stream, pp, la, L0, d_seeds);
+    hipLaunchKernelGGL(spaced_fill_kernel, gp, blk, 0, ctx->stream, rp, pp, la, d_seeds);
     MH_HIP(hipGetLastError());
     return MH_OK;
 }

@@ -143,6 +143,24 @@ def test_match_three_and_four_genomes(ctx, ng, seed):
     assert (gs != 0).sum(axis=1).max() == 2      # pairwise matches: two genomes each
 
 
+@pytest.mark.parametrize("seed", [po.get_seed(15, 0), 0xFFFFF, 0b1101011101110111011])
+@pytest.mark.parametrize("share", [0, 40, 1500, 9000])
+def test_match_few_seeds_in_long_genomes(ctx, seed, share):
+    """Runs of seeds looked for by seed where fewer than one position in 32
+    holds one, by position above: no common stretch but by chance, one
+    window or so, stretches on both strands, and more than a 32nd."""
+    rng = np.random.default_rng(share + (seed & 0xFF))
+    a = synth.BASES[rng.integers(0, 4, 200_000)]
+    b = synth.BASES[rng.integers(0, 4, 190_000)]
+    b[:share] = a[:share]                                  # to the sequences' start
+    b[100_000:100_000 + share] = synth.revcomp(a[150_000:150_000 + share])
+    b[50_000:50_000 + share] = a[70_000:70_000 + share]
+    b[50_000 + share // 2:50_000 + share // 2 + 20:7] = ord("A")
+    _compare(ctx, a.tobytes(), b.tobytes(), seed)
+    few = _compare.last_stats.seed_tuples < len(a) // 32
+    assert few == (share < 9000)
+
+
 @pytest.mark.parametrize("ng,seed", [(2, po.get_seed(17, 3)), (2, po.get_seed(15, 0)), (2, 0xFFF),
                                      (3, po.get_seed(15, 3)), (4, po.get_seed(15, 0))])
 def test_match_bucket_keys_without_starts_and_lines(ctx, monkeypatch, ng, seed):
