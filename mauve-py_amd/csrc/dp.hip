@@ -1905,6 +1905,18 @@ static bool fixed_takes(const DpItem &it, const mh_dp_job *jobs, const FixedScra
 // 2,048 columns 4.9 ms, spread 5.3).  A banded job's stripe starts when the one
 // before it has sent the row the stripe starts at, its row shift and the lanes'
 // skew later, so more parts than a stripe's steps over that lag would only wait.
+// Jobs over all 64 lanes leave fewer SIMDs idle but take two to three times the
+// steps, so a round with enough of them is better off without (10,000 banded
+// jobs of 1,000 columns, 4 to 100 wide: 0.8 to 2.6 ms without, 2.8 to 6.0 with;
+// 50 of 4,000, 100 wide: 5.8 and 1.9).  Where there are such jobs, the round's
+// time is estimated with all its long jobs spread, with those of 64 lanes
+// alone, and with none, in cycles as measured: a step of a job alone on its SIMD 630
+// with one or two columns a lane, 760 or 6.5 an instruction with 16 lanes, 6 an
+// instruction in a part; of several on a SIMD 4.2 (4.6 with 16 lanes) an
+// instruction, 4 for each of 60 + 14 a column with one or two columns.  The
+// estimates fit 60 rounds (equal jobs of 300 to 4,000 columns, log-uniform ones
+// up to 1,000, 5,000 and 20,000) to a fifth; the plan that spreads all has to be
+// 7% ahead, since rounds at 6% lost by it.
 // Pipelined jobs start first.  items[0, n): the round's stripe jobs (every lane
 // shape), longest first; other: its remaining wavefronts.  MH_DP_PIPE = P (p_env)
 // instead gives P wavefronts to the first 64-lane jobs with at least P stripes,
@@ -1963,8 +1975,10 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
     auto step_cost = [](uint32_t cols) { return 24.0 + 12.4 * cols; };
     struct Opt {
         double own, stripe;    // time on its own; of one stripe when pipelined
-        uint32_t ns, pmax;
+        double steps, lead;    // steps on its own; between stripes' starts at least, when pipelined
+        uint32_t ns, pmax, c2; // c2: columns a lane when pipelined
         float weight;
+        bool widen;
     };
     std::vector<Opt> opt(n);
     double total = 0, longest = 0;
@@ -1977,16 +1991,18 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
         o.own = steps * step_cost(c);
         o.ns = (jb.b_len + sw - 1) / sw;
         o.weight = group(it) ? 0.25f : 1.0f;
+        o.steps = steps;
         o.pmax = 0;
-        const bool widen = tagged && group(it) && it.band != 0 && (c == 4 || c == 8);
-        if (o.ns > 1 && (g == 64 || widen)) {
-            const uint32_t c2 = widen ? c / 4 : c;
+        o.widen = tagged && group(it) && it.band != 0 && (c == 4 || c == 8);
+        if (o.ns > 1 && (g == 64 || o.widen)) {
+            o.c2 = o.widen ? c / 4 : c;
             const double rows = steps / o.ns - (g - 1);
-            o.stripe = (rows + 63) * step_cost(c2);
+            o.stripe = (rows + 63) * step_cost(o.c2);
             o.pmax = std::min(DP_PIPE_MAX, o.ns);
+            o.lead = 0;
             if (it.band) {
-                const double lag = (double)jb.a_len * sw / jb.b_len + 63 + (c2 <= 2 ? 16 : 64);
-                o.pmax = std::min<uint32_t>(o.pmax, (uint32_t)std::max(1.0, std::ceil((rows + 63) / lag)));
+                o.lead = (double)jb.a_len * sw / jb.b_len + 63 + (o.c2 <= 2 ? 16 : 64);
+                o.pmax = std::min<uint32_t>(o.pmax, (uint32_t)std::max(1.0, std::ceil((rows + 63) / o.lead)));
             }
         }
         total += o.own * o.weight;
@@ -1994,15 +2010,48 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
     }
     const double share = total / slots, T = 0.25 * share;
     if (longest <= 1.1 * share) return;
+    int spread = 2;     // 0: no job, 1: those of 64 lanes, 2: all
+    bool up = false;
     auto parts_of = [&](const Opt &o, bool up) -> uint32_t {
-        if (o.own <= T || !o.pmax) return 0;
+        if (o.own <= T || !o.pmax || spread < (o.widen ? 2 : 1)) return 0;
         const double m = std::max(1.0, up ? std::ceil(T / o.stripe) : std::floor(T / o.stripe));   // stripes a part
         return std::min<uint32_t>(o.pmax, (uint32_t)std::ceil(o.ns / m));
     };
     // parts past the slots would run after the others: fewer, longer ones then
-    double all = 0;
-    for (const Opt &o : opt) all += parts_of(o, false);
-    const bool up = all > slots;
+    auto plan = [&] {
+        double all = 0;
+        for (const Opt &o : opt) all += parts_of(o, false);
+        up = all > slots;
+    };
+    plan();
+    if (std::any_of(opt.begin(), opt.end(), [&](const Opt &o) { return o.widen && parts_of(o, up); })) {
+        // cycles of the round: the SIMDs' issue shared evenly, or the longest
+        // job's own steps, after the pipelined ones' issue where it is not one
+        double cycles[3];
+        for (spread = 2; spread >= 0; --spread) {
+            plan();
+            double issue = 0, issue_piped = 0, longest_piped = 0, longest_own = 0;
+            for (const Opt &o : opt) {
+                const uint32_t p = parts_of(o, up);
+                if (!p || (p == 1 && !o.widen)) {
+                    const bool g16 = o.weight < 1.0f;
+                    issue += (g16 ? 4.6 : 4.2) * o.own * o.weight;
+                    longest_own = std::max(longest_own, g16 ? std::max(6.5 * o.own, 760.0 * o.steps) : 7.5 * o.own);
+                } else {
+                    const double st = o.stripe / step_cost(o.c2);     // steps of a stripe
+                    const double i = o.ns * st * 4.0 * (o.widen ? 60.0 + 14.0 * o.c2 : step_cost(o.c2));
+                    issue += i;
+                    issue_piped += i;
+                    longest_piped = std::max(longest_piped, std::max(std::ceil((double)o.ns / p) * st, (o.ns - 1) * o.lead + st) *
+                                                                (o.widen ? 630.0 : 6.0 * step_cost(o.c2)));
+                }
+            }
+            cycles[spread] = std::max({issue / (double)simds, longest_piped, issue_piped / (double)simds + longest_own});
+        }
+        spread = cycles[0] <= cycles[1] ? 0 : 1;
+        if (cycles[2] < 0.93 * cycles[spread]) spread = 2;
+        plan();
+    }
     for (uint64_t x = 0; x < n; ++x) {
         DpItem &it = items[x];
         const uint32_t p = parts_of(opt[x], up);

@@ -161,6 +161,33 @@ def test_narrow_banded_stripes_over_all_lanes(ctx, dp_env):
     assert got["1"] == got["auto"]
 
 
+@pytest.mark.parametrize("n,length,band,spread", [(8, 3000, 50, True), (4000, 300, 32, False), (60, 1000, 4, False)])
+def test_narrow_banded_jobs_spread_where_it_gains(ctx, dp_env, n, length, band, spread):
+    """Jobs of 16-lane stripes are spread over all lanes where SIMDs would be
+    idle, and left four a wavefront where the round has enough of them or their
+    bands are so narrow that a stripe waits for the one before it; either way
+    the paths, scores and deviations of one wavefront a job."""
+    rng = np.random.default_rng(n)
+    pairs = [_related(rng, length, length, 0.05) for _ in range(n)]
+    A, B, jobs = _batch(pairs)
+    bands = np.full(n, band, dtype=np.uint32)
+    os.environ.pop("MH_DP_COLS", None)
+    os.environ["MH_DP_BAND_KIND"] = "stripes"
+    got = {}
+    for P in ("1", "auto"):
+        if P == "auto":
+            os.environ.pop("MH_DP_PIPE", None)
+        else:
+            os.environ["MH_DP_PIPE"] = P
+        ctx.set_timing(True)
+        ctx.reset_kernel_times()
+        paths, res, dev, st = mauvehip.global_align_banded(ctx, A, B, jobs, bands, flags=mauvehip.BAND_NO_FALLBACK)
+        assert _pipe_parts(ctx) == (n if spread and P == "auto" else 0)
+        ctx.set_timing(False)
+        got[P] = [(mauvehip.path_of(paths, res, k), int(res[k]["score"]), int(dev[k])) for k in range(n)]
+    assert got["1"] == got["auto"]
+
+
 @pytest.mark.parametrize("budget_gb", ["0.002", "0.004", "0.02"])
 def test_rounds_of_spread_banded_jobs_stay_within_the_budget(ctx, dp_env, monkeypatch, budget_gb):
     """A job spread over wavefronts takes more memory (a boundary four times as
