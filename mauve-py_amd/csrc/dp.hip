@@ -1924,7 +1924,7 @@ static bool fixed_takes(const DpItem &it, const mh_dp_job *jobs, const FixedScra
 // A pipelined job's boundary takes four times the memory, and a byte a column
 // holds half a byte where a lane has one: spare is what the round's bytes may
 // still grow by (item_bytes), and the jobs that would pass it, the longest
-// first, keep one wavefront.
+// first, keep one wavefront.  Returns the bytes it grew by.
 //
 // Measured, with the parts' priorities (dp_job): 4,000 jobs of 10-20,000 columns
 // (at most 8 parts a job, all the round's wavefronts fitting the slots together,
@@ -1932,9 +1932,10 @@ static bool fixed_takes(const DpItem &it, const mh_dp_job *jobs, const FixedScra
 // ms.  Left: a part alone on its SIMD issues an instruction every six cycles
 // instead of four, and a banded job's stripes wait for each other (9 ms for 20,000
 // columns).
-static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_t other, uint64_t simds, int wpe,
-                       int p_env, uint64_t spare)
+static int64_t plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_t other, uint64_t simds, int wpe,
+                          int p_env, uint64_t spare)
 {
+    int64_t grown = 0;
     auto group = [](const DpItem &it) { return it.cols > GROUP_TAG; };
     auto cols_of = [&](const DpItem &it) { return group(it) ? it.cols - GROUP_TAG : it.cols; };
     double est = 0;     // wavefronts of the round as it stands
@@ -1954,14 +1955,14 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
             w.cols = cols_of(it) / 4;
             w.tb_bytes = dp_steps(jobs[it.job].a_len, jobs[it.job].b_len, it.band, w.cols, 64) * 64 * lane_bytes_of(w.cols);
         }
-        const uint64_t had = item_bytes(it, jobs), has = item_bytes(w, jobs);
-        if (has > had && has - had > spare) return false;
-        spare -= has - had;     // (back to spare where a shape takes less)
+        const int64_t more = (int64_t)item_bytes(w, jobs) - (int64_t)item_bytes(it, jobs);
+        if (more > 0 && grown + more > (int64_t)spare) return false;
+        grown += more;
         it = w;
         return true;
     };
     if (p_env > 1) {
-        if (est >= slots) return;
+        if (est >= slots) return 0;
         double used = est;
         for (uint64_t x = 0; x < n; ++x) {
             DpItem &it = items[x];
@@ -1969,7 +1970,7 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
             if (group(it) || ns < (uint64_t)p_env || used + p_env - 1 > slots) continue;
             if (give(it, (uint32_t)p_env)) used += p_env - 1;
         }
-        return;
+        return grown;
     }
     // instructions of a step: about 24 around the cells, 12.4 a cell
     auto step_cost = [](uint32_t cols) { return 24.0 + 12.4 * cols; };
@@ -2009,7 +2010,7 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
         longest = std::max(longest, o.own);
     }
     const double share = total / slots, T = 0.25 * share;
-    if (longest <= 1.1 * share) return;
+    if (longest <= 1.1 * share) return 0;
     int spread = 2;     // 0: no job, 1: those of 64 lanes, 2: all
     bool up = false;
     auto parts_of = [&](const Opt &o, bool up) -> uint32_t {
@@ -2057,6 +2058,7 @@ static void plan_parts(const mh_dp_job *jobs, DpItem *items, uint64_t n, uint64_
         const uint32_t p = parts_of(opt[x], up);
         if (p && (p > 1 || group(it))) give(it, p);
     }
+    return grown;
 }
 
 static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b, const mh_dp_job *jobs,
@@ -2130,11 +2132,6 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
     // round ends on its longest job (100,000 jobs of 10-20,000 columns 1.33 s, 1.07
     // with it)
     uint64_t room = budget;
-    if (!fx) {
-        uint64_t all = 0;
-        for (const DpItem &it : items) all += item_bytes(it, jobs);
-        if (all > budget) room -= budget / 32;
-    }
     for (uint64_t first = 0; first < nitems;) {
         // one round: as many jobs (in schedule order) as fit the trace budget
         uint64_t tbb = 0, bi = 0, last = first;
@@ -2147,6 +2144,10 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
             bi += b;
             ++last;
         }
+        if (last < nitems && room == budget && budget >= 32) {
+            room -= budget / 32;     // (and the first round again)
+            continue;
+        }
         const uint64_t n = last - first;
         // stripe jobs, then sliding-window jobs, then one-lane jobs, each in order
         std::stable_partition(items.begin() + (ptrdiff_t)first, items.begin() + (ptrdiff_t)last,
@@ -2157,18 +2158,12 @@ static int dp_run_items(mh_context *ctx, const uint8_t *d_a, const uint8_t *d_b,
                               [](const DpItem &it) { return it.cols < WINDOW_TAG; });
         uint64_t nstripe = 0;
         while (nstripe < nbig && items[first + nstripe].cols < WINDOW_TAG) ++nstripe;
-        if (!fx && ncu > 0) {
-            const uint64_t bytes = arena_bytes(tbb, bi);
-            plan_parts(jobs, items.data() + first, nstripe, (nbig - nstripe) + (n - nbig + 63) / 64,
-                       (uint64_t)ncu * 4, form == DpCells::TAGGED ? -1 : FWD_VARIANTS[VARIANT_FLOAT].wpe, pipe_env,
-                       bytes < budget ? budget - bytes : 0);
-        }
-        uint64_t tw = 0, bo = 0;
-        for (uint64_t x = first; x < last; ++x) {
-            tw += (items[x].tb_bytes + 15) & ~15ull;
-            bo += bnd_ints(items[x]);
-        }
-        arena = std::max(arena, arena_bytes(tw, bo));
+        uint64_t bytes = arena_bytes(tbb, bi);
+        if (!fx && ncu > 0)
+            bytes += plan_parts(jobs, items.data() + first, nstripe, (nbig - nstripe) + (n - nbig + 63) / 64,
+                                (uint64_t)ncu * 4, form == DpCells::TAGGED ? -1 : FWD_VARIANTS[VARIANT_FLOAT].wpe, pipe_env,
+                                bytes < budget ? budget - bytes : 0);
+        arena = std::max(arena, bytes);
         rounds.push_back({last, nbig, nstripe});
         first = last;
     }
