@@ -238,9 +238,12 @@ __device__ __forceinline__ uint32_t followed(uint32_t m, uint32_t S)
     return m & a;
 }
 
-// One end by a thread: its distance from the seed's window; false past
-// WALK_CHUNKS chunks.
-template <bool RIGHT, class W> __device__ __forceinline__ bool walk_end(const W &w, uint32_t *end)
+constexpr uint32_t WALK_FAR = 0xFFFFFFFFu;
+
+// One end by a thread: its distance from the seed's window, or one of at least
+// lim once it is known to reach that far; false past WALK_CHUNKS chunks.
+template <bool RIGHT, class W>
+__device__ __forceinline__ bool walk_end(const W &w, uint32_t *end, uint32_t lim = WALK_FAR)
 {
     const uint32_t room = RIGHT ? w.room_right() : w.room_left();
     uint32_t last = 0;
@@ -254,7 +257,7 @@ template <bool RIGHT, class W> __device__ __forceinline__ bool walk_end(const W 
             // the first that none follows within S: the chunk's last, or the end
             const uint32_t lone = m & ~followed(m, w.S);
             last = c + __builtin_ctz(lone);
-            if (lone & (lone - 1)) {
+            if ((lone & (lone - 1)) || last >= lim) {
                 *end = last;
                 return true;
             }
@@ -270,11 +273,14 @@ template <bool RIGHT, class W> __device__ __forceinline__ bool walk_end(const W 
 // The same by WALK_BLOCK threads, a chunk each; the last WALK_AHEAD only show
 // the others whether a match follows within a seed length (of at most 64).
 constexpr uint32_t WALK_AHEAD = 3;
-template <bool RIGHT, class W> __device__ __forceinline__ uint32_t walk_end_block(const W &w, uint32_t *lds)
+constexpr uint32_t WALK_STEP = 32 * (WALK_BLOCK - WALK_AHEAD);      // windows a step
+template <bool RIGHT, class W>
+__device__ __forceinline__ uint32_t walk_end_block(const W &w, uint32_t *lds, uint32_t lim = WALK_FAR)
 {
     const uint32_t room = RIGHT ? w.room_right() : w.room_left(), t = threadIdx.x;
     uint32_t *first = lds, *best = lds + WALK_BLOCK;
-    for (uint64_t c0 = 0; c0 <= room; c0 += 32 * (WALK_BLOCK - WALK_AHEAD)) {
+    for (uint64_t c0 = 0; c0 <= room; c0 += WALK_STEP) {
+        if (lim != WALK_FAR && c0 > lim) return lim;      // every match before it is followed
         const uint64_t c = c0 + 32 * t;
         const uint32_t m = c <= room ? w.template chunk<RIGHT>((uint32_t)c, room) : 0;
         __syncthreads();

@@ -408,30 +408,152 @@ __global__ __launch_bounds__(128) void walk_kernel(SRC src, uint64_t ns, const u
     }
 }
 
-template <class SRC>
+// LIMITED: once the blocks have taken max_steps steps together (work[0], counted
+// 64 at a time) they begin no more walks, and work[1] says that some were left.
+constexpr uint32_t WALK_COUNT = 64;
+
+template <class SRC, bool LIMITED>
 __global__ __launch_bounds__(WALK_BLOCK) void walk_long_kernel(SRC src, WalkEnv env, const uint32_t *__restrict__ rest,
-                                                               const uint32_t *__restrict__ cnt)
+                                                               const uint32_t *__restrict__ cnt,
+                                                               uint32_t *__restrict__ work, uint32_t max_steps)
 {
     __shared__ uint32_t lds[WALK_BLOCK + 1];
     const uint32_t n = *cnt;
+    uint32_t steps = 0;
     for (uint32_t h = blockIdx.x; h < n; h += gridDim.x) {
         const uint64_t x = rest[h];
         Walk<SRC::K, SRC::PAL> w;
         walk_setup(src, x, env, w);
         const uint32_t l = walk_end_block<false>(w, lds), r = walk_end_block<true>(w, lds);
         if (threadIdx.x == 0) src.store(x, w, l, l + r + w.S);
+        if constexpr (LIMITED) {
+            steps += l / WALK_STEP + r / WALK_STEP + 2;
+            if ((uint32_t)__builtin_amdgcn_readfirstlane((int)steps) < min(WALK_COUNT, max_steps)) continue;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                lds[0] = atomicAdd(work, steps) + steps > max_steps && h + gridDim.x < n;
+                if (lds[0]) work[1] = 1;
+            }
+            __syncthreads();
+            if (__builtin_amdgcn_readfirstlane((int)lds[0])) return;
+            steps = 0;
+        }
     }
 }
 
 template <class SRC>
 void launch_walks(mh_context *ctx, const SRC &src, uint64_t ns, const uint32_t *count, const WalkEnv &env,
-                  uint32_t *rest, uint32_t *cnt)
+                  uint32_t *rest, uint32_t *cnt, uint32_t max_steps)
 {
     if (!ns) return;
     const uint64_t blocks = (ns + 127) / 128;
     hipLaunchKernelGGL(walk_kernel<SRC>, dim3((unsigned)(count ? std::min<uint64_t>(blocks, 8192) : blocks)), dim3(128),
                        0, ctx->stream, src, ns, count, env, rest, cnt);
-    hipLaunchKernelGGL(walk_long_kernel<SRC>, dim3(512), dim3(WALK_BLOCK), 0, ctx->stream, src, env, rest, cnt);
+    auto kern = max_steps ? walk_long_kernel<SRC, true> : walk_long_kernel<SRC, false>;
+    hipLaunchKernelGGL(kern, dim3(512), dim3(WALK_BLOCK), 0, ctx->stream, src, env, rest, cnt, cnt + 1, max_steps);
+}
+
+// ---- long walks along shared diagonals ---------------------------------------
+// Heads on one diagonal with no seed length of windows without a match between
+// them extend to the same match, but each walk covers all of it: between close
+// relatives full of repeats (whose mers are no seeds, so that runs end) their
+// number times their length.  Where that gets much, the long walks' heads are
+// sorted by diagonal and position instead; each is walked to the left only until
+// it reaches the one before it, which it then belongs to, and the last of those
+// that belong together to the right.  A thread each up to a walk's
+// WALK_CHUNKS chunks, a block past that (todo, counted in cnt[0]).
+
+struct DiagSort {
+    const uint64_t *key;    // strand, diagonal, position (pb bits), sorted
+    const uint32_t *idx;    // of rest
+    uint64_t n;
+    int pb;
+
+    __device__ __forceinline__ uint32_t pos(uint64_t r) const { return (uint32_t)(key[r] & ((1ull << pb) - 1)); }
+    // the distance to the head before r on its diagonal
+    __device__ __forceinline__ uint32_t before(uint64_t r) const
+    {
+        return r && (key[r] >> pb) == (key[r - 1] >> pb) ? (uint32_t)(key[r] - key[r - 1]) : WALK_FAR;
+    }
+};
+
+template <class SRC>
+__global__ void diag_key_kernel(SRC src, WalkEnv env, const uint32_t *__restrict__ rest, uint64_t n, int pb, int db,
+                                uint64_t *__restrict__ key, uint32_t *__restrict__ val)
+{
+    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= n) return;
+    Walk<SRC::K, SRC::PAL> w;
+    walk_setup(src, rest[x], env, w);
+    const uint64_t diag = (uint64_t)w.p[1] + w.n[0] - w.p[0];
+    key[x] = ((uint64_t)(w.rev != 0) << (db + pb)) | (diag << pb) | w.p[0];
+    val[x] = (uint32_t)x;
+}
+
+// link[r]: the head before r, if r belongs to it, else r and its end; next[r]: the
+// head after it that belongs to it, else r and its end
+template <bool RIGHT>
+__device__ __forceinline__ void diag_put(const DiagSort &d, uint64_t r, uint32_t lim, uint32_t end,
+                                         uint32_t *__restrict__ link, uint32_t *__restrict__ ends)
+{
+    const bool joined = !RIGHT && end >= lim;
+    link[r] = (uint32_t)(joined ? r - 1 : r);
+    if (!joined) ends[r] = end;
+}
+
+template <bool RIGHT, class SRC>
+__global__ __launch_bounds__(128) void diag_walk_kernel(SRC src, WalkEnv env, const uint32_t *__restrict__ rest,
+                                                        DiagSort d, const uint32_t *__restrict__ left_link,
+                                                        uint32_t *__restrict__ link, uint32_t *__restrict__ ends,
+                                                        uint32_t *__restrict__ todo, uint32_t *__restrict__ cnt)
+{
+    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= d.n) return;
+    if (RIGHT && r + 1 < d.n && left_link[r + 1] == (uint32_t)r) {
+        link[r] = (uint32_t)r + 1;
+        return;
+    }
+    const uint32_t lim = RIGHT ? WALK_FAR : d.before(r);
+    Walk<SRC::K, SRC::PAL> w;
+    walk_setup(src, rest[d.idx[r]], env, w);
+    uint32_t end;
+    if (walk_end<RIGHT>(w, &end, lim)) diag_put<RIGHT>(d, r, lim, end, link, ends);
+    else todo[atomicAdd(cnt, 1u)] = (uint32_t)r;
+}
+
+template <bool RIGHT, class SRC>
+__global__ __launch_bounds__(WALK_BLOCK) void diag_walk_long_kernel(SRC src, WalkEnv env,
+                                                                    const uint32_t *__restrict__ rest, DiagSort d,
+                                                                    uint32_t *__restrict__ link,
+                                                                    uint32_t *__restrict__ ends,
+                                                                    const uint32_t *__restrict__ todo,
+                                                                    const uint32_t *__restrict__ cnt)
+{
+    __shared__ uint32_t lds[WALK_BLOCK + 1];
+    const uint32_t n = cnt[0];
+    for (uint32_t h = blockIdx.x; h < n; h += gridDim.x) {
+        const uint64_t r = todo[h];
+        const uint32_t lim = RIGHT ? WALK_FAR : d.before(r);
+        Walk<SRC::K, SRC::PAL> w;
+        walk_setup(src, rest[d.idx[r]], env, w);
+        const uint32_t end = walk_end_block<RIGHT>(w, lds, lim);
+        if (threadIdx.x == 0) diag_put<RIGHT>(d, r, lim, end, link, ends);
+    }
+}
+
+template <class SRC>
+__global__ void diag_store_kernel(SRC src, WalkEnv env, const uint32_t *__restrict__ rest, DiagSort d,
+                                  const uint32_t *__restrict__ first, const uint32_t *__restrict__ last,
+                                  const uint32_t *__restrict__ left, const uint32_t *__restrict__ right)
+{
+    const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= d.n) return;
+    const uint64_t x = rest[d.idx[r]];
+    Walk<SRC::K, SRC::PAL> w;
+    walk_setup(src, x, env, w);
+    const uint32_t a = first[r], z = last[r];
+    const uint32_t l = d.pos(r) - d.pos(a) + left[a], e = d.pos(z) - d.pos(r) + right[z];
+    src.store(x, w, l, l + e + w.S);
 }
 
 // ---- spaced and even seeds: one walk per run of seeds -------------------------
@@ -1068,10 +1190,62 @@ static bool walk_env(mh_context *ctx, const mh_sml *const *smls, int k, DevBuf *
 // 2,482, 3.2 million 2,604 and 3,092, 6.1 million 4,728 and 3,401.
 constexpr uint64_t SEEDS_FEW = 32;
 
+// Steps the blocks of a pair's long walks take before the walks go by diagonal
+// instead (MH_LONG_STEPS sets it): 0.9 ms of them, where 25,000 walks by diagonal
+// take 1.2.  Identical genomes of 4 million bases, twenty copies of one stretch
+// with a difference in 100 positions (25,000 walks of all of it): one by one 21.2 ms, 2.2
+// in this way; in 300, 8.9 and 1.9.
+constexpr uint32_t LONG_STEPS = 1u << 17;
+
+// The n walks of rest by diagonal (the diag_* kernels).
+template <class SRC>
+static int walk_by_diagonal(mh_context *ctx, const SRC &src, const WalkEnv &env, const uint32_t *rest, uint64_t n)
+{
+    DevBuf *g = ctx->grid_scratch;
+    int rc;
+    for (int q = 0; q < 2; ++q)
+        if ((rc = g[q].ensure(n * 8 + 64)) != MH_OK) return rc;
+    for (int q = 2; q < 6; ++q)
+        if ((rc = g[q].ensure(n * 8 + 64)) != MH_OK) return rc;
+    if ((rc = g[10].ensure(64)) != MH_OK) return rc;
+    int pb = 1, db = 1;
+    while ((1ull << pb) <= env.L[0]) ++pb;
+    while ((1ull << db) <= (uint64_t)env.L[0] + env.L[1]) ++db;
+    uint64_t *k0 = g[0].as<uint64_t>(), *k1 = g[1].as<uint64_t>();
+    uint32_t *v0 = g[2].as<uint32_t>(), *v1 = v0 + n;
+    uint32_t *link = g[3].as<uint32_t>(), *next = link + n, *ends_l = g[4].as<uint32_t>(), *ends_r = ends_l + n;
+    uint32_t *todo = g[5].as<uint32_t>(), *spare = todo + n, *cnt = g[10].as<uint32_t>();
+    const dim3 grid((unsigned)((n + 255) / 256)), blk(256), wg((unsigned)((n + 127) / 128));
+    MH_HIP(hipMemsetAsync(cnt, 0, 8, ctx->stream));
+    hipLaunchKernelGGL(diag_key_kernel<SRC>, grid, blk, 0, ctx->stream, src, env, rest, n, pb, db, k0, v0);
+    uint64_t *sk = nullptr;
+    uint32_t *sv = nullptr;
+    if ((rc = radix_sort_kv(ctx, k0, v0, k1, v1, n, 1 + db + pb, &sk, &sv)) != MH_OK) return rc;
+    const DiagSort d{sk, sv, n, pb};
+    hipLaunchKernelGGL((diag_walk_kernel<false, SRC>), wg, dim3(128), 0, ctx->stream, src, env, rest, d,
+                       (const uint32_t *)nullptr, link, ends_l, todo, cnt);
+    hipLaunchKernelGGL((diag_walk_long_kernel<false, SRC>), dim3(512), dim3(WALK_BLOCK), 0, ctx->stream, src, env, rest, d,
+                       link, ends_l, todo, cnt);
+    hipLaunchKernelGGL((diag_walk_kernel<true, SRC>), wg, dim3(128), 0, ctx->stream, src, env, rest, d, link, next, ends_r,
+                       todo, cnt + 1);
+    hipLaunchKernelGGL((diag_walk_long_kernel<true, SRC>), dim3(512), dim3(WALK_BLOCK), 0, ctx->stream, src, env, rest, d,
+                       next, ends_r, todo, cnt + 1);
+    // each list's ends by jumps of eight links
+    for (uint32_t **l : {&link, &next})
+        for (uint64_t reach = 1; reach < n; reach *= 8) {
+            hipLaunchKernelGGL(grid_jump_kernel, grid, blk, 0, ctx->stream, *l, spare, n);
+            std::swap(*l, spare);
+        }
+    hipLaunchKernelGGL(diag_store_kernel<SRC>, grid, blk, 0, ctx->stream, src, env, rest, d, link, next, ends_l, ends_r);
+    MH_HIP(hipGetLastError());
+    return MH_OK;
+}
+
 // Seeds of a pair, other than odd solid ones, in HashMatch order with their
-// extensions (the kernels above).  cnt[0, 2): cleared; heads, long walks.
+// extensions (the kernels above).  cnt[0, 4): cleared; walked: heads, long walks.
+template <bool PAL>
 static int extend_by_runs(mh_context *ctx, const mh_sml *a, const mh_sml *b, const uint32_t *oi, const uint32_t *oj,
-                          uint64_t ns, SeedRec *d_seeds, uint32_t *cnt)
+                          uint64_t ns, const WalkEnv &env, SeedRec *d_seeds, uint32_t *cnt, uint32_t walked[2])
 {
     const uint64_t L0 = a->len, S = (uint64_t)a->seed_length;
     DevBuf *rs = ctx->run_scratch;
@@ -1082,11 +1256,6 @@ static int extend_by_runs(mh_context *ctx, const mh_sml *a, const mh_sml *b, con
     uint2 *pp = rs[0].as<uint2>();
     uint32_t *la = (uint32_t *)(pp + L0), *lb = la + L0;
     uint32_t *heads = ctx->grid_scratch[7].as<uint32_t>(), *rest = ctx->grid_scratch[6].as<uint32_t>();
-    const mh_sml *smls[2] = {a, b};
-    DevBuf *bufs[2] = {nullptr, &ctx->mf_scratch[7]};
-    WalkEnv env;
-    const bool pal = walk_env(ctx, smls, 2, bufs, &env, &rc);
-    if (rc != MH_OK) return rc;
     RunPos rp{L0, nullptr, nullptr};
     if (ns < L0 / SEEDS_FEW) rp = {ns, oi, a->d_pos};
     const dim3 gs((unsigned)((ns + 255) / 256)), gp((unsigned)((rp.n + 255) / 256)), blk(256);
@@ -1101,14 +1270,23 @@ static int extend_by_runs(mh_context *ctx, const mh_sml *a, const mh_sml *b, con
         std::swap(la, lb);
     }
     hipLaunchKernelGGL(spaced_heads_kernel, gp, blk, 0, ctx->stream, rp, pp, la, heads, cnt);
-    if (pal)
-        launch_walks(ctx, PairWalks<true>{heads, oi, oj, a->d_keys, b->d_keys, a->d_pos, b->d_pos, d_seeds}, ns, cnt,
-                     env, rest, cnt + 1);
-    else
-        launch_walks(ctx, PairWalks<false>{heads, oi, oj, a->d_keys, b->d_keys, a->d_pos, b->d_pos, d_seeds}, ns, cnt,
-                     env, rest, cnt + 1);
+    const PairWalks<PAL> src{heads, oi, oj, a->d_keys, b->d_keys, a->d_pos, b->d_pos, d_seeds};
+    const char *le = getenv("MH_LONG_STEPS");
+    launch_walks(ctx, src, ns, cnt, env, rest, cnt + 1, le ? (uint32_t)std::max(1, atoi(le)) : LONG_STEPS);
     hipLaunchKernelGGL(spaced_fill_kernel, gp, blk, 0, ctx->stream, rp, pp, la, d_seeds);
     MH_HIP(hipGetLastError());
+    uint32_t h[4];
+    MH_HIP(hipMemcpyAsync(h, cnt, 16, hipMemcpyDeviceToHost, ctx->stream));
+    const double t0 = now_ms();
+    MH_HIP(hipStreamSynchronize(ctx->stream));
+    host_time(ctx, "host_wait_seeds", now_ms() - t0);
+    walked[0] = h[0];
+    walked[1] = h[1];
+    if (!h[3]) return MH_OK;
+    if ((rc = walk_by_diagonal(ctx, src, env, rest, h[1])) != MH_OK) return rc;
+    hipLaunchKernelGGL(spaced_fill_kernel, gp, blk, 0, ctx->stream, rp, pp, la, d_seeds);
+    MH_HIP(hipGetLastError());
+    MH_HIP(hipStreamSynchronize(ctx->stream));
     return MH_OK;
 }
 
@@ -1301,7 +1479,7 @@ int join_and_extend(mh_context *ctx, const mh_sml *a, const mh_sml *b, const Liv
     uint32_t *flag = ctx->mf_scratch[0].as<uint32_t>();
     uint32_t *partner = ctx->mf_scratch[1].as<uint32_t>();
     uint32_t *tiles = ctx->mf_scratch[2].as<uint32_t>();
-    uint32_t *cnt = ctx->mf_scratch[3].as<uint32_t>();   // [1] total seeds, [4], [5] walk_kernel's
+    uint32_t *cnt = ctx->mf_scratch[3].as<uint32_t>();   // [1] total seeds, [4, 8) extend_by_runs's
     // live ranges other than the whole list go to the device
     LivePair lp;
     std::memset(&lp, 0, sizeof(lp));
@@ -1378,6 +1556,7 @@ int join_and_extend(mh_context *ctx, const mh_sml *a, const mh_sml *b, const Liv
                            oi, oj);
     }
     const bool solid_odd = a->seed_length == a->seed_weight && (a->seed_length & 1);
+    uint32_t walked[2] = {(uint32_t)ns, 0};
     if (solid_odd) {
         if ((rc = ctx->mf_scratch[7].ensure(b->n_words * 4 + 64)) != MH_OK) return rc;
         uint32_t *wbrc = ctx->mf_scratch[7].as<uint32_t>();
@@ -1409,13 +1588,19 @@ int join_and_extend(mh_context *ctx, const mh_sml *a, const mh_sml *b, const Liv
         MH_HIP(hipGetLastError());
     } else {
         TimedLaunch tl(ctx, "extend");
-        if ((rc = extend_by_runs(ctx, a, b, oi, oj, ns, d_seeds, cnt + 4)) != MH_OK) return rc;
+        const mh_sml *smls[2] = {a, b};
+        DevBuf *bufs[2] = {nullptr, &ctx->mf_scratch[7]};
+        WalkEnv env;
+        const bool pal = walk_env(ctx, smls, 2, bufs, &env, &rc);
+        if (rc != MH_OK) return rc;
+        auto extend = pal ? extend_by_runs<true> : extend_by_runs<false>;
+        if ((rc = extend(ctx, a, b, oi, oj, ns, env, d_seeds, cnt + 4, walked)) != MH_OK) return rc;
     }
-    uint32_t walked[2] = {(uint32_t)ns, 0};
-    if (!solid_odd) MH_HIP(hipMemcpyAsync(walked, cnt + 4, 8, hipMemcpyDeviceToHost, ctx->stream));
-    const double t0 = now_ms();
-    MH_HIP(hipStreamSynchronize(ctx->stream));
-    host_time(ctx, "host_wait_seeds", now_ms() - t0);
+    if (solid_odd) {
+        const double t0 = now_ms();
+        MH_HIP(hipStreamSynchronize(ctx->stream));
+        host_time(ctx, "host_wait_seeds", now_ms() - t0);
+    }
     ctx->last_walks = walked[0];
     ctx->last_long_walks = walked[1];
     *seeds_out = d_seeds;
@@ -1750,9 +1935,9 @@ template <bool P>
 void uq_launch_walks(mh_context *ctx, const uint32_t *heads, uint64_t nh, const WalkEnv &env, int k,
                      const int32_t *d_sst, int32_t *d_est, uint32_t *d_len, uint32_t *rest, uint32_t *cnt)
 {
-    if (k <= 4) launch_walks(ctx, UqWalks<4, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt);
-    else if (k <= 8) launch_walks(ctx, UqWalks<8, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt);
-    else launch_walks(ctx, UqWalks<16, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt);
+    if (k <= 4) launch_walks(ctx, UqWalks<4, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt, 0);
+    else if (k <= 8) launch_walks(ctx, UqWalks<8, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt, 0);
+    else launch_walks(ctx, UqWalks<16, P>{heads, k, d_sst, d_est, d_len}, nh, nullptr, env, rest, cnt, 0);
 }
 
 // every other seed copies its head's extension

@@ -161,6 +161,37 @@ def test_match_few_seeds_in_long_genomes(ctx, seed, share):
     assert few == (share < 9000)
 
 
+@pytest.mark.parametrize("seed", [po.get_seed(15, 0), 0xFFFFFF, 0b1101011101110111011])
+@pytest.mark.parametrize("snp", [0.0, 0.001, 0.01])
+def test_match_long_walks_by_diagonal(ctx, monkeypatch, seed, snp):
+    """Close relatives of a hundred copies of one stretch: seeds only where the
+    copies differ, so many heads whose walks cover the same diagonals, on both
+    strands.  Past a number of chunks (one here) the long walks go by diagonal:
+    the oracle's list, and that of walks one by one."""
+    rng = np.random.default_rng(seed & 0xFFF)
+
+    def mutate(x, rate):
+        x = x.copy()
+        hit = rng.random(len(x)) < rate
+        x[hit] = synth.BASES[(np.searchsorted(synth.BASES, x[hit]) + rng.integers(1, 4, hit.sum())) % 4]
+        return x
+
+    unit = synth.BASES[rng.integers(0, 4, 2000)]
+    a = np.concatenate([mutate(unit, 0.01) for _ in range(100)])
+    b = mutate(a, snp)
+    b[90_000:150_000] = synth.revcomp(b[90_000:150_000])
+    b = np.concatenate([b[:40_000], synth.BASES[rng.integers(0, 4, 50)], b[40_000:]])
+    _compare(ctx, a.tobytes(), b.tobytes(), seed)
+    one = _compare.last_stats
+    monkeypatch.setenv("MH_LONG_STEPS", "1")
+    _compare(ctx, a.tobytes(), b.tobytes(), seed)
+    st = _compare.last_stats
+    assert st.long_walks == one.long_walks
+    # more than one a block, so that a block stops (a substitution ends a solid seed's walk)
+    if snp == 0.0 or seed != 0xFFFFFF:
+        assert st.long_walks > 512
+
+
 @pytest.mark.parametrize("ng,seed", [(2, po.get_seed(17, 3)), (2, po.get_seed(15, 0)), (2, 0xFFF),
                                      (3, po.get_seed(15, 3)), (4, po.get_seed(15, 0))])
 def test_match_bucket_keys_without_starts_and_lines(ctx, monkeypatch, ng, seed):
