@@ -135,7 +135,7 @@ typedef struct {
     int64_t repeat_runs;     /* SearchRange restarts after runs above
                                 MER_REPEAT_LIMIT (LM/MatchFinder.cpp:253-276)  */
     int64_t walks;           /* seeds extended by a walk of their own        */
-    int64_t long_walks;      /* of those, long walks a whole block finished  */
+    int64_t long_walks;      /* of those, walks too long for one thread      */
 } mh_match_stats;
 
 /* Replaces PairwiseMatchFinder/MemHash::FindMatches (LM/MemHash.cpp:109-127,

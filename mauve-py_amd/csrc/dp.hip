@@ -745,7 +745,7 @@ __device__ __forceinline__ uint32_t qk_per_item(uint32_t kind)
 // Cells outside the window are -infinity: the result is the exact DP over the
 // window region.  Per row: the previous row's M, D', I' shift left by
 // s = base(i) - base(i-1) columns (DPP wave_shl:1 per column step), M and D'
-// follow from the previous row (right-to-left register pass, as dp_job), and
+// follow from the previous row (a right-to-left register pass), and
 // I' -- a running maximum along the row since the gap extension is 0 -- is a
 // lane-local prefix maximum joined by a cross-lane exclusive prefix maximum
 // (DPP row_shr within 16-lane rows, readlane across rows).  Trace: C*4 bits
@@ -1435,7 +1435,9 @@ struct DpItem {
 // runs pick more 16-column stripes, whose wide kernel then slows the round's
 // other jobs.  These weights were chosen by timing whole banded runs (learned
 // and constant bands, edge fallback included) over 100k training gaps: the
-// fastest learned-band run of the sets tried.
+// fastest learned-band run of the sets tried, on cells of 348 instructions a
+// 16-column step.  They decide the regions, and so the results of bands without
+// the fallback, and were not measured again on the present cells.
 constexpr double COST_PER_CELL[3] = {1.34, 1.00, 1.30};   // 64-lane stripes of cols 4, 8, 16
 constexpr double COST_PER_CELL_G16[2] = {2.40, 1.50};      // 16-lane stripes of cols 4, 8
 
@@ -1928,7 +1930,7 @@ static bool fixed_takes(const DpItem &it, const mh_dp_job *jobs, const FixedScra
 //
 // Measured, with the parts' priorities (dp_job): 4,000 jobs of 10-20,000 columns
 // (at most 8 parts a job, all the round's wavefronts fitting the slots together,
-// before) 75.9 -> 46.4 ms, a learned band's run over 6,000 such jobs 55.8 -> 19.7
+// before) 75.9 -> 46.4 ms, a learned band's run over 6,000 such jobs 55.8 -> 20
 // ms.  Left: a part alone on its SIMD issues an instruction every six cycles
 // instead of four, and a banded job's stripes wait for each other (9 ms for 20,000
 // columns).

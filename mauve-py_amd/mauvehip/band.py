@@ -33,13 +33,14 @@ def est_cells(la, lb, w):
     return band_cells(la, lb, w).astype(np.float64)
 
 
-# Time model of a banded run on one MI355X (seconds), from measurements of the
-# DP kernels the committed model was calibrated on (they have become faster; the
-# constants stay, since they decide delta): each pass of the fallback costs its cells at the batch rate
-# (~950 GCUPS of region cells) or its largest job at the rate of one
-# wavefront (a job runs on one wavefront: ~1.7 GCUPS), whichever is longer;
-# then the trace-back, whose longest walk takes ~0.6 us per step; plus a
-# fixed cost for planning and synchronisation.
+# Time model of a banded run on one MI355X (seconds), as measured on the DP
+# kernels of the committed model's calibration: each pass of the fallback costs
+# its cells at the batch rate (~950 GCUPS of region cells) or its largest job at
+# the rate of one wavefront (~1.7 GCUPS), whichever is longer; then the
+# trace-back, whose longest walk takes ~0.6 us per step; plus a fixed cost for
+# planning and synchronisation.  The present kernels run at about 2 TCUPS and
+# spread a large job over wavefronts; the constants stay, since they decide the
+# delta that train() chooses.
 BATCH_CELLS_PER_S = 0.95e12
 WAVE_CELLS_PER_S = 1.7e9
 TRACE_STEP_SECONDS = 0.6e-6
