@@ -1917,8 +1917,8 @@ static bool fixed_takes(const DpItem &it, const mh_dp_job *jobs, const FixedScra
 // instruction in a part; of several on a SIMD 4.2 (4.6 with 16 lanes) an
 // instruction, 4 for each of 60 + 14 a column with one or two columns.  The
 // estimates fit 60 rounds (equal jobs of 300 to 4,000 columns, log-uniform ones
-// up to 1,000, 5,000 and 20,000) to a fifth; the plan that spreads all has to be
-// 7% ahead, since rounds at 6% lost by it.
+// up to 1,000, 5,000 and 20,000) to about a quarter; the plan that spreads all
+// has to be 7% ahead, since rounds at 6% lost by it.
 // Pipelined jobs start first.  items[0, n): the round's stripe jobs (every lane
 // shape), longest first; other: its remaining wavefronts.  MH_DP_PIPE = P (p_env)
 // instead gives P wavefronts to the first 64-lane jobs with at least P stripes,
